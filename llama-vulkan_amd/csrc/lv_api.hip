@@ -24,6 +24,7 @@
 #include "lv_gemm.h"
 #include "lv_gemv_wide.h"
 #include "lv_attn_batch.h"
+#include "lv_short.h"
 
 using namespace lv;
 
@@ -135,6 +136,7 @@ static void uncached_give(int device, void *ptr, size_t bytes, bool pooled)
 struct LayerWeights {
     lv_matrix wq, wk, wv, wo, w1, w2, w3;
     const float *attn_norm = nullptr, *ffn_norm = nullptr;
+    const uint8_t *short_qkv = nullptr, *short_wo = nullptr, *short_gate_up = nullptr, *short_down = nullptr;   // copies for short batches (lv_short.h)
     const uint16_t *gate_up16 = nullptr;   // pair copy of w3 and w1 (in place of their own prompt copies) where they can share one
 };
 
@@ -161,6 +163,10 @@ struct lv_model {
     BlockModel *block = nullptr;    // a block model (lv_block.h): then nothing above but ctx and hp's vocab, dim and layers is set
     int output_state = 0;           // the same for the prompt copy of the output matrix, which only steps that keep every row's logits need
     uint16_t *output_copy = nullptr;
+    bool short_ok = false;          // steps of a few tokens can take the kernels of lv_short.h
+    int short_state = 0;            // their copy of the matrices, as prompt_state
+    uint8_t *short_arena = nullptr;
+    const uint8_t *short_output = nullptr;
 };
 
 // Shape classes the persistent kernel is compiled for: LLaMA-7B and LLaMA-13B layer shapes, q4_0 and q8_0.
@@ -221,6 +227,7 @@ struct lv_session {
     uint16_t *pf_xh = nullptr, *pf_xl = nullptr;
     uint16_t *pf_fh = nullptr, *pf_fl = nullptr;   // the feed-forward's inner activations (their producer still reads pf_xh / pf_xl)
     float *pf_xs = nullptr;   // per token: the power of two the halves written by prefill_norm_kernel are scaled down by
+    uint8_t *short_ws = nullptr;   // workspace of short batches (ShortBuffers), allocated at first use
     // operand planes of the batched attention (one layer's worth, rewritten per layer): four of attn_plane_halfs() each
     uint16_t *pf_planes = nullptr;
     size_t pf_plane_halfs = 0;
@@ -1249,6 +1256,8 @@ static const lv_tensor_desc *find_desc(const lv_tensor_desc *t, uint32_t n, cons
 
 // Persistent-kernel form of the weights: a second copy laid out as per-wave tile streams (lv_mega.h).
 // Built when the model has a compiled shape class and all matrices have one type and one kind of scale plane.
+static bool short_usable(const lv_model *m);
+
 template <class S>
 static int build_mega_stream(lv_model *m)
 {
@@ -1445,6 +1454,7 @@ extern "C" int lv_model_upload(lv_ctx *c, const void *base, uint64_t base_size, 
         delete m;
         return rc;
     }
+    m->short_ok = short_usable(m);
     *out = m;
     return LV_OK;
 }
@@ -1477,6 +1487,7 @@ extern "C" int lv_model_destroy(lv_model *m)
     (void)hipSetDevice(m->ctx->device);
     block_model_destroy(m->block);
     (void)hipFree(m->prompt_arena);
+    (void)hipFree(m->short_arena);
     (void)hipFree(m->output_copy);
     (void)hipFree(m->mega_stream);
     (void)hipFree(m->mega_norms);
@@ -1524,7 +1535,7 @@ extern "C" int lv_session_destroy(lv_session *s)
     block_session_destroy(s->block);
     void *dev[] = {s->kv, s->trig, s->trig_abs, s->x, s->xn, s->q, s->k, s->v, s->vo, s->ff, s->logits, s->attn_part, s->attn_counters,
                    s->cfg, s->argmax_dev, s->trace_buf, s->trace_attn, s->pf_x, s->pf_xn, s->pf_q, s->pf_k, s->pf_v, s->pf_vo, s->pf_g1, s->pf_g2,
-                   s->pf_xh, s->pf_xl, s->pf_xs, s->pf_planes, s->pf_fh, s->pf_fl, s->logits_all};
+                   s->pf_xh, s->pf_xl, s->pf_xs, s->pf_planes, s->pf_fh, s->pf_fl, s->logits_all, s->short_ws};
     for (void *p : dev) (void)hipFree(p);
     for (int i = 0; i < 2; i++) {
         uncached_give(s->model->ctx->device, s->xchg[i], s->xchg_bytes, s->xchg_pooled[i]);
@@ -2155,6 +2166,278 @@ static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_he
     return LV_OK;
 }
 
+
+// ---- short batches (lv_short.h) --------------------------------------------------------------------------------
+// What the kernels need of a model: layer matrices of one quantised type and file version, rows a whole number of chunks of
+// four blocks (both D and F multiples of 128).  Other models' short steps go token by token below kPrefillMin tokens, through the
+// GEMM above.
+static bool short_usable(const lv_model *m)
+{
+    const lv_hparams &hp = m->hp;
+    const uint32_t qt = m->layers.empty() ? LV_F32 : m->layers[0].wq.ftype;
+    if ((qt != LV_Q4_0 && qt != LV_Q8_0) || hp.dim % 128 || hp.ff % 128 || hp.dim > 8192 || (hp.rot != 32 && hp.rot != 64 && hp.rot != 128)) return false;
+    for (const LayerWeights &lw : m->layers)
+        for (const lv_matrix *x : {&lw.wq, &lw.wk, &lw.wv, &lw.wo, &lw.w1, &lw.w2, &lw.w3}) {
+            const bool wide = x == &lw.w2, tall = x == &lw.w1 || x == &lw.w3;
+            if (x->ftype != qt || !x->view.scales_f32 != !m->layers[0].wq.view.scales_f32 || x->view.rows != (tall ? hp.ff : hp.dim) || x->view.cols != (wide ? hp.ff : hp.dim)) return false;
+        }
+    return true;
+}
+
+constexpr uint32_t kShortSplits = 16;      // parts the attention's positions are cut in at most
+
+struct ShortBuffers {
+    float *x, *q, *parts[kShortSlices], *xscale, *num, *den;
+    uint8_t *act, *ff;
+};
+static size_t short_layout(const lv_hparams &hp, uint8_t *base, ShortBuffers *b)
+{
+    const size_t D = hp.dim, row = D * 4 * kShortTokens;
+    size_t at = 0;
+    auto take = [&](size_t bytes) { uint8_t *p = base ? base + at : nullptr; at += (bytes + 255) / 256 * 256; return p; };
+    b->x = (float *)take(row);
+    b->q = (float *)take(row);
+    for (float *&p : b->parts) p = (float *)take(row);
+    b->xscale = (float *)take(kShortTokens * 4);
+    b->num = (float *)take(row * kShortSplits);
+    b->den = (float *)take((size_t)kShortTokens * hp.heads * kShortSplits * 4);
+    b->act = take(short_act_bytes(hp.dim, kShortTokens));
+    b->ff = take(short_act_bytes(hp.ff, kShortTokens));
+    return at;
+}
+
+template <int QT, int T, int RT>
+static void launch_short_kernel(hipStream_t st, const ShortArgs &a, uint32_t slices, bool sf32)
+{
+    if (sf32) short_gemm_kernel<QT, true, T, RT><<<dim3((a.tiles + RT - 1) / RT, slices), dim3(kShortWaves * 64), 0, st>>>(a);
+    else short_gemm_kernel<QT, false, T, RT><<<dim3((a.tiles + RT - 1) / RT, slices), dim3(kShortWaves * 64), 0, st>>>(a);
+}
+template <int QT, int T>
+static void launch_short_rows(hipStream_t st, const ShortArgs &a, uint32_t rt, uint32_t slices, bool sf32)
+{
+    if (rt == 2) launch_short_kernel<QT, T, 2>(st, a, slices, sf32);
+    if constexpr (short_fits(QT, T, 3))
+        if (rt == 3) launch_short_kernel<QT, T, 3>(st, a, slices, sf32);
+    if constexpr (short_fits(QT, T, 4))
+        if (rt == 4) launch_short_kernel<QT, T, 4>(st, a, slices, sf32);
+    if constexpr (short_fits(QT, T, 6))
+        if (rt == 6) launch_short_kernel<QT, T, 6>(st, a, slices, sf32);
+}
+
+// Row tiles per workgroup (RT) and K slices of a product.  A workgroup's step (eight waves, a chunk each) costs its row tiles plus the
+// activations, worth about 1.5 row tiles; up to 16 tokens and 3 row tiles two workgroups share a CU, else one.  What counts is how
+// many of them a CU works off one after the other; a slice more is written and read again.  Measured in us (7B, T token tiles):
+//   q4_0 gate and up, 1376 tiles: T 1 RT 2/3/4/6 22/18/21/20, T 2 32/29/32/25, T 4 49/43/47/41; q, k and v, 768: T 2 22/16/17/22
+//   q4_0 down, 256 tiles, RT 4 slices 1/2/3/4: T 1 28/16/13/11, T 4 53/29/24/20, RT 2: T 1 24/14/13/12, T 4 40/23/29/24
+static void short_plan(uint32_t tiles, uint32_t nb, uint32_t T, int qt, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
+{
+    const uint32_t chunks = nb / 4;
+    double best = 1e30;
+    for (uint32_t rt : {2u, 3u, 4u, 6u}) {
+        if (!short_fits(qt, T, rt)) continue;
+        const uint32_t shared = T <= 1 && rt <= 3 ? 2 : 1;
+        for (uint32_t s = 1; s <= (sliced ? (uint32_t)kShortSlices : 1u); s++) {
+            const uint32_t per = (chunks + s - 1) / s;
+            if ((chunks + per - 1) / per != s) continue;
+            const uint32_t steps = (per + kShortWaves - 1) / kShortWaves, held = ((tiles + rt - 1) / rt * s + 255) / 256;
+            const uint32_t rounds = (held + shared - 1) / shared, at_once = held < shared ? held : shared;
+            const double cost = rounds * steps * (at_once * rt + 1.5) + 0.25 * (T ? T : 1) * (s - 1);
+            if (cost < best) { best = cost; *best_rt = rt; *best_chunks = per; }
+        }
+    }
+}
+
+static int launch_short_gemm(hipStream_t st, ShortArgs a, uint32_t ftype, bool sf32, bool sliced, uint32_t *slices_out = nullptr)
+{
+    const uint32_t T = short_tiles(a.n);
+    const int qt = ftype == LV_Q4_0 ? 4 : 8;
+    uint32_t rt = 2;
+    if (!a.w) return fail(LV_ERR_STATE, "short batch: the matrix has no copy");
+    short_plan(a.tiles, a.nb, T, qt, sliced, &rt, &a.slice_chunks);
+    const uint32_t slices = (a.nb / 4 + a.slice_chunks - 1) / a.slice_chunks;
+    if (slices_out) *slices_out = slices;
+#define LV_SHORT(QT, TT) case QT * 8 + TT: launch_short_rows<QT, TT>(st, a, rt, slices, sf32); break;
+    switch (qt * 8 + T) {
+        LV_SHORT(4, 0) LV_SHORT(4, 1) LV_SHORT(4, 2) LV_SHORT(4, 3) LV_SHORT(4, 4)
+        LV_SHORT(8, 0) LV_SHORT(8, 1) LV_SHORT(8, 2) LV_SHORT(8, 3) LV_SHORT(8, 4)
+    default: return fail(LV_ERR_STATE, "short batch of %u tokens", a.n);
+    }
+#undef LV_SHORT
+    HIP_TRY(hipGetLastError());
+    return LV_OK;
+}
+
+// The short copy of the layer matrices (lv_short.h), made when a model evaluates its first short batch; false when the device has no
+// room for it, short batches then take the paths they would have without it.
+static int launch_short_pack(hipStream_t st, uint8_t *dst, const lv_matrix &w, const lv_matrix *pair)
+{
+    const uint32_t tiles = w.view.rows / (pair ? 8 : 16);
+    const dim3 grid((unsigned)(((uint64_t)tiles * (w.view.cols / 128) * 64 + 255) / 256));
+    const MatView &m2 = pair ? pair->view : w.view;
+    if (w.ftype == LV_Q4_0) pair ? short_pack_kernel<4, true><<<grid, dim3(256), 0, st>>>(dst, w.view, m2, tiles) : short_pack_kernel<4, false><<<grid, dim3(256), 0, st>>>(dst, w.view, m2, tiles);
+    else pair ? short_pack_kernel<8, true><<<grid, dim3(256), 0, st>>>(dst, w.view, m2, tiles) : short_pack_kernel<8, false><<<grid, dim3(256), 0, st>>>(dst, w.view, m2, tiles);
+    HIP_TRY(hipGetLastError());
+    return LV_OK;
+}
+static size_t short_copy_bytes(const lv_matrix &w, uint32_t rows, uint32_t cols) { return rows / 16 * short_tile_bytes(w.ftype == LV_Q4_0 ? 4 : 8, w.view.scales_f32 != nullptr, cols / 32); }
+
+static bool ensure_short_copy(lv_model *m)
+{
+    std::lock_guard<std::mutex> lock(m->prompt_mutex);
+    if (m->short_state) return m->short_state > 0;
+    m->short_state = -1;
+    const lv_hparams &hp = m->hp;
+    const lv_matrix &like = m->layers[0].wq;
+    const size_t dd = short_copy_bytes(like, hp.dim, hp.dim), fd = short_copy_bytes(like, 2 * hp.ff, hp.dim), df = short_copy_bytes(like, hp.dim, hp.ff);
+    // all rows' logits go through the same kernel where the output matrix has the layers' form
+    const bool out = m->output.ftype == like.ftype && !m->output.view.scales_f32 == !like.view.scales_f32 && m->output.view.rows % 16 == 0;
+    const size_t vd = out ? short_copy_bytes(like, m->output.view.rows, hp.dim) : 0;
+    if (hipMalloc(reinterpret_cast<void **>(&m->short_arena), hp.layers * (4 * dd + fd + df) + vd) != hipSuccess) {
+        (void)hipGetLastError();
+        m->short_arena = nullptr;
+        return false;
+    }
+    uint8_t *at = m->short_arena;
+    hipStream_t st = m->ctx->stream;
+    for (LayerWeights &lw : m->layers) {
+        lw.short_qkv = at;
+        for (const lv_matrix *x : {&lw.wq, &lw.wk, &lw.wv, &lw.wo}) {
+            if (x == &lw.wo) lw.short_wo = at;
+            if (launch_short_pack(st, at, *x, nullptr) != LV_OK) return false;
+            at += dd;
+        }
+        lw.short_gate_up = at;
+        if (launch_short_pack(st, at, lw.w3, &lw.w1) != LV_OK) return false;
+        at += fd;
+        lw.short_down = at;
+        if (launch_short_pack(st, at, lw.w2, nullptr) != LV_OK) return false;
+        at += df;
+    }
+    if (out) {
+        if (launch_short_pack(st, at, m->output, nullptr) != LV_OK) return false;
+        m->short_output = at;
+    }
+    if (hipStreamSynchronize(st) != hipSuccess) return false;
+    m->short_state = 1;
+    return true;
+}
+
+static int launch_short_norm(hipStream_t st, const ShortBuffers &b, const float *w, uint32_t n, uint32_t D, uint32_t pending, uint32_t ftype)
+{
+    ShortNormArgs a{};
+    a.x = b.x; a.nparts = pending; a.w = w; a.act = b.act; a.xscale = b.xscale; a.dim = D; a.tiles = short_tiles(n);
+    for (uint32_t i = 0; i < pending; i++) a.parts[i] = b.parts[i];
+    const dim3 threads((D / 8 + 63) / 64 * 64);
+    if (ftype == LV_Q4_0) short_norm_kernel<4><<<dim3(n), threads, 0, st>>>(a);
+    else short_norm_kernel<8><<<dim3(n), threads, 0, st>>>(a);
+    HIP_TRY(hipGetLastError());
+    return LV_OK;
+}
+
+static int launch_short_attention(hipStream_t st, const lv_session *s, const ShortBuffers &b, uint32_t layer, uint32_t pos, uint32_t n, uint32_t ftype)
+{
+    const lv_hparams &hp = s->model->hp;
+    const uint32_t tiles = (pos + n + kAttnBatchK - 1) / kAttnBatchK, want = hp.heads < 512 ? 512 / hp.heads : 1;
+    const uint32_t most = want < kShortSplits ? want : kShortSplits, per = (tiles + most - 1) / most, splits = (tiles + per - 1) / per;
+    ShortAttnArgs a{};
+    a.kcache = kv_ptr(s, layer, 0); a.vcache = kv_ptr(s, layer, 1); a.q = b.q; a.trig_abs = s->trig_abs;
+    a.pos0 = pos; a.n = n; a.heads = hp.heads; a.backlog = s->backlog; a.tiles_per_split = per; a.num = b.num; a.den = b.den;
+    if (splits == 1) { a.act = b.act; a.tiles = short_tiles(n); a.q8 = ftype == LV_Q8_0; }
+    const size_t lds = (size_t)512 * hp.rot;
+    switch (hp.rot) {
+#define LV_SHORT_ATTN(R)                                                                                                              \
+    case R:                                                                                                                           \
+        HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(short_attn_kernel<R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+        short_attn_kernel<R><<<dim3(hp.heads, splits), dim3(256), lds, st>>>(a);                                                      \
+        break;
+        LV_SHORT_ATTN(32)
+        LV_SHORT_ATTN(64)
+        LV_SHORT_ATTN(128)
+#undef LV_SHORT_ATTN
+    default: return fail(LV_ERR_ARG, "attention: head size %u (32, 64 and 128 are built)", hp.rot);
+    }
+    HIP_TRY(hipGetLastError());
+    if (splits == 1) return LV_OK;
+    ShortCombineArgs c{};
+    c.num = b.num; c.den = b.den; c.splits = splits; c.n = n; c.heads = hp.heads; c.rot = hp.rot; c.tiles = short_tiles(n); c.act = b.act;
+    const dim3 grid((hp.dim / 8 + 255) / 256, n);
+    if (ftype == LV_Q4_0) short_attn_combine_kernel<4><<<grid, dim3(256), 0, st>>>(c);
+    else short_attn_combine_kernel<8><<<grid, dim3(256), 0, st>>>(c);
+    HIP_TRY(hipGetLastError());
+    return LV_OK;
+}
+
+// rows idx0 .. idx0 + n - 1 of the step, n <= kShortTokens; pos: the cache row of row idx0
+static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, bool with_head, uint32_t row_base)
+{
+    const lv_model *m = s->model;
+    const lv_hparams &hp = m->hp;
+    const uint32_t D = hp.dim, F = hp.ff, ft = m->layers[0].wq.ftype;
+    const bool sf32 = m->layers[0].wq.view.scales_f32 != nullptr;
+    hipStream_t st = s->stream;
+    ShortBuffers b;
+    if (!s->short_ws) {
+        const hipError_t e = hipMalloc(reinterpret_cast<void **>(&s->short_ws), short_layout(hp, nullptr, &b));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            s->short_ws = nullptr;
+            return fail(e == hipErrorOutOfMemory ? LV_ERR_OOM : LV_ERR_HIP, "workspace of short batches: %s", hipGetErrorString(e));
+        }
+    }
+    short_layout(hp, s->short_ws, &b);
+    const uint32_t *tok_ptr = s->cfg + 1 + idx0;
+    if (m->tok_ftype == LV_F32) embed_f32_kernel<<<dim3((D + 255) / 256, n), dim3(256), 0, st>>>(b.x, m->tok_f32, tok_ptr, D);
+    else if (m->tok_ftype == LV_Q4_0) embed_quant_kernel<4><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, st>>>(b.x, m->tok_quant.view, tok_ptr);
+    else embed_quant_kernel<8><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, st>>>(b.x, m->tok_quant.view, tok_ptr);
+    HIP_TRY(hipGetLastError());
+
+    uint32_t pending = 0;       // K slices in b.parts that the next norm adds to the residual stream
+    for (uint32_t li = 0; li < hp.layers; li++) {
+        const LayerWeights &lw = m->layers[li];
+        LV_TRY(launch_short_norm(st, b, lw.attn_norm, n, D, pending, ft));
+        ShortArgs a{};
+        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = b.xscale;
+        a.mode = kShortQkv;
+        a.w = lw.short_qkv;
+        a.tiles_m = D / 16; a.tiles = 3 * a.tiles_m; a.out[0] = b.q; a.ldo = D;
+        a.cache[0] = kv_ptr(s, li, 0); a.cache[1] = kv_ptr(s, li, 1); a.pos_ptr = s->cfg; a.pos_add = idx0; a.backlog = s->backlog;
+        LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
+        LV_TRY(launch_short_attention(st, s, b, li, pos, n, ft));
+        ShortArgs o{};
+        o.x = b.act; o.n = n; o.nb = D / 32; o.mode = kShortStore; o.w = lw.short_wo; o.tiles_m = o.tiles = D / 16; o.ldo = D;
+        for (int i = 0; i < kShortSlices; i++) o.out[i] = b.parts[i];
+        LV_TRY(launch_short_gemm(st, o, ft, sf32, true, &pending));
+        LV_TRY(launch_short_norm(st, b, lw.ffn_norm, n, D, pending, ft));
+        ShortArgs f{};
+        f.x = b.act; f.n = n; f.nb = D / 32; f.xscale = b.xscale; f.mode = kShortSilu;
+        f.w = lw.short_gate_up; f.tiles_m = f.tiles = F / 8; f.ff = b.ff;
+        LV_TRY(launch_short_gemm(st, f, ft, sf32, false));
+        ShortArgs d = o;
+        d.x = b.ff; d.nb = F / 32; d.w = lw.short_down;
+        LV_TRY(launch_short_gemm(st, d, ft, sf32, true, &pending));
+    }
+    float *parts[kGemmMaxMats];
+    for (int i = 0; i < kShortSlices; i++) parts[i] = b.parts[i];
+    float *all = s->all_logits ? s->logits_all + (size_t)(row_base + idx0) * hp.vocab : nullptr;
+    const lv_matrix &ow = m->output;
+    if (all && m->short_output) {
+        LV_TRY(launch_short_norm(st, b, m->norm, n, D, pending, ft));
+        ShortArgs a{};
+        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = b.xscale; a.mode = kShortStore; a.w = m->short_output;
+        a.tiles_m = a.tiles = hp.vocab / 16; a.out[0] = all; a.ldo = hp.vocab;
+        LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
+    } else if (all || with_head) {
+        // only the last row's logits are ever read (llava_session.cpp:131-139), unless all are asked for
+        LV_TRY(launch_gemm_reduce(st, b.x, D, parts, pending, D, n, true));
+        const uint32_t first = all ? 0 : n - 1, rows = n - first;
+        normalize_kernel<<<dim3(rows), dim3(256), 0, st>>>(b.q, b.x + (size_t)first * D, m->norm, D);
+        HIP_TRY(hipGetLastError());
+        LV_TRY(launch_gemv(st, all ? all : s->logits, ow, nullptr, b.q, rows, kGemvStore));
+    }
+    if (all && with_head) HIP_TRY(hipMemcpyAsync(s->logits, all + (size_t)(n - 1) * hp.vocab, (size_t)hp.vocab * 4, hipMemcpyDeviceToDevice, st));
+    return LV_OK;
+}
+
 extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, uint32_t pos)
 {
     if (!s || !tokens) return fail(LV_ERR_ARG, "lv_step_begin: null argument");
@@ -2199,7 +2482,8 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     (void)lv_session_path(s, &path);
     // the persistent kernel also takes the short steps (a few prompt or add_text tokens) below the size at which the
     // batched path pays: one launch per token, each 1.7 x faster than the operator chain's token
-    bool persistent = n < kPrefillMin && path == LV_PATH_PERSISTENT && !s->trace;
+    const bool few = n >= 2 && n <= kShortTokens && s->model->short_ok && !s->trace && ensure_short_copy(s->model);
+    bool persistent = n < kPrefillMin && path == LV_PATH_PERSISTENT && !s->trace && !few;
     s->mega_step = false;
     if (persistent) {
         uint32_t done = 0;
@@ -2235,6 +2519,8 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     }
     if (persistent) {
         // launched above
+    } else if (few) {
+        LV_TRY(record_short(s, 0, n, pos, true, row_base));
     } else if (n == 1 && (path == LV_PATH_GRAPH || (path == LV_PATH_PERSISTENT && s->use_graph)) && !s->trace) {
         if (!s->graph_exec) {
             HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));

@@ -1,0 +1,701 @@
+// lv_short.h — short batches (2 .. 64 tokens: a command, the next message of a chat) of LLaMA models: products with the
+// quantised matrices as the operator path stores them, and attention split over cache positions.
+//
+// What bounds such a step is reading the weights once.  The GEMM of lv_gemm.h reads a copy of 2.1 bytes a weight and works on tiles
+// of 128 tokens; the persistent kernel reads all weights per token.  Here every weight is read once, in its 4.5 or 8.5 bits, and
+// unpacked to fp16 in registers on its way into the matrix cores.  Arithmetic as in lv_gemm.h: activations as two fp16 halves,
+// every product exact, a block's 32 products summed in fp32, then times the block's scale and added to the fp32 result.
+//
+// short_gemm_kernel.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
+// tokens; its waves deal the K range among themselves, four quant blocks at a time, and add up through LDS at the end.  A wave so
+// reads activations nobody else in the workgroup reads, straight into MFMA operand form, and reuses them for its RT tiles: no
+// LDS, no barrier, nothing but loads in flight in the main loop.
+//   weights ("short copy", made when a model evaluates its first short batch; as many bytes as the file has):
+//       [row tile of 16][chunk of 4 blocks][64 lanes][dwords of blocks 0 .. 3][16 rows][4 scales, fp16 or (version-1 files) fp32]
+//       A lane's codes of a block are the eight it feeds to one MFMA (v_mfma_f32_16x16x32_f16: lane l holds row l % 16, k group l / 16), so
+//       a load is 1 KB in a row and nothing crosses lanes.  Read from the operator path's planes instead, a load touches 16 rows,
+//       16 consecutive lanes 16 cache lines: the address path, not HBM, then sets the time (7B q4_0 gate and up for 8 tokens: 21.5 us that way, 15.8 so).
+//   order: the eight codes a lane feeds to an MFMA come in the order that unpacks cheapest (short_slot); the activations are
+//          written in that order.
+//   activations: [block][16-token tile][high, low half][group][token][8 halfs]: 1 KB per operand, a lane's 16 bytes at 16 l.
+// Rows of tokens past the batch are not written; a token only meets its own row of the result.
+//
+// Measured (us per launch, 7B layer, 8 tokens q4_0 / 45 tokens q8_0): q, k and v 11 / 28, attention output 4.5 / 10, gate and up
+// 16 / 47, down 9 / 22; about 3 of them launch and sum.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.07 ms (eight launches of the
+// persistent kernel before); 45 tokens behind 619, 8 layers of 7B q8_0: 2.77 -> 1.24 ms (128-token GEMM tiles before).
+#pragma once
+
+#include "lv_attn_batch.h"
+#include "lv_gemm.h"
+
+namespace lv {
+
+constexpr uint32_t kShortTokens = 64;
+constexpr int kShortWaves = 8;
+constexpr int kShortSlices = kGemmMaxMats;
+
+typedef _Float16 lv_h2 __attribute__((ext_vector_type(2)));
+typedef uint32_t lv_u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t lv_u2 __attribute__((ext_vector_type(2)));
+
+// tiles of 16 tokens; 0: up to 8 tokens, whose high and low halves share one operand
+__host__ __device__ constexpr uint32_t short_tiles(uint32_t n) { return n <= 8 ? 0 : (n + 15) / 16; }
+__host__ __device__ constexpr uint32_t short_block_bytes(uint32_t tiles) { return tiles ? tiles * 2048 : 1024; }
+// bytes of the activations of K columns
+__host__ __device__ constexpr size_t short_act_bytes(uint32_t K, uint32_t n) { return (size_t)(K / 32) * short_block_bytes(short_tiles(n)); }
+
+// Element k of a block (0 .. 31) -> slot 8 g + e of the operand, and back.  q8_0: bytes in order.  q4_0: group g holds bytes
+// 4g .. 4g + 3 of the block, whose low nibbles are elements 4g .. 4g + 3 and whose high ones are 16 higher; a masked dword leaves
+// nibbles 0 and 4 (then 1 and 5, 2 and 6, 3 and 7) in the two halves of a register.
+template <int QT>
+__host__ __device__ constexpr uint32_t short_slot(uint32_t k)
+{
+    if constexpr (QT == 8) return k;
+    const uint32_t g = (k & 15) >> 2, j = k & 3, hi = k >> 4;
+    return 8 * g + (j & 1) * 4 + hi * 2 + (j >> 1);
+}
+// the elements of group g, slots 0 .. 7, from two runs of four consecutive elements a (from 4g or 8g on) and b (16 or 4 further)
+template <int QT>
+__device__ __forceinline__ void short_order(float (&f)[8], const float4 &a, const float4 &b)
+{
+    if constexpr (QT == 8) {
+        f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
+    } else {
+        f[0] = a.x; f[1] = a.z; f[2] = b.x; f[3] = b.z; f[4] = a.y; f[5] = a.w; f[6] = b.y; f[7] = b.w;
+    }
+}
+template <int QT> __host__ __device__ constexpr uint32_t short_run_a(uint32_t g) { return QT == 8 ? 8 * g : 4 * g; }
+template <int QT> __host__ __device__ constexpr uint32_t short_run_b(uint32_t g) { return QT == 8 ? 8 * g + 4 : 16 + 4 * g; }
+
+// where the high halves of (block, token, group) lie, and how much further the low ones
+__device__ __forceinline__ size_t short_act_offset(uint32_t block, uint32_t token, uint32_t g, uint32_t tiles)
+{
+    return (size_t)block * short_block_bytes(tiles) + token / 16 * 2048 + (g * 16 + token % 16) * 16;
+}
+__host__ __device__ constexpr uint32_t short_act_low(uint32_t tiles) { return tiles ? 1024 : 128; }
+
+enum ShortMode { kShortStore = 0, kShortQkv = 1, kShortSilu = 2 };
+
+struct ShortArgs {
+    const uint8_t *x;          // activations
+    const uint8_t *w;          // short copy of the matrices: kShortQkv: q, k, v one behind the other; kShortSilu: W3 and W1 in pairs
+    uint32_t tiles_m, tiles;   // row tiles of a matrix, of the launch
+    uint32_t nb;               // blocks of a row, a multiple of 4
+    uint32_t slice_chunks;     // chunks of four blocks per K slice (blockIdx.y)
+    uint32_t n, mode;
+    float *out[kShortSlices];  // [n][ldo], one per slice; kShortQkv: out[0] = q
+    uint32_t ldo;
+    const float *xscale;       // null, or per token the power of two its halves have to be multiplied by
+    uint16_t *cache[2];        // kShortQkv: k and v rows
+    const uint32_t *pos_ptr;
+    uint32_t pos_add, backlog;
+    uint8_t *ff;               // kShortSilu: activations of the next product
+};
+
+// Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights or, where a block's
+// products take long enough to cover an L2 access, two blocks ahead.  More in flight per wave costs registers, hence waves per
+// CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us, q, k and v for 45 with q8_0 28 -> 96).
+template <int T, int RT> constexpr int short_ahead() { return T * RT >= 8 ? 2 : 4; }
+// can RT tiles of rows beside T tiles of tokens keep sums, queues and activations in 256 registers (a few values more is fine)
+__host__ __device__ constexpr bool short_fits(int qt, uint32_t t, uint32_t rt) { return qt == 4 || rt <= (t <= 1 ? 6u : t <= 3 ? 3u : 2u); }
+// row tiles whose sums are put together at a time: up to 64 KB of LDS, whole pairs
+template <int T, int RT> constexpr int short_round()
+{
+    constexpr int most = 8 / (T ? T : 1);
+    return RT <= most ? RT : most;
+}
+__device__ __forceinline__ lv_h8 short_unpack4(uint32_t w)
+{
+    // nibble q in the low bits of a half of pattern 0x6400 is 1024 + q; one place up, 1024 + 16 q: both to q - 8, exactly
+    const uint32_t v = w >> 8;
+    const lv_h2 p0 = __builtin_bit_cast(lv_h2, (w & 0x000f000fu) | 0x64006400u), p1 = __builtin_bit_cast(lv_h2, (w & 0x00f000f0u) | 0x64006400u);
+    const lv_h2 p2 = __builtin_bit_cast(lv_h2, (v & 0x000f000fu) | 0x64006400u), p3 = __builtin_bit_cast(lv_h2, (v & 0x00f000f0u) | 0x64006400u);
+    const lv_h2 c = {(_Float16)-1032.f, (_Float16)-1032.f}, s = {(_Float16)0.0625f, (_Float16)0.0625f}, d = {(_Float16)-72.f, (_Float16)-72.f};
+    union { lv_h2 h[4]; lv_h8 v8; } u;
+    u.h[0] = p0 + c;
+    u.h[1] = __builtin_elementwise_fma(p1, s, d);
+    u.h[2] = p2 + c;
+    u.h[3] = __builtin_elementwise_fma(p3, s, d);
+    return u.v8;
+}
+__device__ __forceinline__ lv_h8 short_unpack8(uint32_t lo, uint32_t hi)
+{
+    // byte b ^ 0x80 under 0x64 is 1024 + 128 + b
+    const uint32_t a = lo ^ 0x80808080u, b = hi ^ 0x80808080u;
+    const lv_h2 c = {(_Float16)-1152.f, (_Float16)-1152.f};
+    union { lv_h2 h[4]; lv_h8 v8; } u;
+    u.h[0] = __builtin_bit_cast(lv_h2, __builtin_amdgcn_perm(0x64646464u, a, 0x04010400u)) + c;
+    u.h[1] = __builtin_bit_cast(lv_h2, __builtin_amdgcn_perm(0x64646464u, a, 0x04030402u)) + c;
+    u.h[2] = __builtin_bit_cast(lv_h2, __builtin_amdgcn_perm(0x64646464u, b, 0x04010400u)) + c;
+    u.h[3] = __builtin_bit_cast(lv_h2, __builtin_amdgcn_perm(0x64646464u, b, 0x04030402u)) + c;
+    return u.v8;
+}
+__host__ __device__ constexpr uint32_t short_chunk_bytes(int qt, bool sf32) { return (qt == 4 ? 1024 : 2048) + (sf32 ? 256 : 128); }
+__host__ __device__ constexpr size_t short_tile_bytes(int qt, bool sf32, uint32_t nb) { return (size_t)(nb / 4) * short_chunk_bytes(qt, sf32); }
+
+// The short copy of a matrix, or (PAIR) of W3 and W1 together: tiles of eight rows of W3 and the same eight of W1, so that a workgroup
+// has both products of a row whatever its number of tiles.  One thread per (tile, chunk, lane); `tiles` row tiles, nb a multiple of 4.
+template <int QT, bool PAIR>
+__global__ __launch_bounds__(256) void short_pack_kernel(uint8_t *__restrict__ dst, MatView m, MatView m2, uint32_t tiles)
+{
+    const uint32_t nb = m.cols / 32, chunks = nb / 4;
+    const uint64_t unit = ((uint64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
+    const uint32_t lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, c = (uint32_t)(unit % chunks), tile = (uint32_t)(unit / chunks);
+    if (tile >= tiles) return;
+    const MatView &src = PAIR && r >= 8 ? m2 : m;
+    const uint64_t b0 = (uint64_t)(PAIR ? tile * 8 + (r & 7) : tile * 16 + r) * nb + c * 4;
+    const bool sf32 = src.scales_f32 != nullptr;
+    uint8_t *out = dst + (size_t)tile * short_tile_bytes(QT, sf32, nb) + (size_t)c * short_chunk_bytes(QT, sf32);
+    uint32_t w[QT];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const uint32_t *b = reinterpret_cast<const uint32_t *>(src.codes + (b0 + s) * (QT / 4));
+        if constexpr (QT == 4) w[s] = b[g];
+        else { w[2 * s] = b[2 * g]; w[2 * s + 1] = b[2 * g + 1]; }
+    }
+#pragma unroll
+    for (int i = 0; i < QT / 4; i++) *reinterpret_cast<uint4 *>(out + i * 1024 + lane * 16) = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+    if (g == 0) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            if (sf32) *reinterpret_cast<float *>(out + QT / 4 * 1024 + r * 16 + s * 4) = src.scales_f32[b0 + s];
+            else *reinterpret_cast<uint16_t *>(out + QT / 4 * 1024 + r * 8 + s * 2) = src.scales[b0 + s];
+        }
+    }
+}
+
+// T: tiles of 16 tokens, 0: up to 8 tokens; RT: tiles of 16 rows per workgroup; SF32: fp32 block scales
+template <int QT, bool SF32, int T, int RT>
+__global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs a)
+{
+    constexpr bool EIGHT = T == 0;                     // one operand holds the high halves of 8 tokens and their low halves
+    constexpr int NT = EIGHT ? 1 : T;
+    constexpr int XB = EIGHT ? 1024 : T * 2048;        // activation bytes of a block
+    constexpr int BB = QT == 4 ? 16 : 32;              // code bytes of a block
+    constexpr int CW = BB / 4;                         // a lane's dwords of a chunk
+    constexpr int CB = short_chunk_bytes(QT, SF32);
+    constexpr int XD = short_ahead<T, RT>();
+    constexpr int PR = short_round<T, RT>();           // row tiles summed at a time
+    __shared__ __attribute__((aligned(16))) float red[PR * NT * kShortWaves * 256];
+    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tile0 = blockIdx.x * RT;
+    const uint32_t c0 = blockIdx.y * a.slice_chunks, chunks = min(a.slice_chunks, a.nb / 4 - c0);
+    const uint32_t steps = chunks > (uint32_t)wave ? (chunks - wave + kShortWaves - 1) / kShortWaves : 0;
+    const uint32_t nb = a.nb;
+
+    // uniform bases of the row tiles (past the last one: the last one again, not stored)
+    const uint8_t *wb[RT];
+#pragma unroll
+    for (int t = 0; t < RT; t++) wb[t] = a.w + (size_t)min(tile0 + t, a.tiles - 1) * short_tile_bytes(QT, SF32, nb) + (size_t)(c0 + wave) * CB;
+    const uint8_t *xb = a.x + (size_t)(c0 + wave) * 4 * XB;
+
+    // Loads of chunk j.  They return in the order they were issued, so activations (L2) are requested as far ahead as weights (HBM).
+    // Past this wave's last chunk: one address for all lanes, which costs next to nothing and keeps the queue free of branches.
+    uint32_t cq[RT][CW];
+    std::conditional_t<SF32, lv_u4, lv_u2> sq[RT];
+    lv_u4 xq[XD][EIGHT ? 1 : 2 * NT];
+    auto fetch_w = [&](uint32_t j) {
+        const uint32_t at = j < steps ? j * (kShortWaves * CB) : 0, lw = j < steps ? lane * 16 : 0, ls = j < steps ? r16 * (SF32 ? 16 : 8) : 0;
+#pragma unroll
+        for (int t = 0; t < RT; t++) {
+#pragma unroll
+            for (int i = 0; i < CW / 4; i++) {
+                const lv_u4 v = *reinterpret_cast<const lv_u4 *>(wb[t] + (lw + at + i * 1024));
+                cq[t][4 * i] = v.x; cq[t][4 * i + 1] = v.y; cq[t][4 * i + 2] = v.z; cq[t][4 * i + 3] = v.w;
+            }
+            sq[t] = *reinterpret_cast<const decltype(sq[0] + sq[0]) *>(wb[t] + (ls + at + CW / 4 * 1024));
+        }
+    };
+    auto fetch_x = [&](int slot, uint32_t j, int s) {  // block s of chunk j
+        const uint8_t *p = xb + (j < steps ? ((size_t)j * (kShortWaves * 4) + s) * XB : 0);
+        const uint32_t l = j < steps ? lane * 16 : 0;
+#pragma unroll
+        for (int t = 0; t < (EIGHT ? 1 : 2 * NT); t++) xq[slot][t] = *reinterpret_cast<const lv_u4 *>(p + l + t * 1024);
+    };
+    lv_f4v acc[RT][NT];
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[i][t] = lv_f4v{0.f, 0.f, 0.f, 0.f};
+    const lv_f4v zero = {0.f, 0.f, 0.f, 0.f};
+
+    if (steps) {
+        fetch_w(0);
+#pragma unroll
+        for (int s = 0; s < XD; s++) fetch_x(s, 0, s);
+        for (uint32_t j = 0; j < steps; j++) {
+            uint32_t w[RT][CW];                        // dword s (q8_0: 2 s and 2 s + 1): this lane's codes of block s
+            float sc[RT][4];
+#pragma unroll
+            for (int t = 0; t < RT; t++) {
+#pragma unroll
+                for (int i = 0; i < CW; i++) w[t][i] = cq[t][i];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if constexpr (SF32) sc[t][i] = __uint_as_float(sq[t][i]);
+                    else sc[t][i] = half_bits_to_float((uint16_t)(sq[t][i / 2] >> (16 * (i & 1))));
+                }
+            }
+            fetch_w(j + 1);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                lv_h8 ax[EIGHT ? 1 : 2 * NT];          // high, low halves tile by tile
+#pragma unroll
+                for (int t = 0; t < (EIGHT ? 1 : 2 * NT); t++) ax[t] = __builtin_bit_cast(lv_h8, xq[s % XD][t]);
+#pragma unroll
+                for (int i = 0; i < RT; i++) {
+                    const lv_h8 b = QT == 4 ? short_unpack4(w[i][s]) : short_unpack8(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
+                    lv_f4v p[NT];
+                    if constexpr (EIGHT) {
+                        p[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax[0], b, zero, 0, 0, 0);
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax[2 * t + 1], b, zero, 0, 0, 0);
+#pragma unroll
+                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax[2 * t], b, p[t], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[i][t][e] = fmaf(p[t][e], sc[i][s], acc[i][t][e]);
+                }
+                fetch_x(s % XD, j + (s + XD) / 4, (s + XD) % 4);
+            }
+        }
+    }
+
+    // ---- the waves' sums, PR row tiles at a time, through LDS: [row tile][token tile][wave][lane] float4 -------------------------
+    // acc[i][t][e]: row r16 of row tile i, token 16 t + 4 g + e (EIGHT: the high half's product of token 4 g + e for g < 2, behind
+    // them the low half's).  A wave adds up every eighth (row tile, token tile).
+    const uint32_t row_at = (a.mode == kShortQkv && a.pos_ptr ? *a.pos_ptr : 0u) + a.pos_add;
+    float *const out = a.out[blockIdx.y];
+    auto total = [&](int u, int from, float (&v)[4], const float4 &xs) {      // lane `from`'s sums of unit u
+        const lv_f4v *src = reinterpret_cast<const lv_f4v *>(red) + (size_t)u * kShortWaves * 64 + from;
+        lv_f4v s = src[0];
+#pragma unroll
+        for (int w = 1; w < kShortWaves; w++) s += src[w * 64];
+        if constexpr (EIGHT) {
+            const lv_f4v *low = src + (from < 32 ? 32 : 0);
+#pragma unroll
+            for (int w = 0; w < kShortWaves; w++) s += low[w * 64];
+        }
+        v[0] = s[0] * xs.x; v[1] = s[1] * xs.y; v[2] = s[2] * xs.z; v[3] = s[3] * xs.w;
+    };
+#pragma unroll
+    for (int i0 = 0; i0 < RT; i0 += PR) {
+        if (i0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PR; i++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                if (i0 + i < RT) *reinterpret_cast<lv_f4v *>(red + (((i * NT + t) * kShortWaves + wave) * 64 + lane) * 4) = acc[i0 + i][t];
+        __syncthreads();
+        for (int u = wave; u < (RT - i0 < PR ? RT - i0 : PR) * NT; u += kShortWaves) {
+            const uint32_t tile = tile0 + i0 + u / NT, tok0 = 16 * (u % NT) + 4 * g;
+            if (tile >= a.tiles || (EIGHT && lane >= 32)) continue;
+            float4 xs = make_float4(1.f, 1.f, 1.f, 1.f);
+            if (a.xscale) xs = *reinterpret_cast<const float4 *>(a.xscale + tok0);
+            float v[4];
+            total(u, lane, v, xs);
+            if (a.mode == kShortSilu) {                // rows 0 .. 7 of the tile are W3's, 8 .. 15 the same ones of W1
+                if (r16 >= 8) continue;
+                float w[4];
+                total(u, lane + 8, w, xs);
+                const uint32_t f = tile * 8 + r16, slot = short_slot<QT>(f & 31);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (tok0 + e >= a.n) continue;
+                    const float y = v[e] * w[e] / (__expf(-w[e]) + 1.f);
+                    const uint16_t h = float_to_half_bits(y), l = float_to_half_bits(y - half_bits_to_float(h));
+                    uint8_t *dst = a.ff + short_act_offset(f / 32, tok0 + e, slot >> 3, T) + (slot & 7) * 2;
+                    *reinterpret_cast<uint16_t *>(dst) = h;
+                    *reinterpret_cast<uint16_t *>(dst + short_act_low(T)) = l;
+                }
+                continue;
+            }
+            const uint32_t z = tile / a.tiles_m, m = tile % a.tiles_m * 16 + r16;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t tok = tok0 + e;
+                if (tok >= a.n) continue;
+                if (z == 0) out[(size_t)tok * a.ldo + m] = v[e];
+                else if (row_at + tok < a.backlog) a.cache[z - 1][(size_t)(row_at + tok) * a.ldo + m] = float_to_half_bits(v[e]);
+            }
+        }
+    }
+}
+
+// x += the K slices of the product before, then normalize(x) * w (normalize.comp:34-64) as the next product's activations, scaled
+// per token as in gemm_row_scale.  One workgroup per token, a thread per 8 elements (dim / 8 threads rounded up to whole waves;
+// dim <= 8192, a multiple of 32): nothing but latency counts here, and a thread's loads are few and all in flight at once.
+struct ShortNormArgs {
+    float *x;
+    const float *parts[kShortSlices];
+    uint32_t nparts;
+    const float *w;
+    uint8_t *act;
+    float *xscale;
+    uint32_t dim, tiles;
+};
+template <int QT>
+__global__ __launch_bounds__(1024) void short_norm_kernel(ShortNormArgs a)
+{
+    __shared__ float lds[48];
+    const uint32_t row = blockIdx.x, i = threadIdx.x;
+    const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const bool ok = i < a.dim / 8;
+    const size_t ro = (size_t)row * a.dim;
+    const uint32_t ic = ok ? i : 0, k[2] = {(ic >> 2) * 32 + short_run_a<QT>(ic & 3), (ic >> 2) * 32 + short_run_b<QT>(ic & 3)};
+    float4 x[2], w[2], p[kShortSlices][2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        w[h] = *reinterpret_cast<const float4 *>(a.w + k[h]);
+        x[h] = *reinterpret_cast<const float4 *>(a.x + ro + k[h]);
+#pragma unroll
+        for (int q = 0; q < kShortSlices; q++)
+            if (q < (int)a.nparts) p[q][h] = *reinterpret_cast<const float4 *>(a.parts[q] + ro + k[h]);
+    }
+    // the largest element of x w goes along with the sum: its exponent decides the row's scale, and 1 / rms multiplies every
+    // element alike
+    float s = 0.f, big = 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (a.nparts) {
+            float4 t = p[0][h];
+#pragma unroll
+            for (int q = 1; q < kShortSlices; q++)
+                if (q < (int)a.nparts) { t.x += p[q][h].x; t.y += p[q][h].y; t.z += p[q][h].z; t.w += p[q][h].w; }
+            x[h].x = t.x + x[h].x; x[h].y = t.y + x[h].y; x[h].z = t.z + x[h].z; x[h].w = t.w + x[h].w;
+            if (ok) *reinterpret_cast<float4 *>(a.x + ro + k[h]) = x[h];
+        }
+        if (!ok) x[h] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s += (x[h].x + x[h].y) + (x[h].z + x[h].w);
+        big = fmaxf(big, fmaxf(fmaxf(fabsf(x[h].x * w[h].x), fabsf(x[h].y * w[h].y)), fmaxf(fabsf(x[h].z * w[h].z), fabsf(x[h].w * w[h].w))));
+    }
+    s = wave_sum(s);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) big = fmaxf(big, __shfl_xor(big, off, 64));
+    if ((threadIdx.x & 63) == 0) { lds[wave] = s; lds[16 + wave] = big; }
+    __syncthreads();
+    s = 0.f;
+    for (int v = 0; v < waves; v++) { s += lds[v]; big = fmaxf(big, lds[16 + v]); }
+    const float mean = s / (float)a.dim;
+    float q = 0.f;
+    if (ok) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float c0 = x[h].x - mean, c1 = x[h].y - mean, c2 = x[h].z - mean, c3 = x[h].w - mean;
+            q = fmaf(c0, c0, q); q = fmaf(c1, c1, q); q = fmaf(c2, c2, q); q = fmaf(c3, c3, q);
+        }
+    }
+    q = wave_sum(q);
+    if ((threadIdx.x & 63) == 0) lds[32 + wave] = q;
+    __syncthreads();
+    q = 0.f;
+    for (int v = 0; v < waves; v++) q += lds[32 + v];
+    const float inv = rsqrtf(q / (float)a.dim);
+    float down;
+    const float up = gemm_row_scale(big * inv, &down);
+    if (threadIdx.x == 0) a.xscale[row] = down;
+    if (!ok) return;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        x[h].x = (x[h].x * w[h].x) * inv; x[h].y = (x[h].y * w[h].y) * inv; x[h].z = (x[h].z * w[h].z) * inv; x[h].w = (x[h].w * w[h].w) * inv;
+    }
+    float f[8];
+    short_order<QT>(f, x[0], x[1]);
+#pragma unroll
+    for (int e = 0; e < 8; e++) f[e] *= up;
+    uint4 h, l;
+    gemm_split8(h, l, f);
+    uint8_t *dst = a.act + short_act_offset(i >> 2, row, i & 3, a.tiles);
+    *reinterpret_cast<uint4 *>(dst) = h;
+    *reinterpret_cast<uint4 *>(dst + short_act_low(a.tiles)) = l;
+}
+
+// Attention of a short batch: attention_batch_kernel's arithmetic, with the cache positions shared out over workgroups and the
+// operand planes made on the way into LDS (a plane would be used once).  Without a running maximum the parts of a row are plain
+// sums: numerators [split][n][H*R] and denominators [split][n][H], put together by short_attn_combine_kernel.  64 KB of LDS: two
+// workgroups a CU.
+struct ShortAttnArgs {
+    const uint16_t *kcache, *vcache;   // [backlog][H*R] fp16, the batch's rows already in them
+    const float *q;                    // [n][H*R]
+    const float2 *trig_abs;            // [backlog][R/2]
+    uint32_t pos0, n, heads, backlog;  // row z sits at pos0 + z
+    uint32_t tiles_per_split;          // tiles of 64 positions
+    float *num, *den;
+    uint8_t *act;                      // with one split: the output projection's activations, `tiles` token tiles, in place of num and den
+    uint32_t tiles, q8;
+};
+// grid (heads, splits)
+template <int R>
+__global__ __launch_bounds__(256, 2) void short_attn_kernel(ShortAttnArgs a)
+{
+    constexpr int TK = kAttnBatchK;
+    constexpr int KS = R / 16, DT = R / 32, C8 = R / 8;
+    constexpr int PLANE = TK * R * 2;
+    constexpr int XS = R + 4;
+    static_assert(64 * XS * 4 <= 4 * PLANE, "the result exchange reuses the tile buffers");
+    extern __shared__ __attribute__((aligned(16))) uint8_t short_lds[];      // kh, kl, v1, v2: 512 R bytes
+    __shared__ float den_s[2][32];
+    const uint32_t h = blockIdx.x, H = a.heads, D = H * R;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int qt = wave & 1, pt = wave >> 1, n32 = lane & 31, hh = lane >> 5;
+    const uint32_t rows = min(a.pos0 + a.n, a.backlog);               // positions that hold data
+    const uint32_t tile_end = min((blockIdx.y + 1) * a.tiles_per_split, (rows + TK - 1) / TK);
+
+    // A tile's rows, requested a tile ahead.  K: thread t takes the 16-byte chunk t % C8 of rows t / C8, + 256 / C8, ...  V: two
+    // dims (4 bytes) of eight positions, whose slots are a 16-byte chunk of either dim's row in the transposed planes.
+    constexpr int PT = C8 * TK / 256, VT = R / 2 * 8 < 256 ? 1 : R / 2 * 8 / 256;     // R 32: half of the threads
+    uint4 kq[PT];
+    uint32_t vq[VT][8];
+    auto vpos = [](int c8, int e) { return ((8 * c8 + e) & ~15) + attn_slot_pos((8 * c8 + e) & 15); };
+    auto fetch = [&](uint32_t it) {
+#pragma unroll
+        for (int i = 0; i < PT; i++) {
+            const uint32_t c = t + i * 256, p = min(it * TK + c / C8, rows - 1);
+            kq[i] = *reinterpret_cast<const uint4 *>(a.kcache + (size_t)p * D + (size_t)h * R + c % C8 * 8);
+        }
+#pragma unroll
+        for (int i = 0; i < VT; i++) {
+            const uint32_t u = t + i * 256, dp = u % (R / 2), c8 = min(u / (R / 2), 7u);
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                vq[i][e] = *reinterpret_cast<const uint32_t *>(a.vcache + (size_t)min(it * TK + vpos(c8, e), rows - 1) * D + (size_t)h * R + dp * 2);
+        }
+    };
+    fetch(blockIdx.y * a.tiles_per_split);
+
+    lv_h8 qh[KS], ql[KS];
+    const uint32_t zq = 32 * qt + n32;
+    const bool zok = zq < a.n;
+    {
+        const uint32_t pq = min(a.pos0 + zq, a.backlog - 1);
+        const float *qr = a.q + (size_t)(zok ? zq : 0) * D + (size_t)h * R;
+        const float2 *tr = a.trig_abs + (size_t)pq * (R / 2);
+#pragma unroll
+        for (int j = 0; j < KS; j++) {
+            const float4 q0 = *reinterpret_cast<const float4 *>(qr + 16 * j + 8 * hh), q1 = *reinterpret_cast<const float4 *>(qr + 16 * j + 8 * hh + 4);
+            const float4 c0 = *reinterpret_cast<const float4 *>(tr + 8 * j + 4 * hh), c1 = *reinterpret_cast<const float4 *>(tr + 8 * j + 4 * hh + 2);
+            float f[8] = {q0.x * c0.x - q0.y * c0.y, q0.x * c0.y + q0.y * c0.x, q0.z * c0.z - q0.w * c0.w, q0.z * c0.w + q0.w * c0.z,
+                          q1.x * c1.x - q1.y * c1.y, q1.x * c1.y + q1.y * c1.x, q1.z * c1.z - q1.w * c1.w, q1.z * c1.w + q1.w * c1.z};
+            if (!zok) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) f[e] = 0.f;
+            }
+            uint4 hi, lo;
+            gemm_split8(hi, lo, f);
+            qh[j] = __builtin_bit_cast(lv_h8, hi);
+            ql[j] = __builtin_bit_cast(lv_h8, lo);
+        }
+    }
+    const float scale = rsqrtf((float)R);
+    lv_f16v acc[DT];
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[d][r] = 0.f;
+    float den = 0.f;
+    const uint32_t limit = a.pos0 + zq;
+    const bool tile_live = 32 * qt < (int)a.n;                        // this wave's 32 queries hold one of the batch
+    const uint32_t wave_last = a.pos0 + min(32u * qt + 31, a.n - 1);
+
+    for (uint32_t it = blockIdx.y * a.tiles_per_split; it < tile_end; it++) {
+        const uint32_t k0 = it * TK;
+        __syncthreads();                                              // the tile before is consumed
+#pragma unroll
+        for (int i = 0; i < PT; i++) {
+            const int c = t + i * 256, c8 = c % C8, row = c / C8;
+            const uint32_t p = k0 + row;
+            float f[8];
+            const bool live = p < rows;                               // rows past the data: zeros, which the masked sums can take
+            const float4 cs0 = *reinterpret_cast<const float4 *>(a.trig_abs + (size_t)min(p, rows - 1) * (R / 2) + c8 * 4);
+            const float4 cs1 = *reinterpret_cast<const float4 *>(a.trig_abs + (size_t)min(p, rows - 1) * (R / 2) + c8 * 4 + 2);
+            const uint32_t kw[4] = {kq[i].x, kq[i].y, kq[i].z, kq[i].w};
+            const float cc[4] = {cs0.x, cs0.z, cs1.x, cs1.z}, ss[4] = {cs0.y, cs0.w, cs1.y, cs1.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float x = half_bits_to_float((uint16_t)(kw[j] & 0xffffu)), y = half_bits_to_float((uint16_t)(kw[j] >> 16));
+                f[2 * j] = live ? x * cc[j] - y * ss[j] : 0.f;
+                f[2 * j + 1] = live ? x * ss[j] + y * cc[j] : 0.f;
+            }
+            uint4 hi, lo;
+            gemm_split8(hi, lo, f);
+            uint8_t *kd = short_lds + row * 2 * R + (c8 ^ attn_kswz<R>(row)) * 16;
+            *reinterpret_cast<uint4 *>(kd) = hi;
+            *reinterpret_cast<uint4 *>(kd + PLANE) = lo;
+        }
+#pragma unroll
+        for (int i = 0; i < VT; i++) {
+            const int u = t + i * 256, dp = u % (R / 2), c8 = u / (R / 2);
+            if (R < 64 && c8 >= 8) break;
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                uint32_t w1[4], w2[4];
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    uint32_t b1[2], b2[2];
+#pragma unroll
+                    for (int x = 0; x < 2; x++) {
+                        const bool live = k0 + vpos(c8, e + x) < rows;
+                        const float v = live ? half_bits_to_float((uint16_t)(vq[i][e + x] >> (16 * half))) : 0.f;
+                        b1[x] = __float_as_uint(v) & 0xffff0000u;
+                        b2[x] = __float_as_uint(v - __uint_as_float(b1[x]));
+                    }
+                    w1[e / 2] = (b1[0] >> 16) | b1[1];
+                    w2[e / 2] = (b2[0] >> 16) | (b2[1] & 0xffff0000u);
+                }
+                const int dim = 2 * dp + half;
+                uint8_t *vd = short_lds + 2 * PLANE + dim * 128 + (c8 ^ (dim & 7)) * 16;
+                *reinterpret_cast<uint4 *>(vd) = make_uint4(w1[0], w1[1], w1[2], w1[3]);
+                *reinterpret_cast<uint4 *>(vd + PLANE) = make_uint4(w2[0], w2[1], w2[2], w2[3]);
+            }
+        }
+        if (it + 1 < tile_end) fetch(it + 1);
+        __syncthreads();
+        if (!tile_live || k0 + 32 * pt > wave_last) continue;         // every pair of this wave's 32 x 32 tile is masked
+        const uint8_t *kb = short_lds, *vb = kb + 2 * PLANE;
+        lv_f16v sc;
+#pragma unroll
+        for (int r = 0; r < 16; r++) sc[r] = 0.f;
+        {
+            const int row = 32 * pt + n32;
+            const uint8_t *kr = kb + row * 2 * R;
+            const int sw = attn_kswz<R>(row);
+#pragma unroll
+            for (int j = 0; j < KS; j++) {
+                const int c = (2 * j + hh) ^ sw;
+                const lv_h8 ah = *reinterpret_cast<const lv_h8 *>(kr + c * 16), al = *reinterpret_cast<const lv_h8 *>(kr + PLANE + c * 16);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ql[j], sc, 0, 0, 0);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, qh[j], sc, 0, 0, 0);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qh[j], sc, 0, 0, 0);
+            }
+        }
+        // register r of sc: position k0 + 32 pt + 8 (r / 4) + 4 hh + r % 4, query n32 of the wave's tile
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) {
+            uint32_t w1[4], w2[4], w3[4];
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                uint32_t b1[2], b2[2], b3[2];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int r = 8 * tt + e + u;
+                    const uint32_t p = k0 + 32 * pt + 8 * (r / 4) + 4 * hh + (r % 4);
+                    const bool ok = zok && p <= limit && p < a.backlog;
+                    float e0 = __expf(sc[r] * scale);
+                    e0 = ok ? e0 : 0.f;
+                    den += e0;
+                    b1[u] = __float_as_uint(e0) & 0xffff0000u;
+                    const float r1 = e0 - __uint_as_float(b1[u]);
+                    b2[u] = __float_as_uint(r1) & 0xffff0000u;
+                    b3[u] = __float_as_uint(r1 - __uint_as_float(b2[u]));
+                }
+                w1[e / 2] = (b1[0] >> 16) | b1[1];
+                w2[e / 2] = (b2[0] >> 16) | b2[1];
+                w3[e / 2] = (b3[0] >> 16) | (b3[1] & 0xffff0000u);
+            }
+            const lv_b8 p1 = __builtin_bit_cast(lv_b8, make_uint4(w1[0], w1[1], w1[2], w1[3]));
+            const lv_b8 p2 = __builtin_bit_cast(lv_b8, make_uint4(w2[0], w2[1], w2[2], w2[3]));
+            const lv_b8 p3 = __builtin_bit_cast(lv_b8, make_uint4(w3[0], w3[1], w3[2], w3[3]));
+#pragma unroll
+            for (int d = 0; d < DT; d++) {
+                const int dim = 32 * d + n32, c = (4 * pt + 2 * tt + hh) ^ (dim & 7);
+                const lv_b8 va = *reinterpret_cast<const lv_b8 *>(vb + dim * 128 + c * 16);
+                const lv_b8 vc = *reinterpret_cast<const lv_b8 *>(vb + PLANE + dim * 128 + c * 16);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p3, va, acc[d], 0, 0, 0);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p2, vc, acc[d], 0, 0, 0);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p2, va, acc[d], 0, 0, 0);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p1, vc, acc[d], 0, 0, 0);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p1, va, acc[d], 0, 0, 0);
+            }
+        }
+    }
+    // ---- the second position tile's sums to the first's waves, then out ---------------------------------------------------------
+    den += __shfl_xor(den, 32, kWave);
+    float *xch = reinterpret_cast<float *>(short_lds);
+    __syncthreads();
+    if (pt == 1) {
+        if (hh == 0) den_s[qt][n32] = den;
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) xch[(32 * qt + 8 * (r / 4) + 4 * hh + (r % 4)) * XS + 32 * d + n32] = acc[d][r];
+    }
+    __syncthreads();
+    if (a.act) {
+        if (pt == 0) {
+            if (hh == 0) den_s[qt][n32] += den;
+#pragma unroll
+            for (int d = 0; d < DT; d++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) xch[(32 * qt + 8 * (r / 4) + 4 * hh + (r % 4)) * XS + 32 * d + n32] += acc[d][r];
+        }
+        __syncthreads();
+        for (uint32_t i = t; i < a.n * C8; i += 256) {
+            const uint32_t z = i / C8, c = i % C8, k = h * R + (c >> 2) * 32, g = c & 3;
+            const float *row = xch + z * XS + (c >> 2) * 32;
+            const float total = den_s[z >> 5][z & 31];
+            float4 va = *reinterpret_cast<const float4 *>(row + (a.q8 ? short_run_a<8>(g) : short_run_a<4>(g)));
+            float4 vb = *reinterpret_cast<const float4 *>(row + (a.q8 ? short_run_b<8>(g) : short_run_b<4>(g)));
+            va.x /= total; va.y /= total; va.z /= total; va.w /= total;
+            vb.x /= total; vb.y /= total; vb.z /= total; vb.w /= total;
+            float f[8];
+            if (a.q8) short_order<8>(f, va, vb);
+            else short_order<4>(f, va, vb);
+            uint4 hi, lo;
+            gemm_split8(hi, lo, f);
+            uint8_t *dst = a.act + short_act_offset(k / 32, z, g, a.tiles);
+            *reinterpret_cast<uint4 *>(dst) = hi;
+            *reinterpret_cast<uint4 *>(dst + short_act_low(a.tiles)) = lo;
+        }
+        return;
+    }
+    if (pt == 1) return;
+    const size_t part = (size_t)blockIdx.y * a.n;
+    if (hh == 0 && zok) a.den[(part + zq) * H + h] = den + den_s[qt][n32];
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const uint32_t z = 32 * qt + 8 * (r / 4) + 4 * hh + (r % 4);
+            if (z < a.n) a.num[(part + z) * D + (size_t)h * R + 32 * d + n32] = acc[d][r] + xch[z * XS + 32 * d + n32];
+        }
+}
+
+// numerators and denominators of all splits, in order -> the output projection's activations.  grid (D / 8 / 256 rounded up, n)
+struct ShortCombineArgs {
+    const float *num, *den;
+    uint32_t splits, n, heads, rot, tiles;
+    uint8_t *act;
+};
+template <int QT>
+__global__ __launch_bounds__(256) void short_attn_combine_kernel(ShortCombineArgs a)
+{
+    const uint32_t D = a.heads * a.rot, i = blockIdx.x * 256 + threadIdx.x, z = blockIdx.y;
+    if (i >= D / 8) return;
+    const uint32_t ka = (i >> 2) * 32 + short_run_a<QT>(i & 3), kb = (i >> 2) * 32 + short_run_b<QT>(i & 3);
+    const uint32_t h = ka / a.rot;                     // a block of 32 lies in one head
+    float4 va = make_float4(0.f, 0.f, 0.f, 0.f), vb = va;
+    float den = 0.f;
+    for (uint32_t s = 0; s < a.splits; s++) {
+        const size_t part = (size_t)s * a.n + z;
+        const float4 pa = *reinterpret_cast<const float4 *>(a.num + part * D + ka), pb = *reinterpret_cast<const float4 *>(a.num + part * D + kb);
+        va.x += pa.x; va.y += pa.y; va.z += pa.z; va.w += pa.w;
+        vb.x += pb.x; vb.y += pb.y; vb.z += pb.z; vb.w += pb.w;
+        den += a.den[part * a.heads + h];
+    }
+    va.x /= den; va.y /= den; va.z /= den; va.w /= den;
+    vb.x /= den; vb.y /= den; vb.z /= den; vb.w /= den;
+    float f[8];
+    short_order<QT>(f, va, vb);
+    uint4 hi, lo;
+    gemm_split8(hi, lo, f);
+    uint8_t *dst = a.act + short_act_offset(i >> 2, z, i & 3, a.tiles);
+    *reinterpret_cast<uint4 *>(dst) = hi;
+    *reinterpret_cast<uint4 *>(dst + short_act_low(a.tiles)) = lo;
+}
+
+}  // namespace lv

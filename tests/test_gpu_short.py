@@ -1,0 +1,76 @@
+"""Short batches (2 .. 64 tokens, csrc/lv_short.h) of LLaMA models against the CPU checker: every edge of the token tiles (16) and of
+the kernels' limit, head sizes 32, 64 and 128, both weight types, K slices, contexts in front of the batch.
+
+Tolerance: the one the path is specified with (test_gpu_model.py): 1e-2 and 1e-3 of the largest logit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    "q4_32": ("Q4_0", dict(vocab=512, dim=384, heads=12, layers=2, ff=640)),
+    "q4_64": ("Q4_0", dict(vocab=500, dim=512, heads=8, layers=2, ff=1408)),      # a vocabulary that 16 does not divide
+    "q4_128": ("Q4_0", dict(vocab=512, dim=2048, heads=16, layers=1, ff=5504)),   # rows of 43 chunks: the waves' shares differ
+    "q8_64": ("Q8_0", dict(vocab=512, dim=384, heads=6, layers=2, ff=896)),
+    "q8_128": ("Q8_0", dict(vocab=512, dim=2048, heads=16, layers=1, ff=5504)),
+}
+
+
+@pytest.fixture(scope="module")
+def models(lva, tmp_path_factory):
+    d = tmp_path_factory.mktemp("short")
+    out = {}
+    for i, (name, (wtype, shape)) in enumerate(SHAPES.items()):
+        out[name] = str(d / f"{name}.ggml")
+        lva.write_model(out[name], wtype=getattr(lva, "LV_" + wtype), seed=60 + i, **shape)
+    return out
+
+
+def close(got, want):
+    err = np.max(np.abs(got - want))
+    assert err <= 1e-2 and err <= 1e-3 * np.max(np.abs(want)), (err, np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("name", list(SHAPES))
+@pytest.mark.parametrize("before,n", [(0, 2), (0, 16), (5, 17), (0, 33), (61, 3), (64, 48), (120, 64), (190, 65), (201, 49)])
+def test_short_batch_matches_oracle(lva, orc, ctx, models, name, before, n):
+    om = orc.Model(models[name])
+    osess = orc.Session(om, 256)
+    model = lva.Model(ctx, models[name])
+    sess = lva.Session(model, 256)
+    toks = lva.synth_tokens(before + n + 1, 3, om.hp["vocab"], seed=before + n)
+    if before:
+        osess.eval(toks[:before])
+        sess.begin(toks[:before], 0)
+        sess.wait()
+        for layer in range(om.hp["layers"]):       # the batch under test starts from the checker's cache
+            for which in (0, 1):
+                sess.kv_write(layer, which, osess.kv(layer, which, before))
+    want = osess.eval(toks[before:before + n])
+    sess.begin(toks[before:before + n], before)
+    close(sess.logits(), want)
+    assert sess.argmax() == int(np.argmax(sess.logits()))
+    for which in (0, 1):                           # its cache rows: at most an fp16 rounding apart in layer 0
+        g, o = (s.kv(0, which, before + n)[before:].view(np.float16).astype(np.float32) for s in (sess, osess))
+        assert np.max(np.abs(g - o)) <= np.max(np.abs(o)) * 2.0 ** -10
+    want = osess.eval(toks[-1:])                   # ... which the next token reads
+    sess.begin(toks[-1:], before + n)
+    close(sess.logits(), want)
+    sess.close(); model.close(); osess.close(); om.close()
+
+
+@pytest.mark.parametrize("name", ["q4_64", "q8_128"])
+@pytest.mark.parametrize("n", [2, 31, 64])
+def test_every_row_of_a_short_batch(lva, ctx, models, name, n):
+    """lv_logits_read_rows against the same tokens one by one: both fp32, the cache rows rounded alike but for ties"""
+    model = lva.Model(ctx, models[name])
+    a, b = lva.Session(model, 128), lva.Session(model, 128)
+    toks = lva.synth_tokens(n, 3, 500, seed=n)
+    a.keep_all_logits()
+    a.begin(toks, 0)
+    rows = a.logits_rows(0, n)
+    assert np.array_equal(rows[-1], a.logits())
+    for i, t in enumerate(toks):
+        b.begin([t], i)
+        close(rows[i], b.logits())
+    a.close(); b.close(); model.close()
