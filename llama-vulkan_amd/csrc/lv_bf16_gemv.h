@@ -67,6 +67,7 @@ struct BfGemvArgs {
     GroupInput group;
     StreamInput streams;
     uint32_t act;                // kGemvGlu: LV_ACT_*
+    uint32_t same_order;         // 1: every row is summed in the same order
     // experts
     const float *z;              // router logits
     uint32_t experts, top, expert_rows;   // expert_rows: weight rows from one expert to the next
@@ -203,6 +204,26 @@ __device__ __forceinline__ void group_input(const GroupInput &a, float *sums, Pu
 __device__ __forceinline__ void top_experts(float *zs, uint32_t n, uint32_t top, uint32_t *ids, float *scores)
 {
     const uint32_t lane = threadIdx.x & 63;
+    // Up to a lane each: a lane counts the experts in front of its own, its place in the order.  n steps that do not wait for one
+    // another; the rounds below are `top` times twelve cross-lane moves one after the other, with every weight load behind them.
+    // Nothing is in front of anything where there is a NaN: the rounds settle those.
+    if (n <= 64) {
+        const float mine = lane < n ? zs[lane] : -INFINITY;
+        if (!__any(mine != mine || mine == -INFINITY && lane < n)) {
+            uint32_t place = 0;
+            for (uint32_t e = 0; e < n; e++) {
+                const float z = zs[e];
+                place += z > mine || (z == mine && e < lane);
+            }
+            if (lane < n && place < top) {
+                ids[place] = lane;
+                scores[place] = sigmoid_f(mine);
+            }
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            return;
+        }
+    }
     for (uint32_t k = 0; k < top; k++) {
         float best = -INFINITY;
         uint32_t at = 0xffffffffu;
@@ -262,10 +283,15 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
         }
     }
 
+    // A wave walks its rows from a step of its own on, round to the one before it: were all to start at column 0, the waves of the
+    // chip, a row each, would ask the few memory channels that hold those columns first and stay in step for most of a launch
+    // (4096 x 11008: 20.0 us from column 0, 18.3 so; 13600 x 4096 22.9 and 22.0).  Not where equal rows have to give equal
+    // results to the last bit, since a choice between them hangs on it: router and head.
+    const uint32_t turn = a.same_order ? 0 : first_task % ksteps;
     uint4 q[DEPTH][NR];
-    uint32_t ftask = first_task, fit = 0, fseg = 0;
+    uint32_t ftask = first_task, fit = 0, fk = turn, fseg = 0;
     auto fetch = [&](uint4 (&slot)[NR]) {
-        const uint32_t kk = fit * 512 + lane * 8;
+        const uint32_t kk = fk * 512 + lane * 8;
         const bool ok = ftask < tasks && kk < kp;
         const uint16_t *p = a.w + kk;
         if constexpr (MODE == kGemvExperts) {
@@ -284,6 +310,7 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
             const size_t off = PAIRS ? (size_t)(r % R + (r / R) * 16) * kp : (size_t)r * kp;
             slot[r] = ok ? load_once(p + off) : make_uint4(0, 0, 0, 0);
         }
+        if (++fk == ksteps) fk = 0;
         if (++fit == ksteps) {
             fit = 0;
             if (MODE != kGemvDown || ++fseg == segs) {
@@ -317,7 +344,7 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
     float acc[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++) acc[r] = 0.f;
-    uint32_t task = first_task, it = 0, k = 0, seg = 0;
+    uint32_t task = first_task, it = 0, k = turn, kit = 0, seg = 0;
     const uint32_t my_tasks = first_task < tasks ? (tasks - first_task + nwaves - 1) / nwaves : 0;
     const uint32_t total = my_tasks * iters;
     for (uint32_t t0 = 0; t0 < total; t0 += DEPTH) {
@@ -338,7 +365,8 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
                     acc[r] = s;
                 }
                 fetch(q[d]);
-                if (++k == ksteps) { k = 0; seg++; }
+                if (++k == ksteps) k = 0;
+                if (++kit == ksteps) { kit = 0; seg++; }
                 if (++it == iters) {
                     float tot[NR];
 #pragma unroll

@@ -782,16 +782,14 @@ template <int MODE, int INPUT, int R, int DEPTH> static int launch_gemv(hipStrea
     return LV_OK;
 }
 
-// Rows a wave walks together: as many as still give every wave of the chip work, fewer where the last round of waves would then be
-// far from full.
-static uint32_t gemv_rows_together(uint32_t units, uint32_t most)
+// Rows a wave walks together: two where there are enough of them, one where the last round of waves would then be far from full
+// (us for two and one: 32000 x 4096 47.9 and 51.2, 18560 x 4096 31.1 and 33.4, 8848 x 2048 12.3 and 10.1; four at a time 60, 41
+// and 11.7).
+static uint32_t gemv_rows_together(uint32_t units)
 {
     constexpr uint32_t kWaves = 512 * kBfGemvWaves;
     auto rows_in_turn = [&](uint32_t r) { return ((units + r - 1) / r + kWaves - 1) / kWaves * r; };      // of the busiest wave
-    uint32_t best = most;
-    for (uint32_t r = most / 2; r; r /= 2)
-        if (rows_in_turn(r) < rows_in_turn(best)) best = r;
-    return best;
+    return units < 8192 || rows_in_turn(1) * 4 <= rows_in_turn(2) * 3 ? 1 : 2;
 }
 
 template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs &a)
@@ -799,12 +797,13 @@ template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs 
     const size_t lds = (size_t)a.kp * (MODE == kGemvDown ? a.top : 1) * 4 + (MODE == kGemvExperts ? a.experts * 4ull : 0) +
                        (INPUT == kInGroups ? group_sums(a.group.groups, kBfGemvWaves) * 4ull : 0);
     if constexpr (MODE == kGemvExperts || MODE == kGemvGlu) {
-        const uint32_t units = MODE == kGemvExperts ? a.top * (a.expert_rows / 2) : a.rows / 2, r = gemv_rows_together(units, units >= 8192 ? 2 : 1);
-        return r == 2 ? launch_gemv<MODE, INPUT, 2, 2>(st, a, units, lds) : launch_gemv<MODE, INPUT, 1, 4>(st, a, units, lds);
+        const uint32_t units = MODE == kGemvExperts ? a.top * (a.expert_rows / 2) : a.rows / 2;
+        return gemv_rows_together(units) == 2 ? launch_gemv<MODE, INPUT, 2, 2>(st, a, units, lds) : launch_gemv<MODE, INPUT, 1, 4>(st, a, units, lds);
     } else {
-        const uint32_t r = gemv_rows_together(a.rows, a.rows >= 16384 ? 4 : a.rows >= 8192 ? 2 : 1);
-        return r == 4 ? launch_gemv<MODE, INPUT, 4, 2>(st, a, a.rows, lds) : r == 2 ? launch_gemv<MODE, INPUT, 2, 4>(st, a, a.rows, lds)
-                                                                                    : launch_gemv<MODE, INPUT, 1, 8>(st, a, a.rows, lds);
+        // one row at a time: eight steps ahead, or a row of up to 2048 columns (8848 x 2048: 11.0 us with eight, 10.1 with four)
+        return gemv_rows_together(a.rows) == 2 ? launch_gemv<MODE, INPUT, 2, 4>(st, a, a.rows, lds)
+               : a.kp <= 2048                  ? launch_gemv<MODE, INPUT, 1, 4>(st, a, a.rows, lds)
+                                               : launch_gemv<MODE, INPUT, 1, 8>(st, a, a.rows, lds);
     }
 }
 
@@ -1163,7 +1162,7 @@ int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *
             LV_TRY((gemv<kGemvRows, kInPlain>(st, dn)));
         } else {
             BfGemvArgs rt{};
-            rt.w = l.router.w; rt.rows = l.spec.moe.experts; rt.kp = Dp; rt.out = s->z;
+            rt.w = l.router.w; rt.rows = l.spec.moe.experts; rt.kp = Dp; rt.out = s->z; rt.same_order = 1;
             res.feed(rt, l.site[1], s->h2);
             LV_TRY(gemv_residual<kGemvRows>(m, st, rt));
             LV_TRY(keep((uint32_t)i, LV_TRACE_POST_ATTN));
@@ -1193,7 +1192,7 @@ int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *
     }
     if (logits) {
         BfGemvArgs h{};
-        h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits;
+        h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits; h.same_order = 1;
         res.feed(h, m->final, nullptr, false);
         LV_TRY(gemv_residual<kGemvRows>(m, st, h));
     }
@@ -1562,6 +1561,7 @@ static int step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32
         if (logits_last) HIP_TRY(hipMemcpyAsync(logits_last, logits_all + (size_t)(n - 1) * m->hp.vocab, m->hp.vocab * 4ull, hipMemcpyDeviceToDevice, st));
     } else if (logits_last) {
         BfGemvArgs h{};
+        h.same_order = 1;
         h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits_last;
         const float *x = w.x + (size_t)(n - 1) * m->copies * Dp;
         if (m->hp.streams) {
