@@ -10,11 +10,17 @@
 // In the MFMA a weight tile is operand A (M = weight row) and the tokens are operand B (N = token): lane l of the result
 // holds token l % 16 and four consecutive weight rows 4 * (l / 16) .. + 3, i.e. one 16-byte store into the token's row.
 //
-// gemm_bf16_kernel<NW>: NW waves of 64 x 64 each, tile 32 NW weight rows x 128 tokens, K step 64.  Both operand tiles go to LDS
-// by direct loads: two stages and two workgroups a CU with four waves, three stages and one workgroup with eight (fewer bytes
-// into LDS per product, loads two steps ahead; for launches that fill the chip with it).  A row of a tile is 128 bytes; its
-// eight 16-byte chunks are stored in the order chunk ^ (row % 8), so that the 16 rows an MFMA operand reads at one k spread over
-// all banks.
+// Tiles, K step 64, both operands in LDS by direct loads, four waves:
+//   gemm_bf16_kernel        128 rows x 128 tokens, waves of 64 x 64, two stages, two workgroups a CU: few tiles, and short K
+//   gemm_wide_kernel<64>    256 rows x 128 tokens, waves of 128 x 64, three stages, one workgroup a CU
+//   gemm_wide_kernel<128>   256 rows x 256 tokens, waves of 128 x 128 (all 256 accumulation registers), two stages
+// A 64 x 64 wave reads 8 KB of LDS per 16 matrix instructions, as long as those take, and the direct loads write LDS as well: LDS
+// bounds it at three quarters of the matrix rate.  Larger waves read 6 or 4 KB.  One wave per SIMD hides nothing by itself: the
+// wide kernels spell the order out, the next half step's operand reads and the direct loads one by one between the products.
+// Measured, us (TFLOP/s): 2048 tokens x 22016 x 4096 468 (788), 392 (943), 355 (1040); x 13600 x 4096 313, 263, 235; x 4096 x 8192
+// 153, 138, 189; 777 x 22016 x 4096 211, 191, 214; 777 x 4096 x 11008 147, 156, 235.
+// A row of a tile is 128 bytes; its eight 16-byte chunks are stored in the order chunk ^ (row % 8), so that the 16 rows an MFMA
+// operand reads at one k spread over all banks.
 #pragma once
 
 #include "../../include/llava_hip.h"
@@ -208,17 +214,18 @@ __device__ __forceinline__ void bf_store_glu(const BfGemmArgs &a, uint32_t posit
     else *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
-// Tile of this workgroup: workgroups are dealt to the 8 XCDs in turn; an XCD takes every eighth row tile and walks the token
-// tiles of one row tile before the next, so that the weight tile is read into its L2 once.
+// Tile of this workgroup: workgroups are dealt to the 8 XCDs in turn; the tiles, token tiles of one row tile one after the other, are
+// cut in eight runs of one length, one for each XCD, so that an XCD reads a weight tile into its L2 once and all have as much to do
+// (row tiles dealt in turn: 73 of them x 7 token tiles are 70 for one XCD and 63 for the others, three rounds instead of two).
 template <bool GROUPED>
 __device__ __forceinline__ bool bf_tile(const BfGemmArgs &a, uint32_t tile_tokens, uint32_t &rt, uint32_t &expert, uint32_t &first, uint32_t &count)
 {
-    const uint32_t pid = blockIdx.x, q = pid >> 3;
-    rt = q / a.token_tiles * 8 + (pid & 7);
-    const uint32_t tt = q % a.token_tiles;
-    if (rt >= a.row_tiles) return false;
+    const uint32_t tt_count = GROUPED ? a.tiles[0] : a.token_tiles, all = a.row_tiles * tt_count, run = (all + 7) / 8, q = blockIdx.x >> 3;
+    const uint32_t at = (blockIdx.x & 7) * run + q;
+    if (q >= run || at >= all) return false;
+    rt = at / tt_count;
+    const uint32_t tt = at % tt_count;
     if constexpr (GROUPED) {
-        if (tt >= a.tiles[0]) return false;
         expert = a.tiles[1 + 3 * tt];
         first = a.tiles[2 + 3 * tt];
         count = a.tiles[3 + 3 * tt];
@@ -229,20 +236,52 @@ __device__ __forceinline__ bool bf_tile(const BfGemmArgs &a, uint32_t tile_token
     }
     return true;
 }
-inline uint32_t bf_grid(const BfGemmArgs &a) { return (a.row_tiles + 7) / 8 * 8 * a.token_tiles; }
+inline uint32_t bf_grid(const BfGemmArgs &a) { return (a.row_tiles * a.token_tiles + 7) / 8 * 8; }
 
 constexpr int kBfTile = 128;       // tokens per workgroup, bf16
 constexpr int kBfStep = 64;
-constexpr int bf_tile_rows(int nw) { return 32 * nw; }
-constexpr int bf_stages(int nw) { return nw == 4 ? 2 : 3; }
-constexpr int bf_stage_bytes(int nw) { return (bf_tile_rows(nw) + kBfTile) * kBfStep * 2; }
-constexpr int bf_lds_bytes(int nw) { return bf_stages(nw) * bf_stage_bytes(nw); }
+constexpr int kBfRows = 128;       // rows of gemm_bf16_kernel's tile
+constexpr int kBfLdsBytes = 2 * (kBfRows + kBfTile) * kBfStep * 2;
 
-template <int EP, bool GROUPED, int NW>
-__global__ __launch_bounds__(NW * 64, 2) void gemm_bf16_kernel(BfGemmArgs a)
+// epilogue of a wave: A x B tiles of 16 rows x 16 tokens, the first at weight row `row0` and token `t0` of the workgroup's tile
+template <int EP, int A, int B>
+__device__ __forceinline__ void bf_store_wave(const BfGemmArgs &a, const lv_f4 (&acc)[A][B], uint32_t row0, uint32_t t0, uint32_t first, uint32_t count)
 {
-    constexpr int RM = bf_tile_rows(NW), NST = bf_stages(NW), STAGE = bf_stage_bytes(NW);
-    constexpr int LW = RM / NW / 8, LX = kBfTile / NW / 8, LPS = LW + LX;      // direct loads per wave and stage, 8 rows (1 KB) each
+    const uint32_t l16 = threadIdx.x & 15, g4 = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int j = 0; j < B; j++) {
+        const uint32_t t = t0 + j * 16 + l16;
+        if (t >= count) continue;
+        const uint32_t p = first + t;
+        if constexpr (EP == kEpGlu) {
+            const float wt = a.weights[a.slots[p]];
+#pragma unroll
+            for (int i = 0; i < A; i += 2) {
+                const uint32_t row = row0 + i * 16;        // the pair's gate block
+                if (row < a.rows) bf_store_glu<uint16_t>(a, p, row / 2 + g4 * 4, wt, acc[i][j], acc[i + 1][j]);
+            }
+        } else if constexpr (EP == kEpDense) {
+#pragma unroll
+            for (int i = 0; i < A; i += 2) {
+                const uint32_t row = row0 + i * 16;
+                if (row < a.rows) bf_store_dense<uint16_t>(a, p, row / 2 + g4 * 4, acc[i][j], acc[i + 1][j]);
+            }
+        } else if constexpr (EP == kEpHeads) {
+#pragma unroll
+            for (int i = 0; i < A; i++) bf_store_heads<uint16_t>(a, p, row0 + i * 16 + g4 * 4, acc[i][j]);
+        } else {
+            const uint32_t orow = EP == kEpScatter ? a.slots[p] : p;
+#pragma unroll
+            for (int i = 0; i < A; i++) bf_store4<EP>(a, orow, row0 + i * 16 + g4 * 4, acc[i][j]);
+        }
+    }
+}
+
+template <int EP, bool GROUPED>
+__global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(BfGemmArgs a)
+{
+    constexpr int RM = kBfRows, STAGE = (RM + kBfTile) * kBfStep * 2;
+    constexpr int LW = RM / 32, LX = kBfTile / 32;          // direct loads per wave and stage, 8 rows (1 KB) each
     extern __shared__ __attribute__((aligned(128))) uint8_t bf_lds[];
     uint32_t rt, expert, first, count;
     if (!bf_tile<GROUPED>(a, kBfTile, rt, expert, first, count)) return;
@@ -253,10 +292,10 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_bf16_kernel(BfGemmArgs a)
     const uint16_t *gw, *gx[LX];
     {
         const int r8 = lane >> 3, c = (lane & 7) ^ r8;
-        gw = a.w + ((size_t)expert * a.expert_rows + (size_t)rt * RM + wave * (RM / NW) + r8) * kp + c * 8;
+        gw = a.w + ((size_t)expert * a.expert_rows + (size_t)rt * RM + wave * (RM / 4) + r8) * kp + c * 8;
 #pragma unroll
         for (int i = 0; i < LX; i++) {
-            const int row = wave * (kBfTile / NW) + i * 8 + r8;
+            const int row = wave * (kBfTile / 4) + i * 8 + r8;
             size_t xr = (size_t)first + row;
             if constexpr (GROUPED) {
                 const uint32_t p = first + min((uint32_t)row, count - 1);
@@ -278,22 +317,21 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_bf16_kernel(BfGemmArgs a)
         for (int i = 0; i < LX; i++) __builtin_amdgcn_global_load_lds((lv_glb_any *)(gx[i] + k0), (lv_lds_any *)(buf + RM * 128 + (wave * LX + i) * 1024), 16, 0, 0);
     };
 
-    const int wm = wave % (NW / 2), wn = wave / (NW / 2);
+    const int wm = wave & 1, wn = wave >> 1;
     lv_f4 acc[4][4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[i][j] = lv_f4{0.f, 0.f, 0.f, 0.f};
 
-#pragma unroll
-    for (int s = 0; s < NST - 1; s++) issue(s, s);
-    uint32_t slot = 0, ahead = NST - 1;
+    issue(0, 0);
+    uint32_t slot = 0;
     for (uint32_t s = 0; s < steps; s++) {
         // this wave's loads of stage s have landed; behind the barrier everyone's have, and everyone is done with stage s - 1
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * LPS) : "memory");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        issue(s + NST - 1, ahead);
+        issue(s + 1, slot ^ 1);
         const uint8_t *bw = bf_lds + slot * STAGE, *bx = bw + RM * 128;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
@@ -308,37 +346,121 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_bf16_kernel(BfGemmArgs a)
 #pragma unroll
                 for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
         }
-        slot = slot + 1 == NST ? 0 : slot + 1;
-        ahead = ahead + 1 == NST ? 0 : ahead + 1;
+        slot ^= 1;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the repeats have landed before the workgroup gives up its LDS
+    bf_store_wave<EP>(a, acc, rt * RM + wm * 64, wn * 64, first, count);
+}
+
+constexpr int wide_tokens(int wn) { return 2 * wn; }
+constexpr int wide_stages(int wn) { return wn == 64 ? 3 : 2; }
+constexpr int wide_lds_bytes(int wn) { return wide_stages(wn) * (256 + wide_tokens(wn)) * kBfStep * 2; }
+
+// c += a b; IN_ACC: c in accumulation registers, where the compiler would move them to and fro around every product.  The compiler
+// does not know of these products what has to lie between them and moves of their registers.  It has moves behind a K step (into and
+// out of the loop, spills) but none within, so a step's first product waits for a move into its registers (2 states) and its last one
+// until every product of the step is written (11 states behind an eight-pass product).
+template <bool IN_ACC>
+__device__ __forceinline__ void wide_product(lv_f4 &c, const lv_bf8 &a, const lv_bf8 &b, bool first = false, bool last = false)
+{
+    if constexpr (IN_ACC) {
+        if (first) asm("s_nop 1\n v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+        else if (last) asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n s_nop 15" : "+a"(c) : "v"(a), "v"(b));
+        else asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    } else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// 256 rows x 2 WN tokens, waves of 128 x WN
+template <int EP, bool GROUPED, int WN>
+__global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemmArgs a)
+{
+    constexpr int TN = wide_tokens(WN), NST = wide_stages(WN), STAGE = (256 + TN) * kBfStep * 2, NJ = WN / 16;
+    constexpr int LW = 8, LX = TN / 32, LPS = LW + LX;      // direct loads per wave and stage, 8 rows (1 KB) each
+    constexpr int NM = 8 * NJ, NR = 8 + NJ;                 // products and operand reads of half a step
+    extern __shared__ __attribute__((aligned(128))) uint8_t bf_lds[];
+    uint32_t rt, expert, first, count;
+    if (!bf_tile<GROUPED>(a, TN, rt, expert, first, count)) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g4 = lane >> 4;
+    const uint32_t kp = a.kp;
+
+    const uint16_t *gw, *gx[LX];
+    {
+        const int r8 = lane >> 3, c = (lane & 7) ^ r8;
+        gw = a.w + ((size_t)expert * a.expert_rows + (size_t)rt * 256 + wave * 64 + r8) * kp + c * 8;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t t = wn * 64 + j * 16 + l16;
-        if (t >= count) continue;
-        const uint32_t p = first + t;
-        if constexpr (EP == kEpGlu) {
-            const float wt = a.weights[a.slots[p]];
-#pragma unroll
-            for (int i = 0; i < 4; i += 2) {
-                const uint32_t row = rt * RM + wm * 64 + i * 16;        // the pair's gate block
-                if (row < a.rows) bf_store_glu<uint16_t>(a, p, row / 2 + g4 * 4, wt, acc[i][j], acc[i + 1][j]);
+        for (int i = 0; i < LX; i++) {
+            const int row = wave * (TN / 4) + i * 8 + r8;
+            size_t xr = (size_t)first + row;
+            if constexpr (GROUPED) {
+                const uint32_t p = first + min((uint32_t)row, count - 1);
+                xr = a.gather ? a.slots[p] / a.top : p;
+            } else if constexpr (TN > kBfTile) {            // activations end at a multiple of kBfTile
+                xr = first + min((uint32_t)row, (count + kBfTile - 1) / kBfTile * kBfTile - 1);
             }
-        } else if constexpr (EP == kEpDense) {
-#pragma unroll
-            for (int i = 0; i < 4; i += 2) {
-                const uint32_t row = rt * RM + wm * 64 + i * 16;
-                if (row < a.rows) bf_store_dense<uint16_t>(a, p, row / 2 + g4 * 4, acc[i][j], acc[i + 1][j]);
-            }
-        } else if constexpr (EP == kEpHeads) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) bf_store_heads<uint16_t>(a, p, rt * RM + wm * 64 + i * 16 + g4 * 4, acc[i][j]);
-        } else {
-            const uint32_t orow = EP == kEpScatter ? a.slots[p] : p;
-#pragma unroll
-            for (int i = 0; i < 4; i++) bf_store4<EP>(a, orow, rt * RM + wm * 64 + i * 16 + g4 * 4, acc[i][j]);
+            gx[i] = static_cast<const uint16_t *>(a.x) + xr * a.ldx + c * 8;
         }
     }
+    const uint32_t k_lo = EP == kEpStore && a.k_slice ? blockIdx.z * a.k_slice : 0;
+    const uint32_t steps = (EP == kEpStore && a.k_slice ? min(a.k_slice, kp - k_lo) : kp) / kBfStep;
+    // direct load p of this wave for stage s; past the end a harmless repeat of the last step into a free buffer
+    auto issue_one = [&](uint32_t s, uint32_t slot, int p) {
+        uint8_t *buf = bf_lds + slot * STAGE;
+        const uint32_t k0 = k_lo + min(s, steps - 1) * kBfStep;
+        if (p < LW) __builtin_amdgcn_global_load_lds((lv_glb_any *)(gw + (size_t)p * 8 * kp + k0), (lv_lds_any *)(buf + (wave * LW + p) * 1024), 16, 0, 0);
+        else __builtin_amdgcn_global_load_lds((lv_glb_any *)(gx[p - LW] + k0), (lv_lds_any *)(buf + 256 * 128 + (wave * LX + p - LW) * 1024), 16, 0, 0);
+    };
+
+    const int wm = wave & 1, wn = wave >> 1;
+    lv_f4 acc[8][NJ];
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = lv_f4{0.f, 0.f, 0.f, 0.f};
+    struct Operands { lv_bf8 a[8], b[NJ]; };
+    auto read_one = [&](Operands &f, const uint8_t *buf, int kk, int r) {      // operand read r of half step kk of a stage
+        const int ch = ((kk * 4 + g4) ^ (l16 & 7)) * 16;
+        if (r < NJ) f.b[r] = *reinterpret_cast<const lv_bf8 *>(buf + 256 * 128 + (wn * WN + r * 16 + l16) * 128 + ch);
+        else f.a[r - NJ] = *reinterpret_cast<const lv_bf8 *>(buf + (wm * 128 + (r - NJ) * 16 + l16) * 128 + ch);
+    };
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int p = 0; p < LPS; p++) issue_one(s, s, p);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    Operands f0, f1;
+#pragma unroll
+    for (int r = 0; r < NR; r++) read_one(f0, bf_lds, 0, r);
+    uint32_t slot = 0;
+    for (uint32_t s = 0; s < steps; s++) {
+        const uint32_t next = slot + 1 == NST ? 0 : slot + 1, free_slot = NST == 2 ? slot : next + 1 == NST ? 0 : next + 1;
+        // first half: with three stages the loads of stage s + 2 go where stage s - 1 was
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f0.a[m / NJ], f0.b[m % NJ], m == 0);
+            if (m % 2 == 0 && m / 2 < NR) read_one(f1, bf_lds + slot * STAGE, 1, m / 2);
+            if (NST == 3 && m % 2 == 1 && m / 2 < LPS) issue_one(s + 2, free_slot, m / 2);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // This wave's loads of stage s + 1 have landed and it holds the rest of stage s in registers; behind the barrier that
+        // goes for everyone: stage s + 1 may be read, and with two stages the loads of stage s + 2 may go where stage s is
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NST == 2 ? 0 : LPS) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f1.a[m / NJ], f1.b[m % NJ], false, m == NM - 1);
+            if (m % 2 == 0 && m / 2 < NR) read_one(f0, bf_lds + next * STAGE, 0, m / 2);
+            if (NST == 2 && m % 4 == 1 && m / 4 < LPS) issue_one(s + 2, free_slot, m / 4);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        slot = next;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the repeats have landed before the workgroup gives up its LDS
+    bf_store_wave<EP>(a, acc, rt * 256 + wm * 128, wn * WN, first, count);
 }
 
 constexpr int kF32Tile = 64;

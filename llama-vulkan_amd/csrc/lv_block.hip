@@ -101,6 +101,7 @@ struct Workspace {                     // of batches; sized for `cap` tokens
          *ek = nullptr, *ev = nullptr, *sx = nullptr, *sb = nullptr, *sc = nullptr, *sbt = nullptr;
     uint32_t *ids = nullptr, *slots = nullptr, *tiles = nullptr;
     uint64_t vt_elems = 0, ek_elems = 0, ev_elems = 0;
+    uint64_t y_vectors = 0;            // sublayer outputs there is room for in y
 };
 
 struct BlockSession {
@@ -766,6 +767,8 @@ int block_session_reserve(BlockSession *s, uint32_t positions)
 // ---------------------------------------------------------------------------------------------------------------------------
 // launches
 // ---------------------------------------------------------------------------------------------------------------------------
+constexpr uint32_t kOutSlices = 4;         // slices of K a sublayer's output may come in
+
 template <class K> static int allow_lds(K kernel, size_t bytes)
 {
     if (bytes > 65536) HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
@@ -807,17 +810,48 @@ template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs 
     }
 }
 
-template <int EP, bool GROUPED, int NW> static int launch_bf_gemm(hipStream_t st, BfGemmArgs a)
+// Which tiles a bf16 product takes, and into how many slices of K it is cut (`slices` at most; the reader of the result adds them up).
+// Time = rounds of workgroups over 256 CUs x K steps x a step's time, plus prologue and epilogue, plus writing and reading a slice more.
+// Measured us a step of 64: 128 x 128 tiles 1.22 where two share a CU, 0.85 alone; 256 x 128 1.02; 256 x 256 1.85, 1.45 where half of
+// the CUs have none.
+enum class BfTiles { k128, kWide, kWidest };
+struct BfPlan {
+    BfTiles tiles;
+    uint32_t slices;
+};
+static BfPlan bf_plan(uint32_t rows, uint32_t n, uint32_t token_tiles, uint32_t kp, bool grouped, uint32_t slices)
 {
-    auto *k = &gemm_bf16_kernel<EP, GROUPED, NW>;
-    a.row_tiles = (a.rows + bf_tile_rows(NW) - 1) / bf_tile_rows(NW);
-    LV_TRY(allow_lds(k, bf_lds_bytes(NW)));
-    k<<<dim3(bf_grid(a), 1, a.k_slice ? (a.kp + a.k_slice - 1) / a.k_slice : 1), dim3(NW * 64), bf_lds_bytes(NW), st>>>(a);
+    BfPlan best{BfTiles::k128, 1};
+    double best_us = 1e30;
+    for (uint32_t s = 1; s <= slices; s++) {
+        const uint32_t steps = (kp / kBfStep + s - 1) / s;
+        if (s > 1 && steps < 8) break;
+        const double more = 4.0 + (s - 1) * (1.0 + 2e-6 * n * rows);
+        auto offer = [&](BfTiles t, uint64_t tiles, double step_us) {
+            const double us = step_us * steps + more;
+            if (tiles && us < best_us) {
+                best_us = us;
+                best = {t, s};
+            }
+        };
+        const uint64_t small = (uint64_t)((rows + 127) / 128) * token_tiles * s, wide = (uint64_t)((rows + 255) / 256) * token_tiles * s;
+        const uint64_t widest = grouped ? 0 : (uint64_t)((rows + 255) / 256) * ((n + 255) / 256) * s;
+        offer(BfTiles::k128, small, small / 512 * 1.22 + (small % 512 > 256 ? 1.22 : small % 512 ? 0.85 : 0.0));
+        offer(BfTiles::kWide, wide, (double)((wide + 255) / 256) * 1.02);
+        offer(BfTiles::kWidest, widest, widest <= 128 ? 1.45 : (double)((widest + 255) / 256) * 1.85);
+    }
+    return best;
+}
+
+template <class K> static int launch_bf(hipStream_t st, K *k, const BfGemmArgs &a, int lds)
+{
+    LV_TRY(allow_lds(k, lds));
+    k<<<dim3(bf_grid(a), 1, a.k_slice ? (a.kp + a.k_slice - 1) / a.k_slice : 1), dim3(256), lds, st>>>(a);
     HIP_TRY(hipGetLastError());
     return LV_OK;
 }
 
-template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t experts = 1)
+template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t experts = 1, BfTiles tiles = BfTiles::k128, bool planned = false)
 {
     const uint32_t tile = f32 ? kF32Tile : kBfTile, token_tiles = (n + tile - 1) / tile;
     a.w = w.w;
@@ -832,10 +866,37 @@ template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemm
         return LV_OK;
     }
     if constexpr (EP != kEpDecay && EP != kEpSigmoid) {      // those two have a few K steps only
-        const uint64_t big_tiles = (uint64_t)((w.rows + 255) / 256) * std::max(token_tiles, GROUPED ? experts : 1u);
-        if (big_tiles >= 256) return launch_bf_gemm<EP, GROUPED, 8>(st, a);
+        // grouped: about half of the experts end in a tile of their own
+        if (!planned && !a.k_slice) tiles = bf_plan(w.rows, n, GROUPED ? std::max(token_tiles + experts / 2, 1u) : token_tiles, w.kp, GROUPED, 1).tiles;
+        if (tiles != BfTiles::k128) {
+            a.row_tiles = (w.rows + 255) / 256;
+            if constexpr (!GROUPED) {
+                if (tiles == BfTiles::kWidest) {
+                    a.token_tiles = (n + wide_tokens(128) - 1) / wide_tokens(128);
+                    return launch_bf(st, &gemm_wide_kernel<EP, false, 128>, a, wide_lds_bytes(128));
+                }
+            }
+            return launch_bf(st, &gemm_wide_kernel<EP, GROUPED, 64>, a, wide_lds_bytes(64));
+        }
     }
-    return launch_bf_gemm<EP, GROUPED, 4>(st, a);
+    a.row_tiles = (w.rows + kBfRows - 1) / kBfRows;
+    return launch_bf(st, &gemm_bf16_kernel<EP, GROUPED>, a, kBfLdsBytes);
+}
+
+// a product into the sublayer outputs `y` ([token][slice][dp], room for `room` vectors), cut in slices of K where its tiles would leave
+// CUs without work; *slices: how many the next norm has to add up
+static int gemm_output(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t dp, uint64_t room, uint32_t *slices)
+{
+    BfPlan p{BfTiles::k128, 1};
+    if (!f32) p = bf_plan(w.rows, n, (n + kBfTile - 1) / kBfTile, w.kp, false, (uint32_t)std::min<uint64_t>(kOutSlices, room / n));
+    if (p.slices > 1) {
+        a.k_slice = (w.kp / kBfStep + p.slices - 1) / p.slices * kBfStep;
+        p.slices = (w.kp + a.k_slice - 1) / a.k_slice;       // every slice has a step
+        a.slice_floats = dp;
+    }
+    a.ldo = dp * p.slices;
+    *slices = p.slices;
+    return gemm<kEpStore, false>(st, f32, a, w, n, 1, p.tiles, true);
 }
 
 // calls fn(element, integral constant DP, integral constant R) for a layer's attention
@@ -1217,7 +1278,8 @@ static int workspace_reserve(BlockSession *s, uint32_t n)
     LV_TRY(dev_zeroed(st, &w.x, T * m->copies * m->dp * 4));
     LV_TRY(dev_zeroed(st, &w.act, T * m->dp * E));
     LV_TRY(dev_zeroed(st, &w.y1, T * mx([](const BlockLayer &l) { return l.in.rows; }) * 4));
-    LV_TRY(dev_zeroed(st, &w.y, T * m->dp * 4 * mx([](const BlockLayer &l) { return std::max(1u, l.spec.moe.top); })));
+    w.y_vectors = T * std::max<uint64_t>(mx([](const BlockLayer &l) { return std::max(1u, l.spec.moe.top); }), !m->f32 && T <= 1024 ? kOutSlices : 1);
+    LV_TRY(dev_zeroed(st, &w.y, w.y_vectors * m->dp * 4));
     LV_TRY(dev_zeroed(st, &w.q, T * E * mx([](const BlockLayer &l) { return std::max(l.spec.attn.heads * l.dp, l.spec.latent.heads * l.dk); })));
     const uint64_t kv = mx([](const BlockLayer &l) { return l.spec.attn.kv_heads * l.dp; });
     LV_TRY(dev_zeroed(st, &w.k, T * E * kv));
@@ -1507,9 +1569,8 @@ static int step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32
         LV_TRY((gemm<kEpStore, false>(st, f32, g, l.in, n)));
         LV_TRY(l.latent ? batch_latent<T>(s, i, pos, n) : l.ssm ? batch_ssm<T>(s, i, pos, n) : batch_branches<T>(s, i, pos, n));
         BfGemmArgs o{};
-        o.x = w.cat; o.ldx = l.out.kp; o.out = w.y; o.ldo = Dp;
-        LV_TRY((gemm<kEpStore, false>(st, f32, o, l.out, n)));
-        parts = 1;
+        o.x = w.cat; o.ldx = l.out.kp; o.out = w.y;
+        LV_TRY(gemm_output(st, f32, o, l.out, n, Dp, w.y_vectors, &parts));
         from = &l.site[0];
         if (!l.ff()) continue;
 
@@ -1521,9 +1582,8 @@ static int step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32
             gu.x = w.act; gu.ldx = Dp; gu.act = w.ff; gu.lda = l.down.kp; gu.activation = l.spec.dense.act;
             LV_TRY((gemm<kEpDense, false>(st, f32, gu, l.gate_up, n)));
             BfGemmArgs dn{};
-            dn.x = w.ff; dn.ldx = l.down.kp; dn.out = w.y; dn.ldo = Dp;
-            LV_TRY((gemm<kEpStore, false>(st, f32, dn, l.down, n)));
-            parts = 1;
+            dn.x = w.ff; dn.ldx = l.down.kp; dn.out = w.y;
+            LV_TRY(gemm_output(st, f32, dn, l.down, n, Dp, w.y_vectors, &parts));
             continue;
         }
         const lv_moe_spec &e = l.spec.moe;
@@ -1565,8 +1625,15 @@ static int step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32
         h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits_last;
         const float *x = w.x + (size_t)(n - 1) * m->copies * Dp;
         if (m->hp.streams) {
-            if (parts > 1) {       // the launch's head takes one vector
-                LV_TRY(norm(m->final, false));
+            if (parts > 1) {       // the launch's head takes one vector: the last token's streams take it in beforehand
+                StreamRowsArgs a{};
+                a.in = stream_in(m, x, m->final);
+                a.parts = parts;
+                a.in.y = w.y + (size_t)(n - 1) * parts * Dp;
+                a.in.spread = from->coef;
+                a.in.x_out = w.x + (size_t)(n - 1) * m->copies * Dp;
+                LV_TRY(stream_rows<T>(st, a, 1));
+                parts = 0;
             }
             h.streams = stream_in(m, x, m->final);
             if (parts) {

@@ -1,0 +1,82 @@
+"""The tiles and K slices of bfloat16 products of many tokens, at sizes around their edges: a feed-forward between an embedding and the
+logits (mixers add nothing), dense and chosen by a router.
+
+The tolerance is the rounding itself: what the plain evaluation moves by when its product operands are rounded to bfloat16, twice over
+(roundings of 32-bit values that fall on the other side).  A tile, a slice or a row in the wrong place is an error of order one."""
+import numpy as np
+import pytest
+
+import block_builder as bb
+import block_oracle as bo
+import zedenex_builder as zb
+import zedenex_oracle as zo
+from block_device import Device, rel, tokens_for
+
+pytestmark = pytest.mark.gpu
+BF16 = 30
+
+
+def rounded(a):
+    return bb.from_bf16(bb.to_bf16(a))
+
+
+def dense_model(toks, W, cfg, r):
+    x = np.stack([zo.embedding(toks, W, cfg["embedding"])] * cfg["streams"])
+    x = zo.spread_streams(x, W["l0.hc1.mix"], W["l0.hc1.out"], 0 * x[0])
+    h = r(zo.norm(zo.gather_streams(x, W["l0.hc2.in"]), W, "l0.norm2", cfg["norm"]["eps"]))
+    a = np.maximum(h @ W["l0.mlp.gate"].T, 0) * (h @ W["l0.mlp.up"].T)
+    x = zo.spread_streams(x, W["l0.hc2.mix"], W["l0.hc2.out"], r(a) @ W["l0.mlp.down"].T)
+    return r(zo.norm(x.sum(0), W, "final.norm", cfg["norm"]["eps"])) @ W["embed"].T
+
+
+# width, feed-forward, tokens.  Columns (64 a K step): 1, 3, 11 and more steps in front of the pipelines' two and three stages; rows and
+# tokens one beside a tile's edge; feed-forwards whose way down is cut into 2, 3 and 4 slices, the last one shorter
+DENSE = [(40, 4100, 1100), (130, 2060, 1030), (700, 2060, 1025), (700, 4100, 1281), (300, 1100, 129), (300, 2113, 127), (257, 4160, 257),
+         (1030, 3000, 255), (128, 2048, 513), (129, 1025, 65)]
+
+
+@pytest.mark.parametrize("width,ff,n", DENSE)
+def test_dense_tiles(lva, ctx, width, ff, n):
+    cfg = zb.config(width=width, streams=2, layers=[zb.layer(zb.ssm(), ff=ff)])
+    W = zb.weights(cfg, seed=n)
+    W["l0.mix.o"][:] = 0
+    toks, F = tokens_for(cfg, n, 1), bb.as_float(W)
+    want = dense_model(toks, F, cfg, lambda a: a)
+    tol = 2 * rel(dense_model(toks, F, cfg, rounded), want)
+    assert tol < 2e-2
+    with Device(lva, zb.upload(ctx, cfg, W, BF16), 2048) as d:
+        assert rel(d.run(toks, (n,)), want) < tol
+        d.sess.keep_all_logits(False)                     # the last token's alone: its streams take in the slices beforehand
+        d.sess.begin(toks, 0)
+        assert rel(d.sess.logits()[None], want[-1:]) < tol * max(1.0, np.sqrt(np.mean(want ** 2) / np.mean(want[-1] ** 2)))
+
+
+@pytest.mark.parametrize("width,ff,n,experts,top", [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4)])
+def test_expert_tiles(lva, ctx, width, ff, n, experts, top):
+    cfg = bb.config(width=width, layers=[bb.layer(experts=experts, top=top, ff=ff)])
+    W = bb.weights(cfg, seed=n)
+    for s in ("left", "right"):
+        W[f"l0.mix.{s}.o"][:] = 0
+    F, eps = bb.as_float(W), cfg["norm"]["eps"]
+
+    def model(toks, r):
+        x = F["embed"][toks]
+        h = bo.rms_norm(x, F["l0.norm2"], eps)
+        y = np.zeros_like(x)
+        z = h @ F["l0.mlp.router"].T                      # the choice by 32-bit scores; tokens whose choice hangs on less are not asked
+        for e in range(experts):
+            t = np.nonzero((bo.choose_experts(z, top) == e).any(1))[0]
+            a = r(bo.sigmoid(z[t, e])[:, None] * h[t])
+            p = f"l0.mlp.e{e}."
+            y[t] += r(bo.silu(a @ F[p + "gate"].T) * (a @ F[p + "up"].T)) @ F[p + "down"].T
+        return r(bo.rms_norm(x + bo.rms_norm(y, F["l0.norm2b"], eps), F["final.norm"], eps)) @ F["head"].T, np.sort(z, 1)[:, ::-1]
+
+    toks = tokens_for(cfg, 4 * n, 1)
+    z = model(toks, lambda a: a)[1]
+    toks = toks[z[:, top - 1] - z[:, top] > 0.02][:n]
+    assert len(toks) == n
+    want = model(toks, lambda a: a)[0]
+    tol = 2 * rel(model(toks, rounded)[0], want)
+    assert tol < 4e-2
+    with Device(lva, bb.upload(ctx, cfg, W, BF16), 2048) as d:
+        assert rel(d.run(toks, (n,)), want) < tol
