@@ -215,8 +215,8 @@ struct lv_session {
     uint32_t *attn_counters = nullptr;
     uint32_t *cfg = nullptr;       // device: [0] = pos, [1..] = token ids of the step
     uint32_t *cfg_host = nullptr;  // pinned staging of the same
-    uint32_t *argmax_dev = nullptr;
-    uint32_t *argmax_host = nullptr;  // pinned
+    float *logits_host = nullptr;     // pinned, written by logits_out_kernel
+    uint32_t *argmax_host = nullptr;  // behind them in the same allocation, written by argmax_kernel
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     bool use_graph = true;
@@ -1534,7 +1534,7 @@ extern "C" int lv_session_destroy(lv_session *s)
     drop_graph(s);
     block_session_destroy(s->block);
     void *dev[] = {s->kv, s->trig, s->trig_abs, s->x, s->xn, s->q, s->k, s->v, s->vo, s->ff, s->logits, s->attn_part, s->attn_counters,
-                   s->cfg, s->argmax_dev, s->trace_buf, s->trace_attn, s->pf_x, s->pf_xn, s->pf_q, s->pf_k, s->pf_v, s->pf_vo, s->pf_g1, s->pf_g2,
+                   s->cfg, s->trace_buf, s->trace_attn, s->pf_x, s->pf_xn, s->pf_q, s->pf_k, s->pf_v, s->pf_vo, s->pf_g1, s->pf_g2,
                    s->pf_xh, s->pf_xl, s->pf_xs, s->pf_planes, s->pf_fh, s->pf_fl, s->logits_all, s->short_ws};
     for (void *p : dev) (void)hipFree(p);
     for (int i = 0; i < 2; i++) {
@@ -1543,7 +1543,7 @@ extern "C" int lv_session_destroy(lv_session *s)
     }
     if (s->status_host) (void)hipHostFree(s->status_host);
     if (s->cfg_host) (void)hipHostFree(s->cfg_host);
-    if (s->argmax_host) (void)hipHostFree(s->argmax_host);
+    if (s->logits_host) (void)hipHostFree(s->logits_host);
     if (s->ev_start) (void)hipEventDestroy(s->ev_start);
     if (s->ev_stop) (void)hipEventDestroy(s->ev_stop);
     if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -1573,8 +1573,8 @@ static int session_alloc(lv_session *s)
     const size_t D = hp.dim, F = hp.ff, V = hp.vocab;
     HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->logits), V * 4));
-    HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->argmax_dev), 4));
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&s->argmax_host), 4, hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&s->logits_host), (V + 1) * 4, hipHostMallocDefault));
+    s->argmax_host = reinterpret_cast<uint32_t *>(s->logits_host + V);
     LV_TRY(cfg_reserve(s, kMaxStepTokens));
     if (s->model->block) return block_session_create(s->model->block, s->stream, &s->block);
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->x), D * 4));
@@ -2587,8 +2587,12 @@ extern "C" int lv_logits_read(lv_session *s, float *dst)
 {
     if (!s || !dst) return fail(LV_ERR_ARG, "lv_logits_read: null argument");
     if (!s->have_logits) return fail(LV_ERR_STATE, "lv_logits_read: no step has produced logits");
-    HIP_TRY(hipMemcpyAsync(dst, s->logits, (size_t)s->model->hp.vocab * 4, hipMemcpyDeviceToHost, s->stream));
-    return lv_step_wait(s);
+    const uint32_t V = s->model->hp.vocab;
+    logits_out_kernel<<<dim3((V + 1023) / 1024), dim3(256), 0, s->stream>>>(s->logits_host, s->logits, V);
+    HIP_TRY(hipGetLastError());
+    LV_TRY(lv_step_wait(s));
+    memcpy(dst, s->logits_host, (size_t)V * 4);
+    return LV_OK;
 }
 
 extern "C" int lv_session_set_all_logits(lv_session *s, int enable)
@@ -2622,9 +2626,8 @@ extern "C" int lv_argmax(lv_session *s, uint32_t *token)
         *token = s->status_host[kStatusToken];
         return LV_OK;
     }
-    argmax_kernel<<<dim3(1), dim3(1024), 0, s->stream>>>(s->logits, s->model->hp.vocab, s->argmax_dev);
+    argmax_kernel<<<dim3(1), dim3(1024), 0, s->stream>>>(s->logits, s->model->hp.vocab, s->argmax_host);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(s->argmax_host, s->argmax_dev, 4, hipMemcpyDeviceToHost, s->stream));
     LV_TRY(lv_step_wait(s));
     *token = *s->argmax_host;
     return LV_OK;

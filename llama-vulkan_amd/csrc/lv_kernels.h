@@ -593,4 +593,15 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
     if (threadIdx.x == 0) *out = bi[0] == 0xffffffffu ? 0u : bi[0];
 }
 
+// A step's logits into pinned memory.  The runtime's copy to ordinary memory goes through its own staging buffer, one piece of work
+// for its copy engine or blit kernel and a wait of its own: behind a kernel of 80 us 93.5 us until 128 KB are there, this kernel, the
+// stream's wait and a memcpy 85; behind one of 5 us 73 against 19.
+__global__ __launch_bounds__(256) void logits_out_kernel(float *__restrict__ host, const float *__restrict__ logits, uint32_t n)
+{
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i + 3 < n) *reinterpret_cast<float4 *>(host + i) = *reinterpret_cast<const float4 *>(logits + i);
+    else
+        for (uint32_t j = i; j < n; j++) host[j] = logits[j];
+}
+
 }  // namespace lv
