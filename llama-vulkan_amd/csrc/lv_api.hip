@@ -1860,8 +1860,35 @@ static BlockTrace block_trace(const lv_session *s)
     return t;
 }
 
-// One token through every layer (llava_layer.cpp:53-73 + llava_command_buffer.cpp:38-39).  The token id is
-// cfg[1 + idx], its cache row cfg[0] + idx.  With_head = also compute the logits.
+// rows of the embedding table (llava_session.cpp:219-223) for the step's tokens `tokens` (of the host), n from number idx on
+static int launch_embed(lv_session *s, float *x, const uint32_t *tokens, uint32_t pos, uint32_t idx, uint32_t n)
+{
+    TokenIds ids{};
+    if (n <= kIdsInArgs) {
+        ids.pos = pos;
+        ids.cfg = s->cfg;
+        memcpy(ids.id, tokens + idx, (size_t)n * 4);
+    } else {
+        ids.batch = s->cfg + 1 + idx;
+    }
+    const lv_model *m = s->model;
+    const uint32_t D = m->hp.dim;
+    if (m->tok_ftype == LV_F32) embed_f32_kernel<<<dim3((D + 255) / 256, n), dim3(256), 0, s->stream>>>(x, m->tok_f32, ids, D);
+    else if (m->tok_ftype == LV_Q4_0) embed_quant_kernel<4><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, s->stream>>>(x, m->tok_quant.view, ids);
+    else embed_quant_kernel<8><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, s->stream>>>(x, m->tok_quant.view, ids);
+    HIP_TRY(hipGetLastError());
+    return LV_OK;
+}
+
+// the token of record_token, at cache row pos + idx; not part of its graph, as its arguments change from step to step
+static int embed_token(lv_session *s, uint32_t pos, uint32_t idx, uint32_t token)
+{
+    if (s->block) return block_embed_token(s->block, s->cfg, pos, idx, token);
+    return launch_embed(s, s->x, &token, pos, 0, 1);
+}
+
+// The embedded token through every layer (llava_layer.cpp:53-73 + llava_command_buffer.cpp:38-39).  Its cache row is
+// cfg[0] + idx.  With_head = also compute the logits.
 static int record_token(lv_session *s, uint32_t idx, bool with_head)
 {
     if (s->block) {
@@ -1872,15 +1899,7 @@ static int record_token(lv_session *s, uint32_t idx, bool with_head)
     const lv_hparams &hp = m->hp;
     const uint32_t D = hp.dim, F = hp.ff;
     hipStream_t st = s->stream;
-    const uint32_t *pos_ptr = s->cfg, *tok_ptr = s->cfg + 1 + idx;
-
-    if (m->tok_ftype == LV_F32)
-        embed_f32_kernel<<<dim3((D + 255) / 256, 1), dim3(256), 0, st>>>(s->x, m->tok_f32, tok_ptr, D);
-    else if (m->tok_ftype == LV_Q4_0)
-        embed_quant_kernel<4><<<dim3((D / 32 + 63) / 64, 1), dim3(64), 0, st>>>(s->x, m->tok_quant.view, tok_ptr);
-    else
-        embed_quant_kernel<8><<<dim3((D / 32 + 63) / 64, 1), dim3(64), 0, st>>>(s->x, m->tok_quant.view, tok_ptr);
-    HIP_TRY(hipGetLastError());
+    const uint32_t *pos_ptr = s->cfg;
 
     const dim3 kv_grid((D + 255) / 256, 1);
     for (uint32_t li = 0; li < hp.layers; li++) {
@@ -2071,16 +2090,9 @@ static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_he
     const lv_hparams &hp = m->hp;
     const uint32_t D = hp.dim, F = hp.ff;
     hipStream_t st = s->stream;
-    const uint32_t *pos_ptr = s->cfg, *tok_ptr = s->cfg + 1 + idx0;
+    const uint32_t *pos_ptr = s->cfg;
     LV_TRY(prefill_reserve(s, n));
-
-    if (m->tok_ftype == LV_F32)
-        embed_f32_kernel<<<dim3((D + 255) / 256, n), dim3(256), 0, st>>>(s->pf_x, m->tok_f32, tok_ptr, D);
-    else if (m->tok_ftype == LV_Q4_0)
-        embed_quant_kernel<4><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, st>>>(s->pf_x, m->tok_quant.view, tok_ptr);
-    else
-        embed_quant_kernel<8><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, st>>>(s->pf_x, m->tok_quant.view, tok_ptr);
-    HIP_TRY(hipGetLastError());
+    LV_TRY(launch_embed(s, s->pf_x, s->cfg_host + 1, s->cfg_host[0], idx0, n));
 
     // q, k and v buffers of a layer are free once attention has run: they take the K slices of the output projection
     // and of the down projection; `pending` of them wait to be added to the residual stream by the next norm
@@ -2385,10 +2397,7 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
         }
     }
     short_layout(hp, s->short_ws, &b);
-    const uint32_t *tok_ptr = s->cfg + 1 + idx0;
-    if (m->tok_ftype == LV_F32) embed_f32_kernel<<<dim3((D + 255) / 256, n), dim3(256), 0, st>>>(b.x, m->tok_f32, tok_ptr, D);
-    else if (m->tok_ftype == LV_Q4_0) embed_quant_kernel<4><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, st>>>(b.x, m->tok_quant.view, tok_ptr);
-    else embed_quant_kernel<8><<<dim3((D / 32 + 63) / 64, n), dim3(64), 0, st>>>(b.x, m->tok_quant.view, tok_ptr);
+    LV_TRY(launch_embed(s, b.x, s->cfg_host + 1, s->cfg_host[0], idx0, n));
     HIP_TRY(hipGetLastError());
 
     uint32_t pending = 0;       // K slices in b.parts that the next norm adds to the residual stream
@@ -2512,10 +2521,13 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
         LV_TRY(cfg_reserve(s, n));
         block_session_invalidate(s->block);      // until all of the step is on the stream
     }
-    if (!persistent) {             // the persistent kernel takes position and token id as launch arguments
+    // steps of a few tokens take position and token ids as launch arguments, and so does a token at a time
+    const uint32_t batch_min = s->block ? kBlockBatchMin : (uint32_t)kPrefillMin, batch_max = s->block ? kBlockBatch : kPrefillChunk;
+    const bool batch = !persistent && !few && n >= batch_min && (!s->trace || s->block) && ensure_prompt_copy(s->model);
+    if (!persistent) {
         s->cfg_host[0] = pos;
         memcpy(s->cfg_host + 1, tokens, (size_t)n * 4);
-        HIP_TRY(hipMemcpyAsync(s->cfg, s->cfg_host, (size_t)(1 + n) * 4, hipMemcpyHostToDevice, s->stream));
+        if (batch) HIP_TRY(hipMemcpyAsync(s->cfg, s->cfg_host, (size_t)(1 + n) * 4, hipMemcpyHostToDevice, s->stream));
     }
     if (persistent) {
         // launched above
@@ -2535,23 +2547,22 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
             s->graph = g;
             HIP_TRY(hipGraphInstantiate(&s->graph_exec, s->graph, nullptr, nullptr, 0));
         }
+        LV_TRY(embed_token(s, pos, 0, tokens[0]));
         HIP_TRY(hipGraphLaunch(s->graph_exec, s->stream));
         if (s->all_logits) HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)row_base * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
+    } else if (batch) {
+        for (uint32_t i = 0; i < n; i += batch_max) {
+            const uint32_t m = n - i < batch_max ? n - i : batch_max;
+            LV_TRY(record_prefill(s, i, m, i + m == n, row_base));
+        }
     } else {
         // rows are evaluated one after the other: row z sees cache rows 0..pos+z, which is what the batched
         // shaders compute (every row's K/V is appended before any row attends, and rows above are masked)
-        const uint32_t batch_min = s->block ? kBlockBatchMin : (uint32_t)kPrefillMin, batch_max = s->block ? kBlockBatch : kPrefillChunk;
-        if (n >= batch_min && (!s->trace || s->block) && ensure_prompt_copy(s->model)) {
-            for (uint32_t i = 0; i < n; i += batch_max) {
-                const uint32_t m = n - i < batch_max ? n - i : batch_max;
-                LV_TRY(record_prefill(s, i, m, i + m == n, row_base));
-            }
-        } else {
-            for (uint32_t i = 0; i < n; i++) {
-                LV_TRY(record_token(s, i, s->all_logits || i + 1 == n));
-                if (s->all_logits)
-                    HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)(row_base + i) * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
-            }
+        for (uint32_t i = 0; i < n; i++) {
+            LV_TRY(embed_token(s, pos, i, tokens[i]));
+            LV_TRY(record_token(s, i, s->all_logits || i + 1 == n));
+            if (s->all_logits)
+                HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)(row_base + i) * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
         }
     }
     if (s->block) block_session_advance(s->block, pos + n);

@@ -209,7 +209,7 @@ __device__ __forceinline__ void top_experts(float *zs, uint32_t n, uint32_t top,
     // Nothing is in front of anything where there is a NaN: the rounds settle those.
     if (n <= 64) {
         const float mine = lane < n ? zs[lane] : -INFINITY;
-        if (!__any(mine != mine || mine == -INFINITY && lane < n)) {
+        if (!__any(mine != mine || (mine == -INFINITY && lane < n))) {
             uint32_t place = 0;
             for (uint32_t e = 0; e < n; e++) {
                 const float z = zs[e];

@@ -1059,10 +1059,9 @@ private:
     const NormSite *from_ = nullptr;
 };
 
-static int embed(BlockSession *s, float *x, const uint32_t *cfg, uint32_t idx, uint32_t n)
+static int embed(BlockSession *s, EmbedArgs e, float *x, uint32_t *cfg, uint32_t idx, uint32_t n)
 {
     const BlockModel *m = s->m;
-    EmbedArgs e{};
     e.x = x; e.table = m->embed; e.ld = m->embed_ld; e.dim = m->hp.dim; e.dp = m->dp; e.streams = m->copies; e.scale = m->hp.embed_scale ? m->hp.embed_scale : 1.f;
     e.cfg = cfg; e.idx = idx; e.bigram = m->bigram; e.buckets = m->hp.bigram_buckets; e.prev = m->hp.bigram_prev; e.cur = m->hp.bigram_cur; e.last = s->last;
     if (n == 1) {
@@ -1073,6 +1072,15 @@ static int embed(BlockSession *s, float *x, const uint32_t *cfg, uint32_t idx, u
     embed_bf16_kernel<<<dim3((std::max(m->dp / 4, e.n_freq) + 255) / 256, n), dim3(256), 0, s->st>>>(e);
     HIP_TRY(hipGetLastError());
     return LV_OK;
+}
+
+int block_embed_token(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx, uint32_t token)
+{
+    EmbedArgs e{};
+    e.one = true;
+    e.token = token;
+    e.pos = pos;
+    return embed(s, e, s->xa, cfg, idx, 1);
 }
 
 // copies the residual of rows `row` .. row + n - 1 of a step (the sum of its streams) to the trace
@@ -1189,7 +1197,6 @@ int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *
     const BlockModel *m = s->m;
     hipStream_t st = s->st;
     const uint32_t D = m->hp.dim, Dp = m->dp;
-    LV_TRY(embed(s, s->xa, cfg, idx, 1));
     TokenResidual res(m, s->xa, s->xb);
     auto keep = [&](uint32_t pass, int which) { return trace_residual(m, st, trace, pass, which, idx, 1, res.cur); };
     auto keep_end = [&](uint32_t pass) -> int {      // the residual behind a pass
@@ -1514,7 +1521,7 @@ template <class T> static int batch_ssm(BlockSession *s, size_t i, uint32_t pos,
 }
 
 template <class T>
-static int step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_all, const BlockTrace *trace)
+static int step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_all, const BlockTrace *trace)
 {
     constexpr bool f32 = sizeof(T) == 4;
     const BlockModel *m = s->m;
@@ -1522,7 +1529,7 @@ static int step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32
     const uint32_t Dp = m->dp;
     LV_TRY(workspace_reserve(s, n));
     Workspace &w = s->ws;
-    LV_TRY(embed(s, w.x, cfg, idx0, n));
+    LV_TRY(embed(s, EmbedArgs{}, w.x, cfg, idx0, n));
     if (m->bigram && n > 1) HIP_TRY(hipMemcpyAsync(s->last + ((pos + n - 1) & 1), cfg + idx0 + n, 4, hipMemcpyDeviceToDevice, st));
     const NormSite *from = nullptr;    // of the sublayer whose output waits to be added to the residual
     uint32_t parts = 0;                // vectors per token in w.y that make it up
@@ -1653,7 +1660,7 @@ static int step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32
     return LV_OK;
 }
 
-int block_step_batch(BlockSession *s, const uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_all, const BlockTrace *trace)
+int block_step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_all, const BlockTrace *trace)
 {
     return s->m->f32 ? step_batch<float>(s, cfg, pos, idx0, n, logits_last, logits_all, trace)
                      : step_batch<uint16_t>(s, cfg, pos, idx0, n, logits_last, logits_all, trace);

@@ -15,8 +15,12 @@ struct EmbedArgs {
     const uint16_t *table;       // rows of `ld` elements
     uint32_t ld, dim, dp, streams;
     float scale;
-    const uint32_t *cfg;         // position of the step's first token, then the step's tokens
+    uint32_t *cfg;               // position of the step's first token, then the step's tokens
     uint32_t idx;                // the launch's first token in the step
+    // one token comes in the arguments, with the step's position, which the launch leaves in cfg[0] for the kernels behind it (copying
+    // both to the device first was a launch of its own, 5 us of a step)
+    bool one;
+    uint32_t token, pos;
     const uint16_t *bigram;      // [buckets + 1][dim]; null: none
     uint32_t buckets, prev, cur;
     uint32_t *last;              // a sequence's last token, at [position % 2]
@@ -33,11 +37,13 @@ __device__ __forceinline__ void quad(float (&f)[4], const uint16_t *p)
 // a thread takes four elements
 static __global__ __launch_bounds__(256) void embed_bf16_kernel(EmbedArgs a)
 {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x, z = blockIdx.y, at = a.idx + z, pos = a.cfg[0] + at, token = a.cfg[1 + at];
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, z = blockIdx.y, at = a.idx + z;
+    const uint32_t pos = (a.one ? a.pos : a.cfg[0]) + at, token = a.one ? a.token : a.cfg[1 + at];
+    if (a.one && i == 0) a.cfg[0] = a.pos;
     const uint16_t *row = a.bigram;
     if (a.bigram) {
         uint32_t r = a.buckets;
-        if (pos) r = (uint32_t)(((uint64_t)(at ? a.cfg[at] : a.last[(pos - 1) & 1]) * a.prev + (uint64_t)token * a.cur) % a.buckets);
+        if (pos) r = (uint32_t)(((uint64_t)(at && !a.one ? a.cfg[at] : a.last[(pos - 1) & 1]) * a.prev + (uint64_t)token * a.cur) % a.buckets);
         row += (size_t)r * a.dim;
         // a launch of one token leaves it for the next; one of several is followed by a copy, since its first row may read the slot
         if (gridDim.y == 1 && i == 0) a.last[pos & 1] = token;

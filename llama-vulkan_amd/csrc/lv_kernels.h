@@ -320,22 +320,39 @@ __global__ void kv_append2_kernel(uint16_t *__restrict__ kcache, uint16_t *__res
 // ---------------------------------------------------------------------------------------------------------
 // Embedding gather (llava_session.cpp:219-223 does this on the host): x[z] = dequant(table[token[z]]).
 // ---------------------------------------------------------------------------------------------------------
-__global__ void embed_f32_kernel(float *__restrict__ x, const float *__restrict__ table, const uint32_t *tokens,
-                                 uint32_t dim)
+// Token ids of an embedding launch: of a batch in device memory; of a few tokens in the arguments, with the step's position, which the
+// launch leaves in cfg[0] for the kernels behind it.  Copying them to the device first was a launch of its own, 5 us of a step.
+constexpr uint32_t kIdsInArgs = 64;
+struct TokenIds {
+    const uint32_t *batch;   // null: in the arguments
+    uint32_t pos;
+    uint32_t *cfg;
+    uint32_t id[kIdsInArgs];
+};
+__device__ __forceinline__ uint32_t token_id(const TokenIds &t, uint32_t z, uint32_t i)
+{
+    if (t.batch) return t.batch[z];
+    if (i == 0 && z == 0) t.cfg[0] = t.pos;
+    return t.id[z];
+}
+
+__global__ void embed_f32_kernel(float *__restrict__ x, const float *__restrict__ table, TokenIds ids, uint32_t dim)
 {
     const uint32_t z = blockIdx.y;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < dim) x[(size_t)z * dim + i] = table[(size_t)tokens[z] * dim + i];
+    const uint32_t token = token_id(ids, z, i);
+    if (i < dim) x[(size_t)z * dim + i] = table[(size_t)token * dim + i];
 }
 
 template <int QT>
-__global__ void embed_quant_kernel(float *__restrict__ x, MatView table, const uint32_t *tokens)
+__global__ void embed_quant_kernel(float *__restrict__ x, MatView table, TokenIds ids)
 {
     const uint32_t z = blockIdx.y;
     const uint32_t nb = table.cols / 32;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;  // block within the row
+    const uint32_t token = token_id(ids, z, i);
     if (i >= nb) return;
-    const uint64_t b = (uint64_t)tokens[z] * nb + i;
+    const uint64_t b = (uint64_t)token * nb + i;
     const float d = mat_scale(table, b);
     float *dst = x + (size_t)z * table.cols + (size_t)i * 32;
     if constexpr (QT == 4) {
