@@ -25,6 +25,14 @@ __device__ __forceinline__ uint4 load_once(const uint16_t *p)
     const u4v v = __builtin_nontemporal_load(reinterpret_cast<const u4v *>(p));
     return make_uint4(v.x, v.y, v.z, v.w);
 }
+// the same 16 bytes of a weight row of `bytes` bytes, zero behind its end: a load that is always issued, whatever there is to load.
+// The compiler can count such loads, and a wait for one issued before them does not wait for them as well.
+__device__ __forceinline__ uint4 load_row(const uint16_t *row, uint32_t bytes, uint32_t at)
+{
+    constexpr int kRaw = 0x00027000, kNonTemporal = 2;
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(row), 0, (int)bytes, kRaw), (int)at, 0, kNonTemporal);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
 
 enum BfInput { kInNorm = 0, kInPlain = 1, kInBranch = 2, kInGroups = 3, kInStreams2 = 4, kInStreams4 = 5, kInStreams8 = 6 };
 enum BfGemvMode { kGemvRows = 0, kGemvExperts = 1, kGemvDown = 2, kGemvGlu = 3 };
@@ -123,6 +131,102 @@ __device__ __forceinline__ void norm_input(const NormInput &a, float *xs, float 
     }
 }
 
+// Loads come back in the order in which they are issued, so what an input needs is asked for before a wave fills its weight queue: the
+// input is then ready while the weights are on their way, not behind them.  The early part of an input, in registers: EARLY quads of a
+// thread; what lies behind them is loaded late.  Us of a launch without and with it: 4096 columns of two mixers to 2048 rows 9.5 and
+// 6.6, four experts of 1024 x 2048 gate and up rows 11.3 and 9.9, norm and 32000 x 2048 28.2 and 25.6.  Streams stay late: their 14 quads
+// leave room for one workgroup a CU instead of two (18560 x 4096 37.8 and 42.8).
+template <int EARLY>
+struct EarlyNorm {
+    float4 x[EARLY], y[EARLY], wpost[EARLY], wpre[EARLY];
+
+    __device__ __forceinline__ void load(const NormInput &a)
+    {
+#pragma unroll
+        for (int j = 0; j < EARLY; j++) {
+            if (j * blockDim.x * 4 >= a.dp) break;
+            const uint32_t i = min((threadIdx.x + j * blockDim.x) * 4, a.dp - 4);
+            if (a.y) y[j] = *reinterpret_cast<const float4 *>(a.y + i);
+            x[j] = *reinterpret_cast<const float4 *>(a.x + i);
+            wpost[j] = a.y && a.wpost ? *reinterpret_cast<const float4 *>(a.wpost + i) : make_float4(1.f, 1.f, 1.f, 1.f);
+            wpre[j] = *reinterpret_cast<const float4 *>(a.wpre + i);
+        }
+    }
+    // norm_input with its sums in its order; several pending vectors (behind a batch) are left to it
+    __device__ __forceinline__ void finish(const NormInput &a, float *xs, float *scratch)
+    {
+        if (a.y && a.parts > 1) {
+            norm_input(a, xs, scratch);
+            return;
+        }
+        const uint32_t dp = a.dp, step = blockDim.x * 4, late = EARLY * step + threadIdx.x * 4;
+        const int nw = blockDim.x >> 6;
+        const bool lead = blockIdx.x == 0;
+        auto square = [](const float4 &v, float s) { return fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, fmaf(v.x, v.x, s)))); };
+        float ypost = 1.f;
+        if (a.y && a.wpost) {
+            float s = 0.f;
+#pragma unroll
+            for (int j = 0; j < EARLY; j++)
+                if (threadIdx.x * 4 + j * step < dp) s = square(y[j], s);
+            for (uint32_t i = late; i < dp; i += step) s = square(*reinterpret_cast<const float4 *>(a.y + i), s);
+            ypost = rsqrtf(block_sum_waves(s, scratch, nw) / (float)a.dim + a.eps);
+        }
+        float s = 0.f;
+        auto add = [&](float4 &v, const float4 &y, const float4 &w) {
+            v.x += y.x * ypost * w.x; v.y += y.y * ypost * w.y; v.z += y.z * ypost * w.z; v.w += y.w * ypost * w.w;
+        };
+#pragma unroll
+        for (int j = 0; j < EARLY; j++) {
+            const uint32_t i = threadIdx.x * 4 + j * step;
+            if (i >= dp) break;
+            if (a.y) add(x[j], y[j], wpost[j]);
+            s = square(x[j], s);
+            if (lead && a.x_out) *reinterpret_cast<float4 *>(a.x_out + i) = x[j];
+        }
+        for (uint32_t i = late; i < dp; i += step) {
+            float4 v = *reinterpret_cast<const float4 *>(a.x + i);
+            if (a.y) add(v, *reinterpret_cast<const float4 *>(a.y + i), a.wpost ? *reinterpret_cast<const float4 *>(a.wpost + i) : make_float4(1.f, 1.f, 1.f, 1.f));
+            s = square(v, s);
+            if (lead && a.x_out) *reinterpret_cast<float4 *>(a.x_out + i) = v;
+            *reinterpret_cast<float4 *>(xs + bf_xs(i, dp)) = v;
+        }
+        const float inv = rsqrtf(block_sum_waves(s, scratch, nw) / (float)a.dim + a.eps);
+        auto put = [&](uint32_t i, float4 v, const float4 &w) {
+            v.x *= inv * w.x; v.y *= inv * w.y; v.z *= inv * w.z; v.w *= inv * w.w;
+            *reinterpret_cast<float4 *>(xs + bf_xs(i, dp)) = v;
+            if (lead && a.h_out) *reinterpret_cast<float4 *>(a.h_out + i) = v;
+        };
+#pragma unroll
+        for (int j = 0; j < EARLY; j++)
+            if (threadIdx.x * 4 + j * step < dp) put(threadIdx.x * 4 + j * step, x[j], wpre[j]);
+        for (uint32_t i = late; i < dp; i += step) put(i, *reinterpret_cast<const float4 *>(xs + bf_xs(i, dp)), *reinterpret_cast<const float4 *>(a.wpre + i));
+    }
+};
+
+// a vector in memory, `segs` of kp elements one behind the other
+template <int EARLY>
+struct EarlyPlain {
+    lv_f4 x[EARLY];
+
+    __device__ __forceinline__ void load(const float *src, uint32_t n)
+    {
+#pragma unroll
+        for (int j = 0; j < EARLY; j++)
+            x[j] = j * kBfGemvThreads * 4u < n ? *reinterpret_cast<const lv_f4 *>(src + min((threadIdx.x + j * kBfGemvThreads) * 4, n - 4)) : lv_f4{};
+    }
+    __device__ __forceinline__ void finish(const float *src, uint32_t n, uint32_t kp, float *xs)
+    {
+        auto put = [&](uint32_t i, const lv_f4 v) { *reinterpret_cast<lv_f4 *>(xs + i / kp * kp + bf_xs(i % kp, kp)) = v; };
+#pragma unroll
+        for (int j = 0; j < EARLY; j++) {
+            const uint32_t i = (threadIdx.x + j * blockDim.x) * 4;
+            if (i < n) put(i, x[j]);
+        }
+        for (uint32_t i = (threadIdx.x + EARLY * blockDim.x) * 4; i < n; i += blockDim.x * 4) put(i, *reinterpret_cast<const lv_f4 *>(src + i));
+    }
+};
+
 // one recurrent head's read-out: divided by its root mean square, weighted, gated, scaled.  A wave per head; put(c, value).
 template <class Put>
 __device__ __forceinline__ void gated_head(const float *o, const float *gate, const float *w, uint32_t vdim, float eps, float scale, Put put)
@@ -134,34 +238,101 @@ __device__ __forceinline__ void gated_head(const float *o, const float *gate, co
     for (uint32_t c = lane; c < vdim; c += 64) put(c, o[c] * inv * w[c] * gate[c] * scale);
 }
 
-__device__ __forceinline__ void branch_input(const BranchInput &a, float *xs, uint32_t kp)
-{
-    for (uint32_t i = threadIdx.x; i < a.left_kp; i += blockDim.x) xs[bf_xs(i, kp)] = i < a.left_n ? a.left[i] * a.left_scale : 0.f;
-    for (uint32_t i = a.left_kp + a.heads * a.vdim + threadIdx.x; i < kp; i += blockDim.x) xs[bf_xs(i, kp)] = 0.f;
-    const uint32_t nw = blockDim.x >> 6;
-    for (uint32_t h = threadIdx.x >> 6; h < a.heads; h += nw) {
-        const uint32_t base = h * a.vdim;
-        gated_head(a.o + base, a.gate + base, a.onorm, a.vdim, a.eps, a.right_scale,
-                   [&](uint32_t c, float v) { xs[bf_xs(a.left_kp + base + c, kp)] = v; });
+// the concatenation; in registers early: eight of a thread's attention outputs, and of up to four heads of a wave up to 128 columns
+struct EarlyBranch {
+    static constexpr int kLeft = 8, kHeads = 4, kCols = 2;
+    float left[kLeft], o[kHeads][kCols], gate[kHeads][kCols], w[kCols];
+
+    __device__ __forceinline__ void load(const BranchInput &a)
+    {
+        if (a.left_n) {
+#pragma unroll
+            for (int j = 0; j < kLeft; j++)
+                if (j * blockDim.x < a.left_n) left[j] = a.left[min(threadIdx.x + j * blockDim.x, a.left_n - 1)];
+        }
+        if (!a.heads) return;
+#pragma unroll
+        for (int c = 0; c < kCols; c++) {
+            const uint32_t col = min((threadIdx.x & 63) + c * 64, a.vdim - 1);
+            w[c] = a.onorm[col];
+#pragma unroll
+            for (int h = 0; h < kHeads; h++) {
+                if (h * (blockDim.x >> 6) >= a.heads) break;
+                const uint32_t at = min((threadIdx.x + h * blockDim.x) >> 6, a.heads - 1) * a.vdim + col;
+                o[h][c] = a.o[at];
+                gate[h][c] = a.gate[at];
+            }
+        }
     }
-}
+    __device__ __forceinline__ void finish(const BranchInput &a, float *xs, uint32_t kp)
+    {
+#pragma unroll
+        for (int j = 0; j < kLeft; j++) {
+            const uint32_t i = threadIdx.x + j * blockDim.x;
+            if (i < a.left_kp) xs[bf_xs(i, kp)] = i < a.left_n ? left[j] * a.left_scale : 0.f;
+        }
+        for (uint32_t i = threadIdx.x + kLeft * blockDim.x; i < a.left_kp; i += blockDim.x) xs[bf_xs(i, kp)] = i < a.left_n ? a.left[i] * a.left_scale : 0.f;
+        for (uint32_t i = a.left_kp + a.heads * a.vdim + threadIdx.x; i < kp; i += blockDim.x) xs[bf_xs(i, kp)] = 0.f;
+        const uint32_t nw = blockDim.x >> 6, lane = threadIdx.x & 63;
+        uint32_t h = threadIdx.x >> 6;
+        if (a.vdim <= kCols * 64) {
+#pragma unroll
+            for (int j = 0; j < kHeads; j++, h += nw) {
+                if (h >= a.heads) break;
+                float s = 0.f;
+#pragma unroll
+                for (int c = 0; c < kCols; c++)
+                    if (lane + c * 64 < a.vdim) s = fmaf(o[j][c], o[j][c], s);
+                const float inv = rsqrtf(wave_sum(s) / (float)a.vdim + a.eps);
+#pragma unroll
+                for (int c = 0; c < kCols; c++)
+                    if (lane + c * 64 < a.vdim) xs[bf_xs(a.left_kp + h * a.vdim + lane + c * 64, kp)] = o[j][c] * inv * w[c] * gate[j][c] * a.right_scale;
+            }
+        }
+        for (; h < a.heads; h += nw) {
+            const uint32_t base = h * a.vdim;
+            gated_head(a.o + base, a.gate + base, a.onorm, a.vdim, a.eps, a.right_scale,
+                       [&](uint32_t c, float v) { xs[bf_xs(a.left_kp + base + c, kp)] = v; });
+        }
+    }
+};
 
 // GroupInput: put(i, value) for one element or, where parts are multiples of four, a float4 of them; get(i, value) the other way.
 // Waves share a group where there are fewer groups than waves; `sums` holds group_sums() floats and every thread keeps to its own
 // elements between the passes.
 __host__ __device__ constexpr uint32_t group_parts(uint32_t groups, uint32_t waves) { return groups >= waves ? 1 : waves / groups; }
 __host__ __device__ constexpr uint32_t group_sums(uint32_t groups, uint32_t waves) { return groups * group_parts(groups, waves); }
-template <class V, class Put, class Get>
-__device__ __forceinline__ void group_passes(const GroupInput &a, float *sums, Put put, Get get)
+// In registers early: four quads of each of a wave's first task, where parts are multiples of four.
+template <int EARLY>
+struct EarlyGroups {
+    float4 o[EARLY], z[EARLY];
+
+    __device__ __forceinline__ void load(const GroupInput &a)
+    {
+        const uint32_t waves = blockDim.x >> 6, parts = group_parts(a.groups, waves), size = a.n / a.groups, k = threadIdx.x >> 6;
+        if (size % 4 || k >= a.groups * parts) return;
+#pragma unroll
+        for (int j = 0; j < EARLY; j++) {
+            if (j * parts * 256 >= size) break;
+            const uint32_t i = k / parts * size + min((k % parts * 64 + (threadIdx.x & 63) + j * parts * 64) * 4, size - 4);
+            o[j] = *reinterpret_cast<const float4 *>(a.o + i);
+            z[j] = *reinterpret_cast<const float4 *>(a.z + i);
+        }
+    }
+};
+template <>
+struct EarlyGroups<0> {
+    float4 *o, *z;
+};
+template <class V, int EARLY, class Put, class Get>
+__device__ __forceinline__ void group_passes(const GroupInput &a, float *sums, const EarlyGroups<EARLY> &early, Put put, Get get)
 {
     constexpr uint32_t N = sizeof(V) / 4;
     const uint32_t lane = threadIdx.x & 63, waves = blockDim.x >> 6, parts = group_parts(a.groups, waves), tasks = a.groups * parts, size = a.n / a.groups;
     for (uint32_t k = threadIdx.x >> 6; k < tasks; k += waves) {
         const uint32_t base = k / parts * size;
         float s = 0.f;
-        for (uint32_t c = (k % parts * 64 + lane) * N; c < size; c += parts * 64 * N) {
-            V v = *reinterpret_cast<const V *>(a.o + base + c);
-            const V z = *reinterpret_cast<const V *>(a.z + base + c);
+        auto gate = [&](uint32_t i, V v, const V z) {
             float *f = reinterpret_cast<float *>(&v);
             const float *g = reinterpret_cast<const float *>(&z);
 #pragma unroll
@@ -169,8 +340,19 @@ __device__ __forceinline__ void group_passes(const GroupInput &a, float *sums, P
                 f[e] *= silu_f(g[e]);
                 s = fmaf(f[e], f[e], s);
             }
-            put(base + c, v);
+            put(i, v);
+        };
+        uint32_t c = (k % parts * 64 + lane) * N;
+        if constexpr (EARLY > 0 && N == 4) {
+            if (k < waves) {
+#pragma unroll
+                for (int j = 0; j < EARLY; j++, c += parts * 64 * N) {
+                    if (c >= size) break;
+                    gate(base + c, early.o[j], early.z[j]);
+                }
+            }
         }
+        for (; c < size; c += parts * 64 * N) gate(base + c, *reinterpret_cast<const V *>(a.o + base + c), *reinterpret_cast<const V *>(a.z + base + c));
         s = wave_sum(s);
         if (lane == 0) sums[k] = s;
     }
@@ -192,11 +374,11 @@ __device__ __forceinline__ void group_passes(const GroupInput &a, float *sums, P
         }
     }
 }
-template <class Put, class Get>
-__device__ __forceinline__ void group_input(const GroupInput &a, float *sums, Put put, Get get)
+template <int EARLY, class Put, class Get>
+__device__ __forceinline__ void group_input(const GroupInput &a, float *sums, const EarlyGroups<EARLY> &early, Put put, Get get)
 {
-    if (a.n / a.groups % 4 == 0) group_passes<float4>(a, sums, put, get);
-    else group_passes<float>(a, sums, put, get);
+    if (a.n / a.groups % 4 == 0) group_passes<float4>(a, sums, early, put, get);
+    else group_passes<float>(a, sums, early, put, get);
 }
 
 // The `top` largest of n router logits, largest first, the lower index on equal values (one wave; zs is consumed).  Scores are
@@ -267,6 +449,14 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
     const uint32_t tasks = (units + R - 1) / R, nwaves = gridDim.x * kBfGemvWaves;
     const uint32_t first_task = blockIdx.x * kBfGemvWaves + wave;
 
+    EarlyNorm<2> norm;
+    EarlyPlain<6> plain;
+    EarlyBranch branch;
+    EarlyGroups<4> group;
+    if constexpr (INPUT == kInNorm) norm.load(a.norm);
+    if constexpr (INPUT == kInBranch) branch.load(a.branch);
+    if constexpr (INPUT == kInGroups) group.load(a.group);
+    if constexpr (INPUT == kInPlain) plain.load(a.x, kp * segs);
     if constexpr (MODE == kGemvDown) {
         if (threadIdx.x < a.top) sel_id[threadIdx.x] = a.ids[threadIdx.x];
         __syncthreads();
@@ -288,28 +478,28 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
     // (4096 x 11008: 20.0 us from column 0, 18.3 so; 13600 x 4096 22.9 and 22.0).  Not where equal rows have to give equal
     // results to the last bit, since a choice between them hangs on it: router and head.
     const uint32_t turn = a.same_order ? 0 : first_task % ksteps;
+    const uint32_t chosen = MODE == kGemvExperts || MODE == kGemvDown ? sel_id[lane < (int)a.top ? lane : 0] : 0;      // expert `lane`
+    auto row_of = [&](uint32_t task, uint32_t seg) -> const uint16_t * {
+        if (task >= tasks) return a.w;
+        if constexpr (MODE == kGemvExperts) {
+            const uint32_t u = task * R, per = kp_units(a), x = u / per, f = u - x * per;
+            return a.w + ((size_t)(uint32_t)__builtin_amdgcn_readlane((int)chosen, (int)x) * a.expert_rows + (f >> 4) * 32 + (f & 15)) * kp;
+        } else if constexpr (MODE == kGemvGlu) {
+            const uint32_t f = task * R;
+            return a.w + ((size_t)(f >> 4) * 32 + (f & 15)) * kp;
+        } else if constexpr (MODE == kGemvDown) {
+            return a.w + ((size_t)task * R + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)chosen, (int)seg) * a.expert_rows) * kp;
+        } else {
+            return a.w + (size_t)task * R * kp;
+        }
+    };
     uint4 q[DEPTH][NR];
     uint32_t ftask = first_task, fit = 0, fk = turn, fseg = 0;
+    const uint16_t *frow = row_of(ftask, 0);
     auto fetch = [&](uint4 (&slot)[NR]) {
-        const uint32_t kk = fk * 512 + lane * 8;
-        const bool ok = ftask < tasks && kk < kp;
-        const uint16_t *p = a.w + kk;
-        if constexpr (MODE == kGemvExperts) {
-            const uint32_t u = ftask * R, per = kp_units(a);
-            const uint32_t s = ok ? u / per : 0, f = ok ? u % per : 0;
-            p += ((size_t)sel_id[s] * a.expert_rows + (f >> 4) * 32 + (f & 15)) * kp;
-        } else if constexpr (MODE == kGemvGlu) {
-            const uint32_t f = ftask * R;
-            p += ((size_t)(f >> 4) * 32 + (f & 15)) * kp;
-        } else {
-            p += (size_t)ftask * R * kp;
-            if constexpr (MODE == kGemvDown) p += (size_t)sel_id[fseg] * a.expert_rows * kp;
-        }
+        const uint32_t bytes = ftask < tasks ? kp * 2 : 0;
 #pragma unroll
-        for (int r = 0; r < NR; r++) {
-            const size_t off = PAIRS ? (size_t)(r % R + (r / R) * 16) * kp : (size_t)r * kp;
-            slot[r] = ok ? load_once(p + off) : make_uint4(0, 0, 0, 0);
-        }
+        for (int r = 0; r < NR; r++) slot[r] = load_row(frow + (PAIRS ? (size_t)(r % R + (r / R) * 16) * kp : (size_t)r * kp), bytes, fk * 1024 + lane * 16);
         if (++fk == ksteps) fk = 0;
         if (++fit == ksteps) {
             fit = 0;
@@ -317,27 +507,25 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
                 fseg = 0;
                 ftask += nwaves;
             }
+            frow = row_of(ftask, fseg);
         }
     };
 #pragma unroll
     for (int d = 0; d < DEPTH; d++) fetch(q[d]);
 
     if constexpr (INPUT == kInNorm) {
-        norm_input(a.norm, xs, scratch);
+        norm.finish(a.norm, xs, scratch);
     } else if constexpr (INPUT == kInBranch) {
-        branch_input(a.branch, xs, kp);
+        branch.finish(a.branch, xs, kp);
     } else if constexpr (INPUT == kInGroups) {
         for (uint32_t i = a.group.n + threadIdx.x; i < kp; i += kBfGemvThreads) xs[bf_xs(i, kp)] = 0.f;
-        group_input(a.group, xs + kp, [&](uint32_t i, auto v) { *reinterpret_cast<decltype(v) *>(xs + bf_xs(i, kp)) = v; },
+        group_input(a.group, xs + kp, group, [&](uint32_t i, auto v) { *reinterpret_cast<decltype(v) *>(xs + bf_xs(i, kp)) = v; },
                     [&](uint32_t i, auto &v) { v = *reinterpret_cast<std::decay_t<decltype(v)> *>(xs + bf_xs(i, kp)); });
     } else if constexpr (INPUT >= kInStreams2) {
         stream_input<2 << (INPUT - kInStreams2)>(a.streams, blockIdx.x == 0, scratch, [&](uint32_t i, const float4 h) { *reinterpret_cast<float4 *>(xs + bf_xs(i, kp)) = h; },
                                                  [&](uint32_t i) { return *reinterpret_cast<const float4 *>(xs + bf_xs(i, kp)); });
     } else {
-        for (uint32_t i = threadIdx.x * 4; i < kp * segs; i += kBfGemvThreads * 4) {
-            const uint32_t sg = i / kp, k = i % kp;
-            *reinterpret_cast<float4 *>(xs + sg * kp + bf_xs(k, kp)) = *reinterpret_cast<const float4 *>(a.x + i);
-        }
+        plain.finish(a.x, kp * segs, kp, xs);
     }
     __syncthreads();
 

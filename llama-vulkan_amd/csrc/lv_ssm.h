@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256) void ssm_gate_kernel(GroupInput g, uint32_t ld
     const size_t row = blockIdx.x;
     g.o += row * g.n;
     g.z += row * ldz;
-    group_input(g, gs + g.n, [&](uint32_t i, auto v) { *reinterpret_cast<decltype(v) *>(gs + i) = v; },
+    group_input(g, gs + g.n, EarlyGroups<0>{}, [&](uint32_t i, auto v) { *reinterpret_cast<decltype(v) *>(gs + i) = v; },
                 [&](uint32_t i, auto &v) { v = *reinterpret_cast<std::decay_t<decltype(v)> *>(gs + i); });
     __syncthreads();
     T *out = act + row * ld;          // ld is a multiple of 64; gs is readable to the next multiple of four

@@ -2,13 +2,17 @@
 sides of 64 experts, where the choice of a token takes another form.
 
 Small integers as embeddings, norm weights of one and router rows that come in equal pairs: an odd number of experts a token cuts a
-pair.  The plain evaluation chooses by the same rule (choose_experts); a wrong pick is an error of order one."""
+pair.  The plain evaluation chooses by the same rule (choose_experts); a wrong pick is an error of order one.
+
+And the inputs of one-token products, on both sides of the sizes up to which they are held in registers."""
 import numpy as np
 import pytest
 
 import block_builder as bb
 import block_device
 import block_oracle as bo
+import zedenex_builder as zb
+import zedenex_oracle as zo
 from block_device import rel, tokens_for
 
 pytestmark = pytest.mark.gpu
@@ -34,3 +38,36 @@ def test_equal_experts_tie(lva, ctx, experts, top, width):
     with block_device.Device(lva, bb.upload(ctx, cfg, W, lva.LV_F32), 512) as d:
         for c in ((1000,), (1,), (16, 3)):
             assert rel(d.run(toks, c), want) < 2e-4, c
+
+
+# What a one-token product's input is made of is held in registers up to a size, and read late behind it: on both sides of the 4096
+# columns of a norm, 4096 attention outputs, 32 recurrent heads of 128 columns, and experts' down projections of 12288 columns together
+WIDE = [
+    (4160, dict(left=bb.attn(heads=2, kv_heads=1, dim=16)), dict(experts=3, top=2, ff=40)),
+    (2112, dict(left=bb.attn(heads=33, kv_heads=3, dim=128, chunk=0)), dict(experts=5, top=4, ff=1100)),
+    (48, dict(right=bb.delta(heads=34, kv_heads=17, dim=12, vdim=128)), dict(experts=2, top=1, ff=1030)),
+    (72, dict(right=bb.delta(heads=36, kv_heads=4, dim=12, vdim=20)), dict(experts=7, top=6, ff=2060)),
+    (64, dict(right=bb.delta(heads=3, kv_heads=3, dim=8, vdim=130)), dict(experts=0)),
+]
+
+
+@pytest.mark.parametrize("width,mix,ff", WIDE)
+def test_inputs_beyond_the_early_part(lva, ctx, width, mix, ff):
+    cfg = bb.config(width=width, layers=[bb.layer(**mix, **ff)])
+    W = bb.weights(cfg, seed=width)
+    toks = tokens_for(cfg, 20, 1)
+    want = bo.forward(toks, bb.as_float(W), cfg)[0]
+    with block_device.Device(lva, bb.upload(ctx, cfg, W, lva.LV_F32), 512) as d:
+        assert rel(d.run(toks, (1,)), want) < 2e-4
+
+
+# a read-out normed in parts: a wave's first task in registers (four quads a lane), the rest of it and further tasks late; parts that are no
+# multiple of four
+@pytest.mark.parametrize("heads,vdim,groups", [(64, 130, 1), (40, 130, 2), (40, 130, 8), (36, 64, 9), (24, 96, 36), (6, 7, 2)])
+def test_grouped_input(lva, ctx, heads, vdim, groups):
+    cfg = zb.config(width=52, streams=2, layers=[zb.layer(zb.ssm(heads=heads, groups=2, state=16, vdim=vdim, norm_groups=groups), 0)])
+    W = zb.weights(cfg, seed=heads + groups)
+    toks = tokens_for(cfg, 20, 1)
+    want = zo.forward(toks, bb.as_float(W), cfg)[0]
+    with block_device.Device(lva, zb.upload(ctx, cfg, W, lva.LV_F32), 512) as d:
+        assert rel(d.run(toks, (1,)), want) < 2e-4

@@ -29,6 +29,13 @@ def dense_model(toks, W, cfg, r):
     return r(zo.norm(x.sum(0), W, "final.norm", cfg["norm"]["eps"])) @ W["embed"].T
 
 
+def check_last(d, toks, want, tol):
+    """the last token's logits alone: it takes in the pending slices or experts in front of the head, on another path than all rows"""
+    d.sess.keep_all_logits(False)
+    d.sess.begin(toks, 0)
+    assert rel(d.sess.logits()[None], want[-1:]) < tol * max(1.0, np.sqrt(np.mean(want ** 2) / np.mean(want[-1] ** 2)))
+
+
 # width, feed-forward, tokens.  Columns (64 a K step): 1, 3, 11 and more steps in front of the pipelines' two and three stages; rows and
 # tokens one beside a tile's edge; feed-forwards whose way down is cut into 2, 3 and 4 slices, the last one shorter
 DENSE = [(40, 4100, 1100), (130, 2060, 1030), (700, 2060, 1025), (700, 4100, 1281), (300, 1100, 129), (300, 2113, 127), (257, 4160, 257),
@@ -46,12 +53,10 @@ def test_dense_tiles(lva, ctx, width, ff, n):
     assert tol < 2e-2
     with Device(lva, zb.upload(ctx, cfg, W, BF16), 2048) as d:
         assert rel(d.run(toks, (n,)), want) < tol
-        d.sess.keep_all_logits(False)                     # the last token's alone: its streams take in the slices beforehand
-        d.sess.begin(toks, 0)
-        assert rel(d.sess.logits()[None], want[-1:]) < tol * max(1.0, np.sqrt(np.mean(want ** 2) / np.mean(want[-1] ** 2)))
+        check_last(d, toks, want, tol)
 
 
-@pytest.mark.parametrize("width,ff,n,experts,top", [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4)])
+@pytest.mark.parametrize("width,ff,n,experts,top", [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4), (64, 24, 17, 3, 2)])
 def test_expert_tiles(lva, ctx, width, ff, n, experts, top):
     cfg = bb.config(width=width, layers=[bb.layer(experts=experts, top=top, ff=ff)])
     W = bb.weights(cfg, seed=n)
@@ -80,3 +85,4 @@ def test_expert_tiles(lva, ctx, width, ff, n, experts, top):
     assert tol < 4e-2
     with Device(lva, bb.upload(ctx, cfg, W, BF16), 2048) as d:
         assert rel(d.run(toks, (n,)), want) < tol
+        check_last(d, toks, want, tol)
