@@ -37,8 +37,11 @@ __device__ __forceinline__ uint4 load_row(const uint16_t *row, uint32_t bytes, u
 enum BfInput { kInNorm = 0, kInPlain = 1, kInBranch = 2, kInGroups = 3, kInStreams2 = 4, kInStreams4 = 5, kInStreams8 = 6 };
 enum BfGemvMode { kGemvRows = 0, kGemvExperts = 1, kGemvDown = 2, kGemvGlu = 3 };
 
-constexpr int kBfGemvThreads = 512;
-constexpr int kBfGemvWaves = kBfGemvThreads / 64;
+// 16 waves a CU: two workgroups, or one where every workgroup reads two or four streams (112 KB of four streams, the pending output and
+// a norm of 4096 columns; with 1024 threads one quad of each, which fits the registers early beside the weight queue, two do not).  Four
+// streams, two workgroups and one: gate and up of 11008 x 4096 35.4 and 32.1 us, 3072 x 4096 11.1 and 9.9.
+constexpr int gemv_threads(int input) { return input == kInStreams2 || input == kInStreams4 ? 1024 : 512; }
+constexpr int gemv_waves(int input) { return gemv_threads(input) / 64; }
 constexpr uint32_t kMaxTop = 64;          // experts a token may use
 constexpr uint32_t kMaxExperts = 4096;
 
@@ -134,8 +137,7 @@ __device__ __forceinline__ void norm_input(const NormInput &a, float *xs, float 
 // Loads come back in the order in which they are issued, so what an input needs is asked for before a wave fills its weight queue: the
 // input is then ready while the weights are on their way, not behind them.  The early part of an input, in registers: EARLY quads of a
 // thread; what lies behind them is loaded late.  Us of a launch without and with it: 4096 columns of two mixers to 2048 rows 9.5 and
-// 6.6, four experts of 1024 x 2048 gate and up rows 11.3 and 9.9, norm and 32000 x 2048 28.2 and 25.6.  Streams stay late: their 14 quads
-// leave room for one workgroup a CU instead of two (18560 x 4096 37.8 and 42.8).
+// 6.6, four experts of 1024 x 2048 gate and up rows 11.3 and 9.9, norm and 32000 x 2048 28.2 and 25.6.
 template <int EARLY>
 struct EarlyNorm {
     float4 x[EARLY], y[EARLY], wpost[EARLY], wpre[EARLY];
@@ -213,7 +215,7 @@ struct EarlyPlain {
     {
 #pragma unroll
         for (int j = 0; j < EARLY; j++)
-            x[j] = j * kBfGemvThreads * 4u < n ? *reinterpret_cast<const lv_f4 *>(src + min((threadIdx.x + j * kBfGemvThreads) * 4, n - 4)) : lv_f4{};
+            x[j] = j * blockDim.x * 4 < n ? *reinterpret_cast<const lv_f4 *>(src + min((threadIdx.x + j * blockDim.x) * 4, n - 4)) : lv_f4{};
     }
     __device__ __forceinline__ void finish(const float *src, uint32_t n, uint32_t kp, float *xs)
     {
@@ -433,12 +435,13 @@ __device__ __forceinline__ uint32_t kp_units(const BfGemvArgs &a) { return a.exp
 
 // R = rows (kGemvExperts: gate and up pairs) a wave works on at a time, DEPTH = queue slots of one 512-column step each
 template <int MODE, int INPUT, int R, int DEPTH>
-__global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
+__global__ __launch_bounds__(gemv_threads(INPUT)) void bf16_gemv_kernel(BfGemvArgs a)
 {
     constexpr bool PAIRS = MODE == kGemvExperts || MODE == kGemvGlu;      // gate and up rows
     constexpr int NR = PAIRS ? 2 * R : R;
     extern __shared__ float xs[];          // kp floats (kGemvDown: top * kp), then kGemvExperts: router logits
-    __shared__ float scratch[kBfGemvWaves];
+    constexpr uint32_t kThreads = gemv_threads(INPUT), kWaves = gemv_waves(INPUT);
+    __shared__ float scratch[kWaves];
     __shared__ uint32_t sel_id[kMaxTop];
     __shared__ float sel_score[kMaxTop];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -446,8 +449,8 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
     const uint32_t segs = MODE == kGemvDown ? a.top : 1;
     const uint32_t ksteps = (kp + 511) / 512, iters = ksteps * segs;
     const uint32_t units = MODE == kGemvExperts ? a.top * kp_units(a) : MODE == kGemvGlu ? a.rows / 2 : a.rows;
-    const uint32_t tasks = (units + R - 1) / R, nwaves = gridDim.x * kBfGemvWaves;
-    const uint32_t first_task = blockIdx.x * kBfGemvWaves + wave;
+    const uint32_t tasks = (units + R - 1) / R, nwaves = gridDim.x * kWaves;
+    const uint32_t first_task = blockIdx.x * kWaves + wave;
 
     EarlyNorm<2> norm;
     EarlyPlain<6> plain;
@@ -456,6 +459,8 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
     if constexpr (INPUT == kInNorm) norm.load(a.norm);
     if constexpr (INPUT == kInBranch) branch.load(a.branch);
     if constexpr (INPUT == kInGroups) group.load(a.group);
+    EarlyStreams<INPUT >= kInStreams2 ? 2 << (INPUT - kInStreams2) : 1> streams;
+    if constexpr (INPUT >= kInStreams2) streams.load(a.streams);
     if constexpr (INPUT == kInPlain) plain.load(a.x, kp * segs);
     if constexpr (MODE == kGemvDown) {
         if (threadIdx.x < a.top) sel_id[threadIdx.x] = a.ids[threadIdx.x];
@@ -463,7 +468,7 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
     }
     if constexpr (MODE == kGemvExperts) {
         float *zs = xs + kp;
-        for (uint32_t e = threadIdx.x; e < a.experts; e += kBfGemvThreads) zs[e] = a.z[e];
+        for (uint32_t e = threadIdx.x; e < a.experts; e += kThreads) zs[e] = a.z[e];
         __syncthreads();
         if (wave == 0) top_experts(zs, a.experts, a.top, sel_id, sel_score);
         __syncthreads();
@@ -518,12 +523,12 @@ __global__ __launch_bounds__(kBfGemvThreads) void bf16_gemv_kernel(BfGemvArgs a)
     } else if constexpr (INPUT == kInBranch) {
         branch.finish(a.branch, xs, kp);
     } else if constexpr (INPUT == kInGroups) {
-        for (uint32_t i = a.group.n + threadIdx.x; i < kp; i += kBfGemvThreads) xs[bf_xs(i, kp)] = 0.f;
+        for (uint32_t i = a.group.n + threadIdx.x; i < kp; i += kThreads) xs[bf_xs(i, kp)] = 0.f;
         group_input(a.group, xs + kp, group, [&](uint32_t i, auto v) { *reinterpret_cast<decltype(v) *>(xs + bf_xs(i, kp)) = v; },
                     [&](uint32_t i, auto &v) { v = *reinterpret_cast<std::decay_t<decltype(v)> *>(xs + bf_xs(i, kp)); });
     } else if constexpr (INPUT >= kInStreams2) {
-        stream_input<2 << (INPUT - kInStreams2)>(a.streams, blockIdx.x == 0, scratch, [&](uint32_t i, const float4 h) { *reinterpret_cast<float4 *>(xs + bf_xs(i, kp)) = h; },
-                                                 [&](uint32_t i) { return *reinterpret_cast<const float4 *>(xs + bf_xs(i, kp)); });
+        stream_input(a.streams, blockIdx.x == 0, scratch, streams, [&](uint32_t i, const float4 h) { *reinterpret_cast<float4 *>(xs + bf_xs(i, kp)) = h; },
+                     [&](uint32_t i) { return *reinterpret_cast<const float4 *>(xs + bf_xs(i, kp)); });
     } else {
         plain.finish(a.x, kp * segs, kp, xs);
     }

@@ -777,10 +777,10 @@ template <class K> static int allow_lds(K kernel, size_t bytes)
 
 template <int MODE, int INPUT, int R, int DEPTH> static int launch_gemv(hipStream_t st, const BfGemvArgs &a, uint32_t units, size_t lds)
 {
-    const uint32_t per_wg = kBfGemvWaves * R, wgs = std::min((units + per_wg - 1) / per_wg, 512u);
+    const uint32_t per_wg = gemv_waves(INPUT) * R, wgs = std::min((units + per_wg - 1) / per_wg, 512u * 512 / gemv_threads(INPUT));
     auto *k = &bf16_gemv_kernel<MODE, INPUT, R, DEPTH>;
     LV_TRY(allow_lds(k, lds));
-    k<<<dim3(wgs), dim3(kBfGemvThreads), lds, st>>>(a);
+    k<<<dim3(wgs), dim3(gemv_threads(INPUT)), lds, st>>>(a);
     HIP_TRY(hipGetLastError());
     return LV_OK;
 }
@@ -790,7 +790,7 @@ template <int MODE, int INPUT, int R, int DEPTH> static int launch_gemv(hipStrea
 // and 11.7).
 static uint32_t gemv_rows_together(uint32_t units)
 {
-    constexpr uint32_t kWaves = 512 * kBfGemvWaves;
+    constexpr uint32_t kWaves = 16 * 256;
     auto rows_in_turn = [&](uint32_t r) { return ((units + r - 1) / r + kWaves - 1) / kWaves * r; };      // of the busiest wave
     return units < 8192 || rows_in_turn(1) * 4 <= rows_in_turn(2) * 3 ? 1 : 2;
 }
@@ -798,13 +798,14 @@ static uint32_t gemv_rows_together(uint32_t units)
 template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs &a)
 {
     const size_t lds = (size_t)a.kp * (MODE == kGemvDown ? a.top : 1) * 4 + (MODE == kGemvExperts ? a.experts * 4ull : 0) +
-                       (INPUT == kInGroups ? group_sums(a.group.groups, kBfGemvWaves) * 4ull : 0);
+                       (INPUT == kInGroups ? group_sums(a.group.groups, gemv_waves(INPUT)) * 4ull : 0);
     if constexpr (MODE == kGemvExperts || MODE == kGemvGlu) {
         const uint32_t units = MODE == kGemvExperts ? a.top * (a.expert_rows / 2) : a.rows / 2;
         return gemv_rows_together(units) == 2 ? launch_gemv<MODE, INPUT, 2, 2>(st, a, units, lds) : launch_gemv<MODE, INPUT, 1, 4>(st, a, units, lds);
     } else {
+        // a workgroup of 16 waves takes one row at a time: 45.0 us with two, 39.4 with one (18560 and 32000 x 4096, four streams)
         // one row at a time: eight steps ahead, or a row of up to 2048 columns (8848 x 2048: 11.0 us with eight, 10.1 with four)
-        return gemv_rows_together(a.rows) == 2 ? launch_gemv<MODE, INPUT, 2, 4>(st, a, a.rows, lds)
+        return gemv_threads(INPUT) == 512 && gemv_rows_together(a.rows) == 2 ? launch_gemv<MODE, INPUT, 2, 4>(st, a, a.rows, lds)
                : a.kp <= 2048                  ? launch_gemv<MODE, INPUT, 1, 4>(st, a, a.rows, lds)
                                                : launch_gemv<MODE, INPUT, 1, 8>(st, a, a.rows, lds);
     }

@@ -68,12 +68,12 @@ struct StreamQuad {
     }
 };
 
-// u of all elements, four at a time: use(i, u).  The next four are on their way meanwhile.
+// u of all elements from number `first` of each thread's quads on, four at a time: use(i, u).  The next four are on their way meanwhile.
 template <int NS, class Use>
-__device__ __forceinline__ void stream_each(const StreamInput &a, bool store, Use use)
+__device__ __forceinline__ void stream_each(const StreamInput &a, bool store, Use use, uint32_t first = 0)
 {
     const uint32_t step = blockDim.x * 4;
-    uint32_t i = threadIdx.x * 4;
+    uint32_t i = threadIdx.x * 4 + first * step;
     if (i >= a.dp) return;
     StreamQuad<NS> next;
     next.load(a, i);
@@ -87,32 +87,67 @@ __device__ __forceinline__ void stream_each(const StreamInput &a, bool store, Us
     } while (i < a.dp);
 }
 
+// A thread's first quad, and the norm's weights there, in registers: asked for ahead of other loads, used behind them.  Not of eight
+// streams, which do not fit beside a weight queue.
+template <int NS>
+struct EarlyStreams {
+    static constexpr uint32_t kQuads = 1;
+    StreamQuad<NS> q;
+    float4 w, b;
+
+    __device__ __forceinline__ void load(const StreamInput &a)
+    {
+        const uint32_t i = min(threadIdx.x * 4, a.dp - 4);
+        q.load(a, i);
+        w = *reinterpret_cast<const float4 *>(a.w + i);
+        b = a.alpha ? *reinterpret_cast<const float4 *>(a.b + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+};
+
+template <>
+struct EarlyStreams<kMaxStreams> {
+    static constexpr uint32_t kQuads = 0;
+    __device__ __forceinline__ void load(const StreamInput &) {}
+};
+
 // The whole input: put(i, h) gets four elements at a time, get(i) returns what put left there.  scratch: a float per wave.
 template <int NS, class Put, class Get>
-__device__ __forceinline__ void stream_input(const StreamInput &a, bool lead, float *scratch, Put put, Get get)
+__device__ __forceinline__ void stream_input(const StreamInput &a, bool lead, float *scratch, const EarlyStreams<NS> &early, Put put, Get get)
 {
+    constexpr uint32_t kEarly = EarlyStreams<NS>::kQuads;
+    const uint32_t first = threadIdx.x * 4, step = blockDim.x * 4;
     if (a.alpha) {
         const float al = *a.alpha;
-        stream_each<NS>(a, lead, [&](uint32_t i, const float4 u) {
-            const float4 w = *reinterpret_cast<const float4 *>(a.w + i), b = *reinterpret_cast<const float4 *>(a.b + i);
+        auto use = [&](uint32_t i, const float4 u, const float4 w, const float4 b) {
             const float4 h = make_float4(fmaf(tanh_f(al * u.x), w.x, b.x), fmaf(tanh_f(al * u.y), w.y, b.y), fmaf(tanh_f(al * u.z), w.z, b.z), fmaf(tanh_f(al * u.w), w.w, b.w));
             put(i, h);
             if (lead && a.h_out) *reinterpret_cast<float4 *>(a.h_out + i) = h;
-        });
+        };
+        if constexpr (kEarly > 0) {
+            if (first < a.dp) use(first, early.q.gather(a, first, lead), early.w, early.b);
+        }
+        stream_each<NS>(a, lead, [&](uint32_t i, const float4 u) { use(i, u, *reinterpret_cast<const float4 *>(a.w + i), *reinterpret_cast<const float4 *>(a.b + i)); }, kEarly);
         return;
     }
     float s = 0.f;
-    stream_each<NS>(a, lead, [&](uint32_t i, const float4 u) {
+    auto square = [&](uint32_t i, const float4 u) {
         s = fmaf(u.x, u.x, s); s = fmaf(u.y, u.y, s); s = fmaf(u.z, u.z, s); s = fmaf(u.w, u.w, s);
         put(i, u);
-    });
+    };
+    if constexpr (kEarly > 0) {
+        if (first < a.dp) square(first, early.q.gather(a, first, lead));
+    }
+    stream_each<NS>(a, lead, square, kEarly);
     const float inv = rsqrtf(block_sum_waves(s, scratch, blockDim.x >> 6) / (float)a.dim + a.eps);
-    for (uint32_t i = threadIdx.x * 4; i < a.dp; i += blockDim.x * 4) {
-        const float4 u = get(i), w = *reinterpret_cast<const float4 *>(a.w + i);
-        const float4 h = make_float4(u.x * inv * w.x, u.y * inv * w.y, u.z * inv * w.z, u.w * inv * w.w);
+    auto scale = [&](uint32_t i, const float4 w) {
+        const float4 u = get(i), h = make_float4(u.x * inv * w.x, u.y * inv * w.y, u.z * inv * w.z, u.w * inv * w.w);
         put(i, h);
         if (lead && a.h_out) *reinterpret_cast<float4 *>(a.h_out + i) = h;
+    };
+    if constexpr (kEarly > 0) {
+        if (first < a.dp) scale(first, early.w);
     }
+    for (uint32_t i = first + kEarly * step; i < a.dp; i += step) scale(i, *reinterpret_cast<const float4 *>(a.w + i));
 }
 
 // A batch: one workgroup per row.  x: [row][stream][dp], y: [row][dp] or, with several vectors per row to be added up,
@@ -157,10 +192,12 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(StreamRowsArgs a)
                                                              (uint32_t)float_to_bf16(h.z) | ((uint32_t)float_to_bf16(h.w) << 16));
         else *reinterpret_cast<float4 *>(act + i) = h;
     };
+    EarlyStreams<NS> early;
+    early.load(in);
     if (in.alpha) {
-        stream_input<NS>(in, true, scratch, store, [](uint32_t) { return make_float4(0.f, 0.f, 0.f, 0.f); });
+        stream_input<NS>(in, true, scratch, early, store, [](uint32_t) { return make_float4(0.f, 0.f, 0.f, 0.f); });
     } else {
-        stream_input<NS>(in, true, scratch, [&](uint32_t i, const float4 h) { *reinterpret_cast<float4 *>(us + i) = h; },
+        stream_input<NS>(in, true, scratch, early, [&](uint32_t i, const float4 h) { *reinterpret_cast<float4 *>(us + i) = h; },
                          [&](uint32_t i) { return *reinterpret_cast<const float4 *>(us + i); });
         for (uint32_t i = threadIdx.x * 4; i < in.dp; i += 1024) store(i, *reinterpret_cast<const float4 *>(us + i));
     }
