@@ -1,6 +1,6 @@
 // lv_bf16_gemv.h — one-token products with bfloat16 weights: out[row] = sum_k W[row][k] * x[k], x and the sums in fp32.
 //
-// A workgroup (8 waves) puts x into LDS once, then its waves walk groups of rows with a register queue of 16-byte weight
+// A workgroup (8 or 16 waves) puts x into LDS once, then its waves walk groups of rows with a register queue of 16-byte weight
 // loads that keeps running from one group to the next and is filled before x is ready.  What x is (the "input") is part of
 // the kernel, so that a layer needs no launches for its norms:
 //   kInNorm    x = norm(residual + postnorm(y)) with the sublayer output y still pending; workgroup 0 also leaves the new
