@@ -2401,11 +2401,12 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
     HIP_TRY(hipGetLastError());
 
     uint32_t pending = 0;       // K slices in b.parts that the next norm adds to the residual stream
+    const float *xscale = short_exact(short_tiles(n)) ? nullptr : b.xscale;
     for (uint32_t li = 0; li < hp.layers; li++) {
         const LayerWeights &lw = m->layers[li];
         LV_TRY(launch_short_norm(st, b, lw.attn_norm, n, D, pending, ft));
         ShortArgs a{};
-        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = b.xscale;
+        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = xscale;
         a.mode = kShortQkv;
         a.w = lw.short_qkv;
         a.tiles_m = D / 16; a.tiles = 3 * a.tiles_m; a.out[0] = b.q; a.ldo = D;
@@ -2418,7 +2419,7 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
         LV_TRY(launch_short_gemm(st, o, ft, sf32, true, &pending));
         LV_TRY(launch_short_norm(st, b, lw.ffn_norm, n, D, pending, ft));
         ShortArgs f{};
-        f.x = b.act; f.n = n; f.nb = D / 32; f.xscale = b.xscale; f.mode = kShortSilu;
+        f.x = b.act; f.n = n; f.nb = D / 32; f.xscale = xscale; f.mode = kShortSilu;
         f.w = lw.short_gate_up; f.tiles_m = f.tiles = F / 8; f.ff = b.ff;
         LV_TRY(launch_short_gemm(st, f, ft, sf32, false));
         ShortArgs d = o;
@@ -2432,7 +2433,7 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
     if (all && m->short_output) {
         LV_TRY(launch_short_norm(st, b, m->norm, n, D, pending, ft));
         ShortArgs a{};
-        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = b.xscale; a.mode = kShortStore; a.w = m->short_output;
+        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = xscale; a.mode = kShortStore; a.w = m->short_output;
         a.tiles_m = a.tiles = hp.vocab / 16; a.out[0] = all; a.ldo = hp.vocab;
         LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
     } else if (all || with_head) {

@@ -3,8 +3,13 @@
 //
 // What bounds such a step is reading the weights once.  The GEMM of lv_gemm.h reads a copy of 2.1 bytes a weight and works on tiles
 // of 128 tokens; the persistent kernel reads all weights per token.  Here every weight is read once, in its 4.5 or 8.5 bits, and
-// unpacked to fp16 in registers on its way into the matrix cores.  Arithmetic as in lv_gemm.h: activations as two fp16 halves,
-// every product exact, a block's 32 products summed in fp32, then times the block's scale and added to the fp32 result.
+// unpacked in registers on its way into the matrix cores.  Every product is exact, a block's 32 products are summed in fp32, then
+// multiplied by the block's scale and added to the fp32 result.  Activations:
+//   up to 16 tokens   three bf16 parts, an exact cut of the fp32 value with all of its range.  Such a step is also evaluated token by
+//                     token (other paths, no room for the copy below), in fp32 throughout, and is held to the same.
+//   17 to 64          two fp16 halves as in lv_gemm.h, which takes longer steps and these without the copy: 22 bits, of the norms'
+//                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.
+// The same line divides the attention: fp32 per query (attention_kernel), or short_attn_kernel on fp16 pairs.
 //
 // short_gemm_kernel.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
 // tokens; its waves deal the K range among themselves, four quant blocks at a time, and add up through LDS at the end.  A wave so
@@ -17,12 +22,15 @@
 //       16 consecutive lanes 16 cache lines: the address path, not HBM, then sets the time (7B q4_0 gate and up for 8 tokens: 21.5 us that way, 15.8 so).
 //   order: the eight codes a lane feeds to an MFMA come in the order that unpacks cheapest (short_slot); the activations are
 //          written in that order.
-//   activations: [block][16-token tile][high, low half][group][token][8 halfs]: 1 KB per operand, a lane's 16 bytes at 16 l.
+//   activations: [block][16-token tile][operand][group][token][8 elements]: 1 KB per operand, a lane's 16 bytes at 16 l.  Up to 8 tokens:
+//          the first two parts share an operand (tokens 0 .. 7 and 8 .. 15 of it), the third is half of one.
 // Rows of tokens past the batch are not written; a token only meets its own row of the result.
 //
 // Measured (us per launch, 7B layer, 8 tokens q4_0 / 45 tokens q8_0): q, k and v 11 / 28, attention output 4.5 / 10, gate and up
-// 16 / 47, down 9 / 22; about 3 of them launch and sum.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.07 ms (eight launches of the
-// persistent kernel before); 45 tokens behind 619, 8 layers of 7B q8_0: 2.77 -> 1.24 ms (128-token GEMM tiles before).
+// 16 / 47, down 9 / 22 with halves; about 3 of them launch and sum.  The third part costs 0 to 2 us of 8 tokens, since activations
+// come through the vector cache as the weights do.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.23 ms (eight launches of the persistent
+// kernel before; 2.04 with halves, which lose products beyond 65504 and below 2^-13); 45 tokens behind 619, 8 layers of 7B q8_0:
+// 2.77 -> 1.20 ms (128-token GEMM tiles before).
 #pragma once
 
 #include "lv_attn_batch.h"
@@ -36,29 +44,33 @@ constexpr int kShortSlices = kGemmMaxMats;
 
 typedef _Float16 lv_h2 __attribute__((ext_vector_type(2)));
 typedef uint32_t lv_u4 __attribute__((ext_vector_type(4)));
+typedef __bf16 lv_b2 __attribute__((ext_vector_type(2)));
 typedef uint32_t lv_u2 __attribute__((ext_vector_type(2)));
 
-// tiles of 16 tokens; 0: up to 8 tokens, whose high and low halves share one operand
+// tiles of 16 tokens; 0: up to 8 tokens, whose parts share operands
 __host__ __device__ constexpr uint32_t short_tiles(uint32_t n) { return n <= 8 ? 0 : (n + 15) / 16; }
-__host__ __device__ constexpr uint32_t short_block_bytes(uint32_t tiles) { return tiles ? tiles * 2048 : 1024; }
+// three bf16 parts, not two fp16 halves
+constexpr uint32_t kShortExact = 16;
+__host__ __device__ constexpr bool short_exact(uint32_t tiles) { return tiles <= 1; }
+__host__ __device__ constexpr uint32_t short_block_bytes(uint32_t tiles) { return tiles == 0 ? 1536 : tiles == 1 ? 3072 : tiles * 2048; }
 // bytes of the activations of K columns
 __host__ __device__ constexpr size_t short_act_bytes(uint32_t K, uint32_t n) { return (size_t)(K / 32) * short_block_bytes(short_tiles(n)); }
 
 // Element k of a block (0 .. 31) -> slot 8 g + e of the operand, and back.  q8_0: bytes in order.  q4_0: group g holds bytes
-// 4g .. 4g + 3 of the block, whose low nibbles are elements 4g .. 4g + 3 and whose high ones are 16 higher; a masked dword leaves
-// nibbles 0 and 4 (then 1 and 5, 2 and 6, 3 and 7) in the two halves of a register.
-template <int QT>
+// 4g .. 4g + 3 of the block, whose low nibbles are elements 4g .. 4g + 3 and whose high ones are 16 higher.  Parts: the low ones, then
+// the high ones.  Halves: a masked dword leaves nibbles 0 and 4 (then 1 and 5, 2 and 6, 3 and 7) in the two halves of a register.
+template <int QT, bool PARTS>
 __host__ __device__ constexpr uint32_t short_slot(uint32_t k)
 {
     if constexpr (QT == 8) return k;
     const uint32_t g = (k & 15) >> 2, j = k & 3, hi = k >> 4;
-    return 8 * g + (j & 1) * 4 + hi * 2 + (j >> 1);
+    return PARTS ? 8 * g + hi * 4 + j : 8 * g + (j & 1) * 4 + hi * 2 + (j >> 1);
 }
 // the elements of group g, slots 0 .. 7, from two runs of four consecutive elements a (from 4g or 8g on) and b (16 or 4 further)
 template <int QT>
-__device__ __forceinline__ void short_order(float (&f)[8], const float4 &a, const float4 &b)
+__device__ __forceinline__ void short_order(float (&f)[8], const float4 &a, const float4 &b, bool parts)
 {
-    if constexpr (QT == 8) {
+    if (QT == 8 || parts) {
         f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
     } else {
         f[0] = a.x; f[1] = a.z; f[2] = b.x; f[3] = b.z; f[4] = a.y; f[5] = a.w; f[6] = b.y; f[7] = b.w;
@@ -67,12 +79,44 @@ __device__ __forceinline__ void short_order(float (&f)[8], const float4 &a, cons
 template <int QT> __host__ __device__ constexpr uint32_t short_run_a(uint32_t g) { return QT == 8 ? 8 * g : 4 * g; }
 template <int QT> __host__ __device__ constexpr uint32_t short_run_b(uint32_t g) { return QT == 8 ? 8 * g + 4 : 16 + 4 * g; }
 
-// where the high halves of (block, token, group) lie, and how much further the low ones
-__device__ __forceinline__ size_t short_act_offset(uint32_t block, uint32_t token, uint32_t g, uint32_t tiles)
+// where part `part` of (block, token, group) lies: 0, 1 and 2, or the halves 0 and 1
+__device__ __forceinline__ size_t short_act_offset(uint32_t block, uint32_t token, uint32_t g, uint32_t tiles, uint32_t part)
 {
-    return (size_t)block * short_block_bytes(tiles) + token / 16 * 2048 + (g * 16 + token % 16) * 16;
+    const size_t at = (size_t)block * short_block_bytes(tiles);
+    if (tiles == 0) return at + (part < 2 ? g * 256 + part * 128 : 1024 + g * 128) + token * 16;
+    return at + token / 16 * 2048 + part * 1024 + (g * 16 + token % 16) * 16;
 }
-__host__ __device__ constexpr uint32_t short_act_low(uint32_t tiles) { return tiles ? 1024 : 128; }
+// x = b[0] + b[1] + b[2], each the upper half of its dword: eight bits a part
+__device__ __forceinline__ void short_cut(uint32_t (&b)[3], float x)
+{
+    b[0] = __float_as_uint(x) & 0xffff0000u;
+    const float r = x - __uint_as_float(b[0]);
+    b[1] = __float_as_uint(r) & 0xffff0000u;
+    b[2] = __float_as_uint(r - __uint_as_float(b[1]));
+}
+// the eight elements of (block, token, group)
+__device__ __forceinline__ void short_put(uint8_t *act, uint32_t block, uint32_t token, uint32_t g, uint32_t tiles, const float (&f)[8])
+{
+    uint4 p[3];
+    if (short_exact(tiles)) {
+        uint32_t w[3][4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t b0[3], b1[3];
+            short_cut(b0, f[2 * j]);
+            short_cut(b1, f[2 * j + 1]);
+#pragma unroll
+            for (int i = 0; i < 3; i++) w[i][j] = (b0[i] >> 16) | (b1[i] & 0xffff0000u);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) p[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+        *reinterpret_cast<uint4 *>(act + short_act_offset(block, token, g, tiles, 2)) = p[2];
+    } else {
+        gemm_split8(p[0], p[1], f);
+    }
+    *reinterpret_cast<uint4 *>(act + short_act_offset(block, token, g, tiles, 0)) = p[0];
+    *reinterpret_cast<uint4 *>(act + short_act_offset(block, token, g, tiles, 1)) = p[1];
+}
 
 enum ShortMode { kShortStore = 0, kShortQkv = 1, kShortSilu = 2 };
 
@@ -85,7 +129,7 @@ struct ShortArgs {
     uint32_t n, mode;
     float *out[kShortSlices];  // [n][ldo], one per slice; kShortQkv: out[0] = q
     uint32_t ldo;
-    const float *xscale;       // null, or per token the power of two its halves have to be multiplied by
+    const float *xscale;       // null, or per token the power of two its halves have to be multiplied by (not with parts)
     uint16_t *cache[2];        // kShortQkv: k and v rows
     const uint32_t *pos_ptr;
     uint32_t pos_add, backlog;
@@ -94,8 +138,10 @@ struct ShortArgs {
 
 // Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights or, where a block's
 // products take long enough to cover an L2 access, two blocks ahead.  More in flight per wave costs registers, hence waves per
-// CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us, q, k and v for 45 with q8_0 28 -> 96).
-template <int T, int RT> constexpr int short_ahead() { return T * RT >= 8 ? 2 : 4; }
+// CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us, q, k and v for 45 with q8_0 28 -> 96).  With
+// the third part, three row tiles of q4_0 and four blocks ahead take 138 registers, one workgroup a CU; two blocks ahead 126 and two
+// (q, k, v and gate and up together, mean: 8 tokens 15.0 -> 14.6 us, 14 tokens 18.2 -> 17.6; q8_0, 146 and 130: 19.9 -> 21.1, so not there).
+template <int QT, int T, int RT> constexpr int short_ahead() { return T * RT >= 8 || (short_exact(T) && QT == 4 && RT >= 3) ? 2 : 4; }
 // can RT tiles of rows beside T tiles of tokens keep sums, queues and activations in 256 registers (a few values more is fine)
 __host__ __device__ constexpr bool short_fits(int qt, uint32_t t, uint32_t rt) { return qt == 4 || rt <= (t <= 1 ? 6u : t <= 3 ? 3u : 2u); }
 // row tiles whose sums are put together at a time: up to 64 KB of LDS, whole pairs
@@ -129,6 +175,29 @@ __device__ __forceinline__ lv_h8 short_unpack8(uint32_t lo, uint32_t hi)
     u.h[2] = __builtin_bit_cast(lv_h2, __builtin_amdgcn_perm(0x64646464u, b, 0x04010400u)) + c;
     u.h[3] = __builtin_bit_cast(lv_h2, __builtin_amdgcn_perm(0x64646464u, b, 0x04030402u)) + c;
     return u.v8;
+}
+// bf16, q4_0: a byte 0x0q is q 2^-9 as an fp8 number.  The codes stay unsigned: 8 times every activation is taken off the sum instead, as
+// with q4_block_dot.
+__device__ __forceinline__ lv_b8 short_unpack4_bf16(uint32_t w)
+{
+    const uint32_t l = w & 0x0f0f0f0fu, h = (w >> 4) & 0x0f0f0f0fu;
+    union { lv_b2 h[4]; lv_b8 v8; } u;
+    u.h[0] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(l, 512.f, false);
+    u.h[1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(l, 512.f, true);
+    u.h[2] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, false);
+    u.h[3] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(h, 512.f, true);
+    return u.v8;
+}
+// q8_0: a signed byte converts to fp32, where a whole number of eight bits leaves the lower half zero
+__device__ __forceinline__ lv_b8 short_unpack8_bf16(uint32_t lo, uint32_t hi)
+{
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t d = (j < 2 ? lo : hi) >> (16 * (j & 1));
+        w[j] = __builtin_amdgcn_perm(__float_as_uint((float)(int8_t)(d >> 8)), __float_as_uint((float)(int8_t)d), 0x07060302u);
+    }
+    return __builtin_bit_cast(lv_b8, lv_u4{w[0], w[1], w[2], w[3]});
 }
 __host__ __device__ constexpr uint32_t short_chunk_bytes(int qt, bool sf32) { return (qt == 4 ? 1024 : 2048) + (sf32 ? 256 : 128); }
 __host__ __device__ constexpr size_t short_tile_bytes(int qt, bool sf32, uint32_t nb) { return (size_t)(nb / 4) * short_chunk_bytes(qt, sf32); }
@@ -168,13 +237,15 @@ __global__ __launch_bounds__(256) void short_pack_kernel(uint8_t *__restrict__ d
 template <int QT, bool SF32, int T, int RT>
 __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs a)
 {
-    constexpr bool EIGHT = T == 0;                     // one operand holds the high halves of 8 tokens and their low halves
+    constexpr bool EIGHT = T == 0;                     // 8 tokens: an operand holds their first parts and their second ones
+    constexpr bool EXACT = short_exact(T);
     constexpr int NT = EIGHT ? 1 : T;
-    constexpr int XB = EIGHT ? 1024 : T * 2048;        // activation bytes of a block
+    constexpr int XB = short_block_bytes(T);           // activation bytes of a block
+    constexpr int NX = EIGHT ? 2 : EXACT ? 3 : 2 * NT; // its operands
     constexpr int BB = QT == 4 ? 16 : 32;              // code bytes of a block
     constexpr int CW = BB / 4;                         // a lane's dwords of a chunk
     constexpr int CB = short_chunk_bytes(QT, SF32);
-    constexpr int XD = short_ahead<T, RT>();
+    constexpr int XD = short_ahead<QT, T, RT>();
     constexpr int PR = short_round<T, RT>();           // row tiles summed at a time
     __shared__ __attribute__((aligned(16))) float red[PR * NT * kShortWaves * 256];
     const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
@@ -194,7 +265,7 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
     // Past this wave's last chunk: one address for all lanes, which costs next to nothing and keeps the queue free of branches.
     uint32_t cq[RT][CW];
     std::conditional_t<SF32, lv_u4, lv_u2> sq[RT];
-    lv_u4 xq[XD][EIGHT ? 1 : 2 * NT];
+    lv_u4 xq[XD][NX];
     auto fetch_w = [&](uint32_t j) {
         const uint32_t at = j < steps ? j * (kShortWaves * CB) : 0, lw = j < steps ? lane * 16 : 0, ls = j < steps ? r16 * (SF32 ? 16 : 8) : 0;
 #pragma unroll
@@ -211,7 +282,10 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
         const uint8_t *p = xb + (j < steps ? ((size_t)j * (kShortWaves * 4) + s) * XB : 0);
         const uint32_t l = j < steps ? lane * 16 : 0;
 #pragma unroll
-        for (int t = 0; t < (EIGHT ? 1 : 2 * NT); t++) xq[slot][t] = *reinterpret_cast<const lv_u4 *>(p + l + t * 1024);
+        for (int t = 0; t < NX; t++) {
+            const uint32_t at = EIGHT && t == 1 ? (j < steps ? g * 128 + (r16 & 7) * 16 : 0) : l;
+            xq[slot][t] = *reinterpret_cast<const lv_u4 *>(p + at + t * 1024);
+        }
     };
     lv_f4v acc[RT][NT];
 #pragma unroll
@@ -219,6 +293,7 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[i][t] = lv_f4v{0.f, 0.f, 0.f, 0.f};
     const lv_f4v zero = {0.f, 0.f, 0.f, 0.f};
+    constexpr uint32_t kOnes = 0x3f803f80u;
 
     if (steps) {
         fetch_w(0);
@@ -240,20 +315,29 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
             fetch_w(j + 1);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                lv_h8 ax[EIGHT ? 1 : 2 * NT];          // high, low halves tile by tile
+                lv_u4 ax[NX];                          // parts, or high and low halves tile by tile
 #pragma unroll
-                for (int t = 0; t < (EIGHT ? 1 : 2 * NT); t++) ax[t] = __builtin_bit_cast(lv_h8, xq[s % XD][t]);
+                for (int t = 0; t < NX; t++) ax[t] = xq[s % XD][t];
+                if constexpr (EIGHT) ax[1] = r16 >= 8 ? ax[1] : lv_u4{0u, 0u, 0u, 0u};       // the third parts beside the second
+                auto times = [&](const lv_b8 &b, lv_f4v c) {       // all parts, the small ones first
+#pragma unroll
+                    for (int t = NX - 1; t >= 0; t--) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lv_b8, ax[t]), b, c, 0, 0, 0);
+                    return c;
+                };
+                lv_f4v from = zero;
+                if constexpr (EXACT && QT == 4) from = times(__builtin_bit_cast(lv_b8, lv_u4{kOnes, kOnes, kOnes, kOnes}), zero) * -8.f;
 #pragma unroll
                 for (int i = 0; i < RT; i++) {
-                    const lv_h8 b = QT == 4 ? short_unpack4(w[i][s]) : short_unpack8(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
                     lv_f4v p[NT];
-                    if constexpr (EIGHT) {
-                        p[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax[0], b, zero, 0, 0, 0);
+                    if constexpr (EXACT) {
+                        const lv_b8 b = QT == 4 ? short_unpack4_bf16(w[i][s]) : short_unpack8_bf16(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
+                        p[0] = times(b, from);
                     } else {
+                        const lv_h8 b = QT == 4 ? short_unpack4(w[i][s]) : short_unpack8(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
 #pragma unroll
-                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax[2 * t + 1], b, zero, 0, 0, 0);
+                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lv_h8, ax[2 * t + 1]), b, zero, 0, 0, 0);
 #pragma unroll
-                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax[2 * t], b, p[t], 0, 0, 0);
+                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lv_h8, ax[2 * t]), b, p[t], 0, 0, 0);
                     }
 #pragma unroll
                     for (int t = 0; t < NT; t++)
@@ -266,8 +350,8 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
     }
 
     // ---- the waves' sums, PR row tiles at a time, through LDS: [row tile][token tile][wave][lane] float4 -------------------------
-    // acc[i][t][e]: row r16 of row tile i, token 16 t + 4 g + e (EIGHT: the high half's product of token 4 g + e for g < 2, behind
-    // them the low half's).  A wave adds up every eighth (row tile, token tile).
+    // acc[i][t][e]: row r16 of row tile i, token 16 t + 4 g + e (EIGHT: the first part's product of token 4 g + e for g < 2, behind
+    // them the others').  A wave adds up every eighth (row tile, token tile).
     const uint32_t row_at = (a.mode == kShortQkv && a.pos_ptr ? *a.pos_ptr : 0u) + a.pos_add;
     float *const out = a.out[blockIdx.y];
     auto total = [&](int u, int from, float (&v)[4], const float4 &xs) {      // lane `from`'s sums of unit u
@@ -302,15 +386,22 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
                 if (r16 >= 8) continue;
                 float w[4];
                 total(u, lane + 8, w, xs);
-                const uint32_t f = tile * 8 + r16, slot = short_slot<QT>(f & 31);
+                const uint32_t f = tile * 8 + r16, slot = short_slot<QT, EXACT>(f & 31);
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     if (tok0 + e >= a.n) continue;
                     const float y = v[e] * w[e] / (__expf(-w[e]) + 1.f);
-                    const uint16_t h = float_to_half_bits(y), l = float_to_half_bits(y - half_bits_to_float(h));
-                    uint8_t *dst = a.ff + short_act_offset(f / 32, tok0 + e, slot >> 3, T) + (slot & 7) * 2;
-                    *reinterpret_cast<uint16_t *>(dst) = h;
-                    *reinterpret_cast<uint16_t *>(dst + short_act_low(T)) = l;
+                    auto put = [&](uint32_t part, uint16_t v) { *reinterpret_cast<uint16_t *>(a.ff + short_act_offset(f / 32, tok0 + e, slot >> 3, T, part) + (slot & 7) * 2) = v; };
+                    if constexpr (EXACT) {
+                        uint32_t b[3];
+                        short_cut(b, y);
+#pragma unroll
+                        for (int i = 0; i < 3; i++) put(i, (uint16_t)(b[i] >> 16));
+                    } else {
+                        const uint16_t h = float_to_half_bits(y);
+                        put(0, h);
+                        put(1, float_to_half_bits(y - half_bits_to_float(h)));
+                    }
                 }
                 continue;
             }
@@ -326,8 +417,8 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
     }
 }
 
-// x += the K slices of the product before, then normalize(x) * w (normalize.comp:34-64) as the next product's activations, scaled
-// per token as in gemm_row_scale.  One workgroup per token, a thread per 8 elements (dim / 8 threads rounded up to whole waves;
+// x += the K slices of the product before, then normalize(x) * w (normalize.comp:34-64) as the next product's activations, halves
+// scaled per token as in gemm_row_scale.  One workgroup per token, a thread per 8 elements (dim / 8 threads rounded up to whole waves;
 // dim <= 8192, a multiple of 32): nothing but latency counts here, and a thread's loads are few and all in flight at once.
 struct ShortNormArgs {
     float *x;
@@ -395,23 +486,22 @@ __global__ __launch_bounds__(1024) void short_norm_kernel(ShortNormArgs a)
     q = 0.f;
     for (int v = 0; v < waves; v++) q += lds[32 + v];
     const float inv = rsqrtf(q / (float)a.dim);
-    float down;
-    const float up = gemm_row_scale(big * inv, &down);
-    if (threadIdx.x == 0) a.xscale[row] = down;
+    float up = 1.f;
+    if (!short_exact(a.tiles)) {
+        float down;
+        up = gemm_row_scale(big * inv, &down);
+        if (threadIdx.x == 0) a.xscale[row] = down;
+    }
     if (!ok) return;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         x[h].x = (x[h].x * w[h].x) * inv; x[h].y = (x[h].y * w[h].y) * inv; x[h].z = (x[h].z * w[h].z) * inv; x[h].w = (x[h].w * w[h].w) * inv;
     }
     float f[8];
-    short_order<QT>(f, x[0], x[1]);
+    short_order<QT>(f, x[0], x[1], short_exact(a.tiles));
 #pragma unroll
     for (int e = 0; e < 8; e++) f[e] *= up;
-    uint4 h, l;
-    gemm_split8(h, l, f);
-    uint8_t *dst = a.act + short_act_offset(i >> 2, row, i & 3, a.tiles);
-    *reinterpret_cast<uint4 *>(dst) = h;
-    *reinterpret_cast<uint4 *>(dst + short_act_low(a.tiles)) = l;
+    short_put(a.act, i >> 2, row, i & 3, a.tiles, f);
 }
 
 // Attention of a short batch: attention_batch_kernel's arithmetic, with the cache positions shared out over workgroups and the
@@ -643,13 +733,9 @@ __global__ __launch_bounds__(256, 2) void short_attn_kernel(ShortAttnArgs a)
             va.x /= total; va.y /= total; va.z /= total; va.w /= total;
             vb.x /= total; vb.y /= total; vb.z /= total; vb.w /= total;
             float f[8];
-            if (a.q8) short_order<8>(f, va, vb);
-            else short_order<4>(f, va, vb);
-            uint4 hi, lo;
-            gemm_split8(hi, lo, f);
-            uint8_t *dst = a.act + short_act_offset(k / 32, z, g, a.tiles);
-            *reinterpret_cast<uint4 *>(dst) = hi;
-            *reinterpret_cast<uint4 *>(dst + short_act_low(a.tiles)) = lo;
+            if (a.q8) short_order<8>(f, va, vb, false);
+            else short_order<4>(f, va, vb, short_exact(a.tiles));
+            short_put(a.act, k / 32, z, g, a.tiles, f);
         }
         return;
     }
@@ -690,12 +776,8 @@ __global__ __launch_bounds__(256) void short_attn_combine_kernel(ShortCombineArg
     va.x /= den; va.y /= den; va.z /= den; va.w /= den;
     vb.x /= den; vb.y /= den; vb.z /= den; vb.w /= den;
     float f[8];
-    short_order<QT>(f, va, vb);
-    uint4 hi, lo;
-    gemm_split8(hi, lo, f);
-    uint8_t *dst = a.act + short_act_offset(i >> 2, z, i & 3, a.tiles);
-    *reinterpret_cast<uint4 *>(dst) = hi;
-    *reinterpret_cast<uint4 *>(dst + short_act_low(a.tiles)) = lo;
+    short_order<QT>(f, va, vb, short_exact(a.tiles));
+    short_put(a.act, i >> 2, z, i & 3, a.tiles, f);
 }
 
 }  // namespace lv

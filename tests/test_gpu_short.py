@@ -74,3 +74,49 @@ def test_every_row_of_a_short_batch(lva, ctx, models, name, n):
         b.begin([t], i)
         close(rows[i], b.logits())
     a.close(); b.close(); model.close()
+
+
+def scaled_file(src, dst, powers):
+    """a copy of a version-3 file with the blocks of some tensors multiplied by powers of two; powers: end of the name -> exponent"""
+    data = np.fromfile(src, dtype=np.uint8)
+    cur = 36
+    for _ in range(int(data[8:12].view(np.uint32)[0])):
+        cur += 8 + int(data[cur:cur + 4].view(np.int32)[0])
+    while cur != len(data):
+        dims, name_len, ftype = (int(v) for v in data[cur:cur + 12].view(np.uint32))
+        count = int(np.prod(data[cur + 12:cur + 12 + 4 * dims].view(np.uint32)))
+        name = data[cur + 12 + 4 * dims:cur + 12 + 4 * dims + name_len].tobytes().decode()
+        cur = (cur + 12 + 4 * dims + name_len + 31) & ~31
+        size = {0: 4 * count, 2: count // 32 * 18, 8: count // 32 * 34}[ftype]
+        for end, e in powers.items():
+            if name.endswith(end + ".weight"):
+                d = data[cur:cur + size].reshape(-1, size // (count // 32))
+                d[:, :2] = (d[:, :2].copy().view(np.float16) * np.float16(2.0 ** e)).view(np.uint8)
+        cur += size
+    data.tofile(dst)
+    return dst
+
+
+# feed-forward products of 1e5 and more, beyond fp16, and of 1e-6, where an fp16 pair has few bits left; the way down evens them out
+MAGNITUDES = {"large": {"w1": 12, "w3": 12, "w2": -8}, "small": {"w1": -8, "w3": -8, "w2": 15}}
+
+
+@pytest.mark.parametrize("size", list(MAGNITUDES))
+@pytest.mark.parametrize("name", ["q4_64", "q8_64"])
+def test_short_batch_keeps_the_range_of_one_token_steps(lva, orc, ctx, models, tmp_path, name, size):
+    path = scaled_file(models[name], str(tmp_path / "scaled.ggml"), MAGNITUDES[size])
+    om = orc.Model(path)
+    model = lva.Model(ctx, path)
+    for n in (2, 8, 9, 15, 16):
+        osess, a, b = orc.Session(om, 128), lva.Session(model, 128), lva.Session(model, 128)
+        toks = lva.synth_tokens(n, 3, 500, seed=n)
+        want = osess.eval(toks)
+        a.begin(toks, 0)
+        for i, t in enumerate(toks):
+            b.begin([t], i)
+            b.wait()
+        assert np.isfinite(want).all()
+        close(b.logits(), want)
+        close(a.logits(), want)
+        a.close(); b.close(); osess.close()
+    model.close(); om.close()
