@@ -9,7 +9,8 @@
 //                     token (other paths, no room for the copy below), in fp32 throughout, and is held to the same.
 //   17 to 64          two fp16 halves as in lv_gemm.h, which takes longer steps and these without the copy: 22 bits, of the norms'
 //                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.
-// The same line divides the attention: fp32 per query (attention_kernel), or short_attn_kernel on fp16 pairs.
+// Attention likewise: up to 15 tokens fp32 per query (attention_kernel), then short_attn_kernel on fp16 pairs as with longer steps (a
+// layer, 8 tokens at the start of a sequence 6.9 against 10.1 us; 15 tokens behind 1900 about 60 against 11).
 //
 // short_gemm_kernel.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
 // tokens; its waves deal the K range among themselves, four quant blocks at a time, and add up through LDS at the end.  A wave so
@@ -28,7 +29,7 @@
 //
 // Measured (us per launch, 7B layer, 8 tokens q4_0 / 45 tokens q8_0): q, k and v 11 / 28, attention output 4.5 / 10, gate and up
 // 16 / 47, down 9 / 22 with halves; about 3 of them launch and sum.  The third part costs 0 to 2 us of 8 tokens, since activations
-// come through the vector cache as the weights do.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.23 ms (eight launches of the persistent
+// come through the vector cache as the weights do.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.10 ms (eight launches of the persistent
 // kernel before; 2.04 with halves, which lose products beyond 65504 and below 2^-13); 45 tokens behind 619, 8 layers of 7B q8_0:
 // 2.77 -> 1.20 ms (128-token GEMM tiles before).
 #pragma once
@@ -49,8 +50,7 @@ typedef uint32_t lv_u2 __attribute__((ext_vector_type(2)));
 
 // tiles of 16 tokens; 0: up to 8 tokens, whose parts share operands
 __host__ __device__ constexpr uint32_t short_tiles(uint32_t n) { return n <= 8 ? 0 : (n + 15) / 16; }
-// three bf16 parts, not two fp16 halves
-constexpr uint32_t kShortExact = 16;
+// three bf16 parts, not two fp16 halves: up to 16 tokens
 __host__ __device__ constexpr bool short_exact(uint32_t tiles) { return tiles <= 1; }
 __host__ __device__ constexpr uint32_t short_block_bytes(uint32_t tiles) { return tiles == 0 ? 1536 : tiles == 1 ? 3072 : tiles * 2048; }
 // bytes of the activations of K columns
@@ -504,7 +504,19 @@ __global__ __launch_bounds__(1024) void short_norm_kernel(ShortNormArgs a)
     short_put(a.act, i >> 2, row, i & 3, a.tiles, f);
 }
 
-// Attention of a short batch: attention_batch_kernel's arithmetic, with the cache positions shared out over workgroups and the
+// rows of `dim` floats as a product's activations.  grid (dim / 8 / 256 rounded up, rows)
+template <int QT>
+__global__ __launch_bounds__(256) void short_rows_kernel(uint8_t *__restrict__ act, const float *__restrict__ x, uint32_t dim, uint32_t tiles)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= dim / 8) return;
+    const float *src = x + (size_t)blockIdx.y * dim + (i >> 2) * 32;
+    float f[8];
+    short_order<QT>(f, *reinterpret_cast<const float4 *>(src + short_run_a<QT>(i & 3)), *reinterpret_cast<const float4 *>(src + short_run_b<QT>(i & 3)), short_exact(tiles));
+    short_put(act, i >> 2, blockIdx.y, i & 3, tiles, f);
+}
+
+// Attention of 16 to 64 tokens: attention_batch_kernel's arithmetic, with the cache positions shared out over workgroups and the
 // operand planes made on the way into LDS (a plane would be used once).  Without a running maximum the parts of a row are plain
 // sums: numerators [split][n][H*R] and denominators [split][n][H], put together by short_attn_combine_kernel.  64 KB of LDS: two
 // workgroups a CU.

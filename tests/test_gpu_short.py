@@ -91,23 +91,25 @@ def scaled_file(src, dst, powers):
         for end, e in powers.items():
             if name.endswith(end + ".weight"):
                 d = data[cur:cur + size].reshape(-1, size // (count // 32))
-                d[:, :2] = (d[:, :2].copy().view(np.float16) * np.float16(2.0 ** e)).view(np.uint8)
+                d[:, :2] = np.ldexp(d[:, :2].copy().view(np.float16).astype(np.float32), e).astype(np.float16).view(np.uint8)
         cur += size
     data.tofile(dst)
     return dst
 
 
-# feed-forward products of 1e5 and more, beyond fp16, and of 1e-6, where an fp16 pair has few bits left; the way down evens them out
-MAGNITUDES = {"large": {"w1": 12, "w3": 12, "w2": -8}, "small": {"w1": -8, "w3": -8, "w2": 15}}
+# feed-forward products of 1e5 and more, beyond fp16, and of 1e-6, where an fp16 pair has few bits left; the way down evens them out.
+# Queries beyond fp16 on small keys; from 16 tokens on they are pairs, as in longer steps
+LARGE, SMALL = {"w1": 12, "w3": 12, "w2": -8}, {"w1": -8, "w3": -8, "w2": 15}
+MAGNITUDES = [("q4_64", LARGE, 16), ("q8_64", LARGE, 16), ("q4_64", SMALL, 16), ("q8_64", SMALL, 16),
+              ("q4_64", {"wq": 20, "wk": -16}, 15), ("q8_64", {"wq": 17, "wk": -14}, 15)]
 
 
-@pytest.mark.parametrize("size", list(MAGNITUDES))
-@pytest.mark.parametrize("name", ["q4_64", "q8_64"])
-def test_short_batch_keeps_the_range_of_one_token_steps(lva, orc, ctx, models, tmp_path, name, size):
-    path = scaled_file(models[name], str(tmp_path / "scaled.ggml"), MAGNITUDES[size])
+@pytest.mark.parametrize("name,powers,most", MAGNITUDES)
+def test_short_batch_keeps_the_range_of_one_token_steps(lva, orc, ctx, models, tmp_path, name, powers, most):
+    path = scaled_file(models[name], str(tmp_path / "scaled.ggml"), powers)
     om = orc.Model(path)
     model = lva.Model(ctx, path)
-    for n in (2, 8, 9, 15, 16):
+    for n in (2, 8, 9, 15, most):
         osess, a, b = orc.Session(om, 128), lva.Session(model, 128), lva.Session(model, 128)
         toks = lva.synth_tokens(n, 3, 500, seed=n)
         want = osess.eval(toks)
