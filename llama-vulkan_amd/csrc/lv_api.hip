@@ -2513,9 +2513,10 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
 
     int path = LV_PATH_AUTO;
     (void)lv_session_path(s, &path);
-    // the persistent kernel also takes the short steps (a few prompt or add_text tokens) below the size at which the
-    // batched path pays: one launch per token, each 1.7 x faster than the operator chain's token
-    const bool few = n >= 2 && n <= kShortTokens && s->model->short_ok && !s->trace && ensure_short_copy(s->model) && short_reserve(s);
+    // Steps of a few tokens (a short prompt, add_text) have kernels of their own.  Without them, and in a session whose path is set, they
+    // go token by token below the size at which the batched path pays: on the persistent kernel one launch per token, each 1.7 x faster
+    // than the operator chain's token.
+    const bool few = n >= 2 && n <= kShortTokens && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && ensure_short_copy(s->model) && short_reserve(s);
     bool persistent = n < kPrefillMin && path == LV_PATH_PERSISTENT && !s->trace && !few;
     s->mega_step = false;
     if (persistent) {

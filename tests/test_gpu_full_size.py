@@ -80,6 +80,7 @@ def test_7b_operator_chain_agrees_with_persistent_kernel(lva, ctx, model_7b):
     """the two execution paths of the library on the same full-size model: same greedy tokens, logits within tolerance"""
     model = lva.Model(ctx, model_7b)
     a, b = lva.Session(model, 128), lva.Session(model, 128)
+    a.set_path(lva.PATH_PERSISTENT)       # the prompt's eight tokens as well
     b.set_path(lva.PATH_GRAPH)
     prompt = lva.synth_tokens(8, 3, SHAPE["vocab"], seed=0)
     a.begin(prompt, 0); b.begin(prompt, 0)
@@ -157,7 +158,7 @@ def test_13b_q4_0_prompt_8_then_8_greedy_steps(lva, orc, ctx):
 
 
 def _prompt_then_steps_on_two_paths(lva, orc, ctx, path, shape, n_prompt, seed, steps):
-    """the prompt as ONE step (batched path: matrix-core GEMMs and batched attention) against the oracle evaluating the same
+    """the prompt as ONE step (matrix-core GEMMs and batched attention) against the oracle evaluating the same
     prompt itself, then greedy steps on the graph path and on the persistent kernel, each against the oracle"""
     om = orc.Model(path)
     osess = orc.Session(om, 256)
@@ -169,7 +170,7 @@ def _prompt_then_steps_on_two_paths(lva, orc, ctx, path, shape, n_prompt, seed, 
     want = osess.eval(prompt)
     worst = 0.0
     for s in (graph, pers):
-        s.begin(prompt, 0)                # n_prompt >= 16: both sessions take the batched prompt path
+        s.begin(prompt, 0)                # the batched prompt path; 32 tokens only where the path is set, the kernels for short steps else
         got = s.logits()
         assert np.all(np.abs(got - want) <= 1e-2 + 1e-3 * np.abs(want)), ("prompt", float(np.max(np.abs(got - want))))
         worst = max(worst, float(np.max(np.abs(got - want))))
@@ -377,6 +378,7 @@ def test_13b_q8_0_prompt_of_512_as_one_batch(lva, orc, ctx):
     ohead = orc.Session(om, 128)
     head_want = ohead.eval(prompt[:32])
     head = lva.Session(model, 128)
+    head.set_path(lva.PATH_GRAPH)         # a batch, not the kernels for short steps
     head.begin(prompt[:32], 0)
     head_got = head.logits()
     d_checker, r_checker = _within(head_want, truth32), _rms(head_want, truth32)

@@ -207,6 +207,7 @@ def test_persistent_kernel_matches_oracle_and_operator_path(lva, orc, ctx, wide_
     model = lva.Model(ctx, wide_model)
     pk, ops = lva.Session(model, 128), lva.Session(model, 128)
     assert pk.path() == lva.PATH_PERSISTENT          # chosen automatically for this shape
+    pk.set_path(lva.PATH_PERSISTENT)                  # ... and once set also for every token of a short step
     ops.set_path(lva.PATH_KERNELS)
     prompt = lva.synth_tokens(8, 3, 2048, seed=1)
     want = osess.eval(prompt)
@@ -462,6 +463,7 @@ def test_logits_of_every_row_of_a_step(lva, orc, ctx, tiny_models, name):
         s.begin([5], 0)
         s.logits_rows(0, 1)                  # the switch is off: nothing was kept
     s.wait()
+    s.set_path(lva.PATH_GRAPH)               # of the models here one would take the kernels for short steps
     s.keep_all_logits()
     toks = lva.synth_tokens(26, 3, om.hp["vocab"], seed=21)
     pos = 0
@@ -489,6 +491,7 @@ def test_logits_of_every_row_on_the_persistent_kernel(lva, orc, ctx, wide_model)
     model = lva.Model(ctx, wide_model)
     s = lva.Session(model, 128)
     assert s.path() == lva.PATH_PERSISTENT
+    s.set_path(lva.PATH_PERSISTENT)          # left to itself the session takes the kernels for short steps
     s.keep_all_logits()
     toks = lva.synth_tokens(9, 3, 2048, seed=22)
     want = osess.eval(toks[:6], all_rows=True)
