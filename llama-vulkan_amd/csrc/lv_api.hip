@@ -2515,8 +2515,11 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     (void)lv_session_path(s, &path);
     // Steps of a few tokens (a short prompt, add_text) have kernels of their own.  Without them, and in a session whose path is set, they
     // go token by token below the size at which the batched path pays: on the persistent kernel one launch per token, each 1.7 x faster
-    // than the operator chain's token.
-    const bool few = n >= 2 && n <= kShortTokens && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && ensure_short_copy(s->model) && short_reserve(s);
+    // than the operator chain's token.  So do two tokens of q4_0 there: reading 4.5 bits a weight twice takes less time than unpacking
+    // them once beside launches of an operator each (7B two launches 1.84 ms, 2.04 so; 13B, 8 layers, 0.72 and 0.75; three tokens
+    // 2.74 and 2.06, 1.07 and 0.75; q8_0, two: 7B, 8 layers, 0.76 and 0.68; 13B 1.10 and 0.93).
+    const uint32_t few_min = path == LV_PATH_PERSISTENT && s->model->layers[0].wq.ftype == LV_Q4_0 ? 3 : 2;
+    const bool few = n >= few_min && n <= kShortTokens && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && ensure_short_copy(s->model) && short_reserve(s);
     bool persistent = n < kPrefillMin && path == LV_PATH_PERSISTENT && !s->trace && !few;
     s->mega_step = false;
     if (persistent) {
