@@ -142,8 +142,13 @@ struct ShortArgs {
 // the third part, three row tiles of q4_0 and four blocks ahead take 138 registers, one workgroup a CU; two blocks ahead 126 and two
 // (q, k, v and gate and up together, mean: 8 tokens 15.0 -> 14.6 us, 14 tokens 18.2 -> 17.6; q8_0, 146 and 130: 19.9 -> 21.1, so not there).
 template <int QT, int T, int RT> constexpr int short_ahead() { return T * RT >= 8 || (short_exact(T) && QT == 4 && RT >= 3) ? 2 : 4; }
-// can RT tiles of rows beside T tiles of tokens keep sums, queues and activations in 256 registers (a few values more is fine)
-__host__ __device__ constexpr bool short_fits(int qt, uint32_t t, uint32_t rt) { return qt == 4 || rt <= (t <= 1 ? 6u : t <= 3 ? 3u : 2u); }
+// can RT tiles of rows beside T tiles of tokens keep sums, queues and activations in 256 registers (a few values more is fine; three
+// tiles of tokens and six of rows of q4_0 left 220 in memory: 40 tokens of 7B 8.7 ms, 3.4 with three)
+__host__ __device__ constexpr bool short_fits(int qt, uint32_t t, uint32_t rt)
+{
+    if (qt == 4) return t != 3 || rt <= 3;
+    return rt <= (t <= 1 ? 6u : t <= 3 ? 3u : 2u);
+}
 // row tiles whose sums are put together at a time: up to 64 KB of LDS, whole pairs
 template <int T, int RT> constexpr int short_round()
 {
