@@ -1101,7 +1101,7 @@ template <class T> static int stream_rows(hipStream_t st, const StreamRowsArgs &
 {
     auto run = [&](auto ns) -> int {
         auto *k = &stream_rows_kernel<T, decltype(ns)::value>;
-        const size_t lds = a.in.dp * (a.in.y && a.parts > 1 ? 8ull : 4ull);
+        const size_t lds = a.in.dp * 4ull;
         LV_TRY(allow_lds(k, lds));
         k<<<dim3(n), dim3(256), lds, st>>>(a);
         HIP_TRY(hipGetLastError());

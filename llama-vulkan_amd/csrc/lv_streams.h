@@ -160,7 +160,7 @@ struct StreamRowsArgs {
 template <class T, int NS>
 __global__ __launch_bounds__(256) void stream_rows_kernel(StreamRowsArgs a)
 {
-    extern __shared__ float us[];      // dp floats, and dp more where parts are added up
+    extern __shared__ float us[];      // dp floats: the parts' sum, in its place then u (a thread keeps to its own elements)
     __shared__ float scratch[4];
     StreamInput in = a.in;
     const size_t row = blockIdx.x;
@@ -169,16 +169,15 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(StreamRowsArgs a)
     if (in.y) {
         in.y += row * a.parts * in.dp;
         if (a.parts > 1) {
-            float *sum = us + in.dp;
             for (uint32_t i = threadIdx.x * 4; i < in.dp; i += 1024) {
                 float4 v = *reinterpret_cast<const float4 *>(in.y + i);
                 for (uint32_t p = 1; p < a.parts; p++) {
                     const float4 u = *reinterpret_cast<const float4 *>(in.y + (size_t)p * in.dp + i);
                     v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
                 }
-                *reinterpret_cast<float4 *>(sum + i) = v;      // every thread reads its own elements again
+                *reinterpret_cast<float4 *>(us + i) = v;
             }
-            in.y = sum;
+            in.y = us;
         }
     }
     if (!a.act) {

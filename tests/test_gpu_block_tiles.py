@@ -40,6 +40,8 @@ def check_last(d, toks, want, tol):
 # tokens one beside a tile's edge; feed-forwards whose way down is cut into 2, 3 and 4 slices, the last one shorter
 DENSE = [(40, 4100, 1100), (130, 2060, 1030), (700, 2060, 1025), (700, 4100, 1281), (300, 1100, 129), (300, 2113, 127), (257, 4160, 257),
          (1030, 3000, 255), (128, 2048, 513), (129, 1025, 65)]
+# streams so wide that the sum of slices and the norm's input would not fit LDS side by side
+DENSE += [(20544, 1152, 33)]
 
 
 @pytest.mark.parametrize("width,ff,n", DENSE)
