@@ -102,6 +102,7 @@ struct Workspace {                     // of batches; sized for `cap` tokens
     uint32_t *ids = nullptr, *slots = nullptr, *tiles = nullptr;
     uint64_t vt_elems = 0, ek_elems = 0, ev_elems = 0;
     uint64_t y_vectors = 0;            // sublayer outputs there is room for in y
+    uint32_t y_for = 0;                // tokens of the batch whose slices y was last asked to hold
 };
 
 struct BlockSession {
@@ -684,7 +685,8 @@ static void workspace_free(Workspace &w)
     for (float **p : {&w.x, &w.y1, &w.y, &w.dq, &w.dk, &w.dv, &w.dg, &w.beta, &w.qk, &w.o, &w.gate, &w.z, &w.scores, &w.y2, &w.sdt, &w.sdecay}) drop(*p);
     for (void **p : {&w.act, &w.q, &w.k, &w.v, &w.vt, &w.a1, &w.g1, &w.cat, &w.ff, &w.cq, &w.ek, &w.ev, &w.sx, &w.sb, &w.sc, &w.sbt}) drop(*p);
     for (uint32_t **p : {&w.ids, &w.slots, &w.tiles}) drop(*p);
-    w.cap = 0;
+    w.cap = w.y_for = 0;
+    w.y_vectors = 0;
     w.vt_elems = w.ek_elems = w.ev_elems = 0;
 }
 
@@ -884,12 +886,16 @@ template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemm
     return launch_bf(st, &gemm_bf16_kernel<EP, GROUPED>, a, kBfLdsBytes);
 }
 
+// of a product into the sublayer outputs, by its sizes alone: the same tokens are summed in the same order whatever the session has
+// evaluated before.  More than 1024 tokens have tiles enough without slices.
+static BfPlan output_plan(const BfMatrix &w, uint32_t n, uint32_t slices = kOutSlices) { return bf_plan(w.rows, n, (n + kBfTile - 1) / kBfTile, w.kp, false, n <= 1024 ? slices : 1); }
+
 // a product into the sublayer outputs `y` ([token][slice][dp], room for `room` vectors), cut in slices of K where its tiles would leave
 // CUs without work; *slices: how many the next norm has to add up
 static int gemm_output(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t dp, uint64_t room, uint32_t *slices)
 {
     BfPlan p{BfTiles::k128, 1};
-    if (!f32) p = bf_plan(w.rows, n, (n + kBfTile - 1) / kBfTile, w.kp, false, (uint32_t)std::min<uint64_t>(kOutSlices, room / n));
+    if (!f32) p = output_plan(w, n, (uint32_t)std::min<uint64_t>(kOutSlices, room / n));
     if (p.slices > 1) {
         a.k_slice = (w.kp / kBfStep + p.slices - 1) / p.slices * kBfStep;
         p.slices = (w.kp + a.k_slice - 1) / a.k_slice;       // every slice has a step
@@ -1272,12 +1278,42 @@ int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *
 constexpr uint32_t kRouterParts = 8, kRouterSlice = 128;
 
 // ---- batches ---------------------------------------------------------------------------------------------------------------
+// room in y for a batch of n and, where the device has it, for its slices (without it they are fewer)
+static int outputs_reserve(BlockSession *s, uint32_t n)
+{
+    const BlockModel *m = s->m;
+    Workspace &w = s->ws;
+    if (n == w.y_for) return LV_OK;
+    uint64_t slices = 1;
+    if (!m->f32)
+        for (const BlockLayer &l : m->layers) {
+            slices = std::max<uint64_t>(slices, output_plan(l.out, n).slices);
+            if (l.dense) slices = std::max<uint64_t>(slices, output_plan(l.down, n).slices);
+        }
+    const uint64_t least = w.cap * std::max(1u, layer_max(m, [](const BlockLayer &l) { return l.spec.moe.top; })), most = std::max(least, n * slices);
+    if (most > w.y_vectors) {
+        if (w.y) HIP_TRY(hipStreamSynchronize(s->st));
+        float *more = nullptr;
+        if (dev_alloc(&more, most * m->dp * 4) == LV_OK) {
+            drop(w.y);
+            w.y = more;
+            w.y_vectors = most;
+        } else if (!w.y) {
+            LV_TRY(dev_alloc(&w.y, least * m->dp * 4));
+            w.y_vectors = least;
+        }
+        LV_TRY(zero_async(w.y, w.y_vectors * m->dp * 4, s->st));
+    }
+    w.y_for = n;
+    return LV_OK;
+}
+
 static int workspace_reserve(BlockSession *s, uint32_t n)
 {
     const BlockModel *m = s->m;
     Workspace &w = s->ws;
     const uint32_t cap = up(n, 128);
-    if (cap <= w.cap) return LV_OK;
+    if (cap <= w.cap) return outputs_reserve(s, n);
     HIP_TRY(hipStreamSynchronize(s->st));
     workspace_free(w);
     const uint64_t T = cap, E = m->elem();
@@ -1286,8 +1322,6 @@ static int workspace_reserve(BlockSession *s, uint32_t n)
     LV_TRY(dev_zeroed(st, &w.x, T * m->copies * m->dp * 4));
     LV_TRY(dev_zeroed(st, &w.act, T * m->dp * E));
     LV_TRY(dev_zeroed(st, &w.y1, T * mx([](const BlockLayer &l) { return l.in.rows; }) * 4));
-    w.y_vectors = T * std::max<uint64_t>(mx([](const BlockLayer &l) { return std::max(1u, l.spec.moe.top); }), !m->f32 && T <= 1024 ? kOutSlices : 1);
-    LV_TRY(dev_zeroed(st, &w.y, w.y_vectors * m->dp * 4));
     LV_TRY(dev_zeroed(st, &w.q, T * E * mx([](const BlockLayer &l) { return std::max(l.spec.attn.heads * l.dp, l.spec.latent.heads * l.dk); })));
     const uint64_t kv = mx([](const BlockLayer &l) { return l.spec.attn.kv_heads * l.dp; });
     LV_TRY(dev_zeroed(st, &w.k, T * E * kv));
@@ -1324,7 +1358,7 @@ static int workspace_reserve(BlockSession *s, uint32_t n)
     // a tile of 128 positions may start at any of the T * top
     LV_TRY(dev_zeroed(st, &w.ff, E * mx([&](const BlockLayer &l) { return (cap * std::max(1u, l.spec.moe.top) + 128) * l.down.kp; })));
     w.cap = cap;
-    return LV_OK;
+    return outputs_reserve(s, n);
 }
 
 // device scratch that follows the number of keys: grown by halves, so that a sequence that gets longer does not allocate every time

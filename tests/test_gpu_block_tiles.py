@@ -58,6 +58,18 @@ def test_dense_tiles(lva, ctx, width, ff, n):
         check_last(d, toks, want, tol)
 
 
+def test_slices_do_not_hang_on_what_came_before(lva, ctx):
+    """the same tokens give the same bits in a new session and behind a batch that has grown its workspace past 1024 tokens"""
+    cfg = zb.config(width=700, streams=2, layers=[zb.layer(zb.ssm(), ff=4100)])
+    W = zb.weights(cfg, seed=4)
+    with Device(lva, zb.upload(ctx, cfg, W, BF16), 2048) as d:
+        for n in (300, 777, 129):
+            toks = tokens_for(cfg, n, 1)
+            first = d.run(toks, (n,))
+            d.run(tokens_for(cfg, 1100, 2), (1100,))
+            assert np.array_equal(d.run(toks, (n,)), first), n
+
+
 @pytest.mark.parametrize("width,ff,n,experts,top", [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4), (64, 24, 17, 3, 2)])
 def test_expert_tiles(lva, ctx, width, ff, n, experts, top):
     cfg = bb.config(width=width, layers=[bb.layer(experts=experts, top=top, ff=ff)])
