@@ -2465,7 +2465,14 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
         const uint32_t first = all ? 0 : n - 1, rows = n - first;
         normalize_kernel<<<dim3(rows), dim3(256), 0, st>>>(b.q, b.x + (size_t)first * D, m->norm, D);
         HIP_TRY(hipGetLastError());
-        LV_TRY(launch_gemv(st, all ? all : s->logits, ow, nullptr, b.q, rows, kGemvStore));
+        // many rows of an output matrix the short copy does not hold: as in longer batches (64 rows of 32001 x 4096 q4_0: a step of two layers
+        // 1.36 ms with a product per row, 0.37 so)
+        if (all && n >= kPrefillMin && ensure_output_copy(s->model) && prefill_reserve(s, n) == LV_OK) {
+            LV_TRY(launch_split(st, s->pf_xh, s->pf_xl, s->pf_xs, b.q, n, D));
+            LV_TRY(launch_gemm_presplit(st, all, hp.vocab, ow, n, s->pf_xh, s->pf_xl, false, s->pf_xs));
+        } else {
+            LV_TRY(launch_gemv(st, all ? all : s->logits, ow, nullptr, b.q, rows, kGemvStore));
+        }
     }
     if (all && with_head) HIP_TRY(hipMemcpyAsync(s->logits, all + (size_t)(n - 1) * hp.vocab, (size_t)hp.vocab * 4, hipMemcpyDeviceToDevice, st));
     return LV_OK;
