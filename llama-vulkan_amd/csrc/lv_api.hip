@@ -2259,23 +2259,24 @@ static void launch_short_rows(hipStream_t st, const ShortArgs &a, uint32_t rt, u
 }
 
 // Row tiles per workgroup (RT) and K slices of a product.  A workgroup's step (eight waves, a chunk each) costs its row tiles plus the
-// activations, worth about 1.5 row tiles; up to 16 tokens and 3 row tiles two workgroups share a CU, else one.  What counts is how
-// many of them a CU works off one after the other; a slice more is written and read again.  Measured in us (7B, T token tiles):
-//   q4_0 gate and up, 1376 tiles: T 1 RT 2/3/4/6 22/18/21/20, T 2 32/29/32/25, T 4 49/43/47/41; q, k and v, 768: T 2 22/16/17/22
-//   q4_0 down, 256 tiles, RT 4 slices 1/2/3/4: T 1 28/16/13/11, T 4 53/29/24/20, RT 2: T 1 24/14/13/12, T 4 40/23/29/24
+// activations, worth about 1.5 row tiles.  What counts is how many of them a CU works off, one after the other or beside one another; a
+// slice more is written and read again.  Measured in us (7B, T token tiles):
+//   q4_0 gate and up, 1376 tiles, RT 2/3/4/6: T 2 32/29/32/25, T 4 49/43/47/41
+//   q4_0 down, 256 tiles, RT 4 slices 1/2/3/4: T 4 53/29/24/20, RT 2: 40/23/29/24
+// and with three parts (T 0 and 1) above the choice, 16 and 19 us gate and up, 11 and 13 q, k and v (768 tiles):
+//   gate and up, RT 2/3/4/6: T 0 3.8/2.4/4.0/0, T 1 7.8/4.6/6.5/0; q, k and v: T 0 3.3/0/0.7/2.9, T 1 5.1/0/0.9/3.4
+//   down, RT 4 slices 1/2/3/4: T 0 9.3/1.2/0/0, T 1 13.5/2.3/0.2/0, RT 2: T 0 4.0/-0.8/1.4/0.5, T 1 8.4/-0.4/3.3/1.3
 static void short_plan(uint32_t tiles, uint32_t nb, uint32_t T, int qt, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
 {
     const uint32_t chunks = nb / 4;
     double best = 1e30;
     for (uint32_t rt : {2u, 3u, 4u, 6u}) {
         if (!short_fits(qt, T, rt)) continue;
-        const uint32_t shared = T <= 1 && rt <= 3 ? 2 : 1;
         for (uint32_t s = 1; s <= (sliced ? (uint32_t)kShortSlices : 1u); s++) {
             const uint32_t per = (chunks + s - 1) / s;
             if ((chunks + per - 1) / per != s) continue;
             const uint32_t steps = (per + kShortWaves - 1) / kShortWaves, held = ((tiles + rt - 1) / rt * s + 255) / 256;
-            const uint32_t rounds = (held + shared - 1) / shared, at_once = held < shared ? held : shared;
-            const double cost = rounds * steps * (at_once * rt + 1.5) + 0.25 * (T ? T : 1) * (s - 1);
+            const double cost = held * steps * (rt + 1.5) + 0.25 * (T ? T : 1) * (s - 1);
             if (cost < best) { best = cost; *best_rt = rt; *best_chunks = per; }
         }
     }

@@ -10,7 +10,7 @@
 //   17 to 64          two fp16 halves as in lv_gemm.h, which takes longer steps and these without the copy: 22 bits, of the norms'
 //                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.
 // Attention likewise: up to 15 tokens fp32 per query (attention_kernel), then short_attn_kernel on fp16 pairs as with longer steps (a
-// layer, 8 tokens at the start of a sequence 6.9 against 10.1 us; 15 tokens behind 1900 about 60 against 11).
+// layer, 8 tokens at the start of a sequence 6.9 against 10.1 us; 15 tokens behind 1900 about 65 against 15).
 //
 // short_gemm_kernel.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
 // tokens; its waves deal the K range among themselves, four quant blocks at a time, and add up through LDS at the end.  A wave so
@@ -27,11 +27,9 @@
 //          the first two parts share an operand (tokens 0 .. 7 and 8 .. 15 of it), the third is half of one.
 // Rows of tokens past the batch are not written; a token only meets its own row of the result.
 //
-// Measured (us per launch, 7B layer, 8 tokens q4_0 / 45 tokens q8_0): q, k and v 11 / 28, attention output 4.5 / 10, gate and up
-// 16 / 47, down 9 / 22 with halves; about 3 of them launch and sum.  The third part costs 0 to 2 us of 8 tokens, since activations
-// come through the vector cache as the weights do.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.10 ms (eight launches of the persistent
-// kernel before; 2.04 with halves, which lose products beyond 65504 and below 2^-13); 45 tokens behind 619, 8 layers of 7B q8_0:
-// 2.77 -> 1.20 ms (128-token GEMM tiles before).
+// Measured (us per launch, 7B layer, 8 tokens q4_0 / 45 tokens q8_0): q, k and v 11 / 28, gate and up 16 / 47, attention output and
+// down together 17 / 32; about 3 of each launch and sum.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.02 ms (eight launches of the
+// persistent kernel before); 45 tokens behind 619, 8 layers of 7B q8_0: 2.77 -> 1.20 ms (128-token GEMM tiles before).
 #pragma once
 
 #include "lv_attn_batch.h"
@@ -138,10 +136,10 @@ struct ShortArgs {
 
 // Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights or, where a block's
 // products take long enough to cover an L2 access, two blocks ahead.  More in flight per wave costs registers, hence waves per
-// CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us, q, k and v for 45 with q8_0 28 -> 96).  With
-// the third part, three row tiles of q4_0 and four blocks ahead take 138 registers, one workgroup a CU; two blocks ahead 126 and two
-// (q, k, v and gate and up together, mean: 8 tokens 15.0 -> 14.6 us, 14 tokens 18.2 -> 17.6; q8_0, 146 and 130: 19.9 -> 21.1, so not there).
-template <int QT, int T, int RT> constexpr int short_ahead() { return T * RT >= 8 || (short_exact(T) && QT == 4 && RT >= 3) ? 2 : 4; }
+// CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us, q, k and v for 45 with q8_0 28 -> 96).  Nor
+// do two workgroups a CU pay: two blocks ahead would let three row tiles of q4_0 and up to 16 tokens into 128 registers (a step of 8
+// tokens of 13B q4_0, 8 layers: 752 us so, 708 with four ahead).
+template <int T, int RT> constexpr int short_ahead() { return T * RT >= 8 ? 2 : 4; }
 // can RT tiles of rows beside T tiles of tokens keep sums, queues and activations in 256 registers (a few values more is fine; three
 // tiles of tokens and six of rows of q4_0 left 220 in memory: 40 tokens of 7B 8.7 ms, 3.4 with three)
 __host__ __device__ constexpr bool short_fits(int qt, uint32_t t, uint32_t rt)
@@ -250,7 +248,7 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
     constexpr int BB = QT == 4 ? 16 : 32;              // code bytes of a block
     constexpr int CW = BB / 4;                         // a lane's dwords of a chunk
     constexpr int CB = short_chunk_bytes(QT, SF32);
-    constexpr int XD = short_ahead<QT, T, RT>();
+    constexpr int XD = short_ahead<T, RT>();
     constexpr int PR = short_round<T, RT>();           // row tiles summed at a time
     __shared__ __attribute__((aligned(16))) float red[PR * NT * kShortWaves * 256];
     const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
