@@ -37,9 +37,11 @@ def check_last(d, toks, want, tol):
 
 
 # width, feed-forward, tokens.  Columns (64 a K step): 1, 3, 11 and more steps in front of the pipelines' two and three stages; rows and
-# tokens one beside a tile's edge; feed-forwards whose way down is cut into 2, 3 and 4 slices, the last one shorter
+# tokens one beside a tile's edge; feed-forwards whose way down is cut into 2 and 4 slices, the last one shorter
 DENSE = [(40, 4100, 1100), (130, 2060, 1030), (700, 2060, 1025), (700, 4100, 1281), (300, 1100, 129), (300, 2113, 127), (257, 4160, 257),
          (1030, 3000, 255), (128, 2048, 513), (129, 1025, 65)]
+# 128 x 128 tiles in 3 slices; 256 x 128 in 1, 2, 3 and 4; 256 x 256 in 3; the last slice shorter
+DENSE += [(1536, 2500, 700), (4100, 1100, 900), (3000, 2060, 900), (2500, 2500, 777), (1536, 3000, 900), (4100, 3000, 900)]
 # streams so wide that the sum of slices and the norm's input would not fit LDS side by side
 DENSE += [(20544, 1152, 33)]
 

@@ -5,6 +5,8 @@ Tolerance: the one the path is specified with (test_gpu_model.py): 1e-2 and 1e-3
 import numpy as np
 import pytest
 
+import ggjt_builder as gb
+
 pytestmark = pytest.mark.gpu
 
 SHAPES = {
@@ -14,15 +16,24 @@ SHAPES = {
     "q8_64": ("Q8_0", dict(vocab=512, dim=384, heads=6, layers=2, ff=896)),
     "q8_128": ("Q8_0", dict(vocab=512, dim=2048, heads=16, layers=1, ff=5504)),
 }
+# wide enough for four and six row tiles a workgroup, as many as 64 tokens and LDS allow at a time
+WIDE = {
+    "q4_wide": ("Q4_0", dict(vocab=512, dim=4096, heads=32, layers=1, ff=11008)),
+    "q8_wide": ("Q8_0", dict(vocab=512, dim=4096, heads=32, layers=1, ff=11008)),
+    "q4_wider": ("Q4_0", dict(vocab=512, dim=5120, heads=40, layers=1, ff=13824)),
+}
 
 
 @pytest.fixture(scope="module")
 def models(lva, tmp_path_factory):
     d = tmp_path_factory.mktemp("short")
     out = {}
-    for i, (name, (wtype, shape)) in enumerate(SHAPES.items()):
+    for i, (name, (wtype, shape)) in enumerate({**SHAPES, **WIDE}.items()):
         out[name] = str(d / f"{name}.ggml")
         lva.write_model(out[name], wtype=getattr(lva, "LV_" + wtype), seed=60 + i, **shape)
+    for name in ("q4_64", "q8_64"):      # file version 1, whose block scales need fp32
+        out[name + "_v1"] = str(d / f"{name}_v1.ggml")
+        gb.convert_to_v1(out[name], out[name + "_v1"], jitter_seed=3)
     return out
 
 
@@ -31,8 +42,12 @@ def close(got, want):
     assert err <= 1e-2 and err <= 1e-3 * np.max(np.abs(want)), (err, np.max(np.abs(want)))
 
 
-@pytest.mark.parametrize("name", list(SHAPES))
-@pytest.mark.parametrize("before,n", [(0, 2), (0, 16), (5, 17), (0, 33), (61, 3), (64, 48), (120, 64), (190, 65), (201, 49)])
+CASES = [(name, b, n) for name in [*SHAPES, "q4_64_v1", "q8_64_v1"]
+         for b, n in [(0, 2), (0, 16), (5, 17), (0, 33), (61, 3), (64, 48), (120, 64), (190, 65), (201, 49)]]
+CASES += [(name, b, n) for name in WIDE for b, n in [(0, 3), (70, 15), (0, 16), (0, 32), (9, 40), (0, 49), (130, 64)]]
+
+
+@pytest.mark.parametrize("name,before,n", CASES)
 def test_short_batch_matches_oracle(lva, orc, ctx, models, name, before, n):
     om = orc.Model(models[name])
     osess = orc.Session(om, 256)
