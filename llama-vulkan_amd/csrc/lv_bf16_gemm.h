@@ -357,9 +357,10 @@ constexpr int wide_stages(int wn) { return wn == 64 ? 3 : 2; }
 constexpr int wide_lds_bytes(int wn) { return wide_stages(wn) * (256 + wide_tokens(wn)) * kBfStep * 2; }
 
 // c += a b; IN_ACC: c in accumulation registers, where the compiler would move them to and fro around every product.  The compiler
-// does not know of these products what has to lie between them and moves of their registers.  It has moves behind a K step (into and
-// out of the loop, spills) but none within, so a step's first product waits for a move into its registers (2 states) and its last one
-// until every product of the step is written (11 states behind an eight-pass product).
+// does not know of these products what has to lie between them and moves of their registers.  It may have moves around a half of a K
+// step (into and out of the loop, at its barrier) but none within, which a test of the built code holds it to: a half's first product
+// waits for a move into its registers (2 states) and its last one until every product of the half is written (11 states behind an
+// eight-pass product).
 template <bool IN_ACC>
 __device__ __forceinline__ void wide_product(lv_f4 &c, const lv_bf8 &a, const lv_bf8 &b, bool first = false, bool last = false)
 {
@@ -439,7 +440,7 @@ __global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemm
         // first half: with three stages the loads of stage s + 2 go where stage s - 1 was
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f0.a[m / NJ], f0.b[m % NJ], m == 0);
+            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f0.a[m / NJ], f0.b[m % NJ], m == 0, m == NM - 1);
             if (m % 2 == 0 && m / 2 < NR) read_one(f1, bf_lds + slot * STAGE, 1, m / 2);
             if (NST == 3 && m % 2 == 1 && m / 2 < LPS) issue_one(s + 2, free_slot, m / 2);
             __builtin_amdgcn_sched_barrier(0);
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemm
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f1.a[m / NJ], f1.b[m % NJ], false, m == NM - 1);
+            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f1.a[m / NJ], f1.b[m % NJ], m == 0, m == NM - 1);
             if (m % 2 == 0 && m / 2 < NR) read_one(f0, bf_lds + next * STAGE, 0, m / 2);
             if (NST == 2 && m % 4 == 1 && m / 4 < LPS) issue_one(s + 2, free_slot, m / 4);
             __builtin_amdgcn_sched_barrier(0);

@@ -43,3 +43,26 @@ def test_short_products_fit_their_registers(spills):
     short = {n: v for n, v in spills.items() if "short_gemm_kernel" in n}
     assert len(short) > 40
     assert {n: v for n, v in short.items() if v > 32} == {}
+
+
+def test_nothing_moves_between_matrix_products_in_inline_assembly(code_objects):
+    """gemm_wide_kernel with 256-token tiles names its matrix instructions in inline assembly, where the compiler knows nothing of the
+    states that have to lie between one of them and a move of its registers: it must have no move, no spill and no other matrix
+    instruction between the first and the last product of a half step, and the waits around a half must be there"""
+    bodies = {}
+    for f in code_objects:
+        text = subprocess.run([tool("llvm-objdump"), "-d", "--no-show-raw-insn", f], check=True, capture_output=True, text=True).stdout
+        parts = re.split(r"\n[0-9a-f]+ <(\S+)>:\n", text)
+        bodies.update((n, b) for n, b in zip(parts[1::2], parts[2::2]) if "gemm_wide_kernel" in n and "ELi128E" in n)
+    assert len(bodies) >= 3
+    for name, body in bodies.items():
+        ins = [line.split("//")[0].strip() for line in body.split("\n") if line.strip()]
+        at = [i for i, x in enumerate(ins) if "mfma" in x]
+        assert len(at) == 128, name
+        for half in (at[:64], at[64:]):
+            inside = ins[half[0]:half[-1] + 1]
+            # operands of the next half come from LDS, its loads go there; addresses are all else that is computed
+            allowed = r"v_mfma_f32_16x16x32_bf16 a\[|ds_read_b128 v\[|global_load_lds_dwordx4|s_|v_(lshl_add_u64|add3_u32|add_u32_e32|add_co_u32|addc_co_u32|lshlrev_b64|mad_u64_u32)"
+            assert [x for x in inside if not re.match(allowed, x)] == [], name
+            assert re.match(r"s_nop [1-9]", ins[half[0] - 1]), (name, ins[half[0] - 1])
+            assert ins[half[-1] + 1] == "s_nop 15", (name, ins[half[-1] + 1])
