@@ -806,10 +806,12 @@ template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs 
         return gemv_rows_together(units) == 2 ? launch_gemv<MODE, INPUT, 2, 2>(st, a, units, lds) : launch_gemv<MODE, INPUT, 1, 4>(st, a, units, lds);
     } else {
         // a workgroup of 16 waves takes one row at a time: 45.0 us with two, 39.4 with one (18560 and 32000 x 4096, four streams)
-        // one row at a time: eight steps ahead, or a row of up to 2048 columns (8848 x 2048: 11.0 us with eight, 10.1 with four)
+        // one row at a time: eight steps ahead, or four, which is a row of up to 2048 columns.  Eight and four, us: 8848 x 2048 11.0 and
+        // 10.1; means of all products of Somesun 2048 behind a norm 7.8 and 7.2, of Zedenex 2048 behind streams 11.6 and 10.9.  Beyond 2048
+        // columns it hangs on the rows: few of them (64 x 4096, a router) 5.7 and 6.3, many (Zedenex 4096 behind streams) 25.9 and 24.6
         return gemv_threads(INPUT) == 512 && gemv_rows_together(a.rows) == 2 ? launch_gemv<MODE, INPUT, 2, 4>(st, a, a.rows, lds)
-               : a.kp <= 2048                  ? launch_gemv<MODE, INPUT, 1, 4>(st, a, a.rows, lds)
-                                               : launch_gemv<MODE, INPUT, 1, 8>(st, a, a.rows, lds);
+               : a.kp <= 2048                                                ? launch_gemv<MODE, INPUT, 1, 4>(st, a, a.rows, lds)
+                                                                             : launch_gemv<MODE, INPUT, 1, 8>(st, a, a.rows, lds);
     }
 }
 
