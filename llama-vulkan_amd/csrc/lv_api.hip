@@ -227,7 +227,7 @@ struct lv_session {
     uint16_t *pf_xh = nullptr, *pf_xl = nullptr;
     uint16_t *pf_fh = nullptr, *pf_fl = nullptr;   // the feed-forward's inner activations (their producer still reads pf_xh / pf_xl)
     float *pf_xs = nullptr;   // per token: the power of two the halves written by prefill_norm_kernel are scaled down by
-    uint8_t *short_ws = nullptr;   // workspace of short batches (ShortBuffers), allocated at first use, sized for the backlog
+    uint8_t *short_ws = nullptr;   // workspace of short batches (ShortBuffers), allocated at first use
     // operand planes of the batched attention (one layer's worth, rewritten per layer): four of attn_plane_halfs() each
     uint16_t *pf_planes = nullptr;
     size_t pf_plane_halfs = 0;
@@ -727,12 +727,12 @@ static size_t attn_part_floats(uint32_t batch, uint32_t heads, uint32_t splits, 
 
 static int launch_attention(hipStream_t st, float *out, const uint16_t *kc, const uint16_t *vc, const float *q,
                             const float2 *trig, float *part, uint32_t *counters, const uint32_t *pos_ptr, uint32_t pos_add,
-                            uint32_t backlog, uint32_t heads, uint32_t rot, uint32_t batch, uint32_t positions = 0)
+                            uint32_t backlog, uint32_t heads, uint32_t rot, uint32_t batch)
 {
     AttnArgs a{};
     a.out = out; a.kcache = kc; a.vcache = vc; a.q = q; a.trig = trig; a.part = part; a.counters = counters;
     a.pos_ptr = pos_ptr; a.pos_add = pos_add; a.heads = heads; a.backlog = backlog; a.chunk = kAttnChunk;
-    a.splits = ((positions ? positions : backlog) + kAttnChunk - 1) / kAttnChunk;     // positions: the launch needs to look at no more
+    a.splits = (backlog + kAttnChunk - 1) / kAttnChunk;
     const dim3 grid(heads, a.splits, batch);
     const size_t lds = sizeof(float) * 4 * (rot + 1);
     switch (rot) {
@@ -1708,8 +1708,6 @@ extern "C" int lv_session_reserve(lv_session *s, uint32_t backlog)
     s->attn_part = nullptr;
     (void)hipFree(s->attn_counters);
     s->attn_counters = nullptr;
-    (void)hipFree(s->short_ws);
-    s->short_ws = nullptr;
     (void)hipFree(s->trace_attn);
     s->trace_attn = nullptr;
     s->backlog = 0;
@@ -2202,10 +2200,9 @@ constexpr uint32_t kShortSplits = 16;      // parts the attention's positions ar
 
 struct ShortBuffers {
     float *x, *q, *parts[kShortSlices], *xscale, *num, *den;
-    uint32_t *counters;      // of attention_kernel, zero between launches
     uint8_t *act, *ff;
 };
-static size_t short_layout(const lv_hparams &hp, uint32_t backlog, uint8_t *base, ShortBuffers *b)
+static size_t short_layout(const lv_hparams &hp, uint8_t *base, ShortBuffers *b)
 {
     const size_t D = hp.dim, row = D * 4 * kShortTokens;
     size_t at = 0;
@@ -2214,9 +2211,8 @@ static size_t short_layout(const lv_hparams &hp, uint32_t backlog, uint8_t *base
     b->q = (float *)take(row);
     for (float *&p : b->parts) p = (float *)take(row);
     b->xscale = (float *)take(kShortTokens * 4);
-    b->num = (float *)take(std::max(row * kShortSplits, 4 * attn_part_floats(kPrefillMin, hp.heads, (backlog + kAttnChunk - 1) / kAttnChunk, hp.rot)));
+    b->num = (float *)take(row * kShortSplits);
     b->den = (float *)take((size_t)kShortTokens * hp.heads * kShortSplits * 4);
-    b->counters = (uint32_t *)take((size_t)kPrefillMin * hp.heads * 4);
     b->act = take(short_act_bytes(hp.dim, kShortTokens));
     b->ff = take(short_act_bytes(hp.ff, kShortTokens));
     return at;
@@ -2226,16 +2222,9 @@ static size_t short_layout(const lv_hparams &hp, uint32_t backlog, uint8_t *base
 static bool short_reserve(lv_session *s)
 {
     if (s->short_ws) return true;
-    const lv_hparams &hp = s->model->hp;
     ShortBuffers b;
-    if (hipMalloc(reinterpret_cast<void **>(&s->short_ws), short_layout(hp, s->backlog, nullptr, &b)) != hipSuccess) {
-        (void)hipGetLastError();
-        s->short_ws = nullptr;
-        return false;
-    }
-    short_layout(hp, s->backlog, s->short_ws, &b);
-    if (zero_async(b.counters, (size_t)kPrefillMin * hp.heads * 4, s->stream) == LV_OK) return true;
-    (void)hipFree(s->short_ws);
+    if (hipMalloc(reinterpret_cast<void **>(&s->short_ws), short_layout(s->model->hp, nullptr, &b)) == hipSuccess) return true;
+    (void)hipGetLastError();
     s->short_ws = nullptr;
     return false;
 }
@@ -2372,15 +2361,6 @@ static int launch_short_norm(hipStream_t st, const ShortBuffers &b, const float 
 static int launch_short_attention(hipStream_t st, const lv_session *s, const ShortBuffers &b, uint32_t layer, uint32_t pos, uint32_t n, uint32_t ftype)
 {
     const lv_hparams &hp = s->model->hp;
-    if (n < kPrefillMin) {
-        float *const out = b.parts[0];       // the norm before has taken it in
-        LV_TRY(launch_attention(st, out, kv_ptr(s, layer, 0), kv_ptr(s, layer, 1), b.q, s->trig, b.num, b.counters, nullptr, pos, s->backlog, hp.heads, hp.rot, n, pos + n));
-        const dim3 grid((hp.dim / 8 + 255) / 256, n);
-        if (ftype == LV_Q4_0) short_rows_kernel<4><<<grid, dim3(256), 0, st>>>(b.act, out, hp.dim, short_tiles(n));
-        else short_rows_kernel<8><<<grid, dim3(256), 0, st>>>(b.act, out, hp.dim, short_tiles(n));
-        HIP_TRY(hipGetLastError());
-        return LV_OK;
-    }
     const uint32_t tiles = (pos + n + kAttnBatchK - 1) / kAttnBatchK, want = hp.heads < 512 ? 512 / hp.heads : 1;
     const uint32_t most = want < kShortSplits ? want : kShortSplits, per = (tiles + most - 1) / most, splits = (tiles + per - 1) / per;
     ShortAttnArgs a{};
@@ -2391,6 +2371,10 @@ static int launch_short_attention(hipStream_t st, const lv_session *s, const Sho
     switch (hp.rot) {
 #define LV_SHORT_ATTN(R)                                                                                                              \
     case R:                                                                                                                           \
+        if (n < kPrefillMin) {                                                                                                        \
+            short_attn_exact_kernel<R><<<dim3(hp.heads, splits), dim3(256), 0, st>>>(a);                                              \
+            break;                                                                                                                    \
+        }                                                                                                                             \
         HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(short_attn_kernel<R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
         short_attn_kernel<R><<<dim3(hp.heads, splits), dim3(256), lds, st>>>(a);                                                      \
         break;
@@ -2420,7 +2404,7 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
     const bool sf32 = m->layers[0].wq.view.scales_f32 != nullptr;
     hipStream_t st = s->stream;
     ShortBuffers b;
-    short_layout(hp, s->backlog, s->short_ws, &b);
+    short_layout(hp, s->short_ws, &b);
     LV_TRY(launch_embed(s, b.x, s->cfg_host + 1, s->cfg_host[0], idx0, n));
     HIP_TRY(hipGetLastError());
 

@@ -9,8 +9,7 @@
 //                     token (other paths, no room for the copy below), in fp32 throughout, and is held to the same.
 //   17 to 64          two fp16 halves as in lv_gemm.h, which takes longer steps and these without the copy: 22 bits, of the norms'
 //                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.
-// Attention likewise: up to 15 tokens fp32 per query (attention_kernel), then short_attn_kernel on fp16 pairs as with longer steps (a
-// layer, 8 tokens at the start of a sequence 6.9 against 10.1 us; 15 tokens behind 1900 about 65 against 15).
+// Attention likewise: up to 15 tokens in fp32 (short_attn_exact_kernel), then short_attn_kernel on fp16 pairs as with longer steps.
 //
 // short_gemm_kernel.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
 // tokens; its waves deal the K range among themselves, four quant blocks at a time, and add up through LDS at the end.  A wave so
@@ -507,18 +506,6 @@ __global__ __launch_bounds__(1024) void short_norm_kernel(ShortNormArgs a)
     short_put(a.act, i >> 2, row, i & 3, a.tiles, f);
 }
 
-// rows of `dim` floats as a product's activations.  grid (dim / 8 / 256 rounded up, rows)
-template <int QT>
-__global__ __launch_bounds__(256) void short_rows_kernel(uint8_t *__restrict__ act, const float *__restrict__ x, uint32_t dim, uint32_t tiles)
-{
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= dim / 8) return;
-    const float *src = x + (size_t)blockIdx.y * dim + (i >> 2) * 32;
-    float f[8];
-    short_order<QT>(f, *reinterpret_cast<const float4 *>(src + short_run_a<QT>(i & 3)), *reinterpret_cast<const float4 *>(src + short_run_b<QT>(i & 3)), short_exact(tiles));
-    short_put(act, i >> 2, blockIdx.y, i & 3, tiles, f);
-}
-
 // Attention of 16 to 64 tokens: attention_batch_kernel's arithmetic, with the cache positions shared out over workgroups and the
 // operand planes made on the way into LDS (a plane would be used once).  Without a running maximum the parts of a row are plain
 // sums: numerators [split][n][H*R] and denominators [split][n][H], put together by short_attn_combine_kernel.  64 KB of LDS: two
@@ -764,6 +751,166 @@ __global__ __launch_bounds__(256, 2) void short_attn_kernel(ShortAttnArgs a)
             const uint32_t z = 32 * qt + 8 * (r / 4) + 4 * hh + (r % 4);
             if (z < a.n) a.num[(part + z) * D + (size_t)h * R + 32 * d + n32] = acc[d][r] + xch[z * XS + 32 * d + n32];
         }
+}
+
+// Attention of 2 to 15 tokens: fp32 throughout, on the fp32 matrix instruction, whose 16 columns are the step's queries.  attention_kernel
+// reads a head's cache rows and rotations again for every query (15 queries behind 1900 positions: 0.9 GB through the L2s); here they are read
+// once, rotated in registers and multiplied with all queries, 64 instructions per 16 positions whatever n is.  A layer of 7B, us with what makes
+// the output projection's operands of it: 15 queries behind 1900 positions 65 and 25, 8 at the start of a sequence 10 and 7.
+// Rotation by absolute positions; tiles, splits, num, den and act as short_attn_kernel.  A wave takes 16 of a tile's 64 positions; nothing is exchanged before the end:
+//   scores    A = K (row: position l % 16), B = q (column: query l % 16), step j contracts dims g R/4 + j of the four lane groups g = l / 16
+//   weighted  the result's register r holds position 4 g + r, which is how B = weights is wanted; A = V, rows m of tile t being dim m R/16 + t
+template <int R>
+__global__ __launch_bounds__(256, 2) void short_attn_exact_kernel(ShortAttnArgs a)
+{
+    constexpr int TK = kAttnBatchK;
+    constexpr int KL = R / 4, VD = R / 16, C8 = R / 8, XS = R + 4;
+    __shared__ __attribute__((aligned(16))) float xch[4 * 16 * XS];
+    __shared__ float den_s[4][16];
+    const uint32_t h = blockIdx.x, H = a.heads, D = H * R;
+    const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t rows = min(a.pos0 + a.n, a.backlog);               // positions that hold data
+    const uint32_t tile_end = min((blockIdx.y + 1) * a.tiles_per_split, (rows + TK - 1) / TK);
+
+    uint4 kq[KL / 8];
+    float4 cs[KL / 4];
+    uint32_t vq[4][VD / 2];
+    auto fetch = [&](uint32_t base) {                                 // past the data: the last row again, masked below
+        const uint32_t p = min(base + l16, rows - 1);
+#pragma unroll
+        for (int i = 0; i < KL / 8; i++) kq[i] = *reinterpret_cast<const uint4 *>(a.kcache + (size_t)p * D + (size_t)h * R + g * KL + i * 8);
+#pragma unroll
+        for (int i = 0; i < KL / 4; i++) cs[i] = *reinterpret_cast<const float4 *>(a.trig_abs + (size_t)p * (R / 2) + g * (KL / 2) + i * 2);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            __builtin_memcpy(vq[r], __builtin_assume_aligned(a.vcache + (size_t)min(base + 4 * g + r, rows - 1) * D + (size_t)h * R + l16 * VD, VD * 2), VD * 2);
+    };
+    fetch(blockIdx.y * a.tiles_per_split * TK + 16 * wave);
+
+    const bool zok = (uint32_t)l16 < a.n;
+    const uint32_t limit = a.pos0 + l16;                              // the last position query l16 sees
+    float q[KL];
+    {
+        const float *qr = a.q + (size_t)(zok ? l16 : 0) * D + (size_t)h * R + g * KL;
+        const float2 *tr = a.trig_abs + (size_t)min(limit, a.backlog - 1) * (R / 2) + g * (KL / 2);
+#pragma unroll
+        for (int i = 0; i < KL / 4; i++) {
+            const float4 x = *reinterpret_cast<const float4 *>(qr + i * 4), c = *reinterpret_cast<const float4 *>(tr + i * 2);
+            q[4 * i] = zok ? x.x * c.x - x.y * c.y : 0.f;
+            q[4 * i + 1] = zok ? x.x * c.y + x.y * c.x : 0.f;
+            q[4 * i + 2] = zok ? x.z * c.z - x.w * c.w : 0.f;
+            q[4 * i + 3] = zok ? x.z * c.w + x.w * c.z : 0.f;
+        }
+    }
+    const float scale = rsqrtf((float)R);
+    lv_f4v acc[VD];
+#pragma unroll
+    for (int d = 0; d < VD; d++) acc[d] = lv_f4v{0.f, 0.f, 0.f, 0.f};
+    float den = 0.f;
+
+    for (uint32_t it = blockIdx.y * a.tiles_per_split; it < tile_end; it++) {
+        const uint32_t base = it * TK + 16 * wave;
+        if (base >= rows) break;
+        float k[KL];
+#pragma unroll
+        for (int i = 0; i < KL / 4; i++) {
+            const uint32_t w0 = i & 1 ? kq[i / 2].z : kq[i / 2].x, w1 = i & 1 ? kq[i / 2].w : kq[i / 2].y;
+            const float x0 = half_bits_to_float((uint16_t)w0), y0 = half_bits_to_float((uint16_t)(w0 >> 16));
+            const float x1 = half_bits_to_float((uint16_t)w1), y1 = half_bits_to_float((uint16_t)(w1 >> 16));
+            k[4 * i] = x0 * cs[i].x - y0 * cs[i].y;
+            k[4 * i + 1] = x0 * cs[i].y + y0 * cs[i].x;
+            k[4 * i + 2] = x1 * cs[i].z - y1 * cs[i].w;
+            k[4 * i + 3] = x1 * cs[i].w + y1 * cs[i].z;
+        }
+        uint32_t v[4][VD / 2];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int i = 0; i < VD / 2; i++) v[r][i] = vq[r][i];
+        if (it + 1 < tile_end) fetch(base + TK);
+        lv_f4v sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < KL; j++) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j], q[j], sc, 0, 0, 0);
+        float e[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uint32_t p = base + 4 * g + r;
+            const float w = __expf(sc[r] * scale);
+            e[r] = zok && p <= limit && p < rows ? w : 0.f;
+            den += e[r];
+        }
+        if (base + 15 > a.pos0) {
+            // Rows that some queries do not see.  A weight of zero times an infinity or a NaN of such a row would reach them: these values
+            // are left to the queries that see them.
+            auto wild = [](uint32_t half) { return (half & 0x7c00u) == 0x7c00u; };
+            bool any = false;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int i = 0; i < VD / 2; i++) {
+                    const bool lo = wild(v[r][i]), hi = wild(v[r][i] >> 16);
+                    any |= lo || hi;
+                    v[r][i] &= (lo ? 0u : 0xffffu) | (hi ? 0u : 0xffff0000u);
+                }
+            if (__any(any)) {
+#pragma unroll
+                for (int m = 0; m < 16; m++) {
+                    const uint32_t p = base + m;
+                    const float w = __shfl(e[m & 3], (m >> 2) * 16 + l16, kWave);
+                    const uint16_t *vr = a.vcache + (size_t)min(p, rows - 1) * D + (size_t)h * R + 4 * g * VD;
+                    if (!zok || p > limit || p >= rows) continue;
+#pragma unroll
+                    for (int i = 0; i < 4 * VD; i++)
+                        if (wild(vr[i])) acc[i % VD][i / VD] = fmaf(w, half_bits_to_float(vr[i]), acc[i % VD][i / VD]);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int d = 0; d < VD; d++)
+                acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(half_bits_to_float((uint16_t)(v[r][d / 2] >> (16 * (d & 1)))), e[r], acc[d], 0, 0, 0);
+    }
+    // acc[d][r]: dim (4 g + r) VD + d of query l16.  The waves' sums, then out
+    den += __shfl_xor(den, 16, kWave);
+    den += __shfl_xor(den, 32, kWave);
+    if (g == 0) den_s[wave][l16] = den;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int d = 0; d < VD; d++) xch[(wave * 16 + l16) * XS + (4 * g + r) * VD + d] = acc[d][r];
+    __syncthreads();
+    auto total = [&](uint32_t z, uint32_t d) {
+        float4 s = *reinterpret_cast<const float4 *>(xch + z * XS + d);
+#pragma unroll
+        for (int w = 1; w < 4; w++) {
+            const float4 x = *reinterpret_cast<const float4 *>(xch + (w * 16 + z) * XS + d);
+            s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+        }
+        return s;
+    };
+    auto weight = [&](uint32_t z) { return (den_s[0][z] + den_s[1][z]) + (den_s[2][z] + den_s[3][z]); };
+    if (a.act) {
+        for (uint32_t i = t; i < a.n * C8; i += 256) {
+            const uint32_t z = i / C8, c = i % C8, d = (c >> 2) * 32, og = c & 3;
+            const float w = weight(z);
+            float4 va = total(z, d + (a.q8 ? short_run_a<8>(og) : short_run_a<4>(og))), vb = total(z, d + (a.q8 ? short_run_b<8>(og) : short_run_b<4>(og)));
+            va.x /= w; va.y /= w; va.z /= w; va.w /= w;
+            vb.x /= w; vb.y /= w; vb.z /= w; vb.w /= w;
+            float f[8];
+            if (a.q8) short_order<8>(f, va, vb, true);
+            else short_order<4>(f, va, vb, true);
+            short_put(a.act, (h * R + d) / 32, z, og, a.tiles, f);
+        }
+        return;
+    }
+    const size_t part = (size_t)blockIdx.y * a.n;
+    for (uint32_t i = t; i < a.n * (R / 4); i += 256) {
+        const uint32_t z = i / (R / 4), d = i % (R / 4) * 4;
+        *reinterpret_cast<float4 *>(a.num + (part + z) * D + (size_t)h * R + d) = total(z, d);
+    }
+    if ((uint32_t)t < a.n) a.den[(part + t) * H + h] = weight(t);
 }
 
 // numerators and denominators of all splits, in order -> the output projection's activations.  grid (D / 8 / 256 rounded up, n)

@@ -43,7 +43,8 @@ def close(got, want):
 
 
 CASES = [(name, b, n) for name in [*SHAPES, "q4_64_v1", "q8_64_v1"]
-         for b, n in [(0, 2), (0, 16), (5, 17), (0, 33), (61, 3), (64, 48), (120, 64), (190, 65), (201, 49)]]
+         for b, n in [(0, 2), (0, 16), (5, 17), (0, 33), (61, 3), (64, 48), (120, 64), (190, 65), (201, 49),
+                       (1, 15), (2, 15), (49, 15), (50, 15), (200, 2), (239, 15)]]      # attention of up to 15 tokens: edges of its 16 and 64 positions
 CASES += [(name, b, n) for name in WIDE for b, n in [(0, 3), (70, 15), (0, 16), (0, 32), (9, 40), (0, 49), (130, 64)]]
 
 
@@ -130,9 +131,8 @@ def test_two_tokens_of_a_wide_model(lva, ctx, tmp_path, wtype, same):
     a.close(); b.close(); model.close()
 
 
-def scaled_file(src, dst, powers):
-    """a copy of a version-3 file with the blocks of some tensors multiplied by powers of two; powers: end of the name -> exponent"""
-    data = np.fromfile(src, dtype=np.uint8)
+def tensors(data):
+    """name, type, elements and bytes of a version-3 file's tensors"""
     cur = 36
     for _ in range(int(data[8:12].view(np.uint32)[0])):
         cur += 8 + int(data[cur:cur + 4].view(np.int32)[0])
@@ -142,11 +142,18 @@ def scaled_file(src, dst, powers):
         name = data[cur + 12 + 4 * dims:cur + 12 + 4 * dims + name_len].tobytes().decode()
         cur = (cur + 12 + 4 * dims + name_len + 31) & ~31
         size = {0: 4 * count, 2: count // 32 * 18, 8: count // 32 * 34}[ftype]
+        yield name, ftype, count, data[cur:cur + size]
+        cur += size
+
+
+def scaled_file(src, dst, powers):
+    """a copy of a version-3 file with the blocks of some tensors multiplied by powers of two; powers: end of the name -> exponent"""
+    data = np.fromfile(src, dtype=np.uint8)
+    for name, _, count, payload in tensors(data):
         for end, e in powers.items():
             if name.endswith(end + ".weight"):
-                d = data[cur:cur + size].reshape(-1, size // (count // 32))
+                d = payload.reshape(-1, len(payload) // (count // 32))
                 d[:, :2] = np.ldexp(d[:, :2].copy().view(np.float16).astype(np.float32), e).astype(np.float16).view(np.uint8)
-        cur += size
     data.tofile(dst)
     return dst
 
@@ -176,3 +183,38 @@ def test_short_batch_keeps_the_range_of_one_token_steps(lva, orc, ctx, models, t
         close(a.logits(), want)
         a.close(); b.close(); osess.close()
     model.close(); om.close()
+
+
+@pytest.mark.parametrize("name", ["q4_32", "q8_64", "q4_128"])
+@pytest.mark.parametrize("n", [2, 6, 15])
+def test_a_token_beyond_fp16_does_not_reach_those_before_it(lva, ctx, models, tmp_path, name, n):
+    """cache rows of infinities (and of NaN in the layer behind) in a step: the tokens that do not see them give the bits they give without"""
+    path, wild = str(tmp_path / "wild.ggml"), 7
+    data = np.fromfile(models[name], dtype=np.uint8)
+    dim = SHAPES[name][1]["dim"]
+    for tensor, ftype, _, payload in tensors(data):
+        if tensor == "tok_embeddings.weight":
+            assert ftype == 0
+            table = payload.view(np.float32).reshape(-1, dim)
+            table[:, 0] = 0
+            table[wild] = np.eye(dim)[0]
+        if tensor == "layers.0.attention_norm.weight":
+            payload.view(np.float32)[0] = 1e8
+    data.tofile(path)
+    model = lva.Model(ctx, path)
+    toks = np.array(lva.synth_tokens(n, 20, 480, seed=n), dtype=np.uint32)
+    rows = []
+    for change in (False, True):
+        s = lva.Session(model, 128)
+        s.keep_all_logits()
+        if change:
+            toks[n - 2 if n > 2 else 1] = wild
+        s.begin(toks, 0)
+        rows.append(s.logits_rows(0, n))
+        if change:
+            assert np.isinf(s.kv(0, 1, n).view(np.float16)).any()
+        s.close()
+    seen = n - 2 if n > 2 else 1
+    assert np.isfinite(rows[0]).all()
+    assert np.array_equal(rows[0][:seen], rows[1][:seen])
+    model.close()
