@@ -27,7 +27,7 @@
 // Rows of tokens past the batch are not written; a token only meets its own row of the result.
 //
 // Measured (us per launch, 7B layer, 8 tokens q4_0 / 45 tokens q8_0): q, k and v 11 / 28, gate and up 16 / 47, attention output and
-// down together 17 / 32; about 3 of each launch and sum.  A step of 8 tokens, 7B q4_0: 7.32 -> 2.02 ms (eight launches of the
+// down together 17 / 32; about 3 of each launch and sum.  A step of 8 tokens, 7B q4_0: 7.31 -> 2.00 ms (eight launches of the
 // persistent kernel before); 45 tokens behind 619, 8 layers of 7B q8_0: 2.77 -> 1.20 ms (128-token GEMM tiles before).
 #pragma once
 
