@@ -200,7 +200,7 @@ int lv_argmax(lv_session *s, uint32_t *token);
 /* Enables/disables hipGraph replay for n == 1 steps (on by default); off = plain stream launches. */
 int lv_session_use_graph(lv_session *s, int enable);
 /* How n == 1 steps are executed, and in a session whose path has been set to another than LV_PATH_AUTO also the tokens of
- * steps of 2 to 15 tokens, one after the other (longer ones as batches).  With LV_PATH_AUTO steps of 2 to 64 tokens have
+ * steps of 2 to 15 tokens, one after the other (longer ones as batches).  With LV_PATH_AUTO steps of 2 to 256 tokens have
  * kernels of their own where the model's shape allows (q4_0 or q8_0, width and feed-forward width multiples of 128).  The reference has one way (replay the recorded command buffers,
  * llava_command_buffer.cpp:47-55); here there are three, all computing the same step:
  *   LV_PATH_KERNELS     one launch per operator on the session's stream

@@ -24,7 +24,7 @@
 #include "lv_gemm.h"
 #include "lv_gemv_wide.h"
 #include "lv_attn_batch.h"
-#include "lv_short.h"
+#include "lv_mid.h"
 
 using namespace lv;
 
@@ -2079,7 +2079,9 @@ static int launch_prefill_norm(hipStream_t st, lv_session *s, const float *w, ui
 
 // Rows idx0 .. idx0+n-1 of the step at once (llava_layer.cpp:39-75 with batch > 1).  Row z sees cache rows
 // 0..pos+z: all K/V rows of the chunk are appended before any row attends, rows above its own are masked.
-static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_head, uint32_t row_base)
+static int record_mid_layers(lv_session *s, uint32_t idx0, uint32_t n, float *const parts[kGemmMaxMats], uint32_t *pending_out);
+// mid: the products of lv_mid.h, n at most kMidTokens
+static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_head, uint32_t row_base, bool mid)
 {
     if (s->block) {
         const BlockTrace t = block_trace(s);
@@ -2098,7 +2100,8 @@ static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_he
     // and of the down projection; `pending` of them wait to be added to the residual stream by the next norm
     float *const parts[kGemmMaxMats] = {s->pf_q, s->pf_k, s->pf_v, s->pf_vo};
     uint32_t pending = 0;
-    for (uint32_t li = 0; li < hp.layers; li++) {
+    if (mid) LV_TRY(record_mid_layers(s, idx0, n, parts, &pending));
+    for (uint32_t li = mid ? hp.layers : 0; li < hp.layers; li++) {
         const LayerWeights &lw = m->layers[li];
         const bool qkv_same = gemm_same(lw.wq, lw.wk) && gemm_same(lw.wq, lw.wv), gate_same = gemm_same(lw.w3, lw.w1);
         const float *xscale = nullptr;
@@ -2239,33 +2242,26 @@ template <int QT, int T>
 static void launch_short_rows(hipStream_t st, const ShortArgs &a, uint32_t rt, uint32_t slices, bool sf32)
 {
     if (rt == 2) launch_short_kernel<QT, T, 2>(st, a, slices, sf32);
-    if constexpr (short_fits(QT, T, 3))
-        if (rt == 3) launch_short_kernel<QT, T, 3>(st, a, slices, sf32);
-    if constexpr (short_fits(QT, T, 4))
-        if (rt == 4) launch_short_kernel<QT, T, 4>(st, a, slices, sf32);
-    if constexpr (short_fits(QT, T, 6))
-        if (rt == 6) launch_short_kernel<QT, T, 6>(st, a, slices, sf32);
+    if (rt == 3) launch_short_kernel<QT, T, 3>(st, a, slices, sf32);
+    if (rt == 4) launch_short_kernel<QT, T, 4>(st, a, slices, sf32);
+    if (rt == 6) launch_short_kernel<QT, T, 6>(st, a, slices, sf32);
 }
 
 // Row tiles per workgroup (RT) and K slices of a product.  A workgroup's step (eight waves, a chunk each) costs its row tiles plus the
 // activations, worth about 1.5 row tiles.  What counts is how many of them a CU works off, one after the other or beside one another; a
-// slice more is written and read again.  Measured in us (7B, T token tiles):
-//   q4_0 gate and up, 1376 tiles, RT 2/3/4/6: T 2 32/29/32/25, T 4 49/43/47/41
-//   q4_0 down, 256 tiles, RT 4 slices 1/2/3/4: T 4 53/29/24/20, RT 2: 40/23/29/24
-// and with three parts (T 0 and 1) above the choice, 16 and 19 us gate and up, 11 and 13 q, k and v (768 tiles):
+// slice more is written and read again.  Measured in us above the choice, 16 and 19 us gate and up, 11 and 13 q, k and v (768 tiles):
 //   gate and up, RT 2/3/4/6: T 0 3.8/2.4/4.0/0, T 1 7.8/4.6/6.5/0; q, k and v: T 0 3.3/0/0.7/2.9, T 1 5.1/0/0.9/3.4
 //   down, RT 4 slices 1/2/3/4: T 0 9.3/1.2/0/0, T 1 13.5/2.3/0.2/0, RT 2: T 0 4.0/-0.8/1.4/0.5, T 1 8.4/-0.4/3.3/1.3
-static void short_plan(uint32_t tiles, uint32_t nb, uint32_t T, int qt, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
+static void short_plan(uint32_t tiles, uint32_t nb, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
 {
     const uint32_t chunks = nb / 4;
     double best = 1e30;
     for (uint32_t rt : {2u, 3u, 4u, 6u}) {
-        if (!short_fits(qt, T, rt)) continue;
         for (uint32_t s = 1; s <= (sliced ? (uint32_t)kShortSlices : 1u); s++) {
             const uint32_t per = (chunks + s - 1) / s;
             if ((chunks + per - 1) / per != s) continue;
             const uint32_t steps = (per + kShortWaves - 1) / kShortWaves, held = ((tiles + rt - 1) / rt * s + 255) / 256;
-            const double cost = held * steps * (rt + 1.5) + 0.25 * (T ? T : 1) * (s - 1);
+            const double cost = held * steps * (rt + 1.5) + 0.25 * (s - 1);
             if (cost < best) { best = cost; *best_rt = rt; *best_chunks = per; }
         }
     }
@@ -2277,18 +2273,155 @@ static int launch_short_gemm(hipStream_t st, ShortArgs a, uint32_t ftype, bool s
     const int qt = ftype == LV_Q4_0 ? 4 : 8;
     uint32_t rt = 2;
     if (!a.w) return fail(LV_ERR_STATE, "short batch: the matrix has no copy");
-    short_plan(a.tiles, a.nb, T, qt, sliced, &rt, &a.slice_chunks);
+    short_plan(a.tiles, a.nb, sliced, &rt, &a.slice_chunks);
     const uint32_t slices = (a.nb / 4 + a.slice_chunks - 1) / a.slice_chunks;
     if (slices_out) *slices_out = slices;
 #define LV_SHORT(QT, TT) case QT * 8 + TT: launch_short_rows<QT, TT>(st, a, rt, slices, sf32); break;
     switch (qt * 8 + T) {
-        LV_SHORT(4, 0) LV_SHORT(4, 1) LV_SHORT(4, 2) LV_SHORT(4, 3) LV_SHORT(4, 4)
-        LV_SHORT(8, 0) LV_SHORT(8, 1) LV_SHORT(8, 2) LV_SHORT(8, 3) LV_SHORT(8, 4)
+        LV_SHORT(4, 0) LV_SHORT(4, 1)
+        LV_SHORT(8, 0) LV_SHORT(8, 1)
     default: return fail(LV_ERR_STATE, "short batch of %u tokens", a.n);
     }
 #undef LV_SHORT
     HIP_TRY(hipGetLastError());
     return LV_OK;
+}
+
+// ---- products of 17 to 256 tokens (lv_mid.h) -------------------------------------------------------------------
+template <int QT, bool SF32, int T, int RG, int RTW>
+static int launch_mid_kernel(hipStream_t st, const MidArgs &a, uint32_t slices, uint32_t groups)
+{
+    constexpr int lds = mid_lds_bytes(T, RG, RTW), rt = RG * RTW;
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&wide_short_gemm_kernel<QT, SF32, T, RG, RTW>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    wide_short_gemm_kernel<QT, SF32, T, RG, RTW><<<dim3((a.tiles + rt - 1) / rt, slices, groups), dim3(512), lds, st>>>(a);
+    HIP_TRY(hipGetLastError());
+    return LV_OK;
+}
+template <int QT, bool SF32, int T>
+static int launch_mid_rows(hipStream_t st, const MidArgs &a, uint32_t rt, uint32_t slices, uint32_t groups)
+{
+    if constexpr (T <= 4)
+        if (rt == 3) return launch_mid_kernel<QT, SF32, T, 1, 3>(st, a, slices, groups);
+    if (rt == 2) return launch_mid_kernel<QT, SF32, T, 2, 1>(st, a, slices, groups);
+    if (rt == 4) return launch_mid_kernel<QT, SF32, T, 2, 2>(st, a, slices, groups);
+    return launch_mid_kernel<QT, SF32, T, 2, 3>(st, a, slices, groups);
+}
+template <int QT, bool SF32>
+static int launch_mid_tokens(hipStream_t st, const MidArgs &a, uint32_t T, uint32_t rt, uint32_t slices, uint32_t groups)
+{
+    switch (T) {
+    case 2: return launch_mid_rows<QT, SF32, 2>(st, a, rt, slices, groups);
+    case 3: return launch_mid_rows<QT, SF32, 3>(st, a, rt, slices, groups);
+    case 4: return launch_mid_rows<QT, SF32, 4>(st, a, rt, slices, groups);
+    case 5: return launch_mid_rows<QT, SF32, 5>(st, a, rt, slices, groups);
+    case 6: return launch_mid_rows<QT, SF32, 6>(st, a, rt, slices, groups);
+    default: return launch_mid_rows<QT, SF32, 8>(st, a, rt, slices, groups);
+    }
+}
+
+// Row tiles per workgroup (RT; three: one row group) and K slices of a product of `groups` times 16 T tokens, and what it costs.  A
+// workgroup's time goes with its chunks (whole rounds of its K groups) times its row tiles and the activations, worth 0.4 T of them; a round
+// of 256 workgroups starts and ends at the price of 20 such units, a slice more is written and read again for 5.  Measured in us, 7B q8_0:
+//   q, k and v, RT 2/3/4/6      48 tokens 31/22/24/30, 128 73/-/39/53, 256 -/-/81/55
+//   gate and up, RT 2/3/4/6     48 tokens 47/41/45/32, 128 112/-/86/54, 256 -/-/127/105
+//   down, RT 4, slices 2/3/4    48 tokens 32/23/20, 128 53/41/33, 256 52/73/62; RT 2, slices 2: 22, 46, 91; RT 6, slices 4: 24, 42, 76
+static double mid_plan(uint32_t tiles, uint32_t nb, uint32_t T, uint32_t groups, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
+{
+    const uint32_t chunks = nb / 4;
+    double best = 1e30;
+    for (uint32_t rt : {2u, 3u, 4u, 6u}) {
+        if (rt == 3 && T > 4) continue;
+        const uint32_t kg = rt == 3 ? 8 : 4;
+        for (uint32_t s = 1; s <= (sliced ? (uint32_t)kShortSlices : 1u); s++) {
+            const uint32_t per = (chunks + s - 1) / s;
+            if ((chunks + per - 1) / per != s) continue;
+            const uint32_t held = ((tiles + rt - 1) / rt * s * groups + 255) / 256;
+            const double cost = held * ((per + kg - 1) / kg * kg * (rt + 0.4 * T) + 20) + 5.0 * (s - 1);
+            if (cost < best) { best = cost; *best_rt = rt; *best_chunks = per; }
+        }
+    }
+    return best;
+}
+// tiles of 16 tokens of a workgroup (2 to 6, 8) and how many such groups cover n tokens
+static void mid_tokens(uint32_t n, uint32_t *T, uint32_t *groups)
+{
+    *groups = n <= 128 ? 1 : 2;
+    const uint32_t t = (n + 16 * *groups - 1) / (16 * *groups);
+    *T = t <= 2 ? 2 : t == 7 ? 8 : t;
+}
+
+// Do the products of n tokens (kShortTokens to kMidTokens) take less time here than in tiles of 128 tokens on the prompt copy (lv_gemm.h)?  There
+// 128 columns of a round of 256 workgroups cost 18.6 of mid_plan's units, whatever a tile holds.  Up to 128 tokens those tiles leave most of
+// the chip idle; above, it depends on how both fill their rounds.  Measured, ms a step of 8 layers of q8_0, tiles of 128 and here:
+//   7B   100 tokens 2.54 and 1.57, 129 2.61 and 1.87, 200 2.65 and 2.46, 256 2.68 and 2.49
+//   13B  100 tokens 3.06 and 2.21, 129 3.16 and 2.86, 200 3.32 and 3.82, 256 3.45 and 3.94
+static bool mid_pays(const lv_hparams &hp, uint32_t n)
+{
+    if (n <= 128) return true;
+    if (n > kMidTokens) return false;
+    const uint32_t D = hp.dim, F = hp.ff;
+    uint32_t T, groups, rt, per;
+    mid_tokens(n, &T, &groups);
+    auto there = [&](uint32_t rows, uint32_t nz, uint32_t K, bool sliced) {
+        const uint32_t tt = (n + kGemmTile - 1) / kGemmTile, rts = (rows + kGemmRows - 1) / kGemmRows, s = sliced ? gemm_k_slices(rts, tt, K / kGemmK) : 1;
+        return (rts * nz * s * tt + 255) / 256 * (K / 128.0 / s * 18.6) + 20 + 5.0 * (s - 1);
+    };
+    const double here = mid_plan(3 * D / 16, D / 32, T, groups, false, &rt, &per) + mid_plan(D / 16, D / 32, T, groups, true, &rt, &per) +
+                        mid_plan(F / 8, D / 32, T, groups, false, &rt, &per) + mid_plan(D / 16, F / 32, T, groups, true, &rt, &per);
+    return here < there(D, 3, D, false) + there(D, 1, D, true) + there(2 * F, 1, D, false) + there(D, 1, F, true);
+}
+
+static int launch_mid_gemm(hipStream_t st, MidArgs a, uint32_t ftype, bool sf32, bool sliced, uint32_t *slices_out = nullptr)
+{
+    if (!a.w) return fail(LV_ERR_STATE, "short batch: the matrix has no copy");
+    if (a.n > kMidTokens) return fail(LV_ERR_STATE, "short batch of %u tokens", a.n);
+    uint32_t T, groups, rt = 2;
+    mid_tokens(a.n, &T, &groups);
+    (void)mid_plan(a.tiles, a.nb, T, groups, sliced, &rt, &a.slice_chunks);
+    const uint32_t slices = (a.nb / 4 + a.slice_chunks - 1) / a.slice_chunks;
+    if (slices_out) *slices_out = slices;
+    if (ftype == LV_Q4_0) return sf32 ? launch_mid_tokens<4, true>(st, a, T, rt, slices, groups) : launch_mid_tokens<4, false>(st, a, T, rt, slices, groups);
+    return sf32 ? launch_mid_tokens<8, true>(st, a, T, rt, slices, groups) : launch_mid_tokens<8, false>(st, a, T, rt, slices, groups);
+}
+
+// activations as the kernels for short steps write them (lv_short.h; more than 16 tokens), as the batched path's do (tile order)
+static void mid_input_short(MidArgs &a, const uint8_t *act)
+{
+    const uint32_t tiles = short_tiles(a.n);
+    a.x[0] = act; a.x[1] = act + 1024;
+    a.xb = tiles * 2048; a.xt = 2048; a.xg = 256; a.x128 = 8 * 2048; a.x_bytes = a.nb * a.xb - 1024;
+}
+static void mid_input_planes(MidArgs &a, const uint16_t *xh, const uint16_t *xl)
+{
+    a.x[0] = reinterpret_cast<const uint8_t *>(xh); a.x[1] = reinterpret_cast<const uint8_t *>(xl);
+    a.xb = 4 * kGemmTile * 16; a.xt = 256; a.xg = kGemmTile * 16; a.x128 = a.nb * a.xb; a.x_bytes = (a.n + kGemmTile - 1) / kGemmTile * a.x128;
+}
+
+// the products of a layer, without their input: q, k and v, a matrix of `rows` rows, gate and up (whose output is laid out as `d`'s input)
+static MidArgs mid_store(uint32_t n, uint32_t K, const uint8_t *w, uint32_t rows, const float *xscale)
+{
+    MidArgs a{};
+    a.n = n; a.nb = K / 32; a.w = w; a.mode = kShortStore; a.tiles_m = a.tiles = rows / 16; a.ldo = rows; a.xscale = xscale;
+    return a;
+}
+static MidArgs mid_qkv(const lv_session *s, uint32_t layer, uint32_t n, uint32_t idx0, float *q, const float *xscale)
+{
+    const uint32_t D = s->model->hp.dim;
+    MidArgs a = mid_store(n, D, s->model->layers[layer].short_qkv, D, xscale);
+    a.mode = kShortQkv; a.tiles = 3 * a.tiles_m; a.out[0] = q;
+    a.cache[0] = kv_ptr(s, layer, 0); a.cache[1] = kv_ptr(s, layer, 1); a.pos_ptr = s->cfg; a.pos_add = idx0; a.backlog = s->backlog;
+    return a;
+}
+static MidArgs mid_silu(const lv_session *s, uint32_t layer, uint32_t n, const float *xscale)
+{
+    MidArgs a = mid_store(n, s->model->hp.dim, s->model->layers[layer].short_gate_up, 2 * s->model->hp.ff, xscale);
+    a.mode = kShortSilu;
+    return a;
+}
+static void mid_output_ff(MidArgs &a, const MidArgs &d)
+{
+    a.ff[0] = const_cast<uint8_t *>(d.x[0]); a.ff[1] = const_cast<uint8_t *>(d.x[1]);
+    a.fb = d.xb; a.ft = d.xt; a.fg = d.xg; a.f128 = d.x128;
 }
 
 // The short copy of the layer matrices (lv_short.h), made when a model evaluates its first short batch; false when the device has no
@@ -2395,55 +2528,31 @@ static int launch_short_attention(hipStream_t st, const lv_session *s, const Sho
     return LV_OK;
 }
 
-// rows idx0 .. idx0 + n - 1 of the step, n <= kShortTokens; pos: the cache row of row idx0
-static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, bool with_head, uint32_t row_base)
+// the logits of record_short's step, `pending` K slices still to be added to the residual stream
+static int record_short_head(lv_session *s, const ShortBuffers &b, uint32_t idx0, uint32_t n, uint32_t pending, bool with_head, uint32_t row_base)
 {
     const lv_model *m = s->model;
     const lv_hparams &hp = m->hp;
-    const uint32_t D = hp.dim, F = hp.ff, ft = m->layers[0].wq.ftype;
+    const uint32_t D = hp.dim, ft = m->layers[0].wq.ftype;
     const bool sf32 = m->layers[0].wq.view.scales_f32 != nullptr;
     hipStream_t st = s->stream;
-    ShortBuffers b;
-    short_layout(hp, s->short_ws, &b);
-    LV_TRY(launch_embed(s, b.x, s->cfg_host + 1, s->cfg_host[0], idx0, n));
-    HIP_TRY(hipGetLastError());
-
-    uint32_t pending = 0;       // K slices in b.parts that the next norm adds to the residual stream
-    const float *xscale = short_exact(short_tiles(n)) ? nullptr : b.xscale;
-    for (uint32_t li = 0; li < hp.layers; li++) {
-        const LayerWeights &lw = m->layers[li];
-        LV_TRY(launch_short_norm(st, b, lw.attn_norm, n, D, pending, ft));
-        ShortArgs a{};
-        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = xscale;
-        a.mode = kShortQkv;
-        a.w = lw.short_qkv;
-        a.tiles_m = D / 16; a.tiles = 3 * a.tiles_m; a.out[0] = b.q; a.ldo = D;
-        a.cache[0] = kv_ptr(s, li, 0); a.cache[1] = kv_ptr(s, li, 1); a.pos_ptr = s->cfg; a.pos_add = idx0; a.backlog = s->backlog;
-        LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
-        LV_TRY(launch_short_attention(st, s, b, li, pos, n, ft));
-        ShortArgs o{};
-        o.x = b.act; o.n = n; o.nb = D / 32; o.mode = kShortStore; o.w = lw.short_wo; o.tiles_m = o.tiles = D / 16; o.ldo = D;
-        for (int i = 0; i < kShortSlices; i++) o.out[i] = b.parts[i];
-        LV_TRY(launch_short_gemm(st, o, ft, sf32, true, &pending));
-        LV_TRY(launch_short_norm(st, b, lw.ffn_norm, n, D, pending, ft));
-        ShortArgs f{};
-        f.x = b.act; f.n = n; f.nb = D / 32; f.xscale = xscale; f.mode = kShortSilu;
-        f.w = lw.short_gate_up; f.tiles_m = f.tiles = F / 8; f.ff = b.ff;
-        LV_TRY(launch_short_gemm(st, f, ft, sf32, false));
-        ShortArgs d = o;
-        d.x = b.ff; d.nb = F / 32; d.w = lw.short_down;
-        LV_TRY(launch_short_gemm(st, d, ft, sf32, true, &pending));
-    }
     float *parts[kGemmMaxMats];
     for (int i = 0; i < kShortSlices; i++) parts[i] = b.parts[i];
     float *all = s->all_logits ? s->logits_all + (size_t)(row_base + idx0) * hp.vocab : nullptr;
     const lv_matrix &ow = m->output;
     if (all && m->short_output) {
         LV_TRY(launch_short_norm(st, b, m->norm, n, D, pending, ft));
-        ShortArgs a{};
-        a.x = b.act; a.n = n; a.nb = D / 32; a.xscale = xscale; a.mode = kShortStore; a.w = m->short_output;
-        a.tiles_m = a.tiles = hp.vocab / 16; a.out[0] = all; a.ldo = hp.vocab;
-        LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
+        if (short_exact(short_tiles(n))) {
+            ShortArgs a{};
+            a.x = b.act; a.n = n; a.nb = D / 32; a.mode = kShortStore; a.w = m->short_output;
+            a.tiles_m = a.tiles = hp.vocab / 16; a.out[0] = all; a.ldo = hp.vocab;
+            LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
+        } else {
+            MidArgs a = mid_store(n, D, m->short_output, hp.vocab, b.xscale);
+            mid_input_short(a, b.act);
+            a.out[0] = all;
+            LV_TRY(launch_mid_gemm(st, a, ft, sf32, false));
+        }
     } else if (all || with_head) {
         // only the last row's logits are ever read (llava_session.cpp:131-139), unless all are asked for
         LV_TRY(launch_gemm_reduce(st, b.x, D, parts, pending, D, n, true));
@@ -2461,6 +2570,117 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
     }
     if (all && with_head) HIP_TRY(hipMemcpyAsync(s->logits, all + (size_t)(n - 1) * hp.vocab, (size_t)hp.vocab * 4, hipMemcpyDeviceToDevice, st));
     return LV_OK;
+}
+
+// record_short's layers for 17 tokens and more: activations as fp16 halves, the products of lv_mid.h
+static int record_short_halves(lv_session *s, const ShortBuffers &b, uint32_t idx0, uint32_t n, uint32_t pos, bool with_head, uint32_t row_base)
+{
+    const lv_model *m = s->model;
+    const lv_hparams &hp = m->hp;
+    const uint32_t D = hp.dim, F = hp.ff, ft = m->layers[0].wq.ftype;
+    const bool sf32 = m->layers[0].wq.view.scales_f32 != nullptr;
+    hipStream_t st = s->stream;
+    uint32_t pending = 0;
+    for (uint32_t li = 0; li < hp.layers; li++) {
+        const LayerWeights &lw = m->layers[li];
+        LV_TRY(launch_short_norm(st, b, lw.attn_norm, n, D, pending, ft));
+        MidArgs a = mid_qkv(s, li, n, idx0, b.q, b.xscale);
+        mid_input_short(a, b.act);
+        LV_TRY(launch_mid_gemm(st, a, ft, sf32, false));
+        LV_TRY(launch_short_attention(st, s, b, li, pos, n, ft));
+        MidArgs o = mid_store(n, D, lw.short_wo, D, nullptr);
+        mid_input_short(o, b.act);
+        for (int i = 0; i < kShortSlices; i++) o.out[i] = b.parts[i];
+        LV_TRY(launch_mid_gemm(st, o, ft, sf32, true, &pending));
+        LV_TRY(launch_short_norm(st, b, lw.ffn_norm, n, D, pending, ft));
+        MidArgs f = mid_silu(s, li, n, b.xscale);
+        mid_input_short(f, b.act);
+        MidArgs d = mid_store(n, F, lw.short_down, D, nullptr);
+        mid_input_short(d, b.ff);
+        mid_output_ff(f, d);
+        LV_TRY(launch_mid_gemm(st, f, ft, sf32, false));
+        for (int i = 0; i < kShortSlices; i++) d.out[i] = b.parts[i];
+        LV_TRY(launch_mid_gemm(st, d, ft, sf32, true, &pending));
+    }
+    return record_short_head(s, b, idx0, n, pending, with_head, row_base);
+}
+
+// record_prefill's layers with the products of lv_mid.h
+static int record_mid_layers(lv_session *s, uint32_t idx0, uint32_t n, float *const parts[kGemmMaxMats], uint32_t *pending_out)
+{
+    const lv_model *m = s->model;
+    const lv_hparams &hp = m->hp;
+    const uint32_t D = hp.dim, F = hp.ff, ft = m->layers[0].wq.ftype;
+    const bool sf32 = m->layers[0].wq.view.scales_f32 != nullptr;
+    hipStream_t st = s->stream;
+    uint32_t pending = 0;
+    const float *xscale = nullptr;
+    for (uint32_t li = 0; li < hp.layers; li++) {
+        const LayerWeights &lw = m->layers[li];
+        LV_TRY(launch_prefill_norm(st, s, lw.attn_norm, n, D, parts, pending, false, &xscale));
+        MidArgs a = mid_qkv(s, li, n, idx0, s->pf_q, xscale);
+        mid_input_planes(a, s->pf_xh, s->pf_xl);
+        LV_TRY(launch_mid_gemm(st, a, ft, sf32, false));
+        LV_TRY(launch_attention_batch(st, nullptr, s->pf_xh, s->pf_xl, D, s->pf_planes, kv_ptr(s, li, 0), kv_ptr(s, li, 1), nullptr, nullptr, s->pf_q, s->trig_abs,
+                                      s->cfg, idx0, n, s->backlog, hp.heads, hp.rot));
+        MidArgs o = mid_store(n, D, lw.short_wo, D, nullptr);
+        mid_input_planes(o, s->pf_xh, s->pf_xl);
+        for (int i = 0; i < kShortSlices; i++) o.out[i] = parts[i];
+        LV_TRY(launch_mid_gemm(st, o, ft, sf32, true, &pending));
+        LV_TRY(launch_prefill_norm(st, s, lw.ffn_norm, n, D, parts, pending, false, &xscale));
+        MidArgs f = mid_silu(s, li, n, xscale);
+        mid_input_planes(f, s->pf_xh, s->pf_xl);
+        MidArgs d = mid_store(n, F, lw.short_down, D, nullptr);
+        mid_input_planes(d, s->pf_fh, s->pf_fl);
+        mid_output_ff(f, d);
+        LV_TRY(launch_mid_gemm(st, f, ft, sf32, false));
+        for (int i = 0; i < kShortSlices; i++) d.out[i] = parts[i];
+        LV_TRY(launch_mid_gemm(st, d, ft, sf32, true, &pending));
+    }
+    *pending_out = pending;
+    return LV_OK;
+}
+
+// rows idx0 .. idx0 + n - 1 of the step, n <= kShortTokens; pos: the cache row of row idx0
+static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, bool with_head, uint32_t row_base)
+{
+    const lv_model *m = s->model;
+    const lv_hparams &hp = m->hp;
+    const uint32_t D = hp.dim, F = hp.ff, ft = m->layers[0].wq.ftype;
+    const bool sf32 = m->layers[0].wq.view.scales_f32 != nullptr;
+    hipStream_t st = s->stream;
+    ShortBuffers b;
+    short_layout(hp, s->short_ws, &b);
+    LV_TRY(launch_embed(s, b.x, s->cfg_host + 1, s->cfg_host[0], idx0, n));
+    HIP_TRY(hipGetLastError());
+
+    uint32_t pending = 0;       // K slices in b.parts that the next norm adds to the residual stream
+    if (!short_exact(short_tiles(n))) return record_short_halves(s, b, idx0, n, pos, with_head, row_base);
+    for (uint32_t li = 0; li < hp.layers; li++) {
+        const LayerWeights &lw = m->layers[li];
+        LV_TRY(launch_short_norm(st, b, lw.attn_norm, n, D, pending, ft));
+        ShortArgs a{};
+        a.x = b.act; a.n = n; a.nb = D / 32;
+        a.mode = kShortQkv;
+        a.w = lw.short_qkv;
+        a.tiles_m = D / 16; a.tiles = 3 * a.tiles_m; a.out[0] = b.q; a.ldo = D;
+        a.cache[0] = kv_ptr(s, li, 0); a.cache[1] = kv_ptr(s, li, 1); a.pos_ptr = s->cfg; a.pos_add = idx0; a.backlog = s->backlog;
+        LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
+        LV_TRY(launch_short_attention(st, s, b, li, pos, n, ft));
+        ShortArgs o{};
+        o.x = b.act; o.n = n; o.nb = D / 32; o.mode = kShortStore; o.w = lw.short_wo; o.tiles_m = o.tiles = D / 16; o.ldo = D;
+        for (int i = 0; i < kShortSlices; i++) o.out[i] = b.parts[i];
+        LV_TRY(launch_short_gemm(st, o, ft, sf32, true, &pending));
+        LV_TRY(launch_short_norm(st, b, lw.ffn_norm, n, D, pending, ft));
+        ShortArgs f{};
+        f.x = b.act; f.n = n; f.nb = D / 32; f.mode = kShortSilu;
+        f.w = lw.short_gate_up; f.tiles_m = f.tiles = F / 8; f.ff = b.ff;
+        LV_TRY(launch_short_gemm(st, f, ft, sf32, false));
+        ShortArgs d = o;
+        d.x = b.ff; d.nb = F / 32; d.w = lw.short_down;
+        LV_TRY(launch_short_gemm(st, d, ft, sf32, true, &pending));
+    }
+    return record_short_head(s, b, idx0, n, pending, with_head, row_base);
 }
 
 extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, uint32_t pos)
@@ -2543,7 +2763,11 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     }
     // steps of a few tokens take position and token ids as launch arguments, and so does a token at a time
     const uint32_t batch_min = s->block ? kBlockBatchMin : (uint32_t)kPrefillMin, batch_max = s->block ? kBlockBatch : kPrefillChunk;
-    const bool batch = !persistent && !few && n >= batch_min && (!s->trace || s->block) && ensure_prompt_copy(s->model);
+    // A step of up to kMidTokens, or what is left of a longer one behind its whole chunks, takes the products of lv_mid.h: by its size alone
+    const uint32_t rest = n <= kPrefillChunk ? n : n % kPrefillChunk;
+    const bool mid = !persistent && !few && n >= kPrefillMin && rest && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && mid_pays(s->model->hp, rest) &&
+                     ensure_short_copy(s->model);
+    const bool batch = !persistent && !few && n >= batch_min && (!s->trace || s->block) && ((mid && n == rest) || ensure_prompt_copy(s->model));
     if (!persistent) {
         s->cfg_host[0] = pos;
         memcpy(s->cfg_host + 1, tokens, (size_t)n * 4);
@@ -2573,7 +2797,7 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     } else if (batch) {
         for (uint32_t i = 0; i < n; i += batch_max) {
             const uint32_t m = n - i < batch_max ? n - i : batch_max;
-            LV_TRY(record_prefill(s, i, m, i + m == n, row_base));
+            LV_TRY(record_prefill(s, i, m, i + m == n, row_base, mid && m == rest));
         }
     } else {
         // rows are evaluated one after the other: row z sees cache rows 0..pos+z, which is what the batched

@@ -8,10 +8,10 @@
 //   up to 16 tokens   three bf16 parts, an exact cut of the fp32 value with all of its range.  Such a step is also evaluated token by
 //                     token (other paths, no room for the copy below), in fp32 throughout, and is held to the same.
 //   17 to 64          two fp16 halves as in lv_gemm.h, which takes longer steps and these without the copy: 22 bits, of the norms'
-//                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.
+//                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.  Their products: lv_mid.h.
 // Attention likewise: up to 15 tokens in fp32 (short_attn_exact_kernel), then short_attn_kernel on fp16 pairs as with longer steps.
 //
-// short_gemm_kernel.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
+// short_gemm_kernel, up to 16 tokens.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
 // tokens; its waves deal the K range among themselves, four quant blocks at a time, and add up through LDS at the end.  A wave so
 // reads activations nobody else in the workgroup reads, straight into MFMA operand form, and reuses them for its RT tiles: no
 // LDS, no barrier, nothing but loads in flight in the main loop.
@@ -20,15 +20,14 @@
 //       A lane's codes of a block are the eight it feeds to one MFMA (v_mfma_f32_16x16x32_f16: lane l holds row l % 16, k group l / 16), so
 //       a load is 1 KB in a row and nothing crosses lanes.  Read from the operator path's planes instead, a load touches 16 rows,
 //       16 consecutive lanes 16 cache lines: the address path, not HBM, then sets the time (7B q4_0 gate and up for 8 tokens: 21.5 us that way, 15.8 so).
-//   order: the eight codes a lane feeds to an MFMA come in the order that unpacks cheapest (short_slot); the activations are
-//          written in that order.
+//   order: the eight codes a lane feeds to an MFMA come in the order that unpacks cheapest (short_slot); activation parts are
+//          written in that order, the nibbles of q4_0 packed so that halves stay in order.
 //   activations: [block][16-token tile][operand][group][token][8 elements]: 1 KB per operand, a lane's 16 bytes at 16 l.  Up to 8 tokens:
 //          the first two parts share an operand (tokens 0 .. 7 and 8 .. 15 of it), the third is half of one.
 // Rows of tokens past the batch are not written; a token only meets its own row of the result.
 //
-// Measured (us per launch, 7B layer, 8 tokens q4_0 / 45 tokens q8_0): q, k and v 11 / 28, gate and up 16 / 47, attention output and
-// down together 17 / 32; about 3 of each launch and sum.  A step of 8 tokens, 7B q4_0: 7.31 -> 2.00 ms (eight launches of the
-// persistent kernel before); 45 tokens behind 619, 8 layers of 7B q8_0: 2.77 -> 1.20 ms (128-token GEMM tiles before).
+// Measured (us per launch, 7B layer, 8 tokens q4_0): q, k and v 11, gate and up 16, attention output and down together 17; about 3 of each
+// launch and sum.  A step of 8 tokens, 7B q4_0: 7.31 -> 2.00 ms (eight launches of the persistent kernel before).
 #pragma once
 
 #include "lv_attn_batch.h"
@@ -53,28 +52,25 @@ __host__ __device__ constexpr uint32_t short_block_bytes(uint32_t tiles) { retur
 // bytes of the activations of K columns
 __host__ __device__ constexpr size_t short_act_bytes(uint32_t K, uint32_t n) { return (size_t)(K / 32) * short_block_bytes(short_tiles(n)); }
 
-// Element k of a block (0 .. 31) -> slot 8 g + e of the operand, and back.  q8_0: bytes in order.  q4_0: group g holds bytes
-// 4g .. 4g + 3 of the block, whose low nibbles are elements 4g .. 4g + 3 and whose high ones are 16 higher.  Parts: the low ones, then
-// the high ones.  Halves: a masked dword leaves nibbles 0 and 4 (then 1 and 5, 2 and 6, 3 and 7) in the two halves of a register.
+// Element k of a block (0 .. 31) -> slot 8 g + e of the operand: group g holds elements 8g .. 8g + 7.  Halves and q8_0: in order.  Parts of
+// q4_0: nibble p of a lane's dword holds element 2 (p % 4) + p / 4 (a masked dword leaves nibbles 0 and 4, then 1 and 5, 2 and 6, 3 and 7 in
+// the two halves of a register, in order), and the conversion from bytes takes the low nibbles first, then the high ones: 0 4 1 5 2 6 3 7.
 template <int QT, bool PARTS>
 __host__ __device__ constexpr uint32_t short_slot(uint32_t k)
 {
-    if constexpr (QT == 8) return k;
-    const uint32_t g = (k & 15) >> 2, j = k & 3, hi = k >> 4;
-    return PARTS ? 8 * g + hi * 4 + j : 8 * g + (j & 1) * 4 + hi * 2 + (j >> 1);
+    if constexpr (QT == 8 || !PARTS) return k;
+    return (k & ~7u) + (k & 3) * 2 + ((k >> 2) & 1);
 }
-// the elements of group g, slots 0 .. 7, from two runs of four consecutive elements a (from 4g or 8g on) and b (16 or 4 further)
+// the elements of a group, slots 0 .. 7, from its two runs of four consecutive elements
 template <int QT>
 __device__ __forceinline__ void short_order(float (&f)[8], const float4 &a, const float4 &b, bool parts)
 {
-    if (QT == 8 || parts) {
+    if (QT == 8 || !parts) {
         f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
     } else {
-        f[0] = a.x; f[1] = a.z; f[2] = b.x; f[3] = b.z; f[4] = a.y; f[5] = a.w; f[6] = b.y; f[7] = b.w;
+        f[0] = a.x; f[1] = b.x; f[2] = a.y; f[3] = b.y; f[4] = a.z; f[5] = b.z; f[6] = a.w; f[7] = b.w;
     }
 }
-template <int QT> __host__ __device__ constexpr uint32_t short_run_a(uint32_t g) { return QT == 8 ? 8 * g : 4 * g; }
-template <int QT> __host__ __device__ constexpr uint32_t short_run_b(uint32_t g) { return QT == 8 ? 8 * g + 4 : 16 + 4 * g; }
 
 // where part `part` of (block, token, group) lies: 0, 1 and 2, or the halves 0 and 1
 __device__ __forceinline__ size_t short_act_offset(uint32_t block, uint32_t token, uint32_t g, uint32_t tiles, uint32_t part)
@@ -126,32 +122,16 @@ struct ShortArgs {
     uint32_t n, mode;
     float *out[kShortSlices];  // [n][ldo], one per slice; kShortQkv: out[0] = q
     uint32_t ldo;
-    const float *xscale;       // null, or per token the power of two its halves have to be multiplied by (not with parts)
     uint16_t *cache[2];        // kShortQkv: k and v rows
     const uint32_t *pos_ptr;
     uint32_t pos_add, backlog;
     uint8_t *ff;               // kShortSilu: activations of the next product
 };
 
-// Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights or, where a block's
-// products take long enough to cover an L2 access, two blocks ahead.  More in flight per wave costs registers, hence waves per
-// CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us, q, k and v for 45 with q8_0 28 -> 96).  Nor
-// do two workgroups a CU pay: two blocks ahead would let three row tiles of q4_0 and up to 16 tokens into 128 registers (a step of 8
-// tokens of 13B q4_0, 8 layers: 752 us so, 708 with four ahead).
-template <int T, int RT> constexpr int short_ahead() { return T * RT >= 8 ? 2 : 4; }
-// can RT tiles of rows beside T tiles of tokens keep sums, queues and activations in 256 registers (a few values more is fine; three
-// tiles of tokens and six of rows of q4_0 left 220 in memory: 40 tokens of 7B 8.7 ms, 3.4 with three)
-__host__ __device__ constexpr bool short_fits(int qt, uint32_t t, uint32_t rt)
-{
-    if (qt == 4) return t != 3 || rt <= 3;
-    return rt <= (t <= 1 ? 6u : t <= 3 ? 3u : 2u);
-}
-// row tiles whose sums are put together at a time: up to 64 KB of LDS, whole pairs
-template <int T, int RT> constexpr int short_round()
-{
-    constexpr int most = 8 / (T ? T : 1);
-    return RT <= most ? RT : most;
-}
+// Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights.  More in flight per wave
+// costs registers, hence waves per CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us).  Nor do two
+// workgroups a CU pay: two blocks ahead would let three row tiles of q4_0 and up to 16 tokens into 128 registers (a step of 8 tokens of
+// 13B q4_0, 8 layers: 752 us so, 708 with four ahead).
 __device__ __forceinline__ lv_h8 short_unpack4(uint32_t w)
 {
     // nibble q in the low bits of a half of pattern 0x6400 is 1024 + q; one place up, 1024 + 16 q: both to q - 8, exactly
@@ -221,7 +201,13 @@ __global__ __launch_bounds__(256) void short_pack_kernel(uint8_t *__restrict__ d
 #pragma unroll
     for (int s = 0; s < 4; s++) {
         const uint32_t *b = reinterpret_cast<const uint32_t *>(src.codes + (b0 + s) * (QT / 4));
-        if constexpr (QT == 4) w[s] = b[g];
+        if constexpr (QT == 4) {
+            // elements 8g .. 8g + 7: the low (groups 0 and 1) or high nibbles of eight bytes, to where short_slot wants them
+            const uint32_t lo = b[(g & 1) * 2] >> (g >> 1) * 4 & 0x0f0f0f0fu, hi = b[(g & 1) * 2 + 1] >> (g >> 1) * 4 & 0x0f0f0f0fu;
+            w[s] = 0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) w[s] |= ((e < 4 ? lo : hi) >> 8 * (e & 3) & 15u) << 4 * ((e >> 1) + 4 * (e & 1));
+        }
         else { w[2 * s] = b[2 * g]; w[2 * s + 1] = b[2 * g + 1]; }
     }
 #pragma unroll
@@ -235,21 +221,19 @@ __global__ __launch_bounds__(256) void short_pack_kernel(uint8_t *__restrict__ d
     }
 }
 
-// T: tiles of 16 tokens, 0: up to 8 tokens; RT: tiles of 16 rows per workgroup; SF32: fp32 block scales
+// T: 0: up to 8 tokens, 1: up to 16; RT: tiles of 16 rows per workgroup; SF32: fp32 block scales
 template <int QT, bool SF32, int T, int RT>
 __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs a)
 {
+    static_assert(short_exact(T), "more tokens: wide_short_gemm_kernel");
     constexpr bool EIGHT = T == 0;                     // 8 tokens: an operand holds their first parts and their second ones
-    constexpr bool EXACT = short_exact(T);
-    constexpr int NT = EIGHT ? 1 : T;
     constexpr int XB = short_block_bytes(T);           // activation bytes of a block
-    constexpr int NX = EIGHT ? 2 : EXACT ? 3 : 2 * NT; // its operands
+    constexpr int NX = EIGHT ? 2 : 3;                  // its operands
     constexpr int BB = QT == 4 ? 16 : 32;              // code bytes of a block
     constexpr int CW = BB / 4;                         // a lane's dwords of a chunk
     constexpr int CB = short_chunk_bytes(QT, SF32);
-    constexpr int XD = short_ahead<T, RT>();
-    constexpr int PR = short_round<T, RT>();           // row tiles summed at a time
-    __shared__ __attribute__((aligned(16))) float red[PR * NT * kShortWaves * 256];
+    constexpr int XD = 4;                              // blocks the activations are requested ahead
+    __shared__ __attribute__((aligned(16))) float red[RT * kShortWaves * 256];
     const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tile0 = blockIdx.x * RT;
@@ -289,11 +273,9 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
             xq[slot][t] = *reinterpret_cast<const lv_u4 *>(p + at + t * 1024);
         }
     };
-    lv_f4v acc[RT][NT];
+    lv_f4v acc[RT];
 #pragma unroll
-    for (int i = 0; i < RT; i++)
-#pragma unroll
-        for (int t = 0; t < NT; t++) acc[i][t] = lv_f4v{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < RT; i++) acc[i] = lv_f4v{0.f, 0.f, 0.f, 0.f};
     const lv_f4v zero = {0.f, 0.f, 0.f, 0.f};
     constexpr uint32_t kOnes = 0x3f803f80u;
 
@@ -317,7 +299,7 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
             fetch_w(j + 1);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                lv_u4 ax[NX];                          // parts, or high and low halves tile by tile
+                lv_u4 ax[NX];                          // parts
 #pragma unroll
                 for (int t = 0; t < NX; t++) ax[t] = xq[s % XD][t];
                 if constexpr (EIGHT) ax[1] = r16 >= 8 ? ax[1] : lv_u4{0u, 0u, 0u, 0u};       // the third parts beside the second
@@ -327,36 +309,25 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
                     return c;
                 };
                 lv_f4v from = zero;
-                if constexpr (EXACT && QT == 4) from = times(__builtin_bit_cast(lv_b8, lv_u4{kOnes, kOnes, kOnes, kOnes}), zero) * -8.f;
+                if constexpr (QT == 4) from = times(__builtin_bit_cast(lv_b8, lv_u4{kOnes, kOnes, kOnes, kOnes}), zero) * -8.f;
 #pragma unroll
                 for (int i = 0; i < RT; i++) {
-                    lv_f4v p[NT];
-                    if constexpr (EXACT) {
-                        const lv_b8 b = QT == 4 ? short_unpack4_bf16(w[i][s]) : short_unpack8_bf16(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
-                        p[0] = times(b, from);
-                    } else {
-                        const lv_h8 b = QT == 4 ? short_unpack4(w[i][s]) : short_unpack8(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
+                    const lv_b8 b = QT == 4 ? short_unpack4_bf16(w[i][s]) : short_unpack8_bf16(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
+                    const lv_f4v p = times(b, from);
 #pragma unroll
-                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lv_h8, ax[2 * t + 1]), b, zero, 0, 0, 0);
-#pragma unroll
-                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lv_h8, ax[2 * t]), b, p[t], 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int t = 0; t < NT; t++)
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[i][t][e] = fmaf(p[t][e], sc[i][s], acc[i][t][e]);
+                    for (int e = 0; e < 4; e++) acc[i][e] = fmaf(p[e], sc[i][s], acc[i][e]);
                 }
                 fetch_x(s % XD, j + (s + XD) / 4, (s + XD) % 4);
             }
         }
     }
 
-    // ---- the waves' sums, PR row tiles at a time, through LDS: [row tile][token tile][wave][lane] float4 -------------------------
-    // acc[i][t][e]: row r16 of row tile i, token 16 t + 4 g + e (EIGHT: the first part's product of token 4 g + e for g < 2, behind
-    // them the others').  A wave adds up every eighth (row tile, token tile).
+    // ---- the waves' sums through LDS: [row tile][wave][lane] float4 ---------------------------------------------------------------
+    // acc[i][e]: row r16 of row tile i, token 4 g + e (EIGHT: the first part's product of token 4 g + e for g < 2, behind them the
+    // others').  A wave adds up every eighth row tile.
     const uint32_t row_at = (a.mode == kShortQkv && a.pos_ptr ? *a.pos_ptr : 0u) + a.pos_add;
     float *const out = a.out[blockIdx.y];
-    auto total = [&](int u, int from, float (&v)[4], const float4 &xs) {      // lane `from`'s sums of unit u
+    auto total = [&](int u, int from) {                // lane `from`'s sums of row tile u
         const lv_f4v *src = reinterpret_cast<const lv_f4v *>(red) + (size_t)u * kShortWaves * 64 + from;
         lv_f4v s = src[0];
 #pragma unroll
@@ -366,55 +337,37 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
 #pragma unroll
             for (int w = 0; w < kShortWaves; w++) s += low[w * 64];
         }
-        v[0] = s[0] * xs.x; v[1] = s[1] * xs.y; v[2] = s[2] * xs.z; v[3] = s[3] * xs.w;
+        return s;
     };
 #pragma unroll
-    for (int i0 = 0; i0 < RT; i0 += PR) {
-        if (i0) __syncthreads();
-#pragma unroll
-        for (int i = 0; i < PR; i++)
-#pragma unroll
-            for (int t = 0; t < NT; t++)
-                if (i0 + i < RT) *reinterpret_cast<lv_f4v *>(red + (((i * NT + t) * kShortWaves + wave) * 64 + lane) * 4) = acc[i0 + i][t];
-        __syncthreads();
-        for (int u = wave; u < (RT - i0 < PR ? RT - i0 : PR) * NT; u += kShortWaves) {
-            const uint32_t tile = tile0 + i0 + u / NT, tok0 = 16 * (u % NT) + 4 * g;
-            if (tile >= a.tiles || (EIGHT && lane >= 32)) continue;
-            float4 xs = make_float4(1.f, 1.f, 1.f, 1.f);
-            if (a.xscale) xs = *reinterpret_cast<const float4 *>(a.xscale + tok0);
-            float v[4];
-            total(u, lane, v, xs);
-            if (a.mode == kShortSilu) {                // rows 0 .. 7 of the tile are W3's, 8 .. 15 the same ones of W1
-                if (r16 >= 8) continue;
-                float w[4];
-                total(u, lane + 8, w, xs);
-                const uint32_t f = tile * 8 + r16, slot = short_slot<QT, EXACT>(f & 31);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    if (tok0 + e >= a.n) continue;
-                    const float y = v[e] * w[e] / (__expf(-w[e]) + 1.f);
-                    auto put = [&](uint32_t part, uint16_t v) { *reinterpret_cast<uint16_t *>(a.ff + short_act_offset(f / 32, tok0 + e, slot >> 3, T, part) + (slot & 7) * 2) = v; };
-                    if constexpr (EXACT) {
-                        uint32_t b[3];
-                        short_cut(b, y);
-#pragma unroll
-                        for (int i = 0; i < 3; i++) put(i, (uint16_t)(b[i] >> 16));
-                    } else {
-                        const uint16_t h = float_to_half_bits(y);
-                        put(0, h);
-                        put(1, float_to_half_bits(y - half_bits_to_float(h)));
-                    }
-                }
-                continue;
-            }
-            const uint32_t z = tile / a.tiles_m, m = tile % a.tiles_m * 16 + r16;
+    for (int i = 0; i < RT; i++) *reinterpret_cast<lv_f4v *>(red + ((i * kShortWaves + wave) * 64 + lane) * 4) = acc[i];
+    __syncthreads();
+    for (int u = wave; u < RT; u += kShortWaves) {
+        const uint32_t tile = tile0 + u, tok0 = 4 * g;
+        if (tile >= a.tiles || (EIGHT && lane >= 32)) continue;
+        const lv_f4v v = total(u, lane);
+        if (a.mode == kShortSilu) {                    // rows 0 .. 7 of the tile are W3's, 8 .. 15 the same ones of W1
+            if (r16 >= 8) continue;
+            const lv_f4v w = total(u, lane + 8);
+            const uint32_t f = tile * 8 + r16, slot = short_slot<QT, true>(f & 31);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const uint32_t tok = tok0 + e;
-                if (tok >= a.n) continue;
-                if (z == 0) out[(size_t)tok * a.ldo + m] = v[e];
-                else if (row_at + tok < a.backlog) a.cache[z - 1][(size_t)(row_at + tok) * a.ldo + m] = float_to_half_bits(v[e]);
+                if (tok0 + e >= a.n) continue;
+                uint32_t b[3];
+                short_cut(b, v[e] * w[e] / (__expf(-w[e]) + 1.f));
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+                    *reinterpret_cast<uint16_t *>(a.ff + short_act_offset(f / 32, tok0 + e, slot >> 3, T, i) + (slot & 7) * 2) = (uint16_t)(b[i] >> 16);
             }
+            continue;
+        }
+        const uint32_t z = tile / a.tiles_m, m = tile % a.tiles_m * 16 + r16;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t tok = tok0 + e;
+            if (tok >= a.n) continue;
+            if (z == 0) out[(size_t)tok * a.ldo + m] = v[e];
+            else if (row_at + tok < a.backlog) a.cache[z - 1][(size_t)(row_at + tok) * a.ldo + m] = float_to_half_bits(v[e]);
         }
     }
 }
@@ -439,7 +392,7 @@ __global__ __launch_bounds__(1024) void short_norm_kernel(ShortNormArgs a)
     const int wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const bool ok = i < a.dim / 8;
     const size_t ro = (size_t)row * a.dim;
-    const uint32_t ic = ok ? i : 0, k[2] = {(ic >> 2) * 32 + short_run_a<QT>(ic & 3), (ic >> 2) * 32 + short_run_b<QT>(ic & 3)};
+    const uint32_t ic = ok ? i : 0, k[2] = {(ic >> 2) * 32 + (ic & 3) * 8, (ic >> 2) * 32 + (ic & 3) * 8 + 4};
     float4 x[2], w[2], p[kShortSlices][2];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -730,8 +683,8 @@ __global__ __launch_bounds__(256, 2) void short_attn_kernel(ShortAttnArgs a)
             const uint32_t z = i / C8, c = i % C8, k = h * R + (c >> 2) * 32, g = c & 3;
             const float *row = xch + z * XS + (c >> 2) * 32;
             const float total = den_s[z >> 5][z & 31];
-            float4 va = *reinterpret_cast<const float4 *>(row + (a.q8 ? short_run_a<8>(g) : short_run_a<4>(g)));
-            float4 vb = *reinterpret_cast<const float4 *>(row + (a.q8 ? short_run_b<8>(g) : short_run_b<4>(g)));
+            float4 va = *reinterpret_cast<const float4 *>(row + 8 * g);
+            float4 vb = *reinterpret_cast<const float4 *>(row + 8 * g + 4);
             va.x /= total; va.y /= total; va.z /= total; va.w /= total;
             vb.x /= total; vb.y /= total; vb.z /= total; vb.w /= total;
             float f[8];
@@ -895,7 +848,7 @@ __global__ __launch_bounds__(256, 2) void short_attn_exact_kernel(ShortAttnArgs 
         for (uint32_t i = t; i < a.n * C8; i += 256) {
             const uint32_t z = i / C8, c = i % C8, d = (c >> 2) * 32, og = c & 3;
             const float w = weight(z);
-            float4 va = total(z, d + (a.q8 ? short_run_a<8>(og) : short_run_a<4>(og))), vb = total(z, d + (a.q8 ? short_run_b<8>(og) : short_run_b<4>(og)));
+            float4 va = total(z, d + 8 * og), vb = total(z, d + 8 * og + 4);
             va.x /= w; va.y /= w; va.z /= w; va.w /= w;
             vb.x /= w; vb.y /= w; vb.z /= w; vb.w /= w;
             float f[8];
@@ -924,7 +877,7 @@ __global__ __launch_bounds__(256) void short_attn_combine_kernel(ShortCombineArg
 {
     const uint32_t D = a.heads * a.rot, i = blockIdx.x * 256 + threadIdx.x, z = blockIdx.y;
     if (i >= D / 8) return;
-    const uint32_t ka = (i >> 2) * 32 + short_run_a<QT>(i & 3), kb = (i >> 2) * 32 + short_run_b<QT>(i & 3);
+    const uint32_t ka = (i >> 2) * 32 + (i & 3) * 8, kb = (i >> 2) * 32 + (i & 3) * 8 + 4;
     const uint32_t h = ka / a.rot;                     // a block of 32 lies in one head
     float4 va = make_float4(0.f, 0.f, 0.f, 0.f), vb = va;
     float den = 0.f;

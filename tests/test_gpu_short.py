@@ -1,4 +1,4 @@
-"""Short batches (2 .. 64 tokens, csrc/lv_short.h) of LLaMA models against the CPU checker: every edge of the token tiles (16) and of
+"""Short batches (2 .. 64 tokens, csrc/lv_short.h; to 256, csrc/lv_mid.h) of LLaMA models against the CPU checker: every edge of the token tiles (16) and of
 the kernels' limit, head sizes 32, 64 and 128, both weight types, K slices, contexts in front of the batch.
 
 Tolerance: the one the path is specified with (test_gpu_model.py): 1e-2 and 1e-3 of the largest logit."""
@@ -73,6 +73,56 @@ def test_short_batch_matches_oracle(lva, orc, ctx, models, name, before, n):
     sess.begin(toks[-1:], before + n)
     close(sess.logits(), want)
     sess.close(); model.close(); osess.close(); om.close()
+
+
+# steps of 65 to 256 tokens (csrc/lv_mid.h), and what is left of a longer one: every edge of the token tiles and of the two groups of them
+MIDDLE = [(name, 0, n) for name in ("q4_64", "q8_128") for n in (65, 80, 81, 96, 97, 128, 129, 160, 161, 192, 193, 256)]
+MIDDLE += [(name, 37, n) for name in [*SHAPES, "q4_64_v1", "q8_64_v1"] for n in (70, 120, 170)]
+MIDDLE += [("q4_64", 0, 513), ("q8_64", 3, 600), ("q4_wide", 0, 129), ("q8_wide", 5, 100), ("q4_wider", 0, 90), ("q4_wider", 0, 200)]
+
+
+@pytest.mark.parametrize("name,before,n", MIDDLE)
+def test_longer_step_matches_oracle(lva, orc, ctx, models, name, before, n):
+    om = orc.Model(models[name])
+    osess = orc.Session(om, 1024)
+    model = lva.Model(ctx, models[name])
+    sess = lva.Session(model, 1024)
+    toks = lva.synth_tokens(before + n + 1, 3, om.hp["vocab"], seed=before + n)
+    if before:
+        osess.eval(toks[:before])
+        sess.begin(toks[:before], 0)
+        sess.wait()
+        for layer in range(om.hp["layers"]):
+            for which in (0, 1):
+                sess.kv_write(layer, which, osess.kv(layer, which, before))
+    want = osess.eval(toks[before:before + n])
+    sess.begin(toks[before:before + n], before)
+    close(sess.logits(), want)
+    for which in (0, 1):
+        g, o = (s.kv(0, which, before + n)[before:].view(np.float16).astype(np.float32) for s in (sess, osess))
+        assert np.max(np.abs(g - o)) <= np.max(np.abs(o)) * 2.0 ** -10
+    want = osess.eval(toks[-1:])                   # reads every cache row the step wrote
+    sess.begin(toks[-1:], before + n)
+    close(sess.logits(), want)
+    sess.close(); model.close(); osess.close(); om.close()
+
+
+@pytest.mark.parametrize("name,n", [("q4_64", 100), ("q8_64", 150)])
+def test_every_row_of_a_longer_step(lva, ctx, models, name, n):
+    """against a session whose path is set, which evaluates them as a batch in tiles of 128 tokens"""
+    model = lva.Model(ctx, models[name])
+    a, b = lva.Session(model, 256), lva.Session(model, 256)
+    b.set_path(lva.PATH_GRAPH)
+    toks = lva.synth_tokens(n, 3, 500, seed=n)
+    rows = []
+    for s in (a, b):
+        s.keep_all_logits()
+        s.begin(toks, 0)
+        rows.append(s.logits_rows(0, n))
+        assert np.array_equal(rows[-1][-1], s.logits())
+    for i in range(n):
+        close(rows[0][i], rows[1][i])
+    a.close(); b.close(); model.close()
 
 
 @pytest.mark.parametrize("name", ["q4_64", "q8_128"])
