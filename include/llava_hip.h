@@ -208,6 +208,8 @@ int lv_session_use_graph(lv_session *s, int enable);
  *   LV_PATH_PERSISTENT  one persistent kernel for the whole token (LLaMA-7B and -13B layer shapes, q4_0 or q8_0, on a
  *                       256-CU device)
  *   LV_PATH_AUTO        persistent when the model has that form, else graph (or kernels if graphs are off)
+ *                       A small model (width up to 1024) left to itself takes one launch of a few workgroups for a token as well, up to
+ *                       131072 / head size rows of context; lv_session_path reports the graph path, which it takes otherwise
  * A session stops using the persistent kernel, and lv_session_path reports the graph path (kernels if graphs are off)
  * from then on, when its 256 workgroups cannot all be resident on the device (the step goes on in the other path and succeeds) or when
  * two steps in a row end with an expired hand-over wait (both report LV_ERR_HIP; the step issued again then succeeds).

@@ -25,6 +25,7 @@
 #include "lv_gemv_wide.h"
 #include "lv_attn_batch.h"
 #include "lv_mid.h"
+#include "lv_small.h"
 
 using namespace lv;
 
@@ -157,6 +158,9 @@ struct lv_model {
     float *mega_norms = nullptr;    // [layers][2][D] + final norm [D]
     float *tok_f32_own = nullptr;   // fp32 copy of a quantised embedding table (the persistent kernel reads rows as fp32)
     // prompt copy of the layer matrices (lv_gemm.h), made when the first batch is evaluated; sessions of several threads share it
+    // a small model's token as one launch (lv_small.h): its matrices as a table on the device, the workgroups of a launch (0: not such a model)
+    SmallLayer *small_layers = nullptr;
+    uint32_t small_wgs = 0;
     std::mutex prompt_mutex;
     int prompt_state = 0;           // 0 not made yet, 1 ready, -1 could not be made (batches then go token by token)
     uint16_t *prompt_arena = nullptr;
@@ -239,6 +243,7 @@ struct lv_session {
     uint32_t *status_host = nullptr;      // pinned, written by the persistent kernel: [0] a poll expired, [kStatusToken] greedy pick
     uint32_t wait_limit = 0;              // polls per hand-over of the persistent kernel; 0 = default
     bool xcd_handover = true;             // the persistent kernel may keep a head's hand-overs inside its XCD (lv_session_set_xcd_handover)
+    bool logits_on_host = false;          // the last step left its logits in logits_host as well
     bool pick_in_status = false;          // the last step ran the persistent kernel, whose greedy pick is in status_host
     bool mega_step = false;               // the step in flight ran the persistent kernel
     int mega_failures = 0;                // steps of the persistent kernel in a row that ended with an expired wait
@@ -1337,6 +1342,42 @@ static int build_mega(lv_model *m)
     return LV_OK;
 }
 
+// Which models take lv_small.h's launch for a token: those whose operator chain has ten launches a layer (below the streaming kernels' 2048
+// rows) and whose work a few workgroups do in less time than those launches take to follow one another.  The longest stretch is a
+// head's three projections, which one workgroup does: at most kSmallHeadTiles tiles a wave.  us a token, launch and chain, 100 rows of
+// context: width 256, 3 tiles, 2 layers 53 and 117; 512, 6 tiles, 8 layers 198 and 361; 768, 12 tiles, 12 layers 464 and 568; 1024 with 16
+// heads, 12 tiles, 4 layers 193 and 218, with 8 heads, 24 tiles, 240 and 221.
+constexpr uint32_t kSmallHeadTiles = 12;
+// One workgroup also walks a head's cache rows, 90 ns of a layer for every 1000 elements of them, where the chain splits them over several:
+// width 512, 4 heads of 128, 4 layers 148 and 191 us behind 100 rows, 199 and 205 behind 1000, 257 and 221 behind 2000; width 256, 4 heads
+// of 64, 76 and 118 behind 2000.
+constexpr uint32_t kSmallRowElements = 131072;
+static int build_small(lv_model *m)
+{
+    const lv_hparams &hp = m->hp;
+    const uint32_t D = hp.dim, F = hp.ff, ft = m->output.ftype;
+    if (m->mega_kind || D > kSmallMaxDim || F > kSmallMaxFf || hp.heads > kSmallMaxWGs || m->ctx->props.multiProcessorCount < (int)kSmallMaxWGs) return LV_OK;
+    if (m->tok_ftype != LV_F32 && m->tok_ftype != LV_Q4_0 && m->tok_ftype != LV_Q8_0) return LV_OK;
+    std::vector<SmallLayer> table;
+    for (const LayerWeights &lw : m->layers) {
+        for (const lv_matrix *x : {&lw.wq, &lw.wk, &lw.wv, &lw.wo, &lw.w1, &lw.w2, &lw.w3})
+            if (x->ftype != ft || (x->view.scales_f32 != nullptr) != (m->output.view.scales_f32 != nullptr)) return LV_OK;
+        table.push_back({lw.wq.view, lw.wk.view, lw.wv.view, lw.wo.view, lw.w1.view, lw.w2.view, lw.w3.view, lw.attn_norm, lw.ffn_norm});
+    }
+    const auto tiles = [](uint32_t rows, uint32_t cols) -> uint32_t {
+        const uint32_t nb = cols / 32, lanes = 1u << small_lanes_log2(nb);
+        return (rows * lanes + 63) / 64 * ((nb + lanes - 1) / lanes);
+    };
+    if (tiles(3 * hp.rot, D) > kSmallHeadTiles * kSmallWaves) return LV_OK;
+    // a pair of tiles a wave in the feed-forward, or four tiles of a large vocabulary
+    const uint32_t most = std::max(tiles(F, D), tiles(hp.vocab, D) / 4);
+    m->small_wgs = std::min(kSmallMaxWGs, std::max(hp.heads, (most + kSmallWaves - 1) / kSmallWaves));
+    HIP_TRY(hipMalloc(reinterpret_cast<void **>(&m->small_layers), table.size() * sizeof(SmallLayer)));
+    HIP_TRY(hipMemcpyAsync(m->small_layers, table.data(), table.size() * sizeof(SmallLayer), hipMemcpyHostToDevice, m->ctx->stream));
+    HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+    return LV_OK;
+}
+
 struct Want {
     std::string name;
     uint32_t rows, cols;   // expected shape (cols == 1 for vectors)
@@ -1446,7 +1487,9 @@ extern "C" int lv_model_upload(lv_ctx *c, const void *base, uint64_t base_size, 
     }
     (void)hipFree(staging);
     if (rc == LV_OK) rc = build_mega(m);
+    if (rc == LV_OK) rc = build_small(m);
     if (rc != LV_OK) {
+        (void)hipFree(m->small_layers);
         (void)hipFree(m->mega_stream);
         (void)hipFree(m->mega_norms);
         (void)hipFree(m->tok_f32_own);
@@ -1491,6 +1534,7 @@ extern "C" int lv_model_destroy(lv_model *m)
     (void)hipFree(m->output_copy);
     (void)hipFree(m->mega_stream);
     (void)hipFree(m->mega_norms);
+    (void)hipFree(m->small_layers);
     (void)hipFree(m->tok_f32_own);
     (void)hipFree(m->arena);
     delete m;
@@ -1584,9 +1628,9 @@ static int session_alloc(lv_session *s)
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->v), D * 4));
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->vo), D * 4));
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->ff), F * 4));
-    if (s->model->mega_kind) {
-        size_t bytes = 0, local_bytes = 0;
-        LV_TRY(mega_dispatch(s->model->mega_kind, [&](auto shape) -> int {
+    if (s->model->mega_kind || s->model->small_wgs) {
+        size_t bytes = (size_t)hp.layers * small_layer_floats(hp.dim, hp.ff) * 4, local_bytes = 0;
+        if (s->model->mega_kind) LV_TRY(mega_dispatch(s->model->mega_kind, [&](auto shape) -> int {
             bytes = ((size_t)hp.layers * decltype(shape)::XCHG_LAYER + decltype(shape)::XCHG_TAIL) * 4;
             local_bytes = (size_t)hp.layers * decltype(shape)::LOCAL_LAYER * 4;
             return LV_OK;
@@ -1595,6 +1639,7 @@ static int session_alloc(lv_session *s)
         for (int i = 0; i < 2; i++) {
             LV_TRY(uncached_take(s->model->ctx->device, reinterpret_cast<void **>(&s->xchg[i]), bytes, &s->xchg_pooled[i]));
             HIP_TRY(hipMemsetAsync(s->xchg[i], 0xff, bytes, s->stream));
+            if (!local_bytes) continue;
             HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->xl[i]), local_bytes));
             HIP_TRY(hipMemsetAsync(s->xl[i], 0xff, local_bytes, s->stream));
         }
@@ -1760,6 +1805,22 @@ extern "C" int lv_session_path(const lv_session *s, int *path)
     return LV_OK;
 }
 
+// Launches whose workgroups wait for each other (mega_mutex is held): behind the last one of another session
+static int mega_turn_begin(lv_session *s)
+{
+    lv_ctx *c = s->model->ctx;
+    if (c->mega_last && c->mega_last != s) HIP_TRY(hipStreamWaitEvent(s->stream, c->mega_done, 0));
+    return LV_OK;
+}
+static int mega_turn_end(lv_session *s)
+{
+    lv_ctx *c = s->model->ctx;
+    if (!c->mega_done) HIP_TRY(hipEventCreateWithFlags(&c->mega_done, hipEventDisableTiming));
+    HIP_TRY(hipEventRecord(c->mega_done, s->stream));
+    c->mega_last = s;
+    return LV_OK;
+}
+
 // One token through the persistent kernel.  Its workgroups hand vectors to each other, so all 256 of them have to be
 // resident at once: one per CU, on a device of at least 256 CUs that grants the kernel a workgroup per CU (lv_ctx::mega_fits
 // asks the runtime once per shape class).  *refused is set, and LV_OK returned, when that does not hold or the launch is
@@ -1790,7 +1851,7 @@ static int launch_mega(lv_session *s, uint32_t pos, uint32_t token, bool *refuse
     void *params[] = {&a};
     lv_ctx *c = m->ctx;
     std::lock_guard<std::mutex> lock(c->mega_mutex);
-    if (c->mega_last && c->mega_last != s) HIP_TRY(hipStreamWaitEvent(s->stream, c->mega_done, 0));
+    LV_TRY(mega_turn_begin(s));
     LV_TRY(mega_dispatch(m->mega_kind, [&](auto shape) -> int {
         using S = decltype(shape);
         const void *kernel = reinterpret_cast<const void *>(&mega_decode_kernel<S>);
@@ -1818,10 +1879,46 @@ static int launch_mega(lv_session *s, uint32_t pos, uint32_t token, bool *refuse
         s->xchg_turn--;
         return LV_OK;
     }
-    if (!c->mega_done) HIP_TRY(hipEventCreateWithFlags(&c->mega_done, hipEventDisableTiming));
-    HIP_TRY(hipEventRecord(c->mega_done, s->stream));
-    c->mega_last = s;
-    return LV_OK;
+    return mega_turn_end(s);
+}
+
+template <int QT, bool SF32>
+static void launch_small_kernel(const SmallArgs &a, uint32_t wgs, uint32_t rot, hipStream_t st)
+{
+    if (rot == 32) small_decode_kernel<QT, SF32, 32><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
+    else if (rot == 64) small_decode_kernel<QT, SF32, 64><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
+    else small_decode_kernel<QT, SF32, 128><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
+}
+
+// One token of a small model.  Its few workgroups wait for each other as the persistent kernel's do and take turns with those.
+static int launch_small(lv_session *s, uint32_t pos, uint32_t token)
+{
+    const lv_model *m = s->model;
+    SmallArgs a{};
+    a.layer = m->small_layers;
+    a.output = m->output.view;
+    a.norm = m->norm;
+    a.tok = m->tok_quant.view;
+    a.tok_f32 = m->tok_ftype == LV_F32 ? m->tok_f32 : nullptr;
+    a.tok_q4 = m->tok_ftype == LV_Q4_0;
+    a.kv = s->kv;
+    a.trig = s->trig;
+    a.xchg = s->xchg[s->xchg_turn & 1];
+    a.xchg_rearm = s->xchg[(s->xchg_turn + 1) & 1];
+    a.logits = s->logits;
+    a.logits_host = s->logits_host;
+    a.status = s->status_host;
+    a.layers = m->hp.layers; a.vocab = m->hp.vocab; a.backlog = s->backlog; a.pos = pos; a.token = token;
+    a.D = m->hp.dim; a.F = m->hp.ff; a.heads = m->hp.heads;
+    a.spin_limit = s->wait_limit ? s->wait_limit : kSpinLimit;
+    std::lock_guard<std::mutex> lock(m->ctx->mega_mutex);
+    LV_TRY(mega_turn_begin(s));
+    const auto launch = m->output.ftype == LV_Q4_0 ? m->output.view.scales_f32 ? launch_small_kernel<4, true> : launch_small_kernel<4, false>
+                                                   : m->output.view.scales_f32 ? launch_small_kernel<8, true> : launch_small_kernel<8, false>;
+    launch(a, m->small_wgs, m->hp.rot, s->stream);
+    HIP_TRY(hipGetLastError());
+    s->xchg_turn++;
+    return mega_turn_end(s);
 }
 
 // -----------------------------------------------------------------------------------------------------------
@@ -2700,6 +2797,7 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
 
     s->have_logits = false;
     s->pick_in_status = false;
+    s->logits_on_host = false;
     s->logits_rows = 0;
     if (s->all_logits) {
         if (n > s->logits_cap) {
@@ -2767,8 +2865,10 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     const uint32_t rest = n <= kPrefillChunk ? n : n % kPrefillChunk;
     const bool mid = !persistent && !few && n >= kPrefillMin && rest && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && mid_pays(s->model->hp, rest) &&
                      ensure_short_copy(s->model);
+    const bool small = n < kPrefillMin && !few && s->model->small_wgs && s->path == LV_PATH_AUTO && path == LV_PATH_GRAPH && !s->trace && !s->mega_off &&
+                       (pos + n) * s->model->hp.rot <= kSmallRowElements;
     const bool batch = !persistent && !few && n >= batch_min && (!s->trace || s->block) && ((mid && n == rest) || ensure_prompt_copy(s->model));
-    if (!persistent) {
+    if (!persistent && !small) {
         s->cfg_host[0] = pos;
         memcpy(s->cfg_host + 1, tokens, (size_t)n * 4);
         if (batch) HIP_TRY(hipMemcpyAsync(s->cfg, s->cfg_host, (size_t)(1 + n) * 4, hipMemcpyHostToDevice, s->stream));
@@ -2777,6 +2877,14 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
         // launched above
     } else if (few) {
         LV_TRY(record_short(s, 0, n, pos, true, row_base));
+    } else if (small) {
+        for (uint32_t i = 0; i < n; i++) {
+            LV_TRY(launch_small(s, pos + i, tokens[i]));
+            s->mega_step = true;
+            s->in_flight = true;
+            if (s->all_logits) HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)i * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
+        }
+        s->logits_on_host = true;
     } else if (n == 1 && (path == LV_PATH_GRAPH || (path == LV_PATH_PERSISTENT && s->use_graph)) && !s->trace) {
         if (!s->graph_exec) {
             HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
@@ -2843,8 +2951,10 @@ extern "C" int lv_logits_read(lv_session *s, float *dst)
     if (!s || !dst) return fail(LV_ERR_ARG, "lv_logits_read: null argument");
     if (!s->have_logits) return fail(LV_ERR_STATE, "lv_logits_read: no step has produced logits");
     const uint32_t V = s->model->hp.vocab;
-    logits_out_kernel<<<dim3((V + 1023) / 1024), dim3(256), 0, s->stream>>>(s->logits_host, s->logits, V);
-    HIP_TRY(hipGetLastError());
+    if (!s->logits_on_host) {
+        logits_out_kernel<<<dim3((V + 1023) / 1024), dim3(256), 0, s->stream>>>(s->logits_host, s->logits, V);
+        HIP_TRY(hipGetLastError());
+    }
     LV_TRY(lv_step_wait(s));
     memcpy(dst, s->logits_host, (size_t)V * 4);
     return LV_OK;

@@ -1,0 +1,86 @@
+"""One token of a small model as one launch (lv_small.h) against the oracle and the operator chain: rows that fill tiles and rows that do not,
+one and several blocks a lane, every head size, contexts on both sides of what the workgroup holds of the cache at once."""
+import numpy as np
+import pytest
+
+import ggjt_builder as gb
+
+pytestmark = pytest.mark.gpu
+
+ABS_TOL, REL_TOL = 1e-2, 1e-3       # of a whole evaluation in fp32 with fp16 cache rows, as in the other tests of whole models
+
+
+def _check(got, want):
+    err = np.max(np.abs(got - want))
+    assert err <= ABS_TOL and err <= REL_TOL * np.max(np.abs(want)), (err, np.max(np.abs(want)))
+
+
+# no width is a multiple of 128 where steps of several tokens are compared: those models have other kernels for such steps
+SHAPES = {
+    "one head, one block": dict(vocab=259, dim=32, heads=1, layers=1, ff=32),
+    "three blocks a row": dict(vocab=500, dim=96, heads=3, layers=2, ff=224),
+    "two columns a lane": dict(vocab=512, dim=256, heads=4, layers=2, ff=2080),
+    "head of 128": dict(vocab=513, dim=256, heads=2, layers=3, ff=704),
+    "sixteen heads": dict(vocab=4099, dim=512, heads=16, layers=2, ff=1376),
+    "widest": dict(vocab=1000, dim=1024, heads=8, layers=2, ff=8160),
+    "more heads than tiles": dict(vocab=260, dim=1024, heads=32, layers=1, ff=64),
+}
+
+
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+@pytest.mark.parametrize("wtype", ["q4_0", "q8_0", "q4_0 version 1"])
+def test_small_model_tokens_match_oracle_and_chain(lva, orc, ctx, tmp_path, shape, wtype):
+    p, c = str(tmp_path / "m.ggml"), SHAPES[shape]
+    lva.write_model(p, wtype=lva.LV_Q8_0 if wtype == "q8_0" else lva.LV_Q4_0, tok_type=lva.LV_Q4_0 if wtype.endswith("1") else lva.LV_F32, seed=31, **c)
+    if wtype.endswith("1"):
+        gb.convert_to_v1(p, str(tmp_path / "v1.ggml"))
+        p = str(tmp_path / "v1.ggml")
+    om = orc.Model(p)
+    osess = orc.Session(om, 512)
+    model = lva.Model(ctx, p)
+    one, other, chain = (lva.Session(model, 512) for _ in range(3))
+    assert one.path() == lva.PATH_GRAPH
+    chain.set_path(lva.PATH_GRAPH)
+    toks = lva.synth_tokens(290, 3, c["vocab"], seed=2)
+    pos = 0
+    # alone, a step of several tokens, up to and across the borders of 64, 128 and 256 cache rows
+    for n in (1, 1, 9, 1, 52, 1, 1, 61, 1, 1, 126, 1, 1, 1):
+        step = toks[pos:pos + n]
+        want = osess.eval(step)
+        for s in (one, other, chain):           # sessions take turns on the device
+            s.begin(step, pos)
+        _check(one.logits(), want)
+        _check(chain.logits(), want)
+        assert np.array_equal(one.logits(), other.logits())
+        assert one.argmax() == int(np.argmax(one.logits()))
+        pos += n
+    s = one
+    s.keep_all_logits()
+    s.begin(toks[:3], 0)
+    rows = s.logits_rows(0, 3)
+    assert np.array_equal(rows[2], s.logits())
+    other.begin(toks[:1], 0)
+    assert np.array_equal(rows[0], other.logits())
+    for which in (0, 1):                        # cache rows of layer 0: the same inputs, sums in another order
+        a, b = one.kv(0, which, 3), chain.kv(0, which, 3)
+        assert np.mean(a != b) < 1e-2
+    for s in (one, other, chain):
+        s.close()
+    model.close(); osess.close(); om.close()
+
+
+def test_small_model_not_a_number_is_a_result_and_no_expired_wait(lva, ctx, tmp_path):
+    """hand-overs wait until a value is there; the bit pattern that stands for `not there yet` is a NaN a model can hold"""
+    p = str(tmp_path / "m.ggml")
+    lva.write_model(p, wtype=lva.LV_Q4_0, seed=3, vocab=512, dim=256, heads=4, layers=2, ff=704)
+    raw = np.fromfile(p, np.uint8)
+    name = b"layers.0.ffn_norm.weight"
+    at = (raw.tobytes().index(name) + len(name) + 31) // 32 * 32
+    raw[at:at + 256 * 4] = 255
+    raw.tofile(p)
+    model = lva.Model(ctx, p)
+    s = lva.Session(model, 128)
+    for i in range(3):
+        s.begin([5 + i], i)
+        assert np.isnan(s.logits()).all()
+    s.close(); model.close()
