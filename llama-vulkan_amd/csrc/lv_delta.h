@@ -305,4 +305,268 @@ __global__ __launch_bounds__(kScanThreads) void delta_scan_kernel(DeltaScanArgs 
     }
 }
 
+// ---- batches in chunks of 16 tokens ---------------------------------------------------------------------------------------
+// The scan above is a chain over tokens, 172 ns each whatever the state's size: 352 us for 2048 tokens and 32 heads of 128 x 128.  In chunks
+// it takes 168: 62 for delta_chunk_kernel, 106 for the chain.  Inside a chunk that starts at state S0, with
+// D(s, t) = g_{s+1} ... g_t per channel,
+//   A[t][s] = (D(s, t) k_s) . k_t for s < t,   B[t][s] = (D(s, t) k_s) . q_t for s <= t
+//   u_t = beta_t (v_t - (D(-1, t) k_t) . S0 - sum_{s<t} A[t][s] u_s)       a triangular system: U = T (V - K' S0)
+//   o_t = (D(-1, t) q_t) . S0 + sum_{s<=t} B[t][s] u_s
+//   S  <- D(-1, 15) S0 + sum_s (D(s, 15) k_s) u_s
+// so the chain is one of matrix products a chunk.  Every D is a running product of decays of tokens in a row, never a quotient: strong
+// decays underflow and nothing overflows; T holds products of contractions (unit keys, beta below 1).  All of it stays fp32, the
+// products on v_mfma_f32_16x16x4_f32.
+//
+// delta_chunk_kernel forms what does not depend on the state, all chunks side by side, in operand order of the instruction (lane = 16 g + m
+// has row m, columns 4 g + i of a first operand in step i), so that every load of the chain is one contiguous run.  Per head and chunk,
+// W = 64 J channels in tiles of 16:
+//   -T K' [tile][lane][i] (token m, channel 4 g + i), D(-1, t) q_t the same, D(s, 15) k_s [tile][lane][i] (channel m, token 4 g + i),
+//   D(-1, 15) [W], T [i][lane] (token m, token 4 g + i), B the same
+constexpr int kChunkTokens = 16, kChunkThreads = 256, kChainThreads = 512;
+template <int J> constexpr int chunk_floats() { return 49 * 64 * J + 512; }
+template <int J> constexpr int chunk_lds_floats() { return 80 * 64 * J + 512 + 16; }
+
+struct DeltaChunkArgs {
+    DeltaSpec s;
+    uint32_t n, chunks;       // tokens, and chunks of them
+    bool fresh;               // the batch starts the sequence: the state is zero
+    const float *q, *k, *v, *g, *beta;    // as DeltaScanArgs
+    float *ops;               // [heads][chunks][chunk_floats]
+    float *o;
+};
+
+// grid (heads, chunks).  Bound by the vector units: 240 running products and dots of W a chunk.  Three workgroups a CU need at most 168
+// registers (31 us for 1024 tokens and 32 heads; with two 44).
+template <int J>
+__global__ __launch_bounds__(kChunkThreads, J <= 2 ? 3 : 1) void delta_chunk_kernel(DeltaChunkArgs a)
+{
+    constexpr int W = 64 * J;
+    extern __shared__ __align__(16) float lds[];
+    float *const lk = lds, *const lq = lk + 16 * W, *const lg = lq + 16 * W, *const la = lg + 16 * W, *const lb = la + 256, *const lbeta = lb + 256, *const out = lbeta + 16;
+    const DeltaSpec &s = a.s;
+    const uint32_t head = blockIdx.x, kvh = head / (s.heads / s.kv_heads), t0 = blockIdx.y * kChunkTokens;
+    const int tid = threadIdx.x;
+    float *const ops = a.ops + ((size_t)head * a.chunks + blockIdx.y) * chunk_floats<J>();
+
+    // tokens past the end do nothing: no key, no query, decay 1.  Channels past the size hold no state
+    for (int i = tid; i < 16 * W / 4; i += kChunkThreads) {
+        const uint32_t r = i / (W / 4), d = i % (W / 4) * 4, t = t0 + r;
+        float4 k = make_float4(0.f, 0.f, 0.f, 0.f), q = k, g = make_float4(1.f, 1.f, 1.f, 1.f);
+        if (t < a.n) {
+            k = *reinterpret_cast<const float4 *>(a.k + ((size_t)t * s.kv_heads + kvh) * W + d);
+            q = *reinterpret_cast<const float4 *>(a.q + ((size_t)t * s.kv_heads + kvh) * W + d);
+            g = *reinterpret_cast<const float4 *>(a.g + ((size_t)t * s.heads + head) * W + d);
+        }
+        if (d >= s.dim) g.x = 0.f;
+        if (d + 1 >= s.dim) g.y = 0.f;
+        if (d + 2 >= s.dim) g.z = 0.f;
+        if (d + 3 >= s.dim) g.w = 0.f;
+        *reinterpret_cast<float4 *>(lk + r * W + d) = k;
+        *reinterpret_cast<float4 *>(lq + r * W + d) = q;
+        *reinterpret_cast<float4 *>(lg + r * W + d) = g;
+    }
+    if (tid < 16) lbeta[tid] = t0 + tid < a.n ? a.beta[(size_t)(t0 + tid) * s.heads + head] : 0.f;
+    __syncthreads();
+
+    // 16 lanes a key s, 4 J of its channels each: r = D(s, t) k_s as t goes on
+    const int src = tid >> 4, l16 = tid & 15;
+    float4 r[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) r[j] = *reinterpret_cast<const float4 *>(lk + src * W + j * 64 + l16 * 4);
+#pragma unroll 2
+    for (int t = 0; t < 16; t++) {
+        float pa = 0.f, pb = 0.f;
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const int at = t * W + j * 64 + l16 * 4;
+            const float4 g = *reinterpret_cast<const float4 *>(lg + at), k = *reinterpret_cast<const float4 *>(lk + at), q = *reinterpret_cast<const float4 *>(lq + at);
+            const bool on = t > src;
+            r[j].x *= on ? g.x : 1.f; r[j].y *= on ? g.y : 1.f; r[j].z *= on ? g.z : 1.f; r[j].w *= on ? g.w : 1.f;
+            pa = fmaf(r[j].x, k.x, pa); pa = fmaf(r[j].y, k.y, pa); pa = fmaf(r[j].z, k.z, pa); pa = fmaf(r[j].w, k.w, pa);
+            pb = fmaf(r[j].x, q.x, pb); pb = fmaf(r[j].y, q.y, pb); pb = fmaf(r[j].z, q.z, pb); pb = fmaf(r[j].w, q.w, pb);
+        }
+        pa = group16_sum(pa);
+        pb = group16_sum(pb);
+        if (l16 == 0) {
+            la[t * 16 + src] = t > src ? pa : 0.f;
+            lb[t * 16 + src] = t >= src ? pb : 0.f;
+        }
+    }
+    __syncthreads();
+
+    // a column of the triangular system a thread: the W of K', then the 16 of the unit matrix.  Results of channels meet in LDS, in operand
+    // order with the 64 floats of a g rotated against bank conflicts
+    for (int x = tid; x < W + 16; x += kChunkThreads) {
+        float w[16], run = 1.f;
+        const int tile = x >> 4, g = (x >> 2) & 3, row = tile * 256 + g * 64, at = (x & 3) + 4 * (g + 4 * tile);
+#pragma unroll
+        for (int t = 0; t < 16; t++) {
+            float rhs;
+            if (x < W) {
+                run *= lg[t * W + x];
+                rhs = lk[t * W + x] * run;
+                out[16 * W + row + ((at + 4 * t) & 63)] = lq[t * W + x] * run;
+            } else rhs = x - W == t ? 1.f : 0.f;
+#pragma unroll
+            for (int e = 0; e < t; e++) rhs = fmaf(-la[t * 16 + e], w[e], rhs);
+            w[t] = lbeta[t] * rhs;
+        }
+        if (x < W) {
+#pragma unroll
+            for (int t = 0; t < 16; t++) out[row + ((at + 4 * t) & 63)] = -w[t];
+            ops[48 * W + x] = run;
+        } else {
+#pragma unroll
+            for (int t = 0; t < 16; t++) ops[49 * W + (x & 3) * 64 + ((x >> 2) & 3) * 16 + t] = w[t];
+        }
+    }
+    ops[49 * W + 256 + tid] = lb[(tid & 15) * 16 + ((tid >> 4) & 3) * 4 + (tid >> 6)];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        float *const k = lk + (j * 4 + (l16 >> 2)) * 256 + ((src >> 2) * 16 + (l16 & 3) * 4) * 4 + (src & 3);
+        k[0] = r[j].x; k[4] = r[j].y; k[8] = r[j].z; k[12] = r[j].w;
+    }
+    for (int i = tid; i < 8 * W; i += kChunkThreads) {           // the 4 W float4 of either
+        const int c = i & (4 * W - 1), from = (i & ~15) + (((i & 15) + ((c >> 4) & 3) + 4 * (c >> 6)) & 15);
+        reinterpret_cast<float4 *>(ops)[i] = reinterpret_cast<const float4 *>(out)[from];
+    }
+    __syncthreads();
+    for (int i = tid; i < 4 * W; i += kChunkThreads) reinterpret_cast<float4 *>(ops + 32 * W)[i] = reinterpret_cast<const float4 *>(lk)[i];
+}
+
+// The chain: grid (heads, vdim / 16 up), 16 columns a workgroup.  The state stays in accumulators, whose layout (channel 4 g + i, column m) is
+// that of a second operand.  Waves 0 to 3 hold a quarter of the channels each and do nothing but the chain: their parts of U meet in LDS,
+// then each adds its part of the update.  Waves 4 to 7 share their SIMDs, fill the waits and do what is beside the chain, on copies of the
+// state in LDS: T V of the chunk to come, and the read-out.  A chunk is 26 instructions of 32 clocks a SIMD, 0.39 us; it takes 0.83, of which
+// loads are 0.14 and the hand-over of U most of the rest.  With everything in four waves and operands in row order it took 1.2.
+template <int J>
+__global__ __launch_bounds__(kChainThreads, 1) void delta_chunk_scan_kernel(DeltaChunkArgs a)
+{
+    constexpr int W = 64 * J, DEPTH = J == 4 ? 3 : J == 3 ? 4 : 6;       // chunks on their way
+    __shared__ __align__(16) lv_f4 pu[2][4][64], po[2][4][64], tv[2][4][64], st[2][4][J][64];       // [chunk parity][wave][lane]
+    const DeltaSpec &s = a.s;
+    const uint32_t head = blockIdx.x, HV = s.heads * s.vdim;
+    const int lane = threadIdx.x & 63, wl = (threadIdx.x >> 6) & 3, w = __builtin_amdgcn_readfirstlane(wl), g = lane >> 4, c16 = lane & 15;
+    const uint32_t col = blockIdx.y * 16 + c16, vcol = min(col, s.vdim - 1), last = a.chunks - 1;
+    const bool live = col < s.vdim;
+    const float *const first = a.ops + (size_t)head * a.chunks * chunk_floats<J>();
+    const auto run_all = [&](auto &&chunk) __attribute__((always_inline)) {      // chunk(place in the queue, chunk)
+        uint32_t ch = 0;
+        for (; ch + DEPTH <= a.chunks; ch += DEPTH) {
+#pragma unroll
+            for (int i = 0; i < DEPTH; i++) chunk(i, ch + i);
+        }
+#pragma unroll
+        for (int i = 0; i < DEPTH - 1; i++)
+            if (ch + i < a.chunks) chunk(i, ch + i);
+    };
+
+    if (threadIdx.x < 256) {
+        float *const colp = s.state + ((size_t)head * s.vdim + vcol) * W + w * 16 * J + 4 * g;
+        lv_f4 S[J], k[DEPTH][J], kt[DEPTH][J], d[DEPTH][J];
+#pragma unroll
+        for (int j = 0; j < J; j++) S[j] = a.fresh || !live ? lv_f4(0.f) : *reinterpret_cast<const lv_f4 *>(colp + 16 * j);
+        const auto fetch = [&](int i, uint32_t ch) __attribute__((always_inline)) {
+            const float *p = first + (size_t)min(ch, last) * chunk_floats<J>() + w * J * 256 + lane * 4;
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                k[i][j] = *reinterpret_cast<const lv_f4 *>(p + j * 256);
+                kt[i][j] = *reinterpret_cast<const lv_f4 *>(p + 32 * W + j * 256);
+                d[i][j] = *reinterpret_cast<const lv_f4 *>(first + (size_t)min(ch, last) * chunk_floats<J>() + 48 * W + (w * J + j) * 16 + 4 * g);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < DEPTH; i++) fetch(i, i);
+        lds_barrier();
+        run_all([&](int q, uint32_t ch) __attribute__((always_inline)) {
+            const int at = ch & 1;
+            lv_f4 u = tv[at][w][lane];
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                st[at][w][j][lane] = S[j];
+#pragma unroll
+                for (int i = 0; i < 4; i++) u = __builtin_amdgcn_mfma_f32_16x16x4f32(k[q][j][i], S[j][i], u, 0, 0, 0);
+            }
+            pu[at][w][lane] = u;
+#pragma unroll
+            for (int j = 0; j < J; j++) S[j] *= d[q][j];
+            lds_barrier();
+            u = (pu[at][0][lane] + pu[at][1][lane]) + (pu[at][2][lane] + pu[at][3][lane]);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < J; j++) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[q][j][i], u[i], S[j], 0, 0, 0);
+            fetch(q, ch + DEPTH);
+        });
+        lds_barrier();
+        if (live) {
+#pragma unroll
+            for (int j = 0; j < J; j++) *reinterpret_cast<lv_f4 *>(colp + 16 * j) = S[j];
+        }
+        return;
+    }
+
+    lv_f4 qq[DEPTH][J];
+    float t[DEPTH], b[DEPTH], v[DEPTH];
+    // t and v of the chunk behind it: they are wanted one chunk earlier
+    const auto fetch_tv = [&](int i, uint32_t ch) __attribute__((always_inline)) {
+        t[i] = first[(size_t)min(ch, last) * chunk_floats<J>() + 49 * W + w * 64 + lane];
+        v[i] = a.v[(size_t)min(ch * kChunkTokens + 4 * g + w, a.n - 1) * HV + head * s.vdim + vcol];     // past the end T is zero
+    };
+    const auto fetch = [&](int i, uint32_t ch) __attribute__((always_inline)) {
+        const float *p = first + (size_t)min(ch, last) * chunk_floats<J>();
+#pragma unroll
+        for (int j = 0; j < J; j++) qq[i][j] = *reinterpret_cast<const lv_f4 *>(p + 16 * W + (w * J + j) * 256 + lane * 4);
+        b[i] = p[49 * W + 256 + w * 64 + lane];
+        fetch_tv(i, ch + 1);
+    };
+    // m (lower triangular) times this wave's rows of the right operand.  The instruction multiplies the zeros above the diagonal as well: a
+    // value that is not finite would reach tokens before its own, and then the products are taken one by one
+    const auto triangular = [&](const float *m, float mine, float x, lv_f4 acc) __attribute__((always_inline)) -> lv_f4 {
+        if (!__any((__float_as_uint(x) & 0x7f800000u) == 0x7f800000u)) return __builtin_amdgcn_mfma_f32_16x16x4f32(mine, x, acc, 0, 0, 0);
+#pragma unroll 1
+        for (int gg = 0; gg < 4; gg++) {
+            const float other = __shfl(x, gg * 16 + c16);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (4 * gg + w <= 4 * g + i) acc[i] = fmaf(m[w * 64 + gg * 16 + 4 * g + i], other, acc[i]);
+        }
+        return acc;
+    };
+    // token 4 g + w of a chunk, from the parts of before the last barrier
+    const auto put = [&](uint32_t ch) __attribute__((always_inline)) {
+        float o = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) o += reinterpret_cast<const float *>(&po[ch & 1][i][lane])[w];
+        const uint32_t at = ch * kChunkTokens + 4 * g + w;
+        if (live && at < a.n) a.o[(size_t)at * HV + head * s.vdim + col] = o;
+    };
+    fetch_tv(0, 0);
+    tv[0][w][lane] = triangular(first + 49 * W, t[0], v[0], lv_f4(0.f));
+#pragma unroll
+    for (int i = 0; i < DEPTH; i++) fetch(i, i);
+    lds_barrier();
+    run_all([&](int q, uint32_t ch) __attribute__((always_inline)) {
+        const int at = ch & 1;
+        tv[at ^ 1][w][lane] = triangular(first + (size_t)min(ch + 1, last) * chunk_floats<J>() + 49 * W, t[q], v[q], lv_f4(0.f));
+        lds_barrier();
+        lv_f4 o = lv_f4(0.f);
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const lv_f4 S = st[at][w][j][lane];
+#pragma unroll
+            for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(qq[q][j][i], S[i], o, 0, 0, 0);
+        }
+        float u = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) u += reinterpret_cast<const float *>(&pu[at][i][lane])[w];
+        po[at][w][lane] = triangular(first + (size_t)ch * chunk_floats<J>() + 49 * W + 256, b[q], u, o);
+        if (ch) put(ch - 1);
+        fetch(q, ch + DEPTH);
+    });
+    lds_barrier();
+    put(last);
+}
+
 }  // namespace lv

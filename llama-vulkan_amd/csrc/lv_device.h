@@ -174,6 +174,15 @@ __device__ __forceinline__ void block_sums_waves(float (&v)[N], float *scratch, 
     }
 }
 
+// Workgroup barrier that orders LDS traffic only: global loads stay in flight across it (__syncthreads would
+// wait for vmcnt(0) and drain a kernel's queue of loads).
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---- fp16 ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ float half_bits_to_float(uint16_t h)
 {

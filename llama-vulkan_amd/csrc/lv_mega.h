@@ -95,15 +95,6 @@ __host__ __device__ __forceinline__ void mega_qkv_row(int b, int t, int &which, 
     row = (hl * 8 + (b & 7)) * S::R + within % S::R;
 }
 
-// Workgroup barrier that orders LDS traffic only: global loads of the weight queue stay in flight across it
-// (__syncthreads would wait for vmcnt(0) and drain the queue at every phase step).
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // A value the compiler has to take as new each time: what is computed from it inside the layer loop (LDS addresses above
 // all) is then computed there, a few instructions each, instead of once in front of the loop and kept in registers.  Used
 // (OPAQUE) by the shape classes whose kernel would otherwise spill; where registers suffice, keeping the values is faster.

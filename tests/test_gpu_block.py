@@ -87,6 +87,37 @@ def test_delta_rule_alone(lva, ctx, k, compute):
     check_model(lva, ctx, cfg, W, 110, compute, cuts=((1000,), (1,), (37, 2, 16, 31, 3)))
 
 
+@pytest.mark.parametrize("k", range(len(DELTA)))
+def test_delta_rule_in_chunks(lva, ctx, k):
+    """bfloat16 batches from 224 tokens on go in chunks of 16 tokens, 1024 tokens at a time: full and partial chunks and stretches, going on from
+    a state, slow and strong decays, against shorter batches, which go token by token.  Both round the same operands to bfloat16 (2^-9 each),
+    so they differ where the sums of 32 bits fall on different sides of a rounding: a few rounding steps of the layer's output"""
+    cfg = bb.config(width=44, layers=[bb.layer(right=bb.delta(**DELTA[k]), experts=0, without=("left",))])
+    W = bb.weights(cfg, seed=20 + k, rank_a=5 + 20 * k, rank_g=70 - 15 * k)
+    for shift in (0, 6, -12):          # one after the other: softplus from 1e-3 to 8, decays from nearly 1 to below 1e-3
+        W["l0.mix.right.dt_bias"] = bb.to_bf16(bb.from_bf16(W["l0.mix.right.dt_bias"]) + shift)
+        toks = tokens_for(cfg, 500 if shift else 1300, 5)
+        with Device(lva, ctx, cfg, W, BF16, 2048) as d:
+            want = d.run(toks, (223,))
+            for c in ((len(toks),), (223, 224, 1000), (5, 255, 240, 1000), (225, 3, 1030)):
+                assert rel(d.run(toks, c), want) < 1e-2, (shift, c)
+
+
+def test_delta_rule_in_chunks_is_causal(lva, ctx):
+    """a token whose values are not finite must not reach the ones before it, also those of its own chunk"""
+    cfg = bb.config(width=44, layers=[bb.layer(right=bb.delta(**DELTA[2]), experts=0, without=("left",))])
+    W = bb.weights(cfg, seed=22, rank_a=45, rank_g=40)
+    bad = 3
+    toks = np.where(tokens_for(cfg, 300, 5) == bad, 4, tokens_for(cfg, 300, 5)).astype(np.uint32)
+    with Device(lva, ctx, cfg, W, BF16) as d:
+        want = d.run(toks, (1000,))
+    W["embed"][bad] = 0x7f80
+    toks[73] = bad
+    with Device(lva, ctx, cfg, W, BF16) as d:
+        got = d.run(toks, (1000,))
+    assert np.array_equal(got[:73], want[:73]) and np.isnan(got[73:]).all()
+
+
 @pytest.mark.parametrize("compute", [F32, BF16])
 @pytest.mark.parametrize("experts,top,ff,width", [(5, 2, 24, 40), (70, 6, 17, 33), (3, 3, 100, 130), (1, 1, 64, 64), (9, 1, 40, 70),
                                                    (256, 1, 20, 64), (257, 2, 136, 48)])      # many experts: tiles of 256 weight rows
