@@ -244,6 +244,7 @@ struct lv_session {
     uint32_t wait_limit = 0;              // polls per hand-over of the persistent kernel; 0 = default
     bool xcd_handover = true;             // the persistent kernel may keep a head's hand-overs inside its XCD (lv_session_set_xcd_handover)
     bool logits_on_host = false;          // the last step left its logits in logits_host as well
+    bool logits_were_read = false;        // lv_logits_read has read the last step's logits: the persistent kernel sends the next step's along
     bool pick_in_status = false;          // the last step ran the persistent kernel, whose greedy pick is in status_host
     bool mega_step = false;               // the step in flight ran the persistent kernel
     int mega_failures = 0;                // steps of the persistent kernel in a row that ended with an expired wait
@@ -1829,7 +1830,7 @@ static int mega_turn_end(lv_session *s)
 // either; the waits inside the kernel are bounded for that), the two launch at the same rate (measured in alternation), and
 // the separate queue the runtime opens for cooperative launches makes a process under rocprofv3 end with a segmentation
 // fault in its exit handlers (a forty-line program with one cooperative launch of an empty kernel does the same).
-static int launch_mega(lv_session *s, uint32_t pos, uint32_t token, bool *refused, float *logits_dst)
+static int launch_mega(lv_session *s, uint32_t pos, uint32_t token, bool *refused, float *logits_dst, float *logits_host)
 {
     const lv_model *m = s->model;
     MegaArgs a{};
@@ -1843,6 +1844,7 @@ static int launch_mega(lv_session *s, uint32_t pos, uint32_t token, bool *refuse
     a.xl = s->xl[s->xchg_turn & 1];
     a.xl_rearm = s->xl[(s->xchg_turn + 1) & 1];
     a.logits = logits_dst;
+    a.logits_host = logits_host;
     a.status = s->status_host;
     a.layers = m->hp.layers; a.vocab = m->hp.vocab; a.backlog = s->backlog; a.pos = pos; a.token = token;
     a.spin_limit = s->wait_limit ? s->wait_limit : kSpinLimit;
@@ -2798,6 +2800,9 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     s->have_logits = false;
     s->pick_in_status = false;
     s->logits_on_host = false;
+    // Whoever has read the last step's logits reads this one's: the persistent kernel then sends them to the host itself
+    const bool send_logits = s->logits_were_read && !s->all_logits;
+    s->logits_were_read = false;
     s->logits_rows = 0;
     if (s->all_logits) {
         if (n > s->logits_cap) {
@@ -2836,7 +2841,9 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
         uint32_t done = 0;
         bool refused = false;
         while (done < n) {
-            LV_TRY(launch_mega(s, pos + done, tokens[done], &refused, s->all_logits ? s->logits_all + (size_t)done * V : s->logits));
+            const bool send = send_logits && done + 1 == n;
+            LV_TRY(launch_mega(s, pos + done, tokens[done], &refused, s->all_logits ? s->logits_all + (size_t)done * V : s->logits, send ? s->logits_host : nullptr));
+            if (!refused) s->logits_on_host = send;
             if (refused) break;
             done++;
             s->mega_step = true;
@@ -2951,6 +2958,7 @@ extern "C" int lv_logits_read(lv_session *s, float *dst)
     if (!s || !dst) return fail(LV_ERR_ARG, "lv_logits_read: null argument");
     if (!s->have_logits) return fail(LV_ERR_STATE, "lv_logits_read: no step has produced logits");
     const uint32_t V = s->model->hp.vocab;
+    s->logits_were_read = true;
     if (!s->logits_on_host) {
         logits_out_kernel<<<dim3((V + 1023) / 1024), dim3(256), 0, s->stream>>>(s->logits_host, s->logits, V);
         HIP_TRY(hipGetLastError());

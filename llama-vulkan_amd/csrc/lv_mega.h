@@ -196,6 +196,8 @@ struct MegaArgs {
     float *xchg_rearm;         // the other set, re-armed to kNotReady during this token
     float *xl, *xl_rearm;      // the same for what stays inside an XCD: [layers] x LOCAL_LAYER floats of ordinary memory (ld_xcd)
     float *logits;             // [vocab]
+    float *logits_host;        // null, or pinned memory that gets them too, in runs of 256 bytes while the pick is made: a launch of its own
+                               // that copies them took 5 to 6 us of a step (7B q4_0 977 and 971 us, 13B q4_0, 8 layers, 374 and 369)
     uint32_t *status;          // host-visible; [0] set non-zero when a poll loop expired, [kStatusToken] = greedy pick
     uint32_t layers, vocab, backlog, pos, token;
     uint32_t spin_limit;       // polls per hand-over before the step is given up (kSpinLimit; tests of the failure path lower it)
@@ -958,6 +960,7 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
             if (n < a.vocab) {
                 const float v = red_row<S::NSD>(red, j) * inv_h;
                 a.logits[n] = v;
+                if (a.logits_host) a.logits_host[n] = v;
                 if (better(v, n, bv, bi)) { bv = v; bi = n; }
             }
         }

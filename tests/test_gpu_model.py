@@ -503,3 +503,24 @@ def test_logits_of_every_row_on_the_persistent_kernel(lva, orc, ctx, wide_model)
     _rows_match(s.logits_rows(0, 1), want)
     _rows_match(s.logits()[None, :], want)
     s.close(); model.close(); osess.close(); om.close()
+
+
+def test_logits_of_persistent_steps_read_or_not(lva, ctx, wide_model):
+    """a step behind one whose logits were read sends its own to the host itself: the same values whatever was read before, from
+    lv_logits_read, from all rows' logits and as the greedy pick"""
+    model = lva.Model(ctx, wide_model)
+    a, b = lva.Session(model, 128), lva.Session(model, 128)
+    a.set_path(lva.PATH_PERSISTENT)
+    b.set_path(lva.PATH_PERSISTENT)
+    toks = lva.synth_tokens(14, 3, 2048, seed=9)
+    pos = 0
+    for i, n in enumerate((1, 1, 1, 1, 2, 1, 1, 3, 1, 1, 1)):
+        b.keep_all_logits(True)
+        b.begin(toks[pos:pos + n], pos)
+        want = b.logits_rows(n - 1, 1)[0]
+        a.begin(toks[pos:pos + n], pos)
+        if i % 4 != 2:                                  # behind step 2, 6 and 10 the next one is not told
+            assert np.array_equal(a.logits(), want) and np.array_equal(a.logits(), want)
+        assert a.argmax() == int(np.argmax(want))
+        pos += n
+    a.close(); b.close(); model.close()
