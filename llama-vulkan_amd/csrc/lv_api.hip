@@ -2593,7 +2593,10 @@ static int launch_short_norm(hipStream_t st, const ShortBuffers &b, const float 
 static int launch_short_attention(hipStream_t st, const lv_session *s, const ShortBuffers &b, uint32_t layer, uint32_t pos, uint32_t n, uint32_t ftype)
 {
     const lv_hparams &hp = s->model->hp;
-    const uint32_t tiles = (pos + n + kAttnBatchK - 1) / kAttnBatchK, want = hp.heads < 512 ? 512 / hp.heads : 1;
+    // At most a workgroup a CU: what each does before and behind its tiles (queries to operands, sums through LDS and out) is more than a
+    // tile, and two on a CU are in each other's way.  us with the kernel that puts the parts together, two a CU and one: 45 tokens behind 619
+    // 27.0 and 22.1, behind 1950 32.4 and 29.9; 8 tokens behind 619 15.6 and 13.3, behind 1100 20.7 and 15.8.
+    const uint32_t tiles = (pos + n + kAttnBatchK - 1) / kAttnBatchK, want = hp.heads < 256 ? 256 / hp.heads : 1;
     const uint32_t most = want < kShortSplits ? want : kShortSplits, per = (tiles + most - 1) / most, splits = (tiles + per - 1) / per;
     ShortAttnArgs a{};
     a.kcache = kv_ptr(s, layer, 0); a.vcache = kv_ptr(s, layer, 1); a.q = b.q; a.trig_abs = s->trig_abs;
