@@ -88,7 +88,7 @@ __device__ __forceinline__ void short_conv8(float (&out)[8], const Spec &s, cons
     for (uint32_t i = 0; i < 8; i++) {
         float v = fmaf(in[i + 3], w[0], b);
 #pragma unroll
-        for (uint32_t j = 1; j < 4; j++) v = fmaf(in[i + 3 - j], w[j], v);
+        for (uint32_t j = 1; j < 4; j++) v = j < s.taps ? fmaf(in[i + 3 - j], w[j], v) : v;     // what lies further back counts nothing, finite or not
         out[i] = t0 + i < n ? silu_f(v) : 0.f;
     }
 }
