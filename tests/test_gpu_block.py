@@ -140,6 +140,23 @@ def test_mixture_alone(lva, ctx, experts, top, ff, width, compute):
             assert rel(d.run(toks, c), want) < TOL[compute], c
 
 
+def test_mixture_of_many_choices_and_experts(lva, ctx):
+    """more choices than the sorting workgroup holds at a time, more experts than it has threads"""
+    cfg = bb.config(vocab=300, width=32, layers=[bb.layer(experts=1100, top=9, ff=16)])
+    W = bb.weights(cfg, seed=77)
+    for n in ("left", "right"):
+        W[f"l0.mix.{n}.o"][:] = 0            # the mixer adds nothing: a token's result is its own
+    F = bb.as_float(W)
+    h = bo.rms_norm(F["embed"], F["l0.norm2"], cfg["norm"]["eps"])
+    z = np.sort(h @ F["l0.mlp.router"].T, axis=1)
+    clear = np.flatnonzero(z[:, -9] - z[:, -10] > 1e-3).astype(np.uint32)        # of 32-bit sums
+    assert len(clear) > 100
+    want = bo.forward(clear, F, cfg)[0]
+    at = np.random.default_rng(1).integers(0, len(clear), 2048)
+    with Device(lva, ctx, cfg, W, F32, 2048) as d:
+        assert rel(d.run(clear[at], (2048,)), want[at]) < TOL[F32]
+
+
 # ---- whole models --------------------------------------------------------------------------------------------------------
 def deep(vocab=67, width=52):
     return bb.config(vocab=vocab, width=width, layers=[
