@@ -283,8 +283,17 @@ __global__ __launch_bounds__(256) void append_kernel(PrepareArgs a, uint32_t n)
         }
     }
     if (a.delta.heads && blockIdx.x < a.delta.taps) {
+        // the only workgroups with more than a few loads a thread: eight at a time (8192 channels, the launch: 19.0 us one by one, 8.9 so)
         const uint32_t C = a.delta.channels();
-        for (uint32_t c = threadIdx.x; c < C; c += 256) a.delta.ring[(size_t)(pos % a.delta.taps) * C + c] = a.y[(size_t)t * a.ldy + a.delta.channel_at(c)];
+        float *const ring = a.delta.ring + (size_t)(pos % a.delta.taps) * C;
+        for (uint32_t base = threadIdx.x; base < C; base += 8 * 256) {
+            float v[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) v[i] = a.y[(size_t)t * a.ldy + a.delta.channel_at(min(base + i * 256, C - 1))];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++)
+                if (base + i * 256 < C) ring[base + i * 256] = v[i];
+        }
     }
 }
 
