@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepareArgs a, uint32_t n)
         const uint32_t c = (col - groups) * 256 + threadIdx.x;
         if (c >= nv) return;
         float v[8];
-        short_conv8(v, s, a.y, a.ldy, 2 * nq + c, a.pos0, first, n);
+        short_conv8<true>(v, s, a.y, a.ldy, 2 * nq + c, a.pos0, first, n);
 #pragma unroll
         for (uint32_t i = 0; i < 8; i++)
             if (i < count) a.dv[(size_t)(first + i) * nv + c] = v[i];
@@ -237,8 +237,8 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepareArgs a, uint32_t n)
 #pragma unroll
         for (int i = 0; i < 8; i++) q[j][i] = k[j][i] = 0.f;
         if (d < s.dim) {
-            short_conv8(q[j], s, a.y, a.ldy, h * s.dim + d, a.pos0, first, n);
-            short_conv8(k[j], s, a.y, a.ldy, nq + h * s.dim + d, a.pos0, first, n);
+            short_conv8<true>(q[j], s, a.y, a.ldy, h * s.dim + d, a.pos0, first, n);
+            short_conv8<true>(k[j], s, a.y, a.ldy, nq + h * s.dim + d, a.pos0, first, n);
         }
     }
 #pragma unroll

@@ -55,8 +55,9 @@ __device__ __forceinline__ float short_conv(const Spec &s, const float *y, size_
 }
 
 // Eight consecutive tokens t0 .. t0 + 7 (t0 a multiple of 8) of a batch of n, whose first row is y and first position pos0; 0 for
-// tokens past the end.  Up to four taps every input is read once.
-template <class Spec>
+// tokens past the end.  Up to four taps every input is read once.  EXACT: fewer than four taps leave out what lies further back instead of
+// multiplying it by zero, which a value that is not finite survives.
+template <bool EXACT, class Spec>
 __device__ __forceinline__ void short_conv8(float (&out)[8], const Spec &s, const float *y, size_t ld, uint32_t c, uint32_t pos0, uint32_t t0, uint32_t n)
 {
     if (s.taps > 4) {
@@ -88,7 +89,7 @@ __device__ __forceinline__ void short_conv8(float (&out)[8], const Spec &s, cons
     for (uint32_t i = 0; i < 8; i++) {
         float v = fmaf(in[i + 3], w[0], b);
 #pragma unroll
-        for (uint32_t j = 1; j < 4; j++) v = j < s.taps ? fmaf(in[i + 3 - j], w[j], v) : v;     // what lies further back counts nothing, finite or not
+        for (uint32_t j = 1; j < 4; j++) v = !EXACT || j < s.taps ? fmaf(in[i + 3 - j], w[j], v) : v;
         out[i] = t0 + i < n ? silu_f(v) : 0.f;
     }
 }

@@ -127,7 +127,7 @@ static __global__ __launch_bounds__(256) void ssm_prepare_kernel(SsmBatchArgs a)
             channel = inner + (which * s.groups + g) * s.n + d;
         }
         float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (!pad) short_conv8(v, s, a.y, a.ldy, channel, a.pos0, first, a.n);
+        if (!pad) short_conv8<false>(v, s, a.y, a.ldy, channel, a.pos0, first, a.n);
 #pragma unroll
         for (uint32_t i = 0; i < kSsmPrepareTokens; i++)
             if (first + i < last) out[(first + i) * ld] = v[i];
@@ -277,7 +277,7 @@ static __global__ __launch_bounds__(256) void ssm_operands_kernel(SsmChunkArgs a
         place = e - d + ssm_place(d);
     }
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (!pad) short_conv8(v, s, a.y, a.ldy, channel, a.pos0, t0, a.n);
+    if (!pad) short_conv8<false>(v, s, a.y, a.ldy, channel, a.pos0, t0, a.n);
     uint16_t h[8];
 #pragma unroll
     for (uint32_t i = 0; i < 8; i++) h[i] = float_to_bf16(v[i]);
