@@ -48,6 +48,15 @@ extern "C" const char *lv_last_error(void) { return g_err; }
 // -----------------------------------------------------------------------------------------------------------
 // objects
 // -----------------------------------------------------------------------------------------------------------
+// Launches of small models under way at once; a process has four hardware queues, more would not overlap.  us a token, each launch behind the
+// others' and so: width 768, 12 layers, 3 sessions 385 and 133, 8 sessions 384 and 147; width 256, 2 layers, 8 sessions 50 and 18.
+constexpr uint32_t kSmallTurns = 4;
+struct SmallTurn {
+    hipEvent_t done = nullptr;
+    const void *session = nullptr;
+    uint64_t clock = 0;                   // of the launch that took it
+};
+
 struct lv_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -75,6 +84,10 @@ struct lv_ctx {
     std::mutex mega_mutex;
     hipEvent_t mega_done = nullptr;
     const void *mega_last = nullptr;      // session whose launch mega_done belongs to
+    // Launches of small models (lv_small.h) wait inside as well, but a few of them fit the device beside one another: as many as there are
+    // turns are under way at once, each turn being the last launch of a session.  Also under mega_mutex.
+    SmallTurn small_turn[kSmallTurns];
+    uint64_t small_clock = 0;
     int mega_fits[8] = {-1, -1, -1, -1, -1, -1, -1, -1};   // per shape class of the persistent kernel: can all its workgroups be resident at once (-1 = not asked yet)
 };
 
@@ -330,6 +343,8 @@ extern "C" int lv_ctx_destroy(lv_ctx *c)
     if (c->ev_start) (void)hipEventDestroy(c->ev_start);
     if (c->ev_stop) (void)hipEventDestroy(c->ev_stop);
     if (c->mega_done) (void)hipEventDestroy(c->mega_done);
+    for (SmallTurn &t : c->small_turn)
+        if (t.done) (void)hipEventDestroy(t.done);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return LV_OK;
@@ -1575,6 +1590,8 @@ extern "C" int lv_session_destroy(lv_session *s)
     {
         std::lock_guard<std::mutex> lock(s->model->ctx->mega_mutex);
         if (s->model->ctx->mega_last == s) s->model->ctx->mega_last = nullptr;   // its last launch has finished (stream synchronised)
+        for (SmallTurn &t : s->model->ctx->small_turn)
+            if (t.session == s) { t.session = nullptr; t.clock = 0; }
     }
     drop_graph(s);
     block_session_destroy(s->block);
@@ -1806,11 +1823,14 @@ extern "C" int lv_session_path(const lv_session *s, int *path)
     return LV_OK;
 }
 
-// Launches whose workgroups wait for each other (mega_mutex is held): behind the last one of another session
+// Launches whose workgroups wait for each other (mega_mutex is held).  The persistent kernel occupies every CU: it runs behind the last
+// launch of every other session.
 static int mega_turn_begin(lv_session *s)
 {
     lv_ctx *c = s->model->ctx;
     if (c->mega_last && c->mega_last != s) HIP_TRY(hipStreamWaitEvent(s->stream, c->mega_done, 0));
+    for (const SmallTurn &t : c->small_turn)
+        if (t.session) HIP_TRY(hipStreamWaitEvent(s->stream, t.done, 0));
     return LV_OK;
 }
 static int mega_turn_end(lv_session *s)
@@ -1819,6 +1839,32 @@ static int mega_turn_end(lv_session *s)
     if (!c->mega_done) HIP_TRY(hipEventCreateWithFlags(&c->mega_done, hipEventDisableTiming));
     HIP_TRY(hipEventRecord(c->mega_done, s->stream));
     c->mega_last = s;
+    return LV_OK;
+}
+
+// A small model's launch runs behind the persistent kernel's last one and, where its session holds no turn, behind the launch whose turn is
+// the oldest: at most kSmallTurns at once, each of at most kSmallMaxWGs workgroups, which one per CU find room however they are spread.
+static int small_turn_begin(lv_session *s, SmallTurn **turn)
+{
+    lv_ctx *c = s->model->ctx;
+    if (c->mega_last) HIP_TRY(hipStreamWaitEvent(s->stream, c->mega_done, 0));
+    const uint32_t turns = std::min(kSmallTurns, (uint32_t)c->props.multiProcessorCount / kSmallMaxWGs);
+    SmallTurn *t = c->small_turn;
+    for (uint32_t i = 0; i < turns; i++) {
+        SmallTurn &o = c->small_turn[i];
+        if (o.session == s) { t = &o; break; }
+        if (o.clock < t->clock) t = &o;      // 0: nobody's
+    }
+    if (t->session && t->session != s) HIP_TRY(hipStreamWaitEvent(s->stream, t->done, 0));
+    *turn = t;
+    return LV_OK;
+}
+static int small_turn_end(lv_session *s, SmallTurn *t)
+{
+    if (!t->done) HIP_TRY(hipEventCreateWithFlags(&t->done, hipEventDisableTiming));
+    HIP_TRY(hipEventRecord(t->done, s->stream));
+    t->session = s;
+    t->clock = ++s->model->ctx->small_clock;
     return LV_OK;
 }
 
@@ -1892,7 +1938,7 @@ static void launch_small_kernel(const SmallArgs &a, uint32_t wgs, uint32_t rot, 
     else small_decode_kernel<QT, SF32, 128><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
 }
 
-// One token of a small model.  Its few workgroups wait for each other as the persistent kernel's do and take turns with those.
+// One token of a small model.  Its few workgroups wait for each other as the persistent kernel's do (turns: small_turn_begin).
 static int launch_small(lv_session *s, uint32_t pos, uint32_t token)
 {
     const lv_model *m = s->model;
@@ -1914,13 +1960,14 @@ static int launch_small(lv_session *s, uint32_t pos, uint32_t token)
     a.D = m->hp.dim; a.F = m->hp.ff; a.heads = m->hp.heads;
     a.spin_limit = s->wait_limit ? s->wait_limit : kSpinLimit;
     std::lock_guard<std::mutex> lock(m->ctx->mega_mutex);
-    LV_TRY(mega_turn_begin(s));
+    SmallTurn *turn = nullptr;
+    LV_TRY(small_turn_begin(s, &turn));
     const auto launch = m->output.ftype == LV_Q4_0 ? m->output.view.scales_f32 ? launch_small_kernel<4, true> : launch_small_kernel<4, false>
                                                    : m->output.view.scales_f32 ? launch_small_kernel<8, true> : launch_small_kernel<8, false>;
     launch(a, m->small_wgs, m->hp.rot, s->stream);
     HIP_TRY(hipGetLastError());
     s->xchg_turn++;
-    return mega_turn_end(s);
+    return small_turn_end(s, turn);
 }
 
 // -----------------------------------------------------------------------------------------------------------

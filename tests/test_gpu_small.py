@@ -1,5 +1,7 @@
 """One token of a small model as one launch (lv_small.h) against the oracle and the operator chain: rows that fill tiles and rows that do not,
 one and several blocks a lane, every head size, contexts on both sides of what the workgroup holds of the cache at once."""
+import time
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,68 @@ def test_small_model_not_a_number_is_a_result_and_no_expired_wait(lva, ctx, tmp_
         s.begin([5 + i], i)
         assert np.isnan(s.logits()).all()
     s.close(); model.close()
+
+
+def test_small_models_sessions_run_beside_one_another(lva, ctx, tmp_path):
+    """A launch takes a quarter of the CUs at most: four sessions' tokens take at most twice what one session's does where two of them
+    share a hardware queue, four times it where each waits for the others' launches.  More sessions than that, each with its own tokens, get what each gets alone."""
+    p, c = str(tmp_path / "m.ggml"), dict(vocab=1000, dim=768, heads=12, layers=8, ff=2048)
+    lva.write_model(p, wtype=lva.LV_Q4_0, seed=8, **c)
+    model = lva.Model(ctx, p)
+    toks = [lva.synth_tokens(24, 3, c["vocab"], seed=i) for i in range(7)]
+    alone, s = [], lva.Session(model, 64)
+    for t in toks:
+        for i in range(24):
+            s.begin(t[i:i + 1], i)
+            s.wait()
+        alone.append(s.logits())
+    s.close()
+    several = [lva.Session(model, 64) for _ in toks]
+    for i in range(24):
+        for s, t in zip(several, toks):
+            s.begin(t[i:i + 1], i)
+        for s in several:
+            s.wait()
+    for s, want in zip(several, alone):
+        assert np.array_equal(s.logits(), want)
+
+    def fastest(sessions):
+        times = []
+        for _ in range(30):
+            start = time.perf_counter()
+            for s in sessions:
+                s.begin(toks[0][:1], 24)
+            for s in sessions:
+                s.wait()
+            times.append(time.perf_counter() - start)
+        return min(times)
+    assert fastest(several[:4]) < 3 * fastest(several[:1])
+    for s in several:
+        s.close()
+    model.close()
+
+
+def test_small_and_persistent_launches_of_one_context(lva, ctx, tmp_path):
+    """the persistent kernel occupies every CU and runs behind all small launches, and these behind it"""
+    small, large = dict(vocab=512, dim=256, heads=4, layers=2, ff=704), dict(vocab=512, dim=4096, heads=32, layers=2, ff=11008)
+    models = []
+    for i, c in enumerate((small, large)):
+        lva.write_model(str(tmp_path / f"{i}.ggml"), wtype=lva.LV_Q4_0, seed=9, **c)
+        models.append(lva.Model(ctx, str(tmp_path / f"{i}.ggml")))
+    toks = lva.synth_tokens(40, 3, 512, seed=4)
+
+    def decode(sessions):
+        for i in range(len(toks)):
+            for s in sessions:
+                s.begin(toks[i:i + 1], i)
+            out = [s.logits() for s in sessions]
+        return out
+    sessions = [lva.Session(models[k], 64) for k in (0, 1, 0, 0, 1, 0, 0, 0)]
+    assert sessions[1].path() == lva.PATH_PERSISTENT
+    want = [decode(sessions[k:k + 1])[0] for k in (0, 1)]
+    for s, got in zip(sessions, decode(sessions)):
+        assert np.array_equal(got, want[0 if s.model is models[0] else 1])
+    for s in sessions:
+        s.close()
+    for m in models:
+        m.close()
