@@ -221,7 +221,8 @@ int lv_session_path(const lv_session *s, int *path);
  * that runs out makes the kernel finish anyway and lv_step_wait return LV_ERR_HIP (the reference's waitForFences
  * timeout, llava_command_buffer.cpp:25-27, is the nearest counterpart).  polls = 0 restores the default bound; tests of
  * that failure path set 1.  The step can simply be issued again afterwards; after two such steps in a row it runs in
- * the graph path (see lv_session_set_path). */
+ * the graph path (see lv_session_set_path).  The bound also holds for the one launch a token of small models, whose step is
+ * then evaluated anew on the operator chain by the call that waits for it, and succeeds. */
 int lv_session_set_wait_limit(lv_session *s, uint32_t polls);
 /* The persistent kernel hands a head's query, key and value rows and its partial sums over inside one XCD (through that
  * XCD's L2 instead of memory) whenever a launch has placed the workgroups that share heads on one XCD; it looks at every

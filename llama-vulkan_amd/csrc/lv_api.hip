@@ -259,9 +259,10 @@ struct lv_session {
     bool logits_on_host = false;          // the last step left its logits in logits_host as well
     bool logits_were_read = false;        // lv_logits_read has read the last step's logits: the persistent kernel sends the next step's along
     bool pick_in_status = false;          // the last step ran the persistent kernel, whose greedy pick is in status_host
-    bool mega_step = false;               // the step in flight ran the persistent kernel
-    int mega_failures = 0;                // steps of the persistent kernel in a row that ended with an expired wait
-    bool mega_off = false;                // the persistent kernel is no longer used by this session (refused launch, or two such steps)
+    bool mega_step = false;               // the step in flight ran the persistent kernel, or that of a small model
+    uint32_t small_n = 0;                 // tokens of the step in flight where it ran the latter; they are in cfg_host
+    int mega_failures = 0;                // steps of these kernels in a row that ended with an expired wait
+    bool mega_off = false;                // neither is any longer used by this session (refused launch, or two such steps)
     bool in_flight = false;
     bool have_logits = false;
     // logits of EVERY row of a step (the reference's output_probs holds batch x vocab, llava_session.cpp:49-79), kept on request
@@ -2887,6 +2888,7 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     const bool few = n >= few_min && n <= kShortTokens && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && ensure_short_copy(s->model) && short_reserve(s);
     bool persistent = n < kPrefillMin && path == LV_PATH_PERSISTENT && !s->trace && !few;
     s->mega_step = false;
+    s->small_n = 0;
     if (persistent) {
         uint32_t done = 0;
         bool refused = false;
@@ -2925,7 +2927,7 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     const bool small = n < kPrefillMin && !few && s->model->small_wgs && s->path == LV_PATH_AUTO && path == LV_PATH_GRAPH && !s->trace && !s->mega_off &&
                        (pos + n) * s->model->hp.rot <= kSmallRowElements;
     const bool batch = !persistent && !few && n >= batch_min && (!s->trace || s->block) && ((mid && n == rest) || ensure_prompt_copy(s->model));
-    if (!persistent && !small) {
+    if (!persistent) {
         s->cfg_host[0] = pos;
         memcpy(s->cfg_host + 1, tokens, (size_t)n * 4);
         if (batch) HIP_TRY(hipMemcpyAsync(s->cfg, s->cfg_host, (size_t)(1 + n) * 4, hipMemcpyHostToDevice, s->stream));
@@ -2938,6 +2940,7 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
         for (uint32_t i = 0; i < n; i++) {
             LV_TRY(launch_small(s, pos + i, tokens[i]));
             s->mega_step = true;
+            s->small_n = i + 1;
             s->in_flight = true;
             if (s->all_logits) HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)i * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
         }
@@ -2981,25 +2984,61 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     return LV_OK;
 }
 
-extern "C" int lv_step_wait(lv_session *s)
+// The step in flight again, token by token on the operator chain, which waits for nothing.  A small model's step comes here when its
+// workgroups were not all resident for as long as their waits last (a device that is shared): such a step cannot fail elsewhere.
+static int small_step_again(lv_session *s, uint32_t n)
 {
-    if (!s) return fail(LV_ERR_ARG, "lv_step_wait: session is null");
+    const bool trace = s->trace;
+    const size_t V = s->model->hp.vocab;
+    int rc = LV_OK;
+    s->trace = false;
+    s->in_flight = true;
+    s->logits_on_host = false;
+    for (uint32_t i = 0; i < n && rc == LV_OK; i++) {
+        rc = embed_token(s, s->cfg_host[0], i, s->cfg_host[1 + i]);
+        if (rc == LV_OK) rc = record_token(s, i, s->all_logits || i + 1 == n);
+        if (rc == LV_OK && s->all_logits && hipMemcpyAsync(s->logits_all + i * V, s->logits, V * 4, hipMemcpyDeviceToDevice, s->stream) != hipSuccess)
+            rc = fail(LV_ERR_HIP, "logits of row %u: %s", i, hipGetErrorString(hipGetLastError()));
+    }
+    s->trace = trace;
+    return rc;
+}
+
+// *again: the step is on its way once more; what followed it on the stream has to follow again
+static int step_wait(lv_session *s, bool *again)
+{
+    *again = false;
     const hipError_t done = hipStreamSynchronize(s->stream);
     if (done != hipSuccess && s->block) block_session_invalidate(s->block);
     HIP_TRY(done);
     s->in_flight = false;
     const bool mega_step = s->mega_step;
+    const uint32_t small_n = s->small_n;
     s->mega_step = false;
+    s->small_n = 0;
     if (s->status_host && *s->status_host) {
         *s->status_host = 0;
-        if (++s->mega_failures >= 2) {
-            s->mega_off = true;
+        const bool off = ++s->mega_failures >= 2;
+        if (off) s->mega_off = true;
+        if (small_n) {
+            *again = true;
+            return small_step_again(s, small_n);
+        }
+        if (off)
             return fail(LV_ERR_HIP, "persistent decode kernel: a hand-over wait expired in two steps in a row; this session now takes the %s path",
                         s->use_graph ? "graph" : "operator");
-        }
         return fail(LV_ERR_HIP, "persistent decode kernel: a hand-over wait expired (workgroups not co-resident?)");
     }
     if (mega_step) s->mega_failures = 0;
+    return LV_OK;
+}
+
+extern "C" int lv_step_wait(lv_session *s)
+{
+    if (!s) return fail(LV_ERR_ARG, "lv_step_wait: session is null");
+    bool again;
+    do LV_TRY(step_wait(s, &again));
+    while (again);
     return LV_OK;
 }
 
@@ -3009,11 +3048,14 @@ extern "C" int lv_logits_read(lv_session *s, float *dst)
     if (!s->have_logits) return fail(LV_ERR_STATE, "lv_logits_read: no step has produced logits");
     const uint32_t V = s->model->hp.vocab;
     s->logits_were_read = true;
-    if (!s->logits_on_host) {
-        logits_out_kernel<<<dim3((V + 1023) / 1024), dim3(256), 0, s->stream>>>(s->logits_host, s->logits, V);
-        HIP_TRY(hipGetLastError());
-    }
-    LV_TRY(lv_step_wait(s));
+    bool again;
+    do {
+        if (!s->logits_on_host) {
+            logits_out_kernel<<<dim3((V + 1023) / 1024), dim3(256), 0, s->stream>>>(s->logits_host, s->logits, V);
+            HIP_TRY(hipGetLastError());
+        }
+        LV_TRY(step_wait(s, &again));
+    } while (again);
     memcpy(dst, s->logits_host, (size_t)V * 4);
     return LV_OK;
 }
@@ -3033,11 +3075,13 @@ extern "C" int lv_logits_read_rows(lv_session *s, uint32_t row0, uint32_t n_rows
     if (!s->have_logits || s->logits_rows == 0) return fail(LV_ERR_STATE, "lv_logits_read_rows: no step has kept the logits of all its rows (lv_session_set_all_logits)");
     if (row0 > s->logits_rows || n_rows > s->logits_rows - row0)
         return fail(LV_ERR_RANGE, "lv_logits_read_rows: rows %u..%u of a step of %u", row0, row0 + n_rows, s->logits_rows);
-    if (n_rows) {
-        const size_t V = s->model->hp.vocab;
-        HIP_TRY(hipMemcpyAsync(dst, s->logits_all + (size_t)row0 * V, (size_t)n_rows * V * 4, hipMemcpyDeviceToHost, s->stream));
-    }
-    return lv_step_wait(s);
+    const size_t V = s->model->hp.vocab;
+    bool again;
+    do {
+        if (n_rows) HIP_TRY(hipMemcpyAsync(dst, s->logits_all + (size_t)row0 * V, (size_t)n_rows * V * 4, hipMemcpyDeviceToHost, s->stream));
+        LV_TRY(step_wait(s, &again));
+    } while (again);
+    return LV_OK;
 }
 
 extern "C" int lv_argmax(lv_session *s, uint32_t *token)
@@ -3049,9 +3093,12 @@ extern "C" int lv_argmax(lv_session *s, uint32_t *token)
         *token = s->status_host[kStatusToken];
         return LV_OK;
     }
-    argmax_kernel<<<dim3(1), dim3(1024), 0, s->stream>>>(s->logits, s->model->hp.vocab, s->argmax_host);
-    HIP_TRY(hipGetLastError());
-    LV_TRY(lv_step_wait(s));
+    bool again;
+    do {
+        argmax_kernel<<<dim3(1), dim3(1024), 0, s->stream>>>(s->logits, s->model->hp.vocab, s->argmax_host);
+        HIP_TRY(hipGetLastError());
+        LV_TRY(step_wait(s, &again));
+    } while (again);
     *token = *s->argmax_host;
     return LV_OK;
 }
@@ -3088,6 +3135,7 @@ extern "C" int lv_session_timer_stop(lv_session *s, float *ms)
 {
     if (!s || !ms) return fail(LV_ERR_ARG, "lv_session_timer_stop: null argument");
     LV_TRY(timer_stop(s->ev_start, s->ev_stop, s->stream, ms));
+    if (s->small_n) return lv_step_wait(s);
     s->in_flight = false;
     return LV_OK;
 }

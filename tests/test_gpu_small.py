@@ -151,3 +151,62 @@ def test_small_and_persistent_launches_of_one_context(lva, ctx, tmp_path):
         s.close()
     for m in models:
         m.close()
+
+
+def _same_cache(dst, src, layers, n):
+    for layer in range(layers):
+        for which in (0, 1):
+            dst.kv_write(layer, which, src.kv(layer, which, n))
+
+
+def test_an_expired_wait_of_a_small_model_goes_unnoticed(lva, ctx, tmp_path):
+    """with the poll bound at 1 every launch gives up; the call that waits evaluates the step on the operator chain, bit for bit what a session
+    whose path is the chain gets, for every way of reading a step.  Two such steps in a row leave the session there, one does not"""
+    p, c = str(tmp_path / "m.ggml"), dict(vocab=1000, dim=256, heads=4, layers=3, ff=704)
+    lva.write_model(p, wtype=lva.LV_Q4_0, seed=12, **c)
+    model = lva.Model(ctx, p)
+    one, chain = lva.Session(model, 64), lva.Session(model, 64)
+    chain.set_path(lva.PATH_KERNELS)
+    toks = lva.synth_tokens(40, 3, c["vocab"], seed=6)
+    pos = 0
+
+    def step(n, read, limit):
+        nonlocal pos
+        _same_cache(one, chain, c["layers"], pos)
+        one.set_wait_limit(limit)
+        got = []
+        for s in (one, chain):
+            s.begin(toks[pos:pos + n], pos)
+            got.append(read(s))
+        pos += n
+        return got
+
+    def rows(s):
+        return s.logits_rows(0, 2)
+
+    def after_wait(s):
+        s.wait()
+        return s.logits()
+
+    def timed(s):
+        s.timer_start()
+        s.timer_stop()
+        return s.logits()
+    differ = 0
+    for n, read in ((1, lva.Session.logits), (3, lva.Session.logits), (1, lva.Session.argmax), (2, rows), (1, after_wait), (1, timed)):
+        for s in (one, chain):
+            s.keep_all_logits(read is rows)
+        a, b = step(n, read, 1)                       # given up, evaluated again
+        assert np.array_equal(a, b), read
+        for s in (one, chain):
+            s.keep_all_logits(False)
+        a, b = step(1, lva.Session.logits, 0)         # not given up: the small models' kernel, whose sums round differently
+        differ += not np.array_equal(a, b)
+        _check(a, b)
+    assert differ > 0
+    for limit in (1, 1, 0, 0):                        # two in a row: the chain from then on
+        a, b = step(1, lva.Session.logits, limit)
+        assert np.array_equal(a, b)
+    one.set_path(lva.PATH_AUTO)                       # another try
+    assert any(not np.array_equal(*step(1, lva.Session.logits, 0)) for _ in range(4))
+    one.close(); chain.close(); model.close()
