@@ -26,6 +26,7 @@
 #include "lv_attn_batch.h"
 #include "lv_mid.h"
 #include "lv_small.h"
+#include "lv_copies.h"
 
 using namespace lv;
 
@@ -2104,6 +2105,15 @@ static int record_token(lv_session *s, uint32_t idx, bool with_head)
 }
 
 // ---- batched prompt evaluation -----------------------------------------------------------------------------
+static uint64_t prompt_copy_bytes(const lv_model *m)
+{
+    uint64_t halfs = 0;
+    for (const LayerWeights &lw : m->layers) {
+        for (const lv_matrix *x : {&lw.wq, &lw.wk, &lw.wv, &lw.wo, &lw.w2}) halfs += prompt_copy_halfs(*x);
+        halfs += gemm_pairable(lw.w3, lw.w1) ? pair_copy_halfs(lw.w3) : prompt_copy_halfs(lw.w1) + prompt_copy_halfs(lw.w3);
+    }
+    return halfs * 2;
+}
 // The prompt copy of every layer matrix, made when a model evaluates its first batch (2 bytes a weight: 13.5 GB for a
 // 7B model; decode never reads it).  False when the device has no room for it: batches then go token by token.
 static bool ensure_prompt_copy(lv_model *m)
@@ -2111,14 +2121,8 @@ static bool ensure_prompt_copy(lv_model *m)
     if (m->block) return true;      // one copy of the weights serves both forms of a step
     std::lock_guard<std::mutex> lock(m->prompt_mutex);
     if (m->prompt_state) return m->prompt_state > 0;
-    uint64_t halfs = 0;
-    for (LayerWeights &lw : m->layers) {
-        const bool pair = gemm_pairable(lw.w3, lw.w1);
-        for (lv_matrix *x : {&lw.wq, &lw.wk, &lw.wv, &lw.wo, &lw.w2}) halfs += prompt_copy_halfs(*x);
-        halfs += pair ? pair_copy_halfs(lw.w3) : prompt_copy_halfs(lw.w1) + prompt_copy_halfs(lw.w3);
-    }
     m->prompt_state = -1;
-    if (hipMalloc(reinterpret_cast<void **>(&m->prompt_arena), halfs * 2) != hipSuccess) {
+    if (hipMalloc(reinterpret_cast<void **>(&m->prompt_arena), prompt_copy_bytes(m)) != hipSuccess) {
         (void)hipGetLastError();
         m->prompt_arena = nullptr;
         return false;
@@ -2166,6 +2170,10 @@ constexpr uint32_t kPrefillChunk = 512;    // tokens evaluated together (bounds 
 
 static int prefill_reserve(lv_session *s, uint32_t n)
 {
+    const auto no_workspace = [](hipError_t e) {
+        (void)hipGetLastError();     // a caller that goes another way must not find it behind its next launch
+        return fail(e == hipErrorOutOfMemory ? LV_ERR_OOM : LV_ERR_HIP, "prompt workspace: %s", hipGetErrorString(e));
+    };
     const lv_hparams &hp = s->model->hp;
     const size_t D = hp.dim, F = hp.ff;
     const uint32_t cap = (n + kGemmTile - 1) / kGemmTile * kGemmTile;
@@ -2181,7 +2189,7 @@ static int prefill_reserve(lv_session *s, uint32_t n)
             (void)hipFree(*bufs[i]);
             *bufs[i] = nullptr;
             hipError_t e = hipMalloc(bufs[i], sizes[i] * cap);
-            if (e != hipSuccess) return fail(e == hipErrorOutOfMemory ? LV_ERR_OOM : LV_ERR_HIP, "prompt workspace: %s", hipGetErrorString(e));
+            if (e != hipSuccess) return no_workspace(e);
         }
         s->pf_cap = cap;
     }
@@ -2192,7 +2200,7 @@ static int prefill_reserve(lv_session *s, uint32_t n)
         s->pf_planes = nullptr;
         s->pf_plane_halfs = 0;
         hipError_t e = hipMalloc(reinterpret_cast<void **>(&s->pf_planes), planes * 2);
-        if (e != hipSuccess) return fail(e == hipErrorOutOfMemory ? LV_ERR_OOM : LV_ERR_HIP, "prompt workspace: %s", hipGetErrorString(e));
+        if (e != hipSuccess) return no_workspace(e);
         s->pf_plane_halfs = planes;
     }
     return LV_OK;
@@ -2585,18 +2593,29 @@ static int launch_short_pack(hipStream_t st, uint8_t *dst, const lv_matrix &w, c
 }
 static size_t short_copy_bytes(const lv_matrix &w, uint32_t rows, uint32_t cols) { return rows / 16 * short_tile_bytes(w.ftype == LV_Q4_0 ? 4 : 8, w.view.scales_f32 != nullptr, cols / 32); }
 
+struct ShortSizes { size_t dd, fd, df, vd, total; };      // of a D x D matrix, gate and up, down, output, everything
+static ShortSizes short_sizes(const lv_model *m)
+{
+    const lv_hparams &hp = m->hp;
+    const lv_matrix &like = m->layers[0].wq;
+    ShortSizes z{};
+    z.dd = short_copy_bytes(like, hp.dim, hp.dim);
+    z.fd = short_copy_bytes(like, 2 * hp.ff, hp.dim);
+    z.df = short_copy_bytes(like, hp.dim, hp.ff);
+    // all rows' logits go through the same kernel where the output matrix has the layers' form
+    if (m->output.ftype == like.ftype && !m->output.view.scales_f32 == !like.view.scales_f32 && m->output.view.rows % 16 == 0)
+        z.vd = short_copy_bytes(like, m->output.view.rows, hp.dim);
+    z.total = hp.layers * (4 * z.dd + z.fd + z.df) + z.vd;
+    return z;
+}
+
 static bool ensure_short_copy(lv_model *m)
 {
     std::lock_guard<std::mutex> lock(m->prompt_mutex);
     if (m->short_state) return m->short_state > 0;
     m->short_state = -1;
-    const lv_hparams &hp = m->hp;
-    const lv_matrix &like = m->layers[0].wq;
-    const size_t dd = short_copy_bytes(like, hp.dim, hp.dim), fd = short_copy_bytes(like, 2 * hp.ff, hp.dim), df = short_copy_bytes(like, hp.dim, hp.ff);
-    // all rows' logits go through the same kernel where the output matrix has the layers' form
-    const bool out = m->output.ftype == like.ftype && !m->output.view.scales_f32 == !like.view.scales_f32 && m->output.view.rows % 16 == 0;
-    const size_t vd = out ? short_copy_bytes(like, m->output.view.rows, hp.dim) : 0;
-    if (hipMalloc(reinterpret_cast<void **>(&m->short_arena), hp.layers * (4 * dd + fd + df) + vd) != hipSuccess) {
+    const ShortSizes z = short_sizes(m);
+    if (hipMalloc(reinterpret_cast<void **>(&m->short_arena), z.total) != hipSuccess) {
         (void)hipGetLastError();
         m->short_arena = nullptr;
         return false;
@@ -2608,22 +2627,35 @@ static bool ensure_short_copy(lv_model *m)
         for (const lv_matrix *x : {&lw.wq, &lw.wk, &lw.wv, &lw.wo}) {
             if (x == &lw.wo) lw.short_wo = at;
             if (launch_short_pack(st, at, *x, nullptr) != LV_OK) return false;
-            at += dd;
+            at += z.dd;
         }
         lw.short_gate_up = at;
         if (launch_short_pack(st, at, lw.w3, &lw.w1) != LV_OK) return false;
-        at += fd;
+        at += z.fd;
         lw.short_down = at;
         if (launch_short_pack(st, at, lw.w2, nullptr) != LV_OK) return false;
-        at += df;
+        at += z.df;
     }
-    if (out) {
+    if (z.vd) {
         if (launch_short_pack(st, at, m->output, nullptr) != LV_OK) return false;
         m->short_output = at;
     }
     if (hipStreamSynchronize(st) != hipSuccess) return false;
     m->short_state = 1;
     return true;
+}
+
+// Can the short copy be made without taking the room of a prompt copy that is not there yet, and of a session's workspace?
+static bool short_copy_leaves_room(lv_model *m)
+{
+    std::lock_guard<std::mutex> lock(m->prompt_mutex);
+    if (m->short_state || m->prompt_state) return true;
+    size_t free_bytes = 0, all = 0;
+    if (hipMemGetInfo(&free_bytes, &all) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return free_bytes >= short_sizes(m).total + prompt_copy_bytes(m) + (1ull << 30);
 }
 
 static int launch_short_norm(hipStream_t st, const ShortBuffers &b, const float *w, uint32_t n, uint32_t D, uint32_t pending, uint32_t ftype)
@@ -2920,13 +2952,19 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     }
     // steps of a few tokens take position and token ids as launch arguments, and so does a token at a time
     const uint32_t batch_min = s->block ? kBlockBatchMin : (uint32_t)kPrefillMin, batch_max = s->block ? kBlockBatch : kPrefillChunk;
-    // A step of up to kMidTokens, or what is left of a longer one behind its whole chunks, takes the products of lv_mid.h: by its size alone
-    const uint32_t rest = n <= kPrefillChunk ? n : n % kPrefillChunk;
-    const bool mid = !persistent && !few && n >= kPrefillMin && rest && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && mid_pays(s->model->hp, rest) &&
-                     ensure_short_copy(s->model);
     const bool small = n < kPrefillMin && !few && s->model->small_wgs && s->path == LV_PATH_AUTO && path == LV_PATH_GRAPH && !s->trace && !s->mega_off &&
                        (pos + n) * s->model->hp.rot <= kSmallRowElements;
-    const bool batch = !persistent && !few && n >= batch_min && (!s->trace || s->block) && ((mid && n == rest) || ensure_prompt_copy(s->model));
+    // A step of up to kMidTokens, or what is left of a longer one behind its whole chunks, takes the products of lv_mid.h: by its size alone
+    const uint32_t rest = n <= kPrefillChunk ? n : n % kPrefillChunk;
+    const bool pays = n >= kPrefillMin && rest && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && mid_pays(s->model->hp, rest);
+    bool batch = false, mid = false;
+    if (!persistent && !few && n >= batch_min && (!s->trace || s->block)) {
+        const BatchCopies c = batch_copies(
+            n != rest, pays, [&] { return ensure_prompt_copy(s->model); },
+            [&] { return prefill_reserve(s, std::min(n, kPrefillChunk)) == LV_OK && ensure_short_copy(s->model); }, [&] { return short_copy_leaves_room(s->model); });
+        batch = c.batch;
+        mid = c.mid;
+    }
     if (!persistent) {
         s->cfg_host[0] = pos;
         memcpy(s->cfg_host + 1, tokens, (size_t)n * 4);
