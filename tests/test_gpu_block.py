@@ -87,6 +87,14 @@ def test_delta_rule_alone(lva, ctx, k, compute):
     check_model(lva, ctx, cfg, W, 110, compute, cuts=((1000,), (1,), (37, 2, 16, 31, 3)))
 
 
+@pytest.mark.parametrize("taps", [5, 8, 9, 15, 16, 17, 30])
+def test_delta_rule_behind_long_convolutions(lva, ctx, taps):
+    """taps are read eight at a time: whole and partial groups of them, inputs of the batch, of the ring and before the sequence"""
+    cfg = bb.config(width=44, layers=[bb.layer(right=bb.delta(heads=2, kv_heads=1, dim=70, vdim=20, conv=taps), experts=0, without=("left",))])
+    W = bb.weights(cfg, seed=40 + taps, rank_a=5, rank_g=9)
+    check_model(lva, ctx, cfg, W, 75, F32, cuts=((1000,), (1,), (16, 17, 1, 3, 16, 22)))
+
+
 @pytest.mark.parametrize("k", range(len(DELTA)))
 def test_delta_rule_in_chunks(lva, ctx, k):
     """bfloat16 batches from 224 tokens on go in chunks of 16 tokens, 1024 tokens at a time: full and partial chunks and stretches, going on from
