@@ -104,14 +104,23 @@ struct lv_matrix {
 
 // Uncached device memory (hipDeviceMallocUncached) for the persistent kernel's device-wide hand-over vectors.  Such memory
 // is never given back to the runtime once a kernel has read it (allocations made after such a free have been seen to hold
-// wrong values); a session that ends leaves its buffers here for the next one of the same size.
+// wrong values); a session that ends leaves its buffers here for the next one whose buffers fall in the same class of sizes, a
+// power of two: small models come in any size, and each size would keep blocks of its own for good.
 struct UncachedBlock { int device; size_t bytes; void *ptr; };
 static std::mutex g_uncached_mutex;
 static std::vector<UncachedBlock> g_uncached_free;
 
+static size_t uncached_class(size_t bytes)
+{
+    size_t c = 4096;
+    while (c < bytes) c *= 2;
+    return c;
+}
+
 static int uncached_take(int device, void **out, size_t bytes, bool *pooled)
 {
     *pooled = true;
+    bytes = uncached_class(bytes);
     {
         std::lock_guard<std::mutex> lock(g_uncached_mutex);
         for (size_t i = 0; i < g_uncached_free.size(); i++)
@@ -145,7 +154,7 @@ static void uncached_give(int device, void *ptr, size_t bytes, bool pooled)
         return;
     }
     std::lock_guard<std::mutex> lock(g_uncached_mutex);
-    g_uncached_free.push_back({device, bytes, ptr});
+    g_uncached_free.push_back({device, uncached_class(bytes), ptr});
 }
 
 struct LayerWeights {

@@ -1,5 +1,6 @@
 """One token of a small model as one launch (lv_small.h) against the oracle and the operator chain: rows that fill tiles and rows that do not,
 one and several blocks a lane, every head size, contexts on both sides of what the workgroup holds of the cache at once."""
+import ctypes as C
 import time
 
 import numpy as np
@@ -210,3 +211,24 @@ def test_an_expired_wait_of_a_small_model_goes_unnoticed(lva, ctx, tmp_path):
     one.set_path(lva.PATH_AUTO)                       # another try
     assert any(not np.array_equal(*step(1, lva.Session.logits, 0)) for _ in range(4))
     one.close(); chain.close(); model.close()
+
+
+def test_hand_over_buffers_of_ended_sessions_serve_models_of_other_sizes(lva, ctx, tmp_path):
+    """they are never given back to the runtime: a process that goes through models of many sizes must not keep a pair for each.  17 to 30
+    layers of 33 KB: 22 MB if each keeps its own, none beyond the first pair if they share one"""
+    def free_memory():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert lva.hip().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+    before = None
+    for layers in (30, *range(17, 30)):
+        p = str(tmp_path / f"{layers}.ggml")
+        lva.write_model(p, wtype=lva.LV_Q4_0, seed=3, vocab=259, dim=32, heads=1, layers=layers, ff=8192)
+        model = lva.Model(ctx, p)
+        s = lva.Session(model, 64)
+        s.begin([5], 0)
+        s.wait()
+        s.close(); model.close()
+        if before is None:
+            before = free_memory()
+    assert before - free_memory() < 8 << 20
