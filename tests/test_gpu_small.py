@@ -25,9 +25,12 @@ SHAPES = {
     "two columns a lane": dict(vocab=512, dim=256, heads=4, layers=2, ff=2080),
     "head of 128": dict(vocab=513, dim=256, heads=2, layers=3, ff=704),
     "sixteen heads": dict(vocab=4099, dim=512, heads=16, layers=2, ff=1376),
-    "widest": dict(vocab=1000, dim=1024, heads=8, layers=2, ff=8160),
+    "widest": dict(vocab=1000, dim=1024, heads=16, layers=2, ff=8160),
+    "longest feed-forward": dict(vocab=600, dim=992, heads=31, layers=2, ff=8192),
     "more heads than tiles": dict(vocab=260, dim=1024, heads=32, layers=1, ff=64),
+    "wide heads of 128": dict(vocab=1000, dim=1024, heads=8, layers=2, ff=8160),       # one workgroup a head would take longer: the chain
 }
+CHAIN = {"wide heads of 128"}
 
 
 @pytest.mark.parametrize("shape", sorted(SHAPES))
@@ -45,7 +48,7 @@ def test_small_model_tokens_match_oracle_and_chain(lva, orc, ctx, tmp_path, shap
     assert one.path() == lva.PATH_GRAPH
     chain.set_path(lva.PATH_GRAPH)
     toks = lva.synth_tokens(290, 3, c["vocab"], seed=2)
-    pos = 0
+    pos, differ = 0, 0
     # alone, a step of several tokens, up to and across the borders of 64, 128 and 256 cache rows
     for n in (1, 1, 9, 1, 52, 1, 1, 61, 1, 1, 126, 1, 1, 1):
         step = toks[pos:pos + n]
@@ -55,8 +58,10 @@ def test_small_model_tokens_match_oracle_and_chain(lva, orc, ctx, tmp_path, shap
         _check(one.logits(), want)
         _check(chain.logits(), want)
         assert np.array_equal(one.logits(), other.logits())
+        differ += not np.array_equal(one.logits(), chain.logits())
         assert one.argmax() == int(np.argmax(one.logits()))
         pos += n
+    assert (differ == 0) == (shape in CHAIN)    # which kernels ran: sums in another order round differently
     s = one
     s.keep_all_logits()
     s.begin(toks[:3], 0)
@@ -232,3 +237,31 @@ def test_hand_over_buffers_of_ended_sessions_serve_models_of_other_sizes(lva, ct
         if before is None:
             before = free_memory()
     assert before - free_memory() < 8 << 20
+
+
+@pytest.mark.parametrize("heads,border", [(2, 1024), (4, 2048)])
+def test_a_small_models_session_moves_to_the_chain_behind_a_long_context(lva, ctx, tmp_path, heads, border):
+    """One workgroup walks all cache rows of a head: from 131072 elements of them on the chain is faster.  On either side of that row, and in a
+    step of several tokens that would cross it, with the same cache rows: bit for bit the chain's logits from there on, others before"""
+    p, c = str(tmp_path / "m.ggml"), dict(vocab=700, dim=256, heads=heads, layers=2, ff=704)
+    lva.write_model(p, wtype=lva.LV_Q8_0, seed=15, **c)
+    model = lva.Model(ctx, p)
+    one, chain = lva.Session(model, border + 64), lva.Session(model, border + 64)
+    chain.set_path(lva.PATH_GRAPH)
+    toks = lva.synth_tokens(border + 40, 3, c["vocab"], seed=7)
+    chain.begin(toks[:border - 8], 0)
+    chain.wait()
+    for pos in range(border - 8, border - 2):
+        chain.begin(toks[pos:pos + 1], pos)
+        chain.wait()
+    fresh, differ = True, {True: 0, False: 0}
+    for pos, n in ((border - 2, 1), (border - 1, 1), (border - 1, 3), (border, 1), (border + 1, 1), (border - 2, 2), (border - 2, 3), (border + 1, 5)):
+        _same_cache(one, chain, c["layers"], border - 2 if fresh else pos)
+        fresh = False
+        for s in (one, chain):
+            s.begin(toks[pos:pos + n], pos)
+        a, b = one.logits(), chain.logits()
+        _check(a, b)
+        differ[pos + n <= border] += not np.array_equal(a, b)
+    assert differ[True] > 0 and differ[False] == 0
+    one.close(); chain.close(); model.close()
