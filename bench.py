@@ -90,11 +90,11 @@ def lavapipe_status():
     return "unavailable: " + ", ".join(missing)
 
 
-def other_cases(lva, ctx, headline_picks=None, headline_first=0):
+def other_cases(lva, ctx, headline_picks=None, headline_first=0, headline_prompt=0):
     """The other configurations under the same clock, after the headline's timed region: isolated GEMVs at the 7B decode
     shapes in both weight types, the 512-token GEMM at the 13B layer shapes, 7B q8_0 at positions 1920..2047, 13B q4_0 with a 32-token prompt and 256 steps (on the
     persistent kernel and on the hipGraph of the operator chain, which have to pick the same tokens), the 7B q4_0 headline
-    workload on the hipGraph path (same tokens as the headline run), and the 13B q8_0 512-token prompt.  Each entry carries
+    workload on the hipGraph path (same tokens as the headline run, where that started behind a prompt of the same length), and the 13B q8_0 512-token prompt.  Each entry carries
     tok_s or ms or us, and frac of the roofline that bounds it (HBM for decode and GEMV; matrix cores for the prompt, where
     frac counts the flops the work needs and executed_frac the flops the kernel issues).  A case that fails leaves an
     entry with its error and the others still run."""
@@ -123,8 +123,9 @@ def other_cases(lva, ctx, headline_picks=None, headline_first=0):
              {"force_path": lva.PATH_GRAPH})):
         def decode(name=name, key=key, other=other, args=args, kw=kw):
             expect = picks.get(other)
-            if other == "headline" and headline_picks is not None and headline_first >= args[5]:
-                # the headline's run fed headline_picks[i] at position headline_first + i; this case starts feeding at args[5]
+            if other == "headline" and headline_picks is not None and headline_prompt == args[5]:
+                # the headline's run fed headline_picks[i] at position headline_first + i; this case starts feeding at args[5].  Behind a
+                # prompt of another length the two feed different tokens and pick different ones
                 expect = [None] * (headline_first - args[5]) + list(headline_picks)
             d = measure.decode_case(ctx, *args, report=q, expect_picks=_known(expect), **kw)
             picks[key] = d["picks"]
@@ -318,7 +319,7 @@ def main():
         out["roofline"]["achievable"] = None
         out["roofline"]["achievable_error"] = f"{type(e).__name__}: {e}"
     if not args.no_cases:
-        out["cases"] = other_cases(lva, ctx, headline_picks=tokens, headline_first=timed_first)
+        out["cases"] = other_cases(lva, ctx, headline_picks=tokens, headline_first=timed_first, headline_prompt=first)
     print(json.dumps(out), flush=True)
     ctx.close()
 
