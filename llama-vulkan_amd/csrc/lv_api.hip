@@ -180,10 +180,10 @@ struct lv_model {
     uint8_t *mega_stream = nullptr;
     float *mega_norms = nullptr;    // [layers][2][D] + final norm [D]
     float *tok_f32_own = nullptr;   // fp32 copy of a quantised embedding table (the persistent kernel reads rows as fp32)
-    // prompt copy of the layer matrices (lv_gemm.h), made when the first batch is evaluated; sessions of several threads share it
     // a small model's token as one launch (lv_small.h): its matrices as a table on the device, the workgroups of a launch (0: not such a model)
     SmallLayer *small_layers = nullptr;
     uint32_t small_wgs = 0;
+    // prompt copy of the layer matrices (lv_gemm.h), made when the first batch is evaluated; sessions of several threads share it
     std::mutex prompt_mutex;
     int prompt_state = 0;           // 0 not made yet, 1 ready, -1 could not be made (batches then go token by token)
     uint16_t *prompt_arena = nullptr;
@@ -2489,6 +2489,8 @@ static int launch_mid_tokens(hipStream_t st, const MidArgs &a, uint32_t T, uint3
 //   q, k and v, RT 2/3/4/6      48 tokens 31/22/24/30, 128 73/-/39/53, 256 -/-/81/55
 //   gate and up, RT 2/3/4/6     48 tokens 47/41/45/32, 128 112/-/86/54, 256 -/-/127/105
 //   down, RT 4, slices 2/3/4    48 tokens 32/23/20, 128 53/41/33, 256 52/73/62; RT 2, slices 2: 22, 46, 91; RT 6, slices 4: 24, 42, 76
+// None of the kernel's instances goes unused: up to 64 tokens (T 2 to 4) gate and up of 7B take RT 6, its q, k and v 3, 13B and the outputs
+// 4, width 2048 2 and 3; beyond (T 5 to 8) 7B and 13B take 4 and 6, width 2048 2, 4 and 6.
 static double mid_plan(uint32_t tiles, uint32_t nb, uint32_t T, uint32_t groups, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
 {
     const uint32_t chunks = nb / 4;

@@ -688,8 +688,8 @@ __global__ __launch_bounds__(256, 2) void short_attn_kernel(ShortAttnArgs a)
             va.x /= total; va.y /= total; va.z /= total; va.w /= total;
             vb.x /= total; vb.y /= total; vb.z /= total; vb.w /= total;
             float f[8];
-            if (a.q8) short_order<8>(f, va, vb, false);
-            else short_order<4>(f, va, vb, short_exact(a.tiles));
+            if (a.q8 || !short_exact(a.tiles)) short_order<8>(f, va, vb, false);
+            else short_order<4>(f, va, vb, true);
             short_put(a.act, k / 32, z, g, a.tiles, f);
         }
         return;
