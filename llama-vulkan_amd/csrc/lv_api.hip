@@ -182,7 +182,7 @@ struct lv_model {
     float *tok_f32_own = nullptr;   // fp32 copy of a quantised embedding table (the persistent kernel reads rows as fp32)
     // a small model's token as one launch (lv_small.h): its matrices as a table on the device, the workgroups of a launch (0: not such a model)
     SmallLayer *small_layers = nullptr;
-    uint32_t small_wgs = 0;
+    uint32_t small_wgs = 0, small_elements = 0;      // cache elements of a head up to which it is the faster way
     // prompt copy of the layer matrices (lv_gemm.h), made when the first batch is evaluated; sessions of several threads share it
     std::mutex prompt_mutex;
     int prompt_state = 0;           // 0 not made yet, 1 ready, -1 could not be made (batches then go token by token)
@@ -1370,14 +1370,17 @@ static int build_mega(lv_model *m)
 }
 
 // Which models take lv_small.h's launch for a token: those whose operator chain has ten launches a layer (below the streaming kernels' 2048
-// rows) and whose work a few workgroups do in less time than those launches take to follow one another.  The longest stretch is a
-// head's three projections, which one workgroup does: at most kSmallHeadTiles tiles a wave.  us a token, launch and chain, 100 rows of
-// context: width 256, 3 tiles, 2 layers 53 and 117; 512, 6 tiles, 8 layers 198 and 361; 768, 12 tiles, 12 layers 464 and 568; 1024 with 16
-// heads, 12 tiles, 4 layers 193 and 218, with 8 heads, 24 tiles, 240 and 221.
+// rows) and whose work a few workgroups do in less time than those launches take to follow one another.  A head's three projections are one
+// workgroup's work, at most kSmallHeadTiles tiles a wave were looked at; then both times are estimated, in us behind 100 rows of context:
+//   launch  17 + layers (9.6 + 1.1 tiles a wave of a head's projections + 0.95 tiles a wave of the other products) + 1.26 of the output's
+//   chain   25 + layers (42 + 0.125 MB) + 0.06 MB of the output
+// a fit of 110 shapes of width 64 to 1024, 300 to 128256 rows of output, 7 % off the launch's and 14 % off the chain's measured times at most.
+// Measured, launch and chain: width 256, 2 layers 53 and 117; 512, 8 layers 198 and 361; 768, 12 layers 464 and 568.  A large vocabulary is
+// what a quarter of the chip is too little for: 640 wide, 4 layers, 128256 rows 260 and 240, 1024, 1 layer, 203 and 116.
 constexpr uint32_t kSmallHeadTiles = 12;
-// One workgroup also walks a head's cache rows, 90 ns of a layer for every 1000 elements of them, where the chain splits them over several:
-// width 512, 4 heads of 128, 4 layers 148 and 191 us behind 100 rows, 199 and 205 behind 1000, 257 and 221 behind 2000; width 256, 4 heads
-// of 64, 76 and 118 behind 2000.
+// One workgroup also walks a head's cache rows, where the chain splits them over several: 80 ns more of a layer for every 1000 elements of
+// them, so what the launch gains bounds the context, and so do the rows that were looked at.  Width 512, 4 heads of 128, 4 layers 148 and
+// 191 us behind 100 rows, 199 and 205 behind 1000, 257 and 221 behind 2000; width 256, 4 heads of 64, 76 and 118 behind 2000.
 constexpr uint32_t kSmallRowElements = 131072;
 static int build_small(lv_model *m)
 {
@@ -1391,14 +1394,22 @@ static int build_small(lv_model *m)
             if (x->ftype != ft || (x->view.scales_f32 != nullptr) != (m->output.view.scales_f32 != nullptr)) return LV_OK;
         table.push_back({lw.wq.view, lw.wk.view, lw.wv.view, lw.wo.view, lw.w1.view, lw.w2.view, lw.w3.view, lw.attn_norm, lw.ffn_norm});
     }
-    const auto tiles = [](uint32_t rows, uint32_t cols) -> uint32_t {
+    // tiles of `waves` waves of a matrix, the longest wave's
+    const auto tiles = [](uint32_t rows, uint32_t cols, uint32_t waves) -> uint32_t {
         const uint32_t nb = cols / 32, lanes = 1u << small_lanes_log2(nb);
-        return (rows * lanes + 63) / 64 * ((nb + lanes - 1) / lanes);
+        return ((rows * lanes + 63) / 64 + waves - 1) / waves * ((nb + lanes - 1) / lanes);
     };
-    if (tiles(3 * hp.rot, D) > kSmallHeadTiles * kSmallWaves) return LV_OK;
+    const uint32_t head = tiles(3 * hp.rot, D, kSmallWaves);
+    if (head > kSmallHeadTiles) return LV_OK;
     // a pair of tiles a wave in the feed-forward, or four tiles of a large vocabulary
-    const uint32_t most = std::max(tiles(F, D), tiles(hp.vocab, D) / 4);
-    m->small_wgs = std::min(kSmallMaxWGs, std::max(hp.heads, (most + kSmallWaves - 1) / kSmallWaves));
+    const uint32_t most = std::max(tiles(F, D, 1), tiles(hp.vocab, D, 1) / 4);
+    const uint32_t wgs = std::min(kSmallMaxWGs, std::max(hp.heads, (most + kSmallWaves - 1) / kSmallWaves)), waves = wgs * kSmallWaves;
+    const double mb = (ft == LV_Q4_0 ? 18 : 34) / 32e6, layer_mb = (4.0 * D * D + 3.0 * D * F) * mb, output_mb = (double)hp.vocab * D * mb;
+    const double launch = 17 + hp.layers * (9.6 + 1.1 * head + 0.95 * (tiles(D, D, waves) + 2 * tiles(F, D, waves) + tiles(D, F, waves))) + 1.26 * tiles(hp.vocab, D, waves);
+    const double chain = 25 + hp.layers * (42 + 0.125 * layer_mb) + 0.06 * output_mb;
+    if (launch >= chain) return LV_OK;
+    m->small_wgs = wgs;
+    m->small_elements = (uint32_t)std::min<double>(kSmallRowElements, (chain - launch) / hp.layers / 0.08 * 1000);
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&m->small_layers), table.size() * sizeof(SmallLayer)));
     HIP_TRY(hipMemcpyAsync(m->small_layers, table.data(), table.size() * sizeof(SmallLayer), hipMemcpyHostToDevice, m->ctx->stream));
     HIP_TRY(hipStreamSynchronize(m->ctx->stream));
@@ -2964,7 +2975,7 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     // steps of a few tokens take position and token ids as launch arguments, and so does a token at a time
     const uint32_t batch_min = s->block ? kBlockBatchMin : (uint32_t)kPrefillMin, batch_max = s->block ? kBlockBatch : kPrefillChunk;
     const bool small = n < kPrefillMin && !few && s->model->small_wgs && s->path == LV_PATH_AUTO && path == LV_PATH_GRAPH && !s->trace && !s->mega_off &&
-                       (pos + n) * s->model->hp.rot <= kSmallRowElements;
+                       (pos + n) * s->model->hp.rot <= s->model->small_elements;
     // A step of up to kMidTokens, or what is left of a longer one behind its whole chunks, takes the products of lv_mid.h: by its size alone
     const uint32_t rest = n <= kPrefillChunk ? n : n % kPrefillChunk;
     const bool pays = n >= kPrefillMin && rest && s->path == LV_PATH_AUTO && s->model->short_ok && !s->trace && mid_pays(s->model->hp, rest);
