@@ -2695,11 +2695,20 @@ static int launch_short_norm(hipStream_t st, const ShortBuffers &b, const float 
 static int launch_short_attention(hipStream_t st, const lv_session *s, const ShortBuffers &b, uint32_t layer, uint32_t pos, uint32_t n, uint32_t ftype)
 {
     const lv_hparams &hp = s->model->hp;
-    // At most a workgroup a CU: what each does before and behind its tiles (queries to operands, sums through LDS and out) is more than a
-    // tile, and two on a CU are in each other's way.  us with the kernel that puts the parts together, two a CU and one: 45 tokens behind 619
-    // 27.0 and 22.1, behind 1950 32.4 and 29.9; 8 tokens behind 619 15.6 and 13.3, behind 1100 20.7 and 15.8.
-    const uint32_t tiles = (pos + n + kAttnBatchK - 1) / kAttnBatchK, want = hp.heads < 256 ? 256 / hp.heads : 1;
-    const uint32_t most = want < kShortSplits ? want : kShortSplits, per = (tiles + most - 1) / most, splits = (tiles + per - 1) / per;
+    // Parts: as many as make a workgroup a CU.  What each does before and behind its tiles (queries to operands, sums through LDS and out) is
+    // more than a tile, and two on a CU are in each other's way: in fp32 always (4 tokens behind 4000 rows, 7B 8 us a layer more, 13B 12).  On
+    // fp16 pairs a tile takes 3 us in a workgroup that has its CU to itself; where all share one, 1.85 for every tile a CU, beyond 32 tokens
+    // 2.2, and 5.5 or 7 more at the ends: faster behind long contexts, and where few heads more than a divisor of 256 leave CUs idle.  us a
+    // layer that one a CU takes more than two: 7B, 32 tokens behind 1900 rows -1.3, behind 4000 4.6, 64 tokens -5 and -3; 13B, 16 tokens behind
+    // 1500 rows 0.3, behind 2700 6.7, behind 4000 8.5; 64 tokens behind 2700 3.0, behind 4000 4.3.
+    const uint32_t tiles = (pos + n + kAttnBatchK - 1) / kAttnBatchK;
+    const auto tiles_of_part = [&](uint32_t wgs) {
+        const uint32_t most = std::min(std::max(wgs / hp.heads, 1u), kShortSplits);
+        return (tiles + most - 1) / most;
+    };
+    const uint32_t one = tiles_of_part(256), two = tiles_of_part(512);
+    const float a_cu = tiles * hp.heads / 256.f, shared = n <= 32 ? 5.5f + 1.85f * a_cu : 7.f + 2.2f * a_cu;
+    const uint32_t per = n >= kPrefillMin && shared < 3.f * one ? two : one, splits = (tiles + per - 1) / per;
     ShortAttnArgs a{};
     a.kcache = kv_ptr(s, layer, 0); a.vcache = kv_ptr(s, layer, 1); a.q = b.q; a.trig_abs = s->trig_abs;
     a.pos0 = pos; a.n = n; a.heads = hp.heads; a.backlog = s->backlog; a.tiles_per_split = per; a.num = b.num; a.den = b.den;

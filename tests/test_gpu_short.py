@@ -75,6 +75,29 @@ def test_short_batch_matches_oracle(lva, orc, ctx, models, name, before, n):
     sess.close(); model.close(); osess.close(); om.close()
 
 
+@pytest.mark.parametrize("before,n", [(1900, 16), (1940, 33), (2040, 16), (2017, 31), (2100, 32), (2200, 33), (2300, 64), (2300, 15)])
+def test_attention_of_short_steps_behind_long_contexts(lva, ctx, tmp_path, before, n):
+    """one or two workgroups a CU, by the context's tiles a workgroup, on either side of where it changes; against the operator chain"""
+    path = str(tmp_path / "forty.ggml")
+    lva.write_model(path, wtype=lva.LV_Q8_0, seed=11, vocab=512, dim=1280, heads=40, layers=1, ff=1408)
+    model = lva.Model(ctx, path)
+    toks = lva.synth_tokens(before + n, 3, 512, seed=n)
+    a, b = lva.Session(model, before + n), lva.Session(model, before + n)
+    b.set_path(lva.PATH_KERNELS)
+    a.begin(toks[:before], 0)
+    a.wait()
+    for which in (0, 1):
+        b.kv_write(0, which, a.kv(0, which, before))
+    for s in (a, b):
+        s.keep_all_logits()
+    a.begin(toks[before:], before)
+    got = a.logits_rows(0, n)
+    for i in range(n):
+        b.begin(toks[before + i:before + i + 1], before + i)
+        close(got[i], b.logits())
+    a.close(); b.close(); model.close()
+
+
 # steps of 65 to 256 tokens (csrc/lv_mid.h), and what is left of a longer one: every edge of the token tiles and of the two groups of them
 MIDDLE = [(name, 0, n) for name in ("q4_64", "q8_128") for n in (65, 80, 81, 96, 97, 128, 129, 160, 161, 192, 193, 256)]
 MIDDLE += [(name, 37, n) for name in [*SHAPES, "q4_64_v1", "q8_64_v1"] for n in (70, 120, 170)]
