@@ -2417,26 +2417,32 @@ template <int QT, int T>
 static void launch_short_rows(hipStream_t st, const ShortArgs &a, uint32_t rt, uint32_t slices, bool sf32)
 {
     if (rt == 2) launch_short_kernel<QT, T, 2>(st, a, slices, sf32);
-    if (rt == 3) launch_short_kernel<QT, T, 3>(st, a, slices, sf32);
-    if (rt == 4) launch_short_kernel<QT, T, 4>(st, a, slices, sf32);
-    if (rt == 6) launch_short_kernel<QT, T, 6>(st, a, slices, sf32);
+    if constexpr (short_fits(QT, T, 3))
+        if (rt == 3) launch_short_kernel<QT, T, 3>(st, a, slices, sf32);
+    if constexpr (short_fits(QT, T, 4))
+        if (rt == 4) launch_short_kernel<QT, T, 4>(st, a, slices, sf32);
+    if constexpr (short_fits(QT, T, 6))
+        if (rt == 6) launch_short_kernel<QT, T, 6>(st, a, slices, sf32);
 }
 
 // Row tiles per workgroup (RT) and K slices of a product.  A workgroup's step (eight waves, a chunk each) costs its row tiles plus the
 // activations, worth about 1.5 row tiles.  What counts is how many of them a CU works off, one after the other or beside one another; a
-// slice more is written and read again.  Measured in us above the choice, 16 and 19 us gate and up, 11 and 13 q, k and v (768 tiles):
+// slice more is written and read again.  Measured in us (7B, T token tiles):
+//   q4_0 gate and up, 1376 tiles, T 2, RT 2/3/4/6: 32/29/32/25
+// and with three parts (T 0 and 1) above the choice, 16 and 19 us gate and up, 11 and 13 q, k and v (768 tiles):
 //   gate and up, RT 2/3/4/6: T 0 3.8/2.4/4.0/0, T 1 7.8/4.6/6.5/0; q, k and v: T 0 3.3/0/0.7/2.9, T 1 5.1/0/0.9/3.4
 //   down, RT 4 slices 1/2/3/4: T 0 9.3/1.2/0/0, T 1 13.5/2.3/0.2/0, RT 2: T 0 4.0/-0.8/1.4/0.5, T 1 8.4/-0.4/3.3/1.3
-static void short_plan(uint32_t tiles, uint32_t nb, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
+static void short_plan(uint32_t tiles, uint32_t nb, uint32_t T, int qt, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
 {
     const uint32_t chunks = nb / 4;
     double best = 1e30;
     for (uint32_t rt : {2u, 3u, 4u, 6u}) {
+        if (!short_fits(qt, T, rt)) continue;
         for (uint32_t s = 1; s <= (sliced ? (uint32_t)kShortSlices : 1u); s++) {
             const uint32_t per = (chunks + s - 1) / s;
             if ((chunks + per - 1) / per != s) continue;
             const uint32_t steps = (per + kShortWaves - 1) / kShortWaves, held = ((tiles + rt - 1) / rt * s + 255) / 256;
-            const double cost = held * steps * (rt + 1.5) + 0.25 * (s - 1);
+            const double cost = held * steps * (rt + 1.5) + 0.25 * (T ? T : 1) * (s - 1);
             if (cost < best) { best = cost; *best_rt = rt; *best_chunks = per; }
         }
     }
@@ -2448,13 +2454,13 @@ static int launch_short_gemm(hipStream_t st, ShortArgs a, uint32_t ftype, bool s
     const int qt = ftype == LV_Q4_0 ? 4 : 8;
     uint32_t rt = 2;
     if (!a.w) return fail(LV_ERR_STATE, "short batch: the matrix has no copy");
-    short_plan(a.tiles, a.nb, sliced, &rt, &a.slice_chunks);
+    short_plan(a.tiles, a.nb, T, qt, sliced, &rt, &a.slice_chunks);
     const uint32_t slices = (a.nb / 4 + a.slice_chunks - 1) / a.slice_chunks;
     if (slices_out) *slices_out = slices;
 #define LV_SHORT(QT, TT) case QT * 8 + TT: launch_short_rows<QT, TT>(st, a, rt, slices, sf32); break;
     switch (qt * 8 + T) {
-        LV_SHORT(4, 0) LV_SHORT(4, 1)
-        LV_SHORT(8, 0) LV_SHORT(8, 1)
+        LV_SHORT(4, 0) LV_SHORT(4, 1) LV_SHORT(4, 2) LV_SHORT(4, 3) LV_SHORT(4, 4)
+        LV_SHORT(8, 0) LV_SHORT(8, 1) LV_SHORT(8, 2) LV_SHORT(8, 3) LV_SHORT(8, 4)
     default: return fail(LV_ERR_STATE, "short batch of %u tokens", a.n);
     }
 #undef LV_SHORT
@@ -2548,8 +2554,29 @@ static bool mid_pays(const lv_hparams &hp, uint32_t n)
     return here < there(D, 3, D, false) + there(D, 1, D, true) + there(2 * F, 1, D, false) + there(D, 1, F, true);
 }
 
-static int launch_mid_gemm(hipStream_t st, MidArgs a, uint32_t ftype, bool sf32, bool sliced, uint32_t *slices_out = nullptr)
+// Do up to 64 tokens (T tiles of 16, 2 to 4) times a product of this size take less time in short_gemm_kernel, whose waves wait for nobody?
+// Filling and draining the LDS stages takes 1 us of wide_short_gemm_kernel, unpacking each weight once pays it back the sooner the more tokens there
+// are, and q8_0 sooner than q4_0.  Widths of 384 to 8192, us here and there, 24 / 56 tokens: q, k and v of width 1024 q4_0 4.9 and 5.9, 6.4
+// and 7.5, of 2560 9.0 and 10.4, 12.0 and 13.1, of 4096 15.2 and 15.0, 21.7 and 20.6; gate and up of 2048 q8_0 12.2 and 12.1, 20.7 and 15.2, of
+// 1024 5.6 and 6.4, 7.4 and 8.0; down of 4096 q4_0 13.7 and 17.3, 19.6 and 19.2, of 3584 q8_0 16.9 and 14.9.
+static bool short_pays(uint32_t T, int qt, uint32_t tiles, uint32_t nb, bool sliced)
 {
+    const uint32_t blocks = tiles * nb;
+    if (T == 2) return sliced ? qt == 4 || blocks <= 49152 : tiles <= (qt == 4 ? 1040u : 672u);
+    if (T == 3) return !sliced && tiles <= (qt == 4 ? 512u : 256u);
+    return T == 4 && (sliced ? blocks <= 18432 : tiles <= (qt == 4 ? 512u : 480u));
+}
+
+// act: its activations lie as the kernels for short steps write them
+static int launch_mid_gemm(hipStream_t st, MidArgs a, uint32_t ftype, bool sf32, bool sliced, bool act, uint32_t *slices_out = nullptr)
+{
+    if (act && short_pays(short_tiles(a.n), ftype == LV_Q4_0 ? 4 : 8, a.tiles, a.nb, sliced)) {
+        ShortArgs b{};
+        b.x = a.x[0]; b.w = a.w; b.tiles_m = a.tiles_m; b.tiles = a.tiles; b.nb = a.nb; b.n = a.n; b.mode = a.mode; b.ldo = a.ldo; b.xscale = a.xscale;
+        for (int i = 0; i < kShortSlices; i++) b.out[i] = a.out[i];
+        b.cache[0] = a.cache[0]; b.cache[1] = a.cache[1]; b.pos_ptr = a.pos_ptr; b.pos_add = a.pos_add; b.backlog = a.backlog; b.ff = a.ff[0];
+        return launch_short_gemm(st, b, ftype, sf32, sliced, slices_out);
+    }
     if (!a.w) return fail(LV_ERR_STATE, "short batch: the matrix has no copy");
     if (a.n > kMidTokens) return fail(LV_ERR_STATE, "short batch of %u tokens", a.n);
     uint32_t T, groups, rt = 2;
@@ -2764,7 +2791,7 @@ static int record_short_head(lv_session *s, const ShortBuffers &b, uint32_t idx0
             MidArgs a = mid_store(n, D, m->short_output, hp.vocab, b.xscale);
             mid_input_short(a, b.act);
             a.out[0] = all;
-            LV_TRY(launch_mid_gemm(st, a, ft, sf32, false));
+            LV_TRY(launch_mid_gemm(st, a, ft, sf32, false, true));
         }
     } else if (all || with_head) {
         // only the last row's logits are ever read (llava_session.cpp:131-139), unless all are asked for
@@ -2785,7 +2812,7 @@ static int record_short_head(lv_session *s, const ShortBuffers &b, uint32_t idx0
     return LV_OK;
 }
 
-// record_short's layers for 17 tokens and more: activations as fp16 halves, the products of lv_mid.h
+// record_short's layers for 17 tokens and more: activations as fp16 halves
 static int record_short_halves(lv_session *s, const ShortBuffers &b, uint32_t idx0, uint32_t n, uint32_t pos, bool with_head, uint32_t row_base)
 {
     const lv_model *m = s->model;
@@ -2799,21 +2826,21 @@ static int record_short_halves(lv_session *s, const ShortBuffers &b, uint32_t id
         LV_TRY(launch_short_norm(st, b, lw.attn_norm, n, D, pending, ft));
         MidArgs a = mid_qkv(s, li, n, idx0, b.q, b.xscale);
         mid_input_short(a, b.act);
-        LV_TRY(launch_mid_gemm(st, a, ft, sf32, false));
+        LV_TRY(launch_mid_gemm(st, a, ft, sf32, false, true));
         LV_TRY(launch_short_attention(st, s, b, li, pos, n, ft));
         MidArgs o = mid_store(n, D, lw.short_wo, D, nullptr);
         mid_input_short(o, b.act);
         for (int i = 0; i < kShortSlices; i++) o.out[i] = b.parts[i];
-        LV_TRY(launch_mid_gemm(st, o, ft, sf32, true, &pending));
+        LV_TRY(launch_mid_gemm(st, o, ft, sf32, true, true, &pending));
         LV_TRY(launch_short_norm(st, b, lw.ffn_norm, n, D, pending, ft));
         MidArgs f = mid_silu(s, li, n, b.xscale);
         mid_input_short(f, b.act);
         MidArgs d = mid_store(n, F, lw.short_down, D, nullptr);
         mid_input_short(d, b.ff);
         mid_output_ff(f, d);
-        LV_TRY(launch_mid_gemm(st, f, ft, sf32, false));
+        LV_TRY(launch_mid_gemm(st, f, ft, sf32, false, true));
         for (int i = 0; i < kShortSlices; i++) d.out[i] = b.parts[i];
-        LV_TRY(launch_mid_gemm(st, d, ft, sf32, true, &pending));
+        LV_TRY(launch_mid_gemm(st, d, ft, sf32, true, true, &pending));
     }
     return record_short_head(s, b, idx0, n, pending, with_head, row_base);
 }
@@ -2833,22 +2860,22 @@ static int record_mid_layers(lv_session *s, uint32_t idx0, uint32_t n, float *co
         LV_TRY(launch_prefill_norm(st, s, lw.attn_norm, n, D, parts, pending, false, &xscale));
         MidArgs a = mid_qkv(s, li, n, idx0, s->pf_q, xscale);
         mid_input_planes(a, s->pf_xh, s->pf_xl);
-        LV_TRY(launch_mid_gemm(st, a, ft, sf32, false));
+        LV_TRY(launch_mid_gemm(st, a, ft, sf32, false, false));
         LV_TRY(launch_attention_batch(st, nullptr, s->pf_xh, s->pf_xl, D, s->pf_planes, kv_ptr(s, li, 0), kv_ptr(s, li, 1), nullptr, nullptr, s->pf_q, s->trig_abs,
                                       s->cfg, idx0, n, s->backlog, hp.heads, hp.rot));
         MidArgs o = mid_store(n, D, lw.short_wo, D, nullptr);
         mid_input_planes(o, s->pf_xh, s->pf_xl);
         for (int i = 0; i < kShortSlices; i++) o.out[i] = parts[i];
-        LV_TRY(launch_mid_gemm(st, o, ft, sf32, true, &pending));
+        LV_TRY(launch_mid_gemm(st, o, ft, sf32, true, false, &pending));
         LV_TRY(launch_prefill_norm(st, s, lw.ffn_norm, n, D, parts, pending, false, &xscale));
         MidArgs f = mid_silu(s, li, n, xscale);
         mid_input_planes(f, s->pf_xh, s->pf_xl);
         MidArgs d = mid_store(n, F, lw.short_down, D, nullptr);
         mid_input_planes(d, s->pf_fh, s->pf_fl);
         mid_output_ff(f, d);
-        LV_TRY(launch_mid_gemm(st, f, ft, sf32, false));
+        LV_TRY(launch_mid_gemm(st, f, ft, sf32, false, false));
         for (int i = 0; i < kShortSlices; i++) d.out[i] = parts[i];
-        LV_TRY(launch_mid_gemm(st, d, ft, sf32, true, &pending));
+        LV_TRY(launch_mid_gemm(st, d, ft, sf32, true, false, &pending));
     }
     *pending_out = pending;
     return LV_OK;

@@ -1,5 +1,5 @@
 // lv_mid.h — products of steps of 17 to 256 tokens of LLaMA models: the short copy's weights (lv_short.h), activations as two fp16
-// halves through LDS.
+// halves through LDS.  Up to 64 tokens the smaller ones stay with lv_short.h (short_pays).
 //
 // Every weight is read once per 128 tokens and unpacked once, for all of a workgroup's tokens; a workgroup of eight waves owns
 // RT = RG RTW tiles of 16 rows, T tiles of 16 tokens and all of K or a slice of it.  RG groups of waves take RTW row tiles each, their

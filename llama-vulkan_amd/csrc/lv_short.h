@@ -8,10 +8,11 @@
 //   up to 16 tokens   three bf16 parts, an exact cut of the fp32 value with all of its range.  Such a step is also evaluated token by
 //                     token (other paths, no room for the copy below), in fp32 throughout, and is held to the same.
 //   17 to 64          two fp16 halves as in lv_gemm.h, which takes longer steps and these without the copy: 22 bits, of the norms'
-//                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.  Their products: lv_mid.h.
+//                     outputs scaled per token; feed-forward and attention outputs unscaled, below 65504.  Their products: lv_mid.h,
+//                     smaller ones here.
 // Attention likewise: up to 15 tokens in fp32 (short_attn_exact_kernel), then short_attn_kernel on fp16 pairs as with longer steps.
 //
-// short_gemm_kernel, up to 16 tokens.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
+// short_gemm_kernel.  A workgroup of 8 waves owns RT tiles of 16 weight rows over all of K (or one of up to 4 slices of it) and all
 // tokens; its waves deal the K range among themselves, four quant blocks at a time, and add up through LDS at the end.  A wave so
 // reads activations nobody else in the workgroup reads, straight into MFMA operand form, and reuses them for its RT tiles: no
 // LDS, no barrier, nothing but loads in flight in the main loop.
@@ -122,16 +123,31 @@ struct ShortArgs {
     uint32_t n, mode;
     float *out[kShortSlices];  // [n][ldo], one per slice; kShortQkv: out[0] = q
     uint32_t ldo;
+    const float *xscale;       // null, or per token the power of two its halves have to be multiplied by (not with parts)
     uint16_t *cache[2];        // kShortQkv: k and v rows
     const uint32_t *pos_ptr;
     uint32_t pos_add, backlog;
     uint8_t *ff;               // kShortSilu: activations of the next product
 };
 
-// Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights.  More in flight per wave
-// costs registers, hence waves per CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us).  Nor do two
-// workgroups a CU pay: two blocks ahead would let three row tiles of q4_0 and up to 16 tokens into 128 registers (a step of 8 tokens of
-// 13B q4_0, 8 layers: 752 us so, 708 with four ahead).
+// Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights or, where a block's
+// products take long enough to cover an L2 access, two blocks ahead.  More in flight per wave costs registers, hence waves per
+// CU, and lost (two chunks of weights: 7B q4_0 gate and up for 8 tokens 15.8 -> 16.5 us).  Nor do two workgroups a CU pay: two blocks
+// ahead would let three row tiles of q4_0 and up to 16 tokens into 128 registers (a step of 8 tokens of 13B q4_0, 8 layers: 752 us so,
+// 708 with four ahead).
+template <int T, int RT> constexpr int short_ahead() { return T * RT >= 8 ? 2 : 4; }
+// RT tiles of rows beside T tiles of tokens that keep sums, queues and activations in 256 registers, and that short_pays asks for
+__host__ __device__ constexpr bool short_fits(int qt, uint32_t t, uint32_t rt)
+{
+    if (t > 2) return rt == 2;
+    return rt <= (qt == 8 && t == 2 ? 3u : 6u);
+}
+// row tiles whose sums are put together at a time: up to 64 KB of LDS, whole pairs
+template <int T, int RT> constexpr int short_round()
+{
+    constexpr int most = 8 / (T ? T : 1);
+    return RT <= most ? RT : most;
+}
 __device__ __forceinline__ lv_h8 short_unpack4(uint32_t w)
 {
     // nibble q in the low bits of a half of pattern 0x6400 is 1024 + q; one place up, 1024 + 16 q: both to q - 8, exactly
@@ -221,19 +237,21 @@ __global__ __launch_bounds__(256) void short_pack_kernel(uint8_t *__restrict__ d
     }
 }
 
-// T: 0: up to 8 tokens, 1: up to 16; RT: tiles of 16 rows per workgroup; SF32: fp32 block scales
+// T: tiles of 16 tokens, 0: up to 8 tokens; RT: tiles of 16 rows per workgroup; SF32: fp32 block scales
 template <int QT, bool SF32, int T, int RT>
 __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs a)
 {
-    static_assert(short_exact(T), "more tokens: wide_short_gemm_kernel");
     constexpr bool EIGHT = T == 0;                     // 8 tokens: an operand holds their first parts and their second ones
+    constexpr bool EXACT = short_exact(T);
+    constexpr int NT = EIGHT ? 1 : T;
     constexpr int XB = short_block_bytes(T);           // activation bytes of a block
-    constexpr int NX = EIGHT ? 2 : 3;                  // its operands
+    constexpr int NX = EIGHT ? 2 : EXACT ? 3 : 2 * NT; // its operands
     constexpr int BB = QT == 4 ? 16 : 32;              // code bytes of a block
     constexpr int CW = BB / 4;                         // a lane's dwords of a chunk
     constexpr int CB = short_chunk_bytes(QT, SF32);
-    constexpr int XD = 4;                              // blocks the activations are requested ahead
-    __shared__ __attribute__((aligned(16))) float red[RT * kShortWaves * 256];
+    constexpr int XD = short_ahead<T, RT>();
+    constexpr int PR = short_round<T, RT>();           // row tiles summed at a time
+    __shared__ __attribute__((aligned(16))) float red[PR * NT * kShortWaves * 256];
     const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tile0 = blockIdx.x * RT;
@@ -273,9 +291,11 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
             xq[slot][t] = *reinterpret_cast<const lv_u4 *>(p + at + t * 1024);
         }
     };
-    lv_f4v acc[RT];
+    lv_f4v acc[RT][NT];
 #pragma unroll
-    for (int i = 0; i < RT; i++) acc[i] = lv_f4v{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[i][t] = lv_f4v{0.f, 0.f, 0.f, 0.f};
     const lv_f4v zero = {0.f, 0.f, 0.f, 0.f};
     constexpr uint32_t kOnes = 0x3f803f80u;
 
@@ -299,7 +319,7 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
             fetch_w(j + 1);
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                lv_u4 ax[NX];                          // parts
+                lv_u4 ax[NX];                          // parts, or high and low halves tile by tile
 #pragma unroll
                 for (int t = 0; t < NX; t++) ax[t] = xq[s % XD][t];
                 if constexpr (EIGHT) ax[1] = r16 >= 8 ? ax[1] : lv_u4{0u, 0u, 0u, 0u};       // the third parts beside the second
@@ -309,25 +329,36 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
                     return c;
                 };
                 lv_f4v from = zero;
-                if constexpr (QT == 4) from = times(__builtin_bit_cast(lv_b8, lv_u4{kOnes, kOnes, kOnes, kOnes}), zero) * -8.f;
+                if constexpr (EXACT && QT == 4) from = times(__builtin_bit_cast(lv_b8, lv_u4{kOnes, kOnes, kOnes, kOnes}), zero) * -8.f;
 #pragma unroll
                 for (int i = 0; i < RT; i++) {
-                    const lv_b8 b = QT == 4 ? short_unpack4_bf16(w[i][s]) : short_unpack8_bf16(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
-                    const lv_f4v p = times(b, from);
+                    lv_f4v p[NT];
+                    if constexpr (EXACT) {
+                        const lv_b8 b = QT == 4 ? short_unpack4_bf16(w[i][s]) : short_unpack8_bf16(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
+                        p[0] = times(b, from);
+                    } else {
+                        const lv_h8 b = QT == 4 ? short_unpack4(w[i][s]) : short_unpack8(w[i][CW / 4 * s], w[i][CW / 4 * s + CW / 8]);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc[i][e] = fmaf(p[e], sc[i][s], acc[i][e]);
+                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lv_h8, ax[2 * t + 1]), b, zero, 0, 0, 0);
+#pragma unroll
+                        for (int t = 0; t < NT; t++) p[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lv_h8, ax[2 * t]), b, p[t], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int t = 0; t < NT; t++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[i][t][e] = fmaf(p[t][e], sc[i][s], acc[i][t][e]);
                 }
                 fetch_x(s % XD, j + (s + XD) / 4, (s + XD) % 4);
             }
         }
     }
 
-    // ---- the waves' sums through LDS: [row tile][wave][lane] float4 ---------------------------------------------------------------
-    // acc[i][e]: row r16 of row tile i, token 4 g + e (EIGHT: the first part's product of token 4 g + e for g < 2, behind them the
-    // others').  A wave adds up every eighth row tile.
+    // ---- the waves' sums, PR row tiles at a time, through LDS: [row tile][token tile][wave][lane] float4 -------------------------
+    // acc[i][t][e]: row r16 of row tile i, token 16 t + 4 g + e (EIGHT: the first part's product of token 4 g + e for g < 2, behind
+    // them the others').  A wave adds up every eighth (row tile, token tile).
     const uint32_t row_at = (a.mode == kShortQkv && a.pos_ptr ? *a.pos_ptr : 0u) + a.pos_add;
     float *const out = a.out[blockIdx.y];
-    auto total = [&](int u, int from) {                // lane `from`'s sums of row tile u
+    auto total = [&](int u, int from, float (&v)[4], const float4 &xs) {      // lane `from`'s sums of unit u
         const lv_f4v *src = reinterpret_cast<const lv_f4v *>(red) + (size_t)u * kShortWaves * 64 + from;
         lv_f4v s = src[0];
 #pragma unroll
@@ -337,37 +368,55 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
 #pragma unroll
             for (int w = 0; w < kShortWaves; w++) s += low[w * 64];
         }
-        return s;
+        v[0] = s[0] * xs.x; v[1] = s[1] * xs.y; v[2] = s[2] * xs.z; v[3] = s[3] * xs.w;
     };
 #pragma unroll
-    for (int i = 0; i < RT; i++) *reinterpret_cast<lv_f4v *>(red + ((i * kShortWaves + wave) * 64 + lane) * 4) = acc[i];
-    __syncthreads();
-    for (int u = wave; u < RT; u += kShortWaves) {
-        const uint32_t tile = tile0 + u, tok0 = 4 * g;
-        if (tile >= a.tiles || (EIGHT && lane >= 32)) continue;
-        const lv_f4v v = total(u, lane);
-        if (a.mode == kShortSilu) {                    // rows 0 .. 7 of the tile are W3's, 8 .. 15 the same ones of W1
-            if (r16 >= 8) continue;
-            const lv_f4v w = total(u, lane + 8);
-            const uint32_t f = tile * 8 + r16, slot = short_slot<QT, true>(f & 31);
+    for (int i0 = 0; i0 < RT; i0 += PR) {
+        if (i0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PR; i++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                if (i0 + i < RT) *reinterpret_cast<lv_f4v *>(red + (((i * NT + t) * kShortWaves + wave) * 64 + lane) * 4) = acc[i0 + i][t];
+        __syncthreads();
+        for (int u = wave; u < (RT - i0 < PR ? RT - i0 : PR) * NT; u += kShortWaves) {
+            const uint32_t tile = tile0 + i0 + u / NT, tok0 = 16 * (u % NT) + 4 * g;
+            if (tile >= a.tiles || (EIGHT && lane >= 32)) continue;
+            float4 xs = make_float4(1.f, 1.f, 1.f, 1.f);
+            if (a.xscale) xs = *reinterpret_cast<const float4 *>(a.xscale + tok0);
+            float v[4];
+            total(u, lane, v, xs);
+            if (a.mode == kShortSilu) {                // rows 0 .. 7 of the tile are W3's, 8 .. 15 the same ones of W1
+                if (r16 >= 8) continue;
+                float w[4];
+                total(u, lane + 8, w, xs);
+                const uint32_t f = tile * 8 + r16, slot = short_slot<QT, EXACT>(f & 31);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (tok0 + e >= a.n) continue;
+                    const float y = v[e] * w[e] / (__expf(-w[e]) + 1.f);
+                    auto put = [&](uint32_t part, uint16_t v) { *reinterpret_cast<uint16_t *>(a.ff + short_act_offset(f / 32, tok0 + e, slot >> 3, T, part) + (slot & 7) * 2) = v; };
+                    if constexpr (EXACT) {
+                        uint32_t b[3];
+                        short_cut(b, y);
+#pragma unroll
+                        for (int i = 0; i < 3; i++) put(i, (uint16_t)(b[i] >> 16));
+                    } else {
+                        const uint16_t h = float_to_half_bits(y);
+                        put(0, h);
+                        put(1, float_to_half_bits(y - half_bits_to_float(h)));
+                    }
+                }
+                continue;
+            }
+            const uint32_t z = tile / a.tiles_m, m = tile % a.tiles_m * 16 + r16;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                if (tok0 + e >= a.n) continue;
-                uint32_t b[3];
-                short_cut(b, v[e] * w[e] / (__expf(-w[e]) + 1.f));
-#pragma unroll
-                for (int i = 0; i < 3; i++)
-                    *reinterpret_cast<uint16_t *>(a.ff + short_act_offset(f / 32, tok0 + e, slot >> 3, T, i) + (slot & 7) * 2) = (uint16_t)(b[i] >> 16);
+                const uint32_t tok = tok0 + e;
+                if (tok >= a.n) continue;
+                if (z == 0) out[(size_t)tok * a.ldo + m] = v[e];
+                else if (row_at + tok < a.backlog) a.cache[z - 1][(size_t)(row_at + tok) * a.ldo + m] = float_to_half_bits(v[e]);
             }
-            continue;
-        }
-        const uint32_t z = tile / a.tiles_m, m = tile % a.tiles_m * 16 + r16;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const uint32_t tok = tok0 + e;
-            if (tok >= a.n) continue;
-            if (z == 0) out[(size_t)tok * a.ldo + m] = v[e];
-            else if (row_at + tok < a.backlog) a.cache[z - 1][(size_t)(row_at + tok) * a.ldo + m] = float_to_half_bits(v[e]);
         }
     }
 }
