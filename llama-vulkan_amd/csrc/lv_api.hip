@@ -2538,6 +2538,7 @@ static void mid_tokens(uint32_t n, uint32_t *T, uint32_t *groups)
 // the chip idle; above, it depends on how both fill their rounds.  Measured, ms a step of 8 layers of q8_0, tiles of 128 and here:
 //   7B   100 tokens 2.54 and 1.57, 129 2.61 and 1.87, 200 2.65 and 2.46, 256 2.68 and 2.49
 //   13B  100 tokens 3.06 and 2.21, 129 3.16 and 2.86, 200 3.32 and 3.82, 256 3.45 and 3.94
+// Estimates this close to each other have told the wrong way (6656 wide, 2 layers of q4_0, 200 tokens 1.22 and 1.27): then the larger tiles.
 static bool mid_pays(const lv_hparams &hp, uint32_t n)
 {
     if (n <= 128) return true;
@@ -2551,7 +2552,7 @@ static bool mid_pays(const lv_hparams &hp, uint32_t n)
     };
     const double here = mid_plan(3 * D / 16, D / 32, T, groups, false, &rt, &per) + mid_plan(D / 16, D / 32, T, groups, true, &rt, &per) +
                         mid_plan(F / 8, D / 32, T, groups, false, &rt, &per) + mid_plan(D / 16, F / 32, T, groups, true, &rt, &per);
-    return here < there(D, 3, D, false) + there(D, 1, D, true) + there(2 * F, 1, D, false) + there(D, 1, F, true);
+    return here < 0.975 * (there(D, 3, D, false) + there(D, 1, D, true) + there(2 * F, 1, D, false) + there(D, 1, F, true));
 }
 
 // Do up to 64 tokens (T tiles of 16, 2 to 4) times a product of this size take less time in short_gemm_kernel, whose waves wait for nobody?
