@@ -1476,7 +1476,7 @@ template <class T> static int batch_branches(BlockSession *s, size_t i, uint32_t
     p.attn = gqa_spec(s, i); p.q = w.q; p.k = w.k; p.v = w.v;
     p.delta = delta_spec(s, i); p.dq = w.dq; p.dk = w.dk; p.dv = w.dv; p.beta = w.beta; p.qk = w.qk; p.a1 = w.a1; p.g1 = w.g1;
     LV_TRY(with_j(l.delta ? l.dstride() / 64 : 1, [&](auto j) -> int {
-        prepare_kernel<T, decltype(j)::value><<<dim3(prepare_grid(p, n)), dim3(256), 0, st>>>(p, n);
+        (p.delta.taps > 4 ? prepare_kernel<T, decltype(j)::value, true> : prepare_kernel<T, decltype(j)::value, false>)<<<dim3(prepare_grid(p, n)), dim3(256), 0, st>>>(p, n);
         HIP_TRY(hipGetLastError());
         return LV_OK;
     }));

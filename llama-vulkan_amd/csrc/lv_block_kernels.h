@@ -155,8 +155,11 @@ struct PrepareArgs {
     void *a1, *g1;               // low-rank activations [n][a_kp], [n][g_kp]
 };
 constexpr uint32_t kPrepareTokens = 8;     // per workgroup of the recurrent branch
-// workgroups: one per token (attention, and what is small), then per 8 tokens one for every four key heads and each 256 value channels
-inline uint32_t prepare_columns(const DeltaSpec &s) { return s.heads ? (s.kv_heads + 3) / 4 + (s.heads * s.vdim + 255) / 256 : 0; }
+// waves that share a key head's eight tokens.  One has 4 J convolutions of them one after the other: us a prompt of 16 / 1030 tokens, width 2048,
+// 2 layers, one wave and two: 2 key heads of 256 412 and 395, 998 and 976; 8 of 192 412 and 402, 969 and 964.  Up to 128 channels one reads less.
+constexpr uint32_t prepare_waves(uint32_t dstride) { return dstride > 128 ? 2 : 1; }
+// workgroups of four waves: one per token (attention, and what is small), then per 8 tokens those of the key heads and one for each 256 value channels
+inline uint32_t prepare_columns(const DeltaSpec &s) { return s.heads ? (s.kv_heads * prepare_waves(s.dstride) + 3) / 4 + (s.heads * s.vdim + 255) / 256 : 0; }
 inline uint32_t prepare_grid(const PrepareArgs &a, uint32_t n) { return n + (n + kPrepareTokens - 1) / kPrepareTokens * prepare_columns(a.delta); }
 
 template <class T> __device__ __forceinline__ void store_pair(T *o, float u, float v)
@@ -206,43 +209,45 @@ __device__ __forceinline__ void prepare_token(const PrepareArgs &a, uint32_t t, 
     }
 }
 
-// J = delta.dstride / 64.  Bound by memory: 2048 tokens of width 4096 (119 MB of projections in, 90 MB out) 61 us; with a thread a channel and
-// token, each input asked for once a tap and the taps again for every token, 94.
-template <class T, int J>
+// J = delta.dstride / 64, LONG: more than four taps.  Bound by memory: 2048 tokens of width 4096 (119 MB of projections in, 90 MB out) 61 us; with
+// a thread a channel and token, each input asked for once a tap and the taps again for every token, 94.
+template <class T, int J, bool LONG>
 __global__ __launch_bounds__(256) void prepare_kernel(PrepareArgs a, uint32_t n)
 {
     __shared__ float scratch[8];
     __shared__ float2 turn[kGqaMaxDim / 2];
     if (blockIdx.x < n) return prepare_token<T>(a, blockIdx.x, turn, scratch);
     const DeltaSpec &s = a.delta;
-    const uint32_t nq = s.kv_heads * s.dim, nv = s.heads * s.vdim, groups = (s.kv_heads + 3) / 4, cols = groups + (nv + 255) / 256;
-    const uint32_t idx = blockIdx.x - n, col = idx % cols, first = idx / cols * kPrepareTokens, count = min(kPrepareTokens, n - first);
+    constexpr uint32_t WAVES = prepare_waves(64 * J), N = kPrepareTokens / WAVES;      // of a key head; tokens of each
+    const uint32_t nq = s.kv_heads * s.dim, nv = s.heads * s.vdim, groups = (s.kv_heads * WAVES + 3) / 4, cols = groups + (nv + 255) / 256;
+    const uint32_t idx = blockIdx.x - n, col = idx % cols, base = idx / cols * kPrepareTokens;
     // a thread takes a channel for all eight tokens: every input read once, all of them asked for at once
     if (col >= groups) {
         const uint32_t c = (col - groups) * 256 + threadIdx.x;
         if (c >= nv) return;
-        float v[8];
-        short_conv8<true>(v, s, a.y, a.ldy, 2 * nq + c, a.pos0, first, n);
+        float v[kPrepareTokens];
+        short_conv_run<true, LONG>(v, s, a.y, a.ldy, 2 * nq + c, a.pos0, base, n);
 #pragma unroll
-        for (uint32_t i = 0; i < 8; i++)
-            if (i < count) a.dv[(size_t)(first + i) * nv + c] = v[i];
+        for (uint32_t i = 0; i < kPrepareTokens; i++)
+            if (base + i < n) a.dv[(size_t)(base + i) * nv + c] = v[i];
         return;
     }
-    const uint32_t lane = threadIdx.x & 63, h = col * 4 + (threadIdx.x >> 6);      // a wave a key head
-    if (h >= s.kv_heads) return;
-    float q[J][8], k[J][8];
+    const uint32_t lane = threadIdx.x & 63, w = col * 4 + (threadIdx.x >> 6), h = w / WAVES, first = base + w % WAVES * N;
+    if (h >= s.kv_heads || first >= n) return;
+    const uint32_t count = min(N, n - first);
+    float q[J][N], k[J][N];
 #pragma unroll
     for (int j = 0; j < J; j++) {
         const uint32_t d = j * 64 + lane;
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[j][i] = k[j][i] = 0.f;
+        for (uint32_t i = 0; i < N; i++) q[j][i] = k[j][i] = 0.f;
         if (d < s.dim) {
-            short_conv8<true>(q[j], s, a.y, a.ldy, h * s.dim + d, a.pos0, first, n);
-            short_conv8<true>(k[j], s, a.y, a.ldy, nq + h * s.dim + d, a.pos0, first, n);
+            short_conv_run<true, LONG>(q[j], s, a.y, a.ldy, h * s.dim + d, a.pos0, first, n);
+            short_conv_run<true, LONG>(k[j], s, a.y, a.ldy, nq + h * s.dim + d, a.pos0, first, n);
         }
     }
 #pragma unroll
-    for (uint32_t i = 0; i < 8; i++) {
+    for (uint32_t i = 0; i < N; i++) {
         if (i >= count) break;
         const size_t row = (size_t)(first + i) * s.kv_heads + h;
         float sq = 0.f, sk = 0.f, sqk = 0.f;

@@ -54,21 +54,21 @@ __device__ __forceinline__ float short_conv(const Spec &s, const float *y, size_
     return v.value(s, y, ld, behind, pos, slot);
 }
 
-// short_conv8 for more than four taps: eight of them at a time
-template <class Spec>
-__device__ __forceinline__ void short_conv8_long(float (&out)[8], const Spec &s, const float *y, size_t ld, uint32_t c, uint32_t pos0, uint32_t t0, uint32_t n)
+// short_conv_run for more than four taps: eight of them at a time
+template <int N, class Spec>
+__device__ __forceinline__ void short_conv_long(float (&out)[N], const Spec &s, const float *y, size_t ld, uint32_t c, uint32_t pos0, uint32_t t0, uint32_t n)
 {
     const uint32_t at = s.channel_at(c);
     const float b = s.conv_bias(c);
 #pragma unroll
-    for (uint32_t i = 0; i < 8; i++) out[i] = b;
+    for (uint32_t i = 0; i < N; i++) out[i] = b;
 #pragma unroll 1
     for (uint32_t j0 = 0; j0 < s.taps; j0 += 8) {
-        float in[15], w[8];      // in[i]: token t0 + i - j0 - 7
+        float in[N + 7], w[8];      // in[i]: token t0 + i - j0 - 7
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++) w[j] = j0 + j < s.taps ? s.conv[(size_t)(s.taps - 1 - j0 - j) * s.channels() + c] : 0.f;
 #pragma unroll
-        for (uint32_t i = 0; i < 15; i++) {
+        for (uint32_t i = 0; i < N + 7; i++) {
             const uint32_t t = t0 + i, back = j0 + 7;
             in[i] = 0.f;
             if (t >= back) {
@@ -78,30 +78,30 @@ __device__ __forceinline__ void short_conv8_long(float (&out)[8], const Spec &s,
             }
         }
 #pragma unroll
-        for (uint32_t i = 0; i < 8; i++)
+        for (uint32_t i = 0; i < N; i++)
 #pragma unroll
             for (uint32_t j = 0; j < 8; j++) out[i] = j0 + j < s.taps ? fmaf(in[i + 7 - j], w[j], out[i]) : out[i];
     }
 #pragma unroll
-    for (uint32_t i = 0; i < 8; i++) out[i] = t0 + i < n ? silu_f(out[i]) : 0.f;
+    for (uint32_t i = 0; i < N; i++) out[i] = t0 + i < n ? silu_f(out[i]) : 0.f;
 }
 
-// Eight consecutive tokens t0 .. t0 + 7 (t0 a multiple of 8) of a batch of n, whose first row is y and first position pos0; 0 for
+// N (4 or 8) consecutive tokens t0 .. t0 + N - 1 (t0 a multiple of N) of a batch of n, whose first row is y and first position pos0; 0 for
 // tokens past the end.  Up to eight taps every input is read once, all of them asked for at once.  EXACT: fewer than four taps leave out
-// what lies further back instead of multiplying it by zero, which a value that is not finite survives.
+// what lies further back instead of multiplying it by zero, which a value that is not finite survives.  LONG: there are more than four.
 // us a prompt of width 2048, 4 layers with the delta rule, more than four taps a token at a time and so: 6 taps, 16 tokens 841 and 786, 200
 // 1174 and 1114, 1500 2497 and 2380; 16 taps 1010 and 792, 1329 and 1115, 2840 and 2438.
-template <bool EXACT, class Spec>
-__device__ __forceinline__ void short_conv8(float (&out)[8], const Spec &s, const float *y, size_t ld, uint32_t c, uint32_t pos0, uint32_t t0, uint32_t n)
+template <bool EXACT, bool LONG, int N, class Spec>
+__device__ __forceinline__ void short_conv_run(float (&out)[N], const Spec &s, const float *y, size_t ld, uint32_t c, uint32_t pos0, uint32_t t0, uint32_t n)
 {
-    if (s.taps > 4) return short_conv8_long(out, s, y, ld, c, pos0, t0, n);
+    if constexpr (LONG) return short_conv_long(out, s, y, ld, c, pos0, t0, n);
     const uint32_t at = s.channel_at(c);
     const float b = s.conv_bias(c);
-    float in[11], w[4];      // in[i]: token t0 + i - 3
+    float in[N + 3], w[4];      // in[i]: token t0 + i - 3
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) w[j] = j < s.taps ? s.conv[(size_t)(s.taps - 1 - j) * s.channels() + c] : 0.f;
 #pragma unroll
-    for (uint32_t i = 0; i < 11; i++) {
+    for (uint32_t i = 0; i < N + 3; i++) {
         const uint32_t back = i < 3 ? 3 - i : 0, t = t0 + i - 3;
         in[i] = 0.f;
         if (t0 || !back) {
@@ -111,12 +111,20 @@ __device__ __forceinline__ void short_conv8(float (&out)[8], const Spec &s, cons
         }
     }
 #pragma unroll
-    for (uint32_t i = 0; i < 8; i++) {
+    for (uint32_t i = 0; i < N; i++) {
         float v = fmaf(in[i + 3], w[0], b);
 #pragma unroll
         for (uint32_t j = 1; j < 4; j++) v = !EXACT || j < s.taps ? fmaf(in[i + 3 - j], w[j], v) : v;
         out[i] = t0 + i < n ? silu_f(v) : 0.f;
     }
+}
+
+// eight tokens, however many taps there are
+template <bool EXACT, class Spec>
+__device__ __forceinline__ void short_conv8(float (&out)[8], const Spec &s, const float *y, size_t ld, uint32_t c, uint32_t pos0, uint32_t t0, uint32_t n)
+{
+    if (s.taps > 4) short_conv_run<EXACT, true>(out, s, y, ld, c, pos0, t0, n);
+    else short_conv_run<EXACT, false>(out, s, y, ld, c, pos0, t0, n);
 }
 
 }  // namespace lv
