@@ -201,15 +201,17 @@ int lv_argmax(lv_session *s, uint32_t *token);
 int lv_session_use_graph(lv_session *s, int enable);
 /* How n == 1 steps are executed, and in a session whose path has been set to another than LV_PATH_AUTO also the tokens of
  * steps of 2 to 15 tokens, one after the other (longer ones as batches).  With LV_PATH_AUTO steps of 2 to 256 tokens have
- * kernels of their own where the model's shape allows (q4_0 or q8_0, width and feed-forward width multiples of 128).  The reference has one way (replay the recorded command buffers,
+ * kernels of their own where the model's shape allows (q4_0 or q8_0, width and feed-forward width multiples of 128), above 128 tokens where those take less
+ * time than a batch, and so has what is left of a step behind its batches of 512.  The reference has one way (replay the recorded command buffers,
  * llava_command_buffer.cpp:47-55); here there are three, all computing the same step:
  *   LV_PATH_KERNELS     one launch per operator on the session's stream
  *   LV_PATH_GRAPH       the same launches captured once into a hipGraph and replayed
  *   LV_PATH_PERSISTENT  one persistent kernel for the whole token (LLaMA-7B and -13B layer shapes, q4_0 or q8_0, on a
  *                       256-CU device)
  *   LV_PATH_AUTO        persistent when the model has that form, else graph (or kernels if graphs are off)
- *                       A small model (width up to 1024) left to itself takes one launch of a few workgroups for a token as well, up to
- *                       131072 / head size rows of context; lv_session_path reports the graph path, which it takes otherwise
+ *                       A small model (width up to 1024) left to itself takes one launch of a few workgroups for a token as well where
+ *                       an estimate from its sizes says that it is the faster way, up to 131072 / head size rows of context or fewer;
+ *                       lv_session_path reports the graph path, which it takes otherwise
  * A session stops using the persistent kernel, and lv_session_path reports the graph path (kernels if graphs are off)
  * from then on, when its 256 workgroups cannot all be resident on the device (the step goes on in the other path and succeeds) or when
  * two steps in a row end with an expired hand-over wait (both report LV_ERR_HIP; the step issued again then succeeds).

@@ -307,7 +307,7 @@ __global__ __launch_bounds__(kScanThreads) void delta_scan_kernel(DeltaScanArgs 
 
 // ---- batches in chunks of 16 tokens ---------------------------------------------------------------------------------------
 // The scan above is a chain over tokens, 172 ns each whatever the state's size: 352 us for 2048 tokens and 32 heads of 128 x 128.  In chunks
-// it takes 168: 62 for delta_chunk_kernel, 106 for the chain.  Inside a chunk that starts at state S0, with
+// it takes 186 in a prompt, 78 for delta_chunk_kernel and 108 for the chain (launched back to back, operands in the caches, 62 and 106).  Inside a chunk that starts at state S0, with
 // D(s, t) = g_{s+1} ... g_t per channel,
 //   A[t][s] = (D(s, t) k_s) . k_t for s < t,   B[t][s] = (D(s, t) k_s) . q_t for s <= t
 //   u_t = beta_t (v_t - (D(-1, t) k_t) . S0 - sum_{s<t} A[t][s] u_s)       a triangular system: U = T (V - K' S0)
@@ -336,7 +336,7 @@ struct DeltaChunkArgs {
 };
 
 // grid (heads, chunks).  Bound by the vector units: 240 running products and dots of W a chunk.  Three workgroups a CU need at most 168
-// registers (31 us for 1024 tokens and 32 heads; with two 44).
+// registers (launched back to back, 1024 tokens and 32 heads 31 us, with two 44; 39 in a prompt).
 template <int J>
 __global__ __launch_bounds__(kChunkThreads, J <= 2 ? 3 : 1) void delta_chunk_kernel(DeltaChunkArgs a)
 {

@@ -35,10 +35,11 @@ CHAIN = {"wide heads of 128", "large vocabulary"}
 
 
 @pytest.mark.parametrize("shape", sorted(SHAPES))
-@pytest.mark.parametrize("wtype", ["q4_0", "q8_0", "q4_0 version 1"])
+@pytest.mark.parametrize("wtype", ["q4_0", "q8_0", "q4_0 version 1", "q8_0 table"])
 def test_small_model_tokens_match_oracle_and_chain(lva, orc, ctx, tmp_path, shape, wtype):
     p, c = str(tmp_path / "m.ggml"), SHAPES[shape]
-    lva.write_model(p, wtype=lva.LV_Q8_0 if wtype == "q8_0" else lva.LV_Q4_0, tok_type=lva.LV_Q4_0 if wtype.endswith("1") else lva.LV_F32, seed=31, **c)
+    table = {"1": lva.LV_Q4_0, "e": lva.LV_Q8_0}.get(wtype[-1], lva.LV_F32)       # of embeddings
+    lva.write_model(p, wtype=lva.LV_Q8_0 if wtype.startswith("q8_0") else lva.LV_Q4_0, tok_type=table, seed=31, **c)
     if wtype.endswith("1"):
         gb.convert_to_v1(p, str(tmp_path / "v1.ggml"))
         p = str(tmp_path / "v1.ggml")
