@@ -22,7 +22,7 @@ constexpr int kSmallThreads = 512, kSmallWaves = kSmallThreads / 64;
 constexpr int kSmallDepth = 4;             // tiles in flight a wave
 constexpr uint32_t kSmallMaxDim = 1024;    // two values of a normalised vector a thread
 constexpr uint32_t kSmallMaxFf = 8192;     // floats of LDS
-constexpr uint32_t kSmallMaxWGs = 64;      // each waits for the others: all of them find room beside one another on any device in use
+constexpr uint32_t kSmallMaxWGs = 64;      // each waits for the others: all of them, of four launches at once, find room beside one another
 
 struct SmallLayer {
     MatView wq, wk, wv, wo, w1, w2, w3;

@@ -21,6 +21,9 @@ WIDE = {
     "q4_wide": ("Q4_0", dict(vocab=512, dim=4096, heads=32, layers=1, ff=11008)),
     "q8_wide": ("Q8_0", dict(vocab=512, dim=4096, heads=32, layers=1, ff=11008)),
     "q4_wider": ("Q4_0", dict(vocab=512, dim=5120, heads=40, layers=1, ff=13824)),
+    # a feed-forward at the limit of what goes to the kernel without LDS stages for 17 to 32 tokens: its largest row tiles
+    "q4_tall": ("Q4_0", dict(vocab=512, dim=384, heads=12, layers=1, ff=8320)),
+    "q8_tall": ("Q8_0", dict(vocab=512, dim=384, heads=6, layers=1, ff=5376)),
 }
 
 
