@@ -13,12 +13,16 @@
 // Tiles, K step 64, both operands in LDS by direct loads, four waves:
 //   gemm_bf16_kernel        128 rows x 128 tokens, waves of 64 x 64, two stages, two workgroups a CU: few tiles, and short K
 //   gemm_wide_kernel<64>    256 rows x 128 tokens, waves of 128 x 64, three stages, one workgroup a CU
+//   gemm_wide_kernel<80>    256 rows x 160 tokens, waves of 128 x 80, three stages
+//   gemm_wide_kernel<96>    256 rows x 192 tokens, waves of 128 x 96, two stages
 //   gemm_wide_kernel<128>   256 rows x 256 tokens, waves of 128 x 128 (all 256 accumulation registers), two stages
+// Several widths, since what a product of some hundred tokens loses is the last round of tiles and the last tile's empty columns: 777
+// tokens x 22016 rows are 602 tiles of 128 (2.4 rounds of 256 CUs, three paid for) or 430 of 160 (1.7 rounds).
 // A 64 x 64 wave reads 8 KB of LDS per 16 matrix instructions, as long as those take, and the direct loads write LDS as well: LDS
 // bounds it at three quarters of the matrix rate.  Larger waves read 6 or 4 KB.  One wave per SIMD hides nothing by itself: the
 // wide kernels spell the order out, the next half step's operand reads and the direct loads one by one between the products.
-// Measured, us (TFLOP/s): 2048 tokens x 22016 x 4096 468 (788), 392 (943), 355 (1040); x 13600 x 4096 313, 263, 235; x 4096 x 8192
-// 153, 138, 189; 777 x 22016 x 4096 211, 191, 214; 777 x 4096 x 11008 147, 156, 235.
+// Measured, us (TFLOP/s): 2048 tokens x 13600 x 4096 240 (952), 239 (957), 196 (1165); x 4096 x 8192
+// 130, 116, 154 (128 x 128, 256 x 128 and 256 x 256; all five: bf_plan).
 // A row of a tile is 128 bytes; its eight 16-byte chunks are stored in the order chunk ^ (row % 8), so that the 16 rows an MFMA
 // operand reads at one k spread over all banks.
 #pragma once
@@ -125,6 +129,7 @@ struct BfGemmArgs {
     const uint32_t *slots;   // position in expert order -> token * top + choice
     const float *weights;    // [token * top + choice]
     uint32_t top, expert_rows;   // weight rows from one expert to the next
+    bool by_expert;          // order of the tiles: an expert after the other, not a row tile after the other
     bool gather;             // x rows are tokens (slots[position] / top), otherwise positions
     void *act;               // kEpGlu, kEpDense, kEpHeads output [position][lda]
     uint32_t lda;
@@ -214,24 +219,28 @@ __device__ __forceinline__ void bf_store_glu(const BfGemmArgs &a, uint32_t posit
     else *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
-// Tile of this workgroup: workgroups are dealt to the 8 XCDs in turn; the tiles, token tiles of one row tile one after the other, are
-// cut in eight runs of one length, one for each XCD, so that an XCD reads a weight tile into its L2 once and all have as much to do
-// (row tiles dealt in turn: 73 of them x 7 token tiles are 70 for one XCD and 63 for the others, three rounds instead of two).
+// Tile of this workgroup: workgroups are dealt to the 8 XCDs in turn; the tiles are cut in eight runs of one length, one for each XCD, so
+// that all have as much to do (row tiles dealt in turn: 73 of them x 7 token tiles are 70 for one XCD and 63 for the others, three rounds
+// instead of two).  A run goes through the token tiles of one row tile after the other, so that an XCD reads a weight tile into its L2
+// once (the batch's rest behind all whole tiles instead, to fill gaps: 777 x 18560 x 4096 122 -> 129 us).
+// by_expert: through the row tiles of one token tile after the other.  An expert's token tiles read its weights at one time, gathered
+// activations come from L2 as well; but experts that are chosen unevenly then make unequal runs.
 template <bool GROUPED>
 __device__ __forceinline__ bool bf_tile(const BfGemmArgs &a, uint32_t tile_tokens, uint32_t &rt, uint32_t &expert, uint32_t &first, uint32_t &count)
 {
     const uint32_t tt_count = GROUPED ? a.tiles[0] : a.token_tiles, all = a.row_tiles * tt_count, run = (all + 7) / 8, q = blockIdx.x >> 3;
     const uint32_t at = (blockIdx.x & 7) * run + q;
     if (q >= run || at >= all) return false;
-    rt = at / tt_count;
-    const uint32_t tt = at % tt_count;
     if constexpr (GROUPED) {
+        const uint32_t inner = a.by_expert ? a.row_tiles : tt_count, o = at / inner, i = at - o * inner, tt = a.by_expert ? o : i;
+        rt = a.by_expert ? i : o;
         expert = a.tiles[1 + 3 * tt];
         first = a.tiles[2 + 3 * tt];
         count = a.tiles[3 + 3 * tt];
     } else {
+        rt = at / tt_count;
         expert = 0;
-        first = tt * tile_tokens;
+        first = (at - rt * tt_count) * tile_tokens;
         count = min(tile_tokens, a.n - first);
     }
     return true;
@@ -277,14 +286,14 @@ __device__ __forceinline__ void bf_store_wave(const BfGemmArgs &a, const lv_f4 (
     }
 }
 
-template <int EP, bool GROUPED>
+template <int EP>
 __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(BfGemmArgs a)
 {
     constexpr int RM = kBfRows, STAGE = (RM + kBfTile) * kBfStep * 2;
     constexpr int LW = RM / 32, LX = kBfTile / 32;          // direct loads per wave and stage, 8 rows (1 KB) each
     extern __shared__ __attribute__((aligned(128))) uint8_t bf_lds[];
     uint32_t rt, expert, first, count;
-    if (!bf_tile<GROUPED>(a, kBfTile, rt, expert, first, count)) return;
+    if (!bf_tile<false>(a, kBfTile, rt, expert, first, count)) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, g4 = lane >> 4;
     const uint32_t kp = a.kp;
@@ -292,16 +301,11 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(BfGemmArgs a)
     const uint16_t *gw, *gx[LX];
     {
         const int r8 = lane >> 3, c = (lane & 7) ^ r8;
-        gw = a.w + ((size_t)expert * a.expert_rows + (size_t)rt * RM + wave * (RM / 4) + r8) * kp + c * 8;
+        gw = a.w + ((size_t)rt * RM + wave * (RM / 4) + r8) * kp + c * 8;
 #pragma unroll
         for (int i = 0; i < LX; i++) {
             const int row = wave * (kBfTile / 4) + i * 8 + r8;
-            size_t xr = (size_t)first + row;
-            if constexpr (GROUPED) {
-                const uint32_t p = first + min((uint32_t)row, count - 1);
-                xr = a.gather ? a.slots[p] / a.top : p;
-            }
-            gx[i] = static_cast<const uint16_t *>(a.x) + xr * a.ldx + c * 8;
+            gx[i] = static_cast<const uint16_t *>(a.x) + ((size_t)first + row) * a.ldx + c * 8;
         }
     }
     const uint32_t k_lo = EP == kEpStore && a.k_slice ? blockIdx.z * a.k_slice : 0;
@@ -353,8 +357,10 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(BfGemmArgs a)
 }
 
 constexpr int wide_tokens(int wn) { return 2 * wn; }
-constexpr int wide_stages(int wn) { return wn == 64 ? 3 : 2; }
-constexpr int wide_lds_bytes(int wn) { return wide_stages(wn) * (256 + wide_tokens(wn)) * kBfStep * 2; }
+constexpr int wide_stages(int wn) { return wn <= 80 ? 3 : 2; }
+constexpr int wide_stage_bytes(int wn) { return wide_stages(wn) * (256 + wide_tokens(wn)) * kBfStep * 2; }
+// the three stages of a rest of 160 tokens are more than two of 192
+constexpr int wide_lds_bytes(int wn) { return wn == 96 ? wide_stage_bytes(80) : wide_stage_bytes(wn); }
 
 // c += a b; IN_ACC: c in accumulation registers, where the compiler would move them to and fro around every product.  The compiler
 // does not know of these products what has to lie between them and moves of their registers.  It may have moves around a half of a K
@@ -371,16 +377,16 @@ __device__ __forceinline__ void wide_product(lv_f4 &c, const lv_bf8 &a, const lv
     } else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// 256 rows x 2 WN tokens, waves of 128 x WN
-template <int EP, bool GROUPED, int WN>
-__global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemmArgs a)
+// one tile of 256 rows x 2 WN tokens, waves of 128 x WN
+template <int EP, bool GROUPED, int WN, bool IN_ACC>
+__device__ __forceinline__ void wide_tile(const BfGemmArgs &a, uint32_t rt, uint32_t expert, uint32_t first, uint32_t count)
 {
     constexpr int TN = wide_tokens(WN), NST = wide_stages(WN), STAGE = (256 + TN) * kBfStep * 2, NJ = WN / 16;
     constexpr int LW = 8, LX = TN / 32, LPS = LW + LX;      // direct loads per wave and stage, 8 rows (1 KB) each
     constexpr int NM = 8 * NJ, NR = 8 + NJ;                 // products and operand reads of half a step
+    constexpr int RP = (NR + NM / 2 - 1) / (NM / 2), LP = (LPS + NM / 2 - 1) / (NM / 2);    // reads, loads between two products
+    constexpr int LD = NM / LPS;
     extern __shared__ __attribute__((aligned(128))) uint8_t bf_lds[];
-    uint32_t rt, expert, first, count;
-    if (!bf_tile<GROUPED>(a, TN, rt, expert, first, count)) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, g4 = lane >> 4;
     const uint32_t kp = a.kp;
@@ -396,7 +402,7 @@ __global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemm
             if constexpr (GROUPED) {
                 const uint32_t p = first + min((uint32_t)row, count - 1);
                 xr = a.gather ? a.slots[p] / a.top : p;
-            } else if constexpr (TN > kBfTile) {            // activations end at a multiple of kBfTile
+            } else if constexpr (TN > 192) {            // activations end at a multiple of kBfTile
                 xr = first + min((uint32_t)row, (count + kBfTile - 1) / kBfTile * kBfTile - 1);
             }
             gx[i] = static_cast<const uint16_t *>(a.x) + xr * a.ldx + c * 8;
@@ -440,9 +446,11 @@ __global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemm
         // first half: with three stages the loads of stage s + 2 go where stage s - 1 was
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f0.a[m / NJ], f0.b[m % NJ], m == 0, m == NM - 1);
-            if (m % 2 == 0 && m / 2 < NR) read_one(f1, bf_lds + slot * STAGE, 1, m / 2);
-            if (NST == 3 && m % 2 == 1 && m / 2 < LPS) issue_one(s + 2, free_slot, m / 2);
+            wide_product<IN_ACC>(acc[m / NJ][m % NJ], f0.a[m / NJ], f0.b[m % NJ], m == 0, m == NM - 1);
+#pragma unroll
+            for (int r = m / 2 * RP; m % 2 == 0 && r < (m / 2 + 1) * RP && r < NR; r++) read_one(f1, bf_lds + slot * STAGE, 1, r);
+#pragma unroll
+            for (int p = m / 2 * LP; NST == 3 && m % 2 == 1 && p < (m / 2 + 1) * LP && p < LPS; p++) issue_one(s + 2, free_slot, p);
             __builtin_amdgcn_sched_barrier(0);
         }
         // This wave's loads of stage s + 1 have landed and it holds the rest of stage s in registers; behind the barrier that
@@ -453,15 +461,36 @@ __global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemm
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            wide_product<(WN > 64)>(acc[m / NJ][m % NJ], f1.a[m / NJ], f1.b[m % NJ], m == 0, m == NM - 1);
-            if (m % 2 == 0 && m / 2 < NR) read_one(f0, bf_lds + next * STAGE, 0, m / 2);
-            if (NST == 2 && m % 4 == 1 && m / 4 < LPS) issue_one(s + 2, free_slot, m / 4);
+            wide_product<IN_ACC>(acc[m / NJ][m % NJ], f1.a[m / NJ], f1.b[m % NJ], m == 0, m == NM - 1);
+#pragma unroll
+            for (int r = m / 2 * RP; m % 2 == 0 && r < (m / 2 + 1) * RP && r < NR; r++) read_one(f0, bf_lds + next * STAGE, 0, r);
+            if (NST == 2 && m % LD == 1 && m / LD < LPS) issue_one(s + 2, free_slot, m / LD);
             __builtin_amdgcn_sched_barrier(0);
         }
         slot = next;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the repeats have landed before the workgroup gives up its LDS
     bf_store_wave<EP>(a, acc, rt * 256 + wm * 128, wn * WN, first, count);
+}
+
+// 256 rows x 2 WN tokens.  Below 128 a tile of fewer tokens, an expert's or the batch's last one, takes as many products and loads as they
+// need, in units of 32 tokens.
+template <int EP, bool GROUPED, int WN>
+__global__ __launch_bounds__(256, WN == 64 ? 2 : 1) void gemm_wide_kernel(BfGemmArgs a)
+{
+    constexpr bool IN_ACC = WN > 64;
+    uint32_t rt, expert, first, count;
+    if (!bf_tile<GROUPED>(a, wide_tokens(WN), rt, expert, first, count)) return;
+    if constexpr (WN < 128) {
+        if (count <= 32) return wide_tile<EP, GROUPED, 16, IN_ACC>(a, rt, expert, first, count);
+        if (count <= 64) return wide_tile<EP, GROUPED, 32, IN_ACC>(a, rt, expert, first, count);
+        if (count <= 96) return wide_tile<EP, GROUPED, 48, IN_ACC>(a, rt, expert, first, count);
+        if constexpr (WN > 64)
+            if (count <= 128) return wide_tile<EP, GROUPED, 64, IN_ACC>(a, rt, expert, first, count);
+        if constexpr (WN > 80)
+            if (count <= 160) return wide_tile<EP, GROUPED, 80, IN_ACC>(a, rt, expert, first, count);
+    }
+    wide_tile<EP, GROUPED, WN, IN_ACC>(a, rt, expert, first, count);
 }
 
 constexpr int kF32Tile = 64;

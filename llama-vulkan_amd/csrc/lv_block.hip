@@ -817,35 +817,72 @@ template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs 
 
 // Which tiles a bf16 product takes, and into how many slices of K it is cut (`slices` at most; the reader of the result adds them up).
 // Time = rounds of workgroups over 256 CUs x K steps x a step's time, plus prologue and epilogue, plus writing and reading a slice more.
-// Measured us a step of 64: 128 x 128 tiles 1.22 where two share a CU, 0.85 alone; 256 x 128 1.02; 256 x 256 1.85, 1.45 where half of
-// the CUs have none.
-enum class BfTiles { k128, kWide, kWidest };
+// Fitted to launches whose weights come from HBM, as a model's do.  us, 128 x 128 tiles and 256 rows x 128, 160, 192 and 256 tokens:
+// 16 x 8848 x 2048 29 25 26 26 46; 100 x 8848 x 2048 32 35 35 35 52; 300 x 22016 x 4096 109 89 78 69 95; 500 x 18560 x 4096 135 124 135 80 108;
+// 777 x 22016 x 4096 193 159 148 145 191; 777 x 18560 x 4096 144 126 157 155 209; 777 x 2112 x 4096 57 53 76 72 101; 777 x 4096 x 11008 in two
+// slices 93 82 109 96 137, in three 124 106 82 79 101; 1000 x 8848 x 2048 63 66 45 46 62; 1100 x 18560 x 4096 204 187 168 174 210;
+// 1900 x 22016 x 4096 346 328 335 324 294; 2048 x 13600 x 4096 279 250 234 244 217; 2048 x 4096 x 8192 144 123 133 130 187.
+enum class BfTiles { k128, kWide, kWide160, kWide192, kWidest };
 struct BfPlan {
     BfTiles tiles;
     uint32_t slices;
 };
-static BfPlan bf_plan(uint32_t rows, uint32_t n, uint32_t token_tiles, uint32_t kp, bool grouped, uint32_t slices)
+static BfPlan bf_plan(uint32_t rows, uint32_t n, uint32_t kp, uint32_t slices)
 {
+    constexpr double kCus = 256;
+    struct Offer {
+        BfTiles tiles;
+        uint32_t tokens;
+        double busy, idle;      // us of a step, every CU at work and few of them
+    };
+    constexpr Offer offers[] = {{BfTiles::kWide, 128, 0.95, 0.75}, {BfTiles::kWide160, 160, 1.20, 1.00}, {BfTiles::kWide192, 192, 1.33, 0.98}, {BfTiles::kWidest, 256, 1.60, 1.42}};
     BfPlan best{BfTiles::k128, 1};
     double best_us = 1e30;
     for (uint32_t s = 1; s <= slices; s++) {
         const uint32_t steps = (kp / kBfStep + s - 1) / s;
         if (s > 1 && steps < 8) break;
-        const double more = 4.0 + (s - 1) * (1.0 + 2e-6 * n * rows);
-        auto offer = [&](BfTiles t, uint64_t tiles, double step_us) {
+        const double more = 8.0 + (s - 1) * (1.0 + 2e-6 * n * rows);
+        auto take = [&](BfTiles t, double step_us) {
             const double us = step_us * steps + more;
-            if (tiles && us < best_us) {
+            if (us < best_us) {
                 best_us = us;
                 best = {t, s};
             }
         };
-        const uint64_t small = (uint64_t)((rows + 127) / 128) * token_tiles * s, wide = (uint64_t)((rows + 255) / 256) * token_tiles * s;
-        const uint64_t widest = grouped ? 0 : (uint64_t)((rows + 255) / 256) * ((n + 255) / 256) * s;
-        offer(BfTiles::k128, small, small / 512 * 1.22 + (small % 512 > 256 ? 1.22 : small % 512 ? 0.85 : 0.0));
-        offer(BfTiles::kWide, wide, (double)((wide + 255) / 256) * 1.02);
-        offer(BfTiles::kWidest, widest, widest <= 128 ? 1.45 : (double)((widest + 255) / 256) * 1.85);
+        // two share a CU
+        const double small = (double)((rows + 127) / 128) * ((n + 127) / 128) * s, left = std::fmod(small, 2 * kCus);
+        take(BfTiles::k128, std::floor(small / (2 * kCus)) * 1.05 + (left > kCus ? 0.95 + 0.1 * left / kCus : left ? 0.78 : 0.0));
+        for (const Offer &o : offers) {
+            const uint32_t whole = n / o.tokens, rest = n % o.tokens;
+            // the batch's rest: what its loads take whatever its tokens, and its products
+            const double part = !rest ? 0.0 : o.tiles == BfTiles::kWidest ? 1.0 : 0.6 + 0.4 * ((rest + 31) / 32 * 32) / o.tokens;
+            const uint32_t token_tiles = whole + (rest != 0);
+            const double tiles = (double)((rows + 255) / 256) * token_tiles * s, last = std::fmod(tiles, kCus);
+            take(o.tiles, (std::floor(tiles / kCus) * o.busy + (last ? o.idle + (o.busy - o.idle) * last / kCus : 0.0)) * (whole + part) / token_tiles);
+        }
     }
     return best;
+}
+
+// Tokens of an expert's tiles, 128 or 160, and their order.  us of gate and up, and of down (64 experts, 8 a token, 2048 x 4096 and
+// 4096 x 1024): tiles of 128, a row tile after the other, then an expert after the other; tiles of 160 likewise.
+//    300 tokens            239 180 241 179   127 121 127 121
+//    900                   273 240 265 199   168 170 166 161
+//   1400                   280 250 327 310   227 198 228 221
+//   2048                   372 356 329 309   259 281 270 242
+//    600, unevenly chosen  226 214 226 219   136 142 133 148
+//   2048, unevenly chosen  356 364 344 372   272 282 257 279
+// Few tokens an expert: the weights' way from HBM counts, an expert after the other; 160 where an expert of the mean number of choices
+// and two standard deviations more then has fewer tiles.  Many: runs of one length whoever is chosen.
+struct ExpertPlan {
+    uint32_t tile;
+    bool by_expert;
+};
+static ExpertPlan expert_plan(uint32_t n, uint32_t top, uint32_t experts)
+{
+    const double mean = (double)n * top / experts, many = mean + 2 * std::sqrt(mean);
+    if (mean >= 192) return {160, false};
+    return {std::ceil(many / 160) < std::ceil(many / 128) ? 160u : 128u, true};
 }
 
 template <class K> static int launch_bf(hipStream_t st, K *k, const BfGemmArgs &a, int lds)
@@ -856,9 +893,19 @@ template <class K> static int launch_bf(hipStream_t st, K *k, const BfGemmArgs &
     return LV_OK;
 }
 
-template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t experts = 1, BfTiles tiles = BfTiles::k128, bool planned = false)
+template <int EP, bool GROUPED, int WN> static int launch_wide(hipStream_t st, BfGemmArgs a)
 {
-    const uint32_t tile = f32 ? kF32Tile : kBfTile, token_tiles = (n + tile - 1) / tile;
+    constexpr uint32_t tokens = wide_tokens(WN);
+    a.row_tiles = (a.rows + 255) / 256;
+    if (!GROUPED) a.token_tiles = (a.n + tokens - 1) / tokens;
+    return launch_bf(st, &gemm_wide_kernel<EP, GROUPED, WN>, a, wide_lds_bytes(WN));
+}
+
+// a product of n tokens.  `plan`: its tiles where they are settled already.  Grouped: `tile` tokens at most a tile of the list
+template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t experts = 1, uint32_t tile = kBfTile, const BfTiles *plan = nullptr)
+{
+    if (f32) tile = kF32Tile;
+    const uint32_t token_tiles = (n + tile - 1) / tile;
     a.w = w.w;
     a.kp = w.kp;
     a.rows = w.rows;
@@ -870,27 +917,26 @@ template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemm
         HIP_TRY(hipGetLastError());
         return LV_OK;
     }
-    if constexpr (EP != kEpDecay && EP != kEpSigmoid) {      // those two have a few K steps only
-        // grouped: about half of the experts end in a tile of their own
-        if (!planned && !a.k_slice) tiles = bf_plan(w.rows, n, GROUPED ? std::max(token_tiles + experts / 2, 1u) : token_tiles, w.kp, GROUPED, 1).tiles;
-        if (tiles != BfTiles::k128) {
-            a.row_tiles = (w.rows + 255) / 256;
-            if constexpr (!GROUPED) {
-                if (tiles == BfTiles::kWidest) {
-                    a.token_tiles = (n + wide_tokens(128) - 1) / wide_tokens(128);
-                    return launch_bf(st, &gemm_wide_kernel<EP, false, 128>, a, wide_lds_bytes(128));
-                }
+    if constexpr (GROUPED) {
+        return tile == kBfTile ? launch_wide<EP, true, 64>(st, a) : launch_wide<EP, true, 80>(st, a);
+    } else {
+        if constexpr (EP != kEpDecay && EP != kEpSigmoid) {      // those two have a few K steps only
+            switch (plan ? *plan : a.k_slice ? BfTiles::k128 : bf_plan(w.rows, n, w.kp, 1).tiles) {
+            case BfTiles::kWide: return launch_wide<EP, false, 64>(st, a);
+            case BfTiles::kWide160: return launch_wide<EP, false, 80>(st, a);
+            case BfTiles::kWide192: return launch_wide<EP, false, 96>(st, a);
+            case BfTiles::kWidest: return launch_wide<EP, false, 128>(st, a);
+            case BfTiles::k128: break;
             }
-            return launch_bf(st, &gemm_wide_kernel<EP, GROUPED, 64>, a, wide_lds_bytes(64));
         }
+        a.row_tiles = (w.rows + kBfRows - 1) / kBfRows;
+        return launch_bf(st, &gemm_bf16_kernel<EP>, a, kBfLdsBytes);
     }
-    a.row_tiles = (w.rows + kBfRows - 1) / kBfRows;
-    return launch_bf(st, &gemm_bf16_kernel<EP, GROUPED>, a, kBfLdsBytes);
 }
 
 // of a product into the sublayer outputs, by its sizes alone: the same tokens are summed in the same order whatever the session has
 // evaluated before.  More than 1024 tokens have tiles enough without slices.
-static BfPlan output_plan(const BfMatrix &w, uint32_t n, uint32_t slices = kOutSlices) { return bf_plan(w.rows, n, (n + kBfTile - 1) / kBfTile, w.kp, false, n <= 1024 ? slices : 1); }
+static BfPlan output_plan(const BfMatrix &w, uint32_t n, uint32_t slices = kOutSlices) { return bf_plan(w.rows, n, w.kp, n <= 1024 ? slices : 1); }
 
 // a product into the sublayer outputs `y` ([token][slice][dp], room for `room` vectors), cut in slices of K where its tiles would leave
 // CUs without work; *slices: how many the next norm has to add up
@@ -905,7 +951,7 @@ static int gemm_output(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w
     }
     a.ldo = dp * p.slices;
     *slices = p.slices;
-    return gemm<kEpStore, false>(st, f32, a, w, n, 1, p.tiles, true);
+    return gemm<kEpStore, false>(st, f32, a, w, n, 1, kBfTile, &p.tiles);
 }
 
 // calls fn(element, integral constant DP, integral constant R) for a layer's attention
@@ -1357,7 +1403,7 @@ static int workspace_reserve(BlockSession *s, uint32_t n)
     LV_TRY(dev_zeroed(st, &w.ids, T * 4 * top));
     LV_TRY(dev_zeroed(st, &w.slots, T * 4 * top));
     LV_TRY(dev_zeroed(st, &w.tiles, 4 * (1 + 3 * (T * top / kF32Tile + experts + 1))));
-    // a tile of 128 positions may start at any of the T * top
+    // a tile of positions may start at any of the T * top
     LV_TRY(dev_zeroed(st, &w.ff, E * mx([&](const BlockLayer &l) { return (cap * std::max(1u, l.spec.moe.top) + 128) * l.down.kp; })));
     w.cap = cap;
     return outputs_reserve(s, n);
@@ -1671,15 +1717,17 @@ static int step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx
         LV_TRY((gemm<kEpStore, false>(st, f32, rt, l.router, n)));
         route_rows_kernel<<<dim3(n), dim3(64), e.experts * 4ull, st>>>(w.z, ldz, z_parts, rt.slice_floats, e.experts, e.top, w.ids, w.scores);
         HIP_TRY(hipGetLastError());
-        sort_experts_kernel<<<dim3(1), dim3(1024), e.experts * 8ull, st>>>(w.ids, total, e.experts, f32 ? kF32Tile : kBfTile, w.slots, w.tiles);
+        const ExpertPlan plan = f32 ? ExpertPlan{kF32Tile, false} : expert_plan(n, e.top, e.experts);
+        sort_experts_kernel<<<dim3(1), dim3(1024), e.experts * 8ull, st>>>(w.ids, total, e.experts, plan.tile, w.slots, w.tiles);
         HIP_TRY(hipGetLastError());
         BfGemmArgs gu{};
-        gu.x = w.act; gu.ldx = Dp; gu.tiles = w.tiles; gu.slots = w.slots; gu.weights = w.scores; gu.top = e.top; gu.expert_rows = l.gu_rows; gu.gather = true;
+        gu.x = w.act; gu.ldx = Dp; gu.tiles = w.tiles; gu.slots = w.slots; gu.weights = w.scores; gu.top = e.top; gu.expert_rows = l.gu_rows; gu.gather = true; gu.by_expert = plan.by_expert;
         gu.act = w.ff; gu.lda = l.down.kp;
-        LV_TRY((gemm<kEpGlu, true>(st, f32, gu, l.gate_up, total, e.experts)));
+        LV_TRY((gemm<kEpGlu, true>(st, f32, gu, l.gate_up, total, e.experts, plan.tile)));
         BfGemmArgs dn{};
         dn.x = w.ff; dn.ldx = l.down.kp; dn.tiles = w.tiles; dn.slots = w.slots; dn.top = e.top; dn.expert_rows = l.down_rows; dn.out = w.y; dn.ldo = Dp;
-        LV_TRY((gemm<kEpScatter, true>(st, f32, dn, l.down, total, e.experts)));
+        dn.by_expert = plan.by_expert;
+        LV_TRY((gemm<kEpScatter, true>(st, f32, dn, l.down, total, e.experts, plan.tile)));
         parts = e.top;
     }
     if (trace || logits_all) {

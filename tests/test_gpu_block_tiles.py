@@ -42,6 +42,10 @@ DENSE = [(40, 4100, 1100), (130, 2060, 1030), (700, 2060, 1025), (700, 4100, 128
          (1030, 3000, 255), (128, 2048, 513), (129, 1025, 65)]
 # 128 x 128 tiles in 3 slices; 256 x 128 in 1, 2, 3 and 4; 256 x 256 in 3; the last slice shorter
 DENSE += [(1536, 2500, 700), (4100, 1100, 900), (3000, 2060, 900), (2500, 2500, 777), (1536, 3000, 900), (4100, 3000, 900)]
+# 256 rows x 160 and x 192 tokens, every number of units of 32 tokens that a rest may have, one token beside a unit's end; 160 in two slices
+DENSE += [(70, 5500, 641), (70, 7000, 513), (70, 8200, 385), (70, 11008, 257), (70, 8200, 449), (70, 4100, 960)]
+DENSE += [(70, 10240, 961), (70, 5500, 801), (70, 7000, 641), (70, 11008, 289), (70, 11008, 321), (70, 11008, 353)]
+DENSE += [(4102, 2500, 897)]
 # streams so wide that the sum of slices and the norm's input would not fit LDS side by side
 DENSE += [(20544, 1152, 33)]
 
@@ -72,7 +76,8 @@ def test_slices_do_not_hang_on_what_came_before(lva, ctx):
             assert np.array_equal(d.run(toks, (n,)), first), n
 
 
-@pytest.mark.parametrize("width,ff,n,experts,top", [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4), (64, 24, 17, 3, 2)])
+@pytest.mark.parametrize("width,ff,n,experts,top", [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4), (64, 24, 17, 3, 2),
+                                                      (130, 520, 230, 4, 2), (70, 300, 375, 3, 2)])      # tiles of 160 tokens
 def test_expert_tiles(lva, ctx, width, ff, n, experts, top):
     cfg = bb.config(width=width, layers=[bb.layer(experts=experts, top=top, ff=ff)])
     W = bb.weights(cfg, seed=n)

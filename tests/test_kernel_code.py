@@ -66,3 +66,28 @@ def test_nothing_moves_between_matrix_products_in_inline_assembly(code_objects):
             assert [x for x in inside if not re.match(allowed, x)] == [], name
             assert re.match(r"s_nop [1-9]", ins[half[0] - 1]), (name, ins[half[0] - 1])
             assert ins[half[-1] + 1] == "s_nop 15", (name, ins[half[-1] + 1])
+
+
+def test_nothing_moves_between_matrix_products_of_tiles_with_units(code_objects):
+    """the same of the tiles of 160 and 192 tokens, whose kernels hold a loop for every number of units of 32 tokens"""
+    allowed = r"v_mfma_f32_16x16x32_bf16 a\[|ds_read_b128 v\[|global_load_lds_dwordx4|s_|v_(lshl_add_u64|add3_u32|add_u32_e32|add_co_u32|addc_co_u32|lshlrev_b64|mad_u64_u32)"
+    seen = 0
+    for f in code_objects:
+        text = subprocess.run([tool("llvm-objdump"), "-d", "--no-show-raw-insn", f], check=True, capture_output=True, text=True).stdout
+        parts = re.split(r"\n[0-9a-f]+ <(\S+)>:\n", text)
+        for name, body in zip(parts[1::2], parts[2::2]):
+            if "gemm_wide_kernel" not in name or not re.search(r"ELi(80|96)E", name):
+                continue
+            seen += 1
+            ins = [line.split("//")[0].strip() for line in body.split("\n") if line.strip()]
+            halves, inside = 0, False
+            for i, x in enumerate(ins):
+                if "mfma" in x and not inside:
+                    assert re.match(r"s_nop [1-9]", ins[i - 1]), (name, ins[i - 1])
+                    inside = True
+                if inside:
+                    assert re.match(allowed, x), (name, x)
+                    if x == "s_nop 15":
+                        inside, halves = False, halves + 1
+            assert not inside and halves == 2 * (5 if "ELi80E" in name else 6), (name, halves)
+    assert seen == 8      # three epilogues of each, and of 160 tokens the experts' two
