@@ -2378,7 +2378,9 @@ constexpr uint32_t kShortSplits = 16;      // parts the attention's positions ar
 
 struct ShortBuffers {
     float *x, *q, *parts[kShortSlices], *xscale, *num, *den;
-    uint8_t *act, *ff;
+    uint8_t *act, *act2, *ff;      // act2: of a product behind a norm, while others still read act
+    float2 *stats;
+    uint32_t *counters;
 };
 static size_t short_layout(const lv_hparams &hp, uint8_t *base, ShortBuffers *b)
 {
@@ -2393,6 +2395,9 @@ static size_t short_layout(const lv_hparams &hp, uint8_t *base, ShortBuffers *b)
     b->den = (float *)take((size_t)kShortTokens * hp.heads * kShortSplits * 4);
     b->act = take(short_act_bytes(hp.dim, kShortTokens));
     b->ff = take(short_act_bytes(hp.ff, kShortTokens));
+    b->act2 = take(short_act_bytes(hp.dim, kShortExact));
+    b->stats = (float2 *)take((size_t)(hp.dim / 32) * kShortExact * 8);
+    b->counters = (uint32_t *)take((size_t)(hp.dim / 32) * 4);
     return at;
 }
 
@@ -2401,8 +2406,14 @@ static bool short_reserve(lv_session *s)
 {
     if (s->short_ws) return true;
     ShortBuffers b;
-    if (hipMalloc(reinterpret_cast<void **>(&s->short_ws), short_layout(s->model->hp, nullptr, &b)) == hipSuccess) return true;
-    (void)hipGetLastError();
+    if (hipMalloc(reinterpret_cast<void **>(&s->short_ws), short_layout(s->model->hp, nullptr, &b)) != hipSuccess) {
+        (void)hipGetLastError();
+        s->short_ws = nullptr;
+        return false;
+    }
+    short_layout(s->model->hp, s->short_ws, &b);
+    if (zero_async(b.counters, (uint64_t)(s->model->hp.dim / 32) * 4, s->stream) == LV_OK) return true;
+    (void)hipFree(s->short_ws);
     s->short_ws = nullptr;
     return false;
 }
@@ -2448,7 +2459,7 @@ static void short_plan(uint32_t tiles, uint32_t nb, uint32_t T, int qt, bool sli
     }
 }
 
-static int launch_short_gemm(hipStream_t st, ShortArgs a, uint32_t ftype, bool sf32, bool sliced, uint32_t *slices_out = nullptr)
+static int launch_short_gemm(hipStream_t st, ShortArgs a, uint32_t ftype, bool sf32, bool sliced, uint32_t *slices_out = nullptr, uint32_t *rows_out = nullptr)
 {
     const uint32_t T = short_tiles(a.n);
     const int qt = ftype == LV_Q4_0 ? 4 : 8;
@@ -2457,6 +2468,7 @@ static int launch_short_gemm(hipStream_t st, ShortArgs a, uint32_t ftype, bool s
     short_plan(a.tiles, a.nb, T, qt, sliced, &rt, &a.slice_chunks);
     const uint32_t slices = (a.nb / 4 + a.slice_chunks - 1) / a.slice_chunks;
     if (slices_out) *slices_out = slices;
+    if (rows_out) *rows_out = rt * 16;
 #define LV_SHORT(QT, TT) case QT * 8 + TT: launch_short_rows<QT, TT>(st, a, rt, slices, sf32); break;
     switch (qt * 8 + T) {
         LV_SHORT(4, 0) LV_SHORT(4, 1) LV_SHORT(4, 2) LV_SHORT(4, 3) LV_SHORT(4, 4)
@@ -2796,7 +2808,7 @@ static int record_short_head(lv_session *s, const ShortBuffers &b, uint32_t idx0
         }
     } else if (all || with_head) {
         // only the last row's logits are ever read (llava_session.cpp:131-139), unless all are asked for
-        LV_TRY(launch_gemm_reduce(st, b.x, D, parts, pending, D, n, true));
+        if (pending) LV_TRY(launch_gemm_reduce(st, b.x, D, parts, pending, D, n, true));
         const uint32_t first = all ? 0 : n - 1, rows = n - first;
         normalize_kernel<<<dim3(rows), dim3(256), 0, st>>>(b.q, b.x + (size_t)first * D, m->norm, D);
         HIP_TRY(hipGetLastError());
@@ -2895,13 +2907,21 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
     LV_TRY(launch_embed(s, b.x, s->cfg_host + 1, s->cfg_host[0], idx0, n));
     HIP_TRY(hipGetLastError());
 
-    uint32_t pending = 0;       // K slices in b.parts that the next norm adds to the residual stream
     if (!short_exact(short_tiles(n))) return record_short_halves(s, b, idx0, n, pos, with_head, row_base);
+    // The output projections leave the residual stream, its activations and its statistics behind: a norm of its own is needed for the
+    // first layer only.
+    ShortBuffers first = b;
+    first.act = b.act2;
+    LV_TRY(launch_short_norm(st, first, m->layers[0].attn_norm, n, D, 0, ft));
+    uint32_t stat_rows = 0;
+    const auto behind_norm = [&](ShortArgs &a) {
+        a.x = b.act2; a.n = n; a.nb = D / 32; a.dim = D;
+        if (stat_rows) { a.stats = b.stats; a.stat_rows = stat_rows; a.stat_groups = (D + stat_rows - 1) / stat_rows; }
+    };
     for (uint32_t li = 0; li < hp.layers; li++) {
         const LayerWeights &lw = m->layers[li];
-        LV_TRY(launch_short_norm(st, b, lw.attn_norm, n, D, pending, ft));
         ShortArgs a{};
-        a.x = b.act; a.n = n; a.nb = D / 32;
+        behind_norm(a);
         a.mode = kShortQkv;
         a.w = lw.short_qkv;
         a.tiles_m = D / 16; a.tiles = 3 * a.tiles_m; a.out[0] = b.q; a.ldo = D;
@@ -2909,19 +2929,21 @@ static int record_short(lv_session *s, uint32_t idx0, uint32_t n, uint32_t pos, 
         LV_TRY(launch_short_gemm(st, a, ft, sf32, false));
         LV_TRY(launch_short_attention(st, s, b, li, pos, n, ft));
         ShortArgs o{};
-        o.x = b.act; o.n = n; o.nb = D / 32; o.mode = kShortStore; o.w = lw.short_wo; o.tiles_m = o.tiles = D / 16; o.ldo = D;
+        o.x = b.act; o.n = n; o.nb = D / 32; o.mode = kShortResidual; o.w = lw.short_wo; o.tiles_m = o.tiles = D / 16; o.ldo = D;
         for (int i = 0; i < kShortSlices; i++) o.out[i] = b.parts[i];
-        LV_TRY(launch_short_gemm(st, o, ft, sf32, true, &pending));
-        LV_TRY(launch_short_norm(st, b, lw.ffn_norm, n, D, pending, ft));
+        o.res = b.x; o.norm_w = lw.ffn_norm; o.act_out = b.act2; o.stats_out = b.stats; o.counters = b.counters;
+        LV_TRY(launch_short_gemm(st, o, ft, sf32, true, nullptr, &stat_rows));
         ShortArgs f{};
-        f.x = b.act; f.n = n; f.nb = D / 32; f.mode = kShortSilu;
+        behind_norm(f);
+        f.mode = kShortSilu;
         f.w = lw.short_gate_up; f.tiles_m = f.tiles = F / 8; f.ff = b.ff;
         LV_TRY(launch_short_gemm(st, f, ft, sf32, false));
         ShortArgs d = o;
         d.x = b.ff; d.nb = F / 32; d.w = lw.short_down;
-        LV_TRY(launch_short_gemm(st, d, ft, sf32, true, &pending));
+        d.norm_w = li + 1 < hp.layers ? m->layers[li + 1].attn_norm : m->norm;
+        LV_TRY(launch_short_gemm(st, d, ft, sf32, true, nullptr, &stat_rows));
     }
-    return record_short_head(s, b, idx0, n, pending, with_head, row_base);
+    return record_short_head(s, b, idx0, n, 0, with_head, row_base);
 }
 
 extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, uint32_t pos)

@@ -27,16 +27,26 @@
 //          the first two parts share an operand (tokens 0 .. 7 and 8 .. 15 of it), the third is half of one.
 // Rows of tokens past the batch are not written; a token only meets its own row of the result.
 //
-// Measured (us per launch, 7B layer, 8 tokens q4_0): q, k and v 11, gate and up 16, attention output and down together 17; about 3 of each
-// launch and sum.  A step of 8 tokens, 7B q4_0: 7.31 -> 2.00 ms (eight launches of the persistent kernel before).
+// Norms of up to 16 tokens have no launch of their own: the norm is (x w) / rms with one number a token.  The last of a row group's K
+// slices to arrive (kShortResidual) adds them to x, writes the parts of x w and the group's sum and squared deviations of x; the next
+// product puts those together while its first weights are on their way, and multiplies its results by 1 / rms.  A norm's launch is one
+// workgroup a token, 5.6 us of latency on eight CUs; putting slices together takes 2.9 at the end of the product (7B q4_0, 8 tokens: a
+// layer's two products and norms 26.8 -> 21.4 us, the step 2.00 -> 1.82 ms).  Halves need the row's largest value before they are made
+// and keep short_norm_kernel.
+//
+// Measured (us per launch, 7B layer, 8 tokens q4_0): q, k and v 11, gate and up 16, attention output 9 and down 12.5; about 3 of each
+// launch and sum.  A step of 8 tokens, 7B q4_0: 7.31 -> 1.82 ms (eight launches of the persistent kernel before).
 #pragma once
 
 #include "lv_attn_batch.h"
 #include "lv_gemm.h"
+#include "lv_mega.h"
 
 namespace lv {
 
 constexpr uint32_t kShortTokens = 64;
+constexpr uint32_t kShortExact = 16;       // tokens of steps on three parts
+constexpr uint32_t kShortStatLanes = 4;    // row groups a lane of a wave adds up: 256 of at least 32 rows, up to 8192
 constexpr int kShortWaves = 8;
 constexpr int kShortSlices = kGemmMaxMats;
 
@@ -48,7 +58,7 @@ typedef uint32_t lv_u2 __attribute__((ext_vector_type(2)));
 // tiles of 16 tokens; 0: up to 8 tokens, whose parts share operands
 __host__ __device__ constexpr uint32_t short_tiles(uint32_t n) { return n <= 8 ? 0 : (n + 15) / 16; }
 // three bf16 parts, not two fp16 halves: up to 16 tokens
-__host__ __device__ constexpr bool short_exact(uint32_t tiles) { return tiles <= 1; }
+__host__ __device__ constexpr bool short_exact(uint32_t tiles) { return tiles <= kShortExact / 16; }
 __host__ __device__ constexpr uint32_t short_block_bytes(uint32_t tiles) { return tiles == 0 ? 1536 : tiles == 1 ? 3072 : tiles * 2048; }
 // bytes of the activations of K columns
 __host__ __device__ constexpr size_t short_act_bytes(uint32_t K, uint32_t n) { return (size_t)(K / 32) * short_block_bytes(short_tiles(n)); }
@@ -112,7 +122,7 @@ __device__ __forceinline__ void short_put(uint8_t *act, uint32_t block, uint32_t
     *reinterpret_cast<uint4 *>(act + short_act_offset(block, token, g, tiles, 1)) = p[1];
 }
 
-enum ShortMode { kShortStore = 0, kShortQkv = 1, kShortSilu = 2 };
+enum ShortMode { kShortStore = 0, kShortQkv = 1, kShortSilu = 2, kShortResidual = 3 };
 
 struct ShortArgs {
     const uint8_t *x;          // activations
@@ -128,6 +138,16 @@ struct ShortArgs {
     const uint32_t *pos_ptr;
     uint32_t pos_add, backlog;
     uint8_t *ff;               // kShortSilu: activations of the next product
+    // kShortResidual, up to 16 tokens: x += the product, x w as the next product's activations, and sum and squared deviations of x by row
+    // groups (a workgroup's rows) and tokens.  The last of a row group's K slices to arrive does it; counters are zero before and after.
+    float *res;                // x, [n][ldo]
+    const float *norm_w;
+    uint8_t *act_out;
+    float2 *stats_out;         // [row group][kShortExact]
+    uint32_t *counters;        // [row group]
+    // Input of parts of x w: the results are multiplied by the tokens' 1 / rms, from these of `stat_groups` groups of `stat_rows` rows
+    const float2 *stats;       // null: the activations are whole
+    uint32_t stat_groups, stat_rows, dim;
 };
 
 // Loads of a chunk are requested while the one before it is multiplied, activations as far ahead as the weights or, where a block's
@@ -252,6 +272,8 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
     constexpr int XD = short_ahead<T, RT>();
     constexpr int PR = short_round<T, RT>();           // row tiles summed at a time
     __shared__ __attribute__((aligned(16))) float red[PR * NT * kShortWaves * 256];
+    __shared__ __attribute__((aligned(16))) float inv_rms[EXACT ? kShortExact : 1];
+    __shared__ uint32_t arrived;
     const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tile0 = blockIdx.x * RT;
@@ -299,10 +321,43 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
     const lv_f4v zero = {0.f, 0.f, 0.f, 0.f};
     constexpr uint32_t kOnes = 0x3f803f80u;
 
+    // a wave's tokens: `wave` and, beyond 8, `wave` + 8.  Asked for before the weights, added up while those are on their way.
+    constexpr int WT = EIGHT ? 1 : 2;
+    float2 st[EXACT ? WT : 1][kShortStatLanes];
+    if constexpr (EXACT) {
+        if (a.stats) {
+#pragma unroll
+            for (int t = 0; t < WT; t++)
+#pragma unroll
+                for (uint32_t j = 0; j < kShortStatLanes; j++) st[t][j] = j * 64 + lane < a.stat_groups ? a.stats[(j * 64 + lane) * kShortExact + wave + 8 * t] : make_float2(0.f, 0.f);
+        }
+    }
     if (steps) {
         fetch_w(0);
 #pragma unroll
         for (int s = 0; s < XD; s++) fetch_x(s, 0, s);
+    }
+    if constexpr (EXACT) {
+        if (a.stats) {
+#pragma unroll
+            for (int t = 0; t < WT; t++) {
+                float sum = 0.f, q = 0.f;
+#pragma unroll
+                for (uint32_t j = 0; j < kShortStatLanes; j++) sum += st[t][j].x;
+                const float mean = wave_sum(sum) / (float)a.dim;
+#pragma unroll
+                for (uint32_t j = 0; j < kShortStatLanes; j++) {
+                    const uint32_t grp = j * 64 + lane;
+                    if (grp >= a.stat_groups) continue;
+                    const float rows = (float)min(a.stat_rows, a.dim - grp * a.stat_rows), d = st[t][j].x / rows - mean;
+                    q += fmaf(rows * d, d, st[t][j].y);
+                }
+                q = wave_sum(q);
+                if (lane == 0) inv_rms[wave + 8 * t] = rsqrtf(q / (float)a.dim);
+            }
+        }
+    }
+    if (steps) {
         for (uint32_t j = 0; j < steps; j++) {
             uint32_t w[RT][CW];                        // dword s (q8_0: 2 s and 2 s + 1): this lane's codes of block s
             float sc[RT][4];
@@ -383,7 +438,11 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
             const uint32_t tile = tile0 + i0 + u / NT, tok0 = 16 * (u % NT) + 4 * g;
             if (tile >= a.tiles || (EIGHT && lane >= 32)) continue;
             float4 xs = make_float4(1.f, 1.f, 1.f, 1.f);
-            if (a.xscale) xs = *reinterpret_cast<const float4 *>(a.xscale + tok0);
+            if constexpr (EXACT) {
+                if (a.stats) xs = *reinterpret_cast<const float4 *>(inv_rms + tok0);
+            } else {
+                if (a.xscale) xs = *reinterpret_cast<const float4 *>(a.xscale + tok0);
+            }
             float v[4];
             total(u, lane, v, xs);
             if (a.mode == kShortSilu) {                // rows 0 .. 7 of the tile are W3's, 8 .. 15 the same ones of W1
@@ -414,15 +473,77 @@ __global__ __launch_bounds__(kShortWaves * 64) void short_gemm_kernel(ShortArgs 
             for (int e = 0; e < 4; e++) {
                 const uint32_t tok = tok0 + e;
                 if (tok >= a.n) continue;
-                if (z == 0) out[(size_t)tok * a.ldo + m] = v[e];
+                if (EXACT && a.mode == kShortResidual) st_dev(out + (size_t)tok * a.ldo + m, v[e]);
+                else if (z == 0) out[(size_t)tok * a.ldo + m] = v[e];
                 else if (row_at + tok < a.backlog) a.cache[z - 1][(size_t)(row_at + tok) * a.ldo + m] = float_to_half_bits(v[e]);
             }
+        }
+    }
+    if constexpr (EXACT) {
+        if (a.mode != kShortResidual) return;
+        // As in attention_kernel: write-through stores, acknowledged, then counted in; the last one reads with device-scope loads.  One
+        // slice: the workgroup is its own last one.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (gridDim.y > 1) {
+            if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(&a.counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (arrived != gridDim.y - 1) return;
+            if (threadIdx.x == 0) a.counters[blockIdx.x] = 0u;
+        }
+        constexpr int ROWS = RT * 16;
+        static_assert(2 * kShortExact * ROWS <= sizeof red / 4, "x and x w of a row group");
+        float *const xl = red, *const yl = red + kShortExact * ROWS;      // [token][row]
+        const uint32_t row0 = tile0 * 16, rows = min((uint32_t)ROWS, a.ldo - row0);
+        for (uint32_t i = threadIdx.x; i < a.n * ROWS; i += kShortWaves * 64) {
+            const uint32_t tok = i / ROWS, r = i % ROWS;
+            if (r >= rows) continue;
+            const size_t at = (size_t)tok * a.ldo + row0 + r;
+            uint32_t p[kShortSlices];
+#pragma unroll
+            for (int q = 0; q < kShortSlices; q++)
+                if (q < (int)gridDim.y) p[q] = ld_dev(reinterpret_cast<const uint32_t *>(a.out[q] + at));
+            const float x0 = a.res[at], w = a.norm_w[row0 + r];
+            float t = __uint_as_float(p[0]);
+#pragma unroll
+            for (int q = 1; q < kShortSlices; q++)
+                if (q < (int)gridDim.y) t += __uint_as_float(p[q]);
+            t += x0;
+            a.res[at] = t;
+            xl[tok * ROWS + r] = t;
+            yl[tok * ROWS + r] = t * w;
+        }
+        __syncthreads();
+        for (uint32_t tok = wave; tok < a.n; tok += kShortWaves) {
+            constexpr int PER = (ROWS + 63) / 64;
+            float v[PER], sum = 0.f, q = 0.f;
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                v[j] = j * 64 + lane < (int)rows ? xl[tok * ROWS + j * 64 + lane] : 0.f;
+                sum += v[j];
+            }
+            sum = wave_sum(sum);
+            const float mean = sum / (float)rows;
+#pragma unroll
+            for (int j = 0; j < PER; j++)
+                if (j * 64 + lane < (int)rows) q = fmaf(v[j] - mean, v[j] - mean, q);
+            q = wave_sum(q);
+            if (lane == 0) a.stats_out[blockIdx.x * kShortExact + tok] = make_float2(sum, q);
+        }
+        for (uint32_t i = threadIdx.x; i < a.n * (ROWS / 8); i += kShortWaves * 64) {
+            const uint32_t tok = i / (ROWS / 8), r = i % (ROWS / 8) * 8, k = row0 + r;
+            if (r >= rows) continue;
+            const float4 *y = reinterpret_cast<const float4 *>(yl + tok * ROWS + r);
+            float f[8];
+            short_order<QT>(f, y[0], y[1], true);
+            short_put(a.act_out, k / 32, tok, k % 32 / 8, T, f);
         }
     }
 }
 
 // x += the K slices of the product before, then normalize(x) * w (normalize.comp:34-64) as the next product's activations, halves
-// scaled per token as in gemm_row_scale.  One workgroup per token, a thread per 8 elements (dim / 8 threads rounded up to whole waves;
+// scaled per token as in gemm_row_scale: in steps of 17 tokens and more, and in front of the first layer.  One workgroup per token, a
+// thread per 8 elements (dim / 8 threads rounded up to whole waves;
 // dim <= 8192, a multiple of 32): nothing but latency counts here, and a thread's loads are few and all in flight at once.
 struct ShortNormArgs {
     float *x;

@@ -25,13 +25,15 @@ WIDE = {
     "q4_tall": ("Q4_0", dict(vocab=512, dim=384, heads=12, layers=1, ff=8320)),
     "q8_tall": ("Q8_0", dict(vocab=512, dim=384, heads=6, layers=1, ff=5376)),
 }
+# six row tiles a workgroup on the way down, the last workgroup two: rows and statistics of part of a row group
+RAGGED = {"q4_ragged": ("Q4_0", dict(vocab=512, dim=6656, heads=52, layers=1, ff=17920))}
 
 
 @pytest.fixture(scope="module")
 def models(lva, tmp_path_factory):
     d = tmp_path_factory.mktemp("short")
     out = {}
-    for i, (name, (wtype, shape)) in enumerate({**SHAPES, **WIDE}.items()):
+    for i, (name, (wtype, shape)) in enumerate({**SHAPES, **WIDE, **RAGGED}.items()):
         out[name] = str(d / f"{name}.ggml")
         lva.write_model(out[name], wtype=getattr(lva, "LV_" + wtype), seed=60 + i, **shape)
     for name in ("q4_64", "q8_64"):      # file version 1, whose block scales need fp32
@@ -48,6 +50,7 @@ def close(got, want):
 CASES = [(name, b, n) for name in [*SHAPES, "q4_64_v1", "q8_64_v1"]
          for b, n in [(0, 2), (0, 16), (5, 17), (0, 33), (61, 3), (64, 48), (120, 64), (190, 65), (201, 49),
                        (1, 15), (2, 15), (49, 15), (50, 15), (200, 2), (239, 15)]]      # attention of up to 15 tokens: edges of its 16 and 64 positions
+CASES += [(name, b, n) for name in RAGGED for b, n in [(0, 3), (3, 9)]]
 CASES += [(name, b, n) for name in WIDE for b, n in [(0, 3), (70, 15), (0, 16), (0, 32), (9, 40), (0, 49), (130, 64)]]
 
 
