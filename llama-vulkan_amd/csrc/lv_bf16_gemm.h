@@ -385,7 +385,7 @@ __device__ __forceinline__ void wide_tile(const BfGemmArgs &a, uint32_t rt, uint
     constexpr int LW = 8, LX = TN / 32, LPS = LW + LX;      // direct loads per wave and stage, 8 rows (1 KB) each
     constexpr int NM = 8 * NJ, NR = 8 + NJ;                 // products and operand reads of half a step
     constexpr int RP = (NR + NM / 2 - 1) / (NM / 2), LP = (LPS + NM / 2 - 1) / (NM / 2);    // reads, loads between two products
-    constexpr int LD = NM / LPS;
+    constexpr int LD = NST == 2 ? NM / LPS : 1;             // two stages: products a load
     extern __shared__ __attribute__((aligned(128))) uint8_t bf_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, g4 = lane >> 4;

@@ -540,51 +540,51 @@ __global__ __launch_bounds__(gemv_threads(INPUT)) void bf16_gemv_kernel(BfGemvAr
     uint32_t task = first_task, it = 0, k = turn, kit = 0, seg = 0;
     const uint32_t my_tasks = first_task < tasks ? (tasks - first_task + nwaves - 1) / nwaves : 0;
     const uint32_t total = my_tasks * iters;
-    for (uint32_t t0 = 0; t0 < total; t0 += DEPTH) {
+    // One way out at every place of the queue: where a step could be passed over and the next one taken, the compiler would not know how many
+    // loads are on their way behind the one it waits for, and wait for them all.
+    for (uint32_t t = 0;;) {
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) {
-            if (t0 + d < total) {
-                const uint32_t c = k * 64 + lane;               // 8-element chunk
-                const float *src = xs + seg * kp + (c * 8 < kp ? c * 4 : 0);
-                const float4 x0 = *reinterpret_cast<const float4 *>(src), x1 = *reinterpret_cast<const float4 *>(src + kp / 2);
+            if (t++ == total) return;
+            const uint32_t c = k * 64 + lane;               // 8-element chunk
+            const float *src = xs + seg * kp + (c * 8 < kp ? c * 4 : 0);
+            const float4 x0 = *reinterpret_cast<const float4 *>(src), x1 = *reinterpret_cast<const float4 *>(src + kp / 2);
 #pragma unroll
-                for (int r = 0; r < NR; r++) {
-                    const uint4 v = q[d][r];
-                    float s = acc[r];
-                    s = fmaf(__uint_as_float(v.x << 16), x0.x, s); s = fmaf(__uint_as_float(v.x & 0xffff0000u), x0.y, s);
-                    s = fmaf(__uint_as_float(v.y << 16), x0.z, s); s = fmaf(__uint_as_float(v.y & 0xffff0000u), x0.w, s);
-                    s = fmaf(__uint_as_float(v.z << 16), x1.x, s); s = fmaf(__uint_as_float(v.z & 0xffff0000u), x1.y, s);
-                    s = fmaf(__uint_as_float(v.w << 16), x1.z, s); s = fmaf(__uint_as_float(v.w & 0xffff0000u), x1.w, s);
-                    acc[r] = s;
-                }
-                fetch(q[d]);
-                if (++k == ksteps) k = 0;
-                if (++kit == ksteps) { kit = 0; seg++; }
-                if (++it == iters) {
-                    float tot[NR];
+            for (int r = 0; r < NR; r++) {
+                const uint4 v = q[d][r];
+                float s = acc[r];
+                s = fmaf(__uint_as_float(v.x << 16), x0.x, s); s = fmaf(__uint_as_float(v.x & 0xffff0000u), x0.y, s);
+                s = fmaf(__uint_as_float(v.y << 16), x0.z, s); s = fmaf(__uint_as_float(v.y & 0xffff0000u), x0.w, s);
+                s = fmaf(__uint_as_float(v.z << 16), x1.x, s); s = fmaf(__uint_as_float(v.z & 0xffff0000u), x1.y, s);
+                s = fmaf(__uint_as_float(v.w << 16), x1.z, s); s = fmaf(__uint_as_float(v.w & 0xffff0000u), x1.w, s);
+                acc[r] = s;
+            }
+            fetch(q[d]);
+            if (++k == ksteps) k = 0;
+            if (++kit == ksteps) { kit = 0; seg++; }
+            if (++it != iters) continue;
+            float tot[NR];
 #pragma unroll
-                    for (int r = 0; r < NR; r++) { tot[r] = wave_sum(acc[r]); acc[r] = 0.f; }
-                    if (lane < R) {
-                        const uint32_t u = task * R + lane;
-                        float v0 = tot[0], v1 = tot[NR - R];
+            for (int r = 0; r < NR; r++) { tot[r] = wave_sum(acc[r]); acc[r] = 0.f; }
+            if (lane < R) {
+                const uint32_t u = task * R + lane;
+                float v0 = tot[0], v1 = tot[NR - R];
 #pragma unroll
-                        for (int r = 1; r < R; r++)
-                            if (lane == r) { v0 = tot[r]; v1 = tot[NR - R + r]; }
-                        if (u < units) {
-                            if constexpr (MODE == kGemvExperts) {
-                                const float wt = sel_score[u / kp_units(a)];
-                                a.out[u] = silu_f(wt * v0) * (wt * v1);
-                            } else if constexpr (MODE == kGemvGlu) {
-                                a.out[u] = glu_f(a.act, v0) * v1;
-                            } else {
-                                a.out[u] = v0;
-                            }
-                        }
+                for (int r = 1; r < R; r++)
+                    if (lane == r) { v0 = tot[r]; v1 = tot[NR - R + r]; }
+                if (u < units) {
+                    if constexpr (MODE == kGemvExperts) {
+                        const float wt = sel_score[u / kp_units(a)];
+                        a.out[u] = silu_f(wt * v0) * (wt * v1);
+                    } else if constexpr (MODE == kGemvGlu) {
+                        a.out[u] = glu_f(a.act, v0) * v1;
+                    } else {
+                        a.out[u] = v0;
                     }
-                    it = 0; seg = 0;
-                    task += nwaves;
                 }
             }
+            it = 0; seg = 0;
+            task += nwaves;
         }
     }
 }

@@ -788,8 +788,8 @@ template <int MODE, int INPUT, int R, int DEPTH> static int launch_gemv(hipStrea
 }
 
 // Rows a wave walks together: two where there are enough of them, one where the last round of waves would then be far from full
-// (us for two and one: 32000 x 4096 47.9 and 51.2, 18560 x 4096 31.1 and 33.4, 8848 x 2048 12.3 and 10.1; four at a time 60, 41
-// and 11.7).
+// (us for two and one: 32000 x 4096 40.9 and 42.5, 16384 x 4096 22.5 and 23.5, 32000 x 2048 22.0 and 23.1, 9000 x 4096 16.3 and 15.4,
+// 8848 x 2048 9.4 and 8.3).
 static uint32_t gemv_rows_together(uint32_t units)
 {
     constexpr uint32_t kWaves = 16 * 256;
@@ -801,17 +801,16 @@ template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs 
 {
     const size_t lds = (size_t)a.kp * (MODE == kGemvDown ? a.top : 1) * 4 + (MODE == kGemvExperts ? a.experts * 4ull : 0) +
                        (INPUT == kInGroups ? group_sums(a.group.groups, gemv_waves(INPUT)) * 4ull : 0);
-    if constexpr (MODE == kGemvExperts || MODE == kGemvGlu) {
-        const uint32_t units = MODE == kGemvExperts ? a.top * (a.expert_rows / 2) : a.rows / 2;
-        return gemv_rows_together(units) == 2 ? launch_gemv<MODE, INPUT, 2, 2>(st, a, units, lds) : launch_gemv<MODE, INPUT, 1, 4>(st, a, units, lds);
-    } else {
-        // a workgroup of 16 waves takes one row at a time: 45.0 us with two, 39.4 with one (18560 and 32000 x 4096, four streams)
-        // one row at a time: eight steps ahead, or four, which is a row of up to 2048 columns.  Eight and four, us: 8848 x 2048 11.0 and
-        // 10.1; means of all products of Somesun 2048 behind a norm 7.8 and 7.2, of Zedenex 2048 behind streams 11.6 and 10.9.  Beyond 2048
-        // columns it hangs on the rows: few of them (64 x 4096, a router) 5.7 and 6.3, many (Zedenex 4096 behind streams) 25.9 and 24.6
-        return gemv_threads(INPUT) == 512 && gemv_rows_together(a.rows) == 2 ? launch_gemv<MODE, INPUT, 2, 4>(st, a, a.rows, lds)
-               : a.kp <= 2048                                                ? launch_gemv<MODE, INPUT, 1, 4>(st, a, a.rows, lds)
-                                                                             : launch_gemv<MODE, INPUT, 1, 8>(st, a, a.rows, lds);
+    // Three or four loads of a wave ahead: enough while every one of them is waited for by itself, and what is asked for first keeps the
+    // input waiting.  us, one row, 2, 3, 4, 5 and 8 ahead: 8848 x 2048 9.0 8.3 8.5 8.9 10.3; 18560 x 4096 behind four streams 27.9 27.8 27.5 28.4
+    // 29.0; 6144 x 1536 5.7 5.7 5.9 7.0 7.1; two rows, 1, 2, 3 and 4 ahead: 32000 x 2048 22.0 22.0 22.1 22.5.  Pairs of gate and up one at a
+    // time (two, one: 8 experts of 2048 x 4096 25.6 and 23.2, 22016 x 4096 32.7 and 30.8), and so a workgroup of 16 waves.
+    if constexpr (MODE == kGemvExperts) return launch_gemv<MODE, INPUT, 1, 3>(st, a, a.top * (a.expert_rows / 2), lds);
+    else if constexpr (MODE == kGemvGlu) return launch_gemv<MODE, INPUT, 1, 3>(st, a, a.rows / 2, lds);
+    else {
+        if constexpr (gemv_threads(INPUT) == 512)
+            if (gemv_rows_together(a.rows) == 2) return launch_gemv<MODE, INPUT, 2, 2>(st, a, a.rows, lds);
+        return launch_gemv<MODE, INPUT, 1, 3>(st, a, a.rows, lds);
     }
 }
 
