@@ -182,6 +182,7 @@ struct lv_model {
     float *tok_f32_own = nullptr;   // fp32 copy of a quantised embedding table (the persistent kernel reads rows as fp32)
     // a small model's token as one launch (lv_small.h): its matrices as a table on the device, the workgroups of a launch (0: not such a model)
     SmallLayer *small_layers = nullptr;
+    uint32_t small_own = 0;          // feed-forward blocks of a workgroup, with partial sums (SmallArgs)
     uint32_t small_wgs = 0, small_elements = 0;      // cache elements of a head up to which it is the faster way
     // prompt copy of the layer matrices (lv_gemm.h), made when the first batch is evaluated; sessions of several threads share it
     std::mutex prompt_mutex;
@@ -1382,6 +1383,11 @@ constexpr uint32_t kSmallHeadTiles = 12;
 // them, so what the launch gains bounds the context, and so do the rows that were looked at.  Width 512, 4 heads of 128, 4 layers 148 and
 // 191 us behind 100 rows, 199 and 205 behind 1000, 257 and 221 behind 2000; width 256, 4 heads of 64, 76 and 118 behind 2000.
 constexpr uint32_t kSmallRowElements = 131072;
+// Partial sums (lv_small.h) save two hand-overs a layer, 4 to 5 us, and every workgroup reads this many floats a layer instead of 3 D + F.
+// us a token, 4 layers unless said, without and with them (floats): width 256, ff 704, 2 layers 57 and 47 (6656), 8 layers 169 and 132; 256 and
+// 4096 90 and 78 (17408, two blocks a workgroup); 448 and 1216 107 and 98 (20160), q8_0 108 and 104; 384 and 2048 94 and 88 (29184), q8_0 96
+// and 93; 576 and 1536 140 and 142 (32832); 512 and 2048 101 and 102 (36864); 768 and 2048 143 and 155 (58368).
+constexpr uint32_t kSmallPartFloats = 30000;
 static int build_small(lv_model *m)
 {
     const lv_hparams &hp = m->hp;
@@ -1409,6 +1415,11 @@ static int build_small(lv_model *m)
     const double chain = 25 + hp.layers * (42 + 0.125 * layer_mb) + 0.06 * output_mb;
     if (launch >= chain) return LV_OK;
     m->small_wgs = wgs;
+    const uint32_t own = small_parts(F, 1) <= kSmallMaxWGs ? 1 : 2, parts = small_parts(F, own);
+    if (parts <= kSmallMaxWGs && D * std::max(own, hp.rot / 32) <= kSmallPartBlocks * kSmallThreads && (hp.heads + parts) * D <= kSmallPartFloats) {
+        m->small_own = own;
+        m->small_wgs = std::max(wgs, parts);
+    }
     m->small_elements = (uint32_t)std::min<double>(kSmallRowElements, (chain - launch) / hp.layers / 0.08 * 1000);
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&m->small_layers), table.size() * sizeof(SmallLayer)));
     HIP_TRY(hipMemcpyAsync(m->small_layers, table.data(), table.size() * sizeof(SmallLayer), hipMemcpyHostToDevice, m->ctx->stream));
@@ -1669,7 +1680,7 @@ static int session_alloc(lv_session *s)
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->vo), D * 4));
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&s->ff), F * 4));
     if (s->model->mega_kind || s->model->small_wgs) {
-        size_t bytes = (size_t)hp.layers * small_layer_floats(hp.dim, hp.ff) * 4, local_bytes = 0;
+        size_t bytes = (size_t)hp.layers * small_layer_floats(hp.dim, hp.ff, hp.heads, s->model->small_own) * 4, local_bytes = 0;
         if (s->model->mega_kind) LV_TRY(mega_dispatch(s->model->mega_kind, [&](auto shape) -> int {
             bytes = ((size_t)hp.layers * decltype(shape)::XCHG_LAYER + decltype(shape)::XCHG_TAIL) * 4;
             local_bytes = (size_t)hp.layers * decltype(shape)::LOCAL_LAYER * 4;
@@ -1979,7 +1990,7 @@ static int launch_small(lv_session *s, uint32_t pos, uint32_t token)
     a.logits_host = s->logits_host;
     a.status = s->status_host;
     a.layers = m->hp.layers; a.vocab = m->hp.vocab; a.backlog = s->backlog; a.pos = pos; a.token = token;
-    a.D = m->hp.dim; a.F = m->hp.ff; a.heads = m->hp.heads;
+    a.D = m->hp.dim; a.F = m->hp.ff; a.heads = m->hp.heads; a.own = m->small_own;
     a.spin_limit = s->wait_limit ? s->wait_limit : kSpinLimit;
     std::lock_guard<std::mutex> lock(m->ctx->mega_mutex);
     SmallTurn *turn = nullptr;

@@ -8,7 +8,11 @@
 //   per layer: a workgroup a head forms its query, key and value rows and attends, all inside the workgroup -> o
 //              all workgroups: x += Wo o -> x1; norm, gate and up -> ff; x1 += W2 ff -> x2
 //
-// 53 us a token, 17.5 of them a layer: four hand-overs of about 1.5 us, and the latency of weights, rows and norms between them.
+// With partial sums, two hand-overs a layer instead of four: a head's workgroup multiplies its own o by its columns of Wo, a workgroup its
+// own blocks of ff by their columns of W2, and every reader adds the parts up.  More values are handed over, (heads + workgroups) D a
+// layer: for narrow models only (build_small).
+//
+// Width 256, 2 layers: 53.6 us a token with four hand-overs a layer, 18.7 of them a layer; 47.9 with two, 14.2.
 // A wave takes tiles of 64 blocks: L lanes a row (a power of two, 8 to 64), 64 / L rows; the first kSmallDepth tiles of a phase are
 // asked for before the vector they are multiplied with is waited for.
 #pragma once
@@ -42,9 +46,13 @@ struct SmallArgs {
     float *logits, *logits_host;   // on the device and in pinned memory: no launch of its own copies them
     uint32_t *status;
     uint32_t layers, vocab, backlog, pos, token, D, F, heads, spin_limit;
+    uint32_t own;              // 0, or with partial sums: feed-forward blocks of a workgroup, a power of two
 };
 
-__host__ __device__ __forceinline__ uint32_t small_layer_floats(uint32_t D, uint32_t F) { return 3 * D + F; }
+// o, x1, ff, x2; with partial sums: one vector of every head and of every workgroup that has feed-forward blocks
+__host__ __device__ __forceinline__ uint32_t small_parts(uint32_t F, uint32_t own) { return (F / 32 + own - 1) / own; }
+__host__ __device__ __forceinline__ uint32_t small_layer_floats(uint32_t D, uint32_t F, uint32_t heads, uint32_t own) { return own ? (heads + small_parts(F, own)) * D : 3 * D + F; }
+constexpr uint32_t kSmallPartBlocks = 4;   // blocks a thread multiplies of a workgroup's own columns of Wo or W2, at most
 // lanes a row of nb blocks, as a power of two
 __host__ __device__ __forceinline__ int small_lanes_log2(uint32_t nb) { return nb <= 8 ? 3 : nb <= 16 ? 4 : nb <= 32 ? 5 : 6; }
 
@@ -248,6 +256,87 @@ __device__ __forceinline__ void small_stage(const float *src, uint32_t n, float 
     lds_barrier();
 }
 
+// v += `count` vectors of D floats one behind the other (D a multiple of 4), in an order that hangs on D alone
+__device__ __forceinline__ void small_add_parts(float (&v)[2], const float *src, uint32_t count, uint32_t D, float *sums, const SmallArgs &a)
+{
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    constexpr int AHEAD = 4;
+    const uint32_t quads = D / 4, groups = kSmallThreads / quads, grp = threadIdx.x / quads, q = threadIdx.x - grp * quads;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), 0, (int)(count * D * 4), 0x00020000);
+    float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t p0 = grp; p0 < count && grp < groups; p0 += AHEAD * groups) {
+        u4 u[AHEAD];
+        uint32_t spins = 0;
+        bool pending;
+        do {
+            pending = false;
+            asm volatile("" ::: "memory");      // every turn issues the loads again; behind the last part they return zeros
+#pragma unroll
+            for (int j = 0; j < AHEAD; j++) {
+                u[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(((p0 + j * groups) * D + q * 4) * 4), 0, 16 /* device scope */);
+                pending |= (u[j].x == kNotReady) | (u[j].y == kNotReady) | (u[j].z == kNotReady) | (u[j].w == kNotReady);
+            }
+        } while (pending && ++spins < a.spin_limit);
+        if (pending) *a.status = 1u;
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) {
+            t.x += __uint_as_float(u[j].x); t.y += __uint_as_float(u[j].y); t.z += __uint_as_float(u[j].z); t.w += __uint_as_float(u[j].w);
+        }
+    }
+    lds_barrier();                   // other waves may still read the last sums
+    if (grp < groups) *reinterpret_cast<float4 *>(sums + (grp * quads + q) * 4) = t;
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const uint32_t i = threadIdx.x + j * kSmallThreads;
+        if (i < D)
+            for (uint32_t g = 0; g < groups; g++) v[j] += sums[g * D + i];
+    }
+}
+
+// A workgroup's columns of a matrix of D rows of nb blocks: blocks c0 .. c0 + n - 1 of every row, `wide` (n rounded up to a power of two) lanes
+// a row.  Asked for early, multiplied with a vector in LDS, the rows' sums published.
+template <int QT, bool SF32>
+struct SmallColumns {
+    SmallRaw<QT> q[kSmallPartBlocks];
+
+    __device__ __forceinline__ void fetch(const SmallView &m, uint32_t nb, uint32_t c0, uint32_t n, uint32_t wide, uint32_t D)
+    {
+#pragma unroll
+        for (uint32_t j = 0; j < kSmallPartBlocks; j++) {
+            const uint32_t i = threadIdx.x + j * kSmallThreads, r = i / wide, k = i - r * wide, b = r < D && k < n ? r * nb + c0 + k : 0;
+            if constexpr (QT == 4) q[j].c = m.codes[b];
+            else { q[j].c = m.codes[2 * b]; q[j].c2 = m.codes[2 * b + 1]; }
+            if constexpr (SF32) q[j].d = ((const __attribute__((address_space(1))) uint32_t *)m.scales)[b];
+            else q[j].d = ((const __attribute__((address_space(1))) uint16_t *)m.scales)[b];
+        }
+    }
+    __device__ __forceinline__ void publish(const float *x, uint32_t n, uint32_t wide, uint32_t D, float *out)
+    {
+#pragma unroll
+        for (uint32_t j = 0; j < kSmallPartBlocks; j++) {
+            if (j * kSmallThreads >= D * wide) break;
+            const uint32_t i = threadIdx.x + j * kSmallThreads, r = i / wide, k = i - r * wide;
+            float xr[32], xsum = 0.f;
+            const float4 *src = reinterpret_cast<const float4 *>(x + (k < n ? k : 0) * 32);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float4 f = src[e];
+                xr[4 * e] = f.x; xr[4 * e + 1] = f.y; xr[4 * e + 2] = f.z; xr[4 * e + 3] = f.w;
+                xsum += (f.x + f.y) + (f.z + f.w);
+            }
+            const float d = SF32 ? __uint_as_float(q[j].d) : half_bits_to_float((uint16_t)q[j].d);
+            const uint4 qa = make_uint4(q[j].c.x, q[j].c.y, q[j].c.z, q[j].c.w);
+            float s;
+            if constexpr (QT == 4) s = (q4_block_dot(qa, xr) - 8.f * xsum) * d;
+            else s = (q8_block_dot(qa, make_uint4(q[j].c2.x, q[j].c2.y, q[j].c2.z, q[j].c2.w), xr) - 128.f * xsum) * d;
+            s = k < n ? s : 0.f;
+            for (uint32_t off = 1; off < wide; off <<= 1) s += __shfl_xor(s, (int)off, kWave);
+            if (k == 0 && r < D) small_publish(out + r, s);
+        }
+    }
+};
+
 template <int QT, bool SF32, int R>
 __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a)
 {
@@ -261,7 +350,10 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
     const uint32_t D = a.D, F = a.F, nbD = D / 32, nbF = F / 32, G = gridDim.x, cur = a.pos;
     const uint32_t gw = blockIdx.x + wave * G, waves = G * kSmallWaves;   // consecutive tiles on different CUs
     const bool attends = blockIdx.x < a.heads;
-    const uint32_t per = small_layer_floats(D, F);
+    const uint32_t per = small_layer_floats(D, F, a.heads, a.own);
+    // with partial sums: this workgroup's feed-forward blocks
+    const uint32_t parts = a.own ? small_parts(F, a.own) : 0, c0 = blockIdx.x * a.own, nown = blockIdx.x < parts ? min(a.own, nbF - c0) : 0;
+    float *const sums = xs;          // of parts, before xs is the norm
 
     for (uint32_t i = blockIdx.x * kSmallThreads + tid; i < a.layers * per; i += G * kSmallThreads) st_dev(a.xchg_rearm + i, __uint_as_float(kNotReady));
 
@@ -286,6 +378,8 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
         const SmallLayer &l = a.layer[ph == 4 ? 0 : li];
         float *const o = a.xchg + (size_t)li * per, *const x1 = o + D, *const ff = x1 + D, *const x2 = ff + F;   // o - D: the layer before's x2
         if (ph == 0 && !attends) continue;
+        if (a.own && (ph == 1 || ph == 3)) continue;
+        float *const part1 = o, *const part2 = o + a.heads * D;      // with partial sums; part1 - parts D: the layer before's part2
 
         SmallGemv<QT, SF32> g;
         g.kind = ph == 2 ? kSmallPair : kSmallStacked;
@@ -300,7 +394,12 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
             g.part = R;
         }
         if (ph == 2) g.m1 = small_view<SF32>(&l.w1);
-        g.start(ph == 0 ? wave : gw, ph == 0 ? kSmallWaves : waves, ph == 3 ? nbF : nbD, ph == 0 ? 3 * R : ph == 2 ? F : ph == 4 ? a.vocab : D);
+        const bool mine = ph == 0 || (ph == 2 && a.own);             // a product of this workgroup alone
+        if (ph == 2 && a.own) g.row0 = 32 * c0;
+        g.start(mine ? wave : gw, mine ? kSmallWaves : waves, ph == 3 ? nbF : nbD, ph == 0 ? 3 * R : ph == 2 ? (a.own ? 32 * nown : F) : ph == 4 ? a.vocab : D);
+        SmallColumns<QT, SF32> cols;
+        if (a.own && ph == 0) cols.fetch(small_view<SF32>(&l.wo), nbD, blockIdx.x * (R / 32), R / 32, R / 32, D);
+        if (a.own && ph == 2) cols.fetch(small_view<SF32>(&l.w2), nbF, c0, nown, a.own, D);
 
         // the first cache rows come on their way before anything is waited for; the new row is in LDS only
         uint16_t *const kc = a.kv + (size_t)(2 * li) * a.backlog * D + blockIdx.x * R, *const vc = kc + (size_t)a.backlog * D;
@@ -325,7 +424,10 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
         const bool x_phase = ph != 1 && ph != 3;
         if (x_phase || (ph == 1 && !attends)) {
             const float *src = ph == 2 ? x1 : o - D;
-            if (ph == 2 || li) small_poll_x(v, src, D, a);
+            if (a.own) {
+                if (li && !(ph == 2 && attends)) small_add_parts(v, o - parts * D, parts, D, sums, a);
+                if (ph == 2) small_add_parts(v, part1, a.heads, D, sums, a);
+            } else if (ph == 2 || li) small_poll_x(v, src, D, a);
             lds_barrier();           // other waves still read xs and xraw
             const small_float_p w = ph == 4 ? (small_float_p)a.norm : ph == 2 ? small_norm(&l.ffn_norm) : ph == 0 ? small_norm(&l.attn_norm) : nullptr;
             small_stage_x(v, D, w, xraw, xs, red);
@@ -340,9 +442,17 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
             } else if (ph == 4) {
                 a.logits[r] = s;
                 a.logits_host[r] = s;
-            } else if (ph == 2) small_publish(ff + r, up * s / (__expf(-s) + 1.f));
+            } else if (ph == 2) {
+                const float f = up * s / (__expf(-s) + 1.f);
+                if (a.own) xraw[r] = f;          // the residual is in registers
+                else small_publish(ff + r, f);
+            }
             else small_publish((ph == 1 ? x1 : x2) + r, xraw[r] + s);
         });
+        if (a.own && ph == 2) {
+            lds_barrier();
+            if (nown) cols.publish(xraw, nown, a.own, D, part2 + blockIdx.x * D);
+        }
         if (ph != 0) continue;
 
         lds_barrier();
@@ -404,7 +514,12 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
                 num += part[w][tid];
                 all += part[w][R];
             }
-            small_publish(o + blockIdx.x * R + tid, num / all);
+            if (a.own) xraw[tid] = num / all;
+            else small_publish(o + blockIdx.x * R + tid, num / all);
+        }
+        if (a.own) {
+            lds_barrier();
+            cols.publish(xraw, R / 32, R / 32, D, part1 + blockIdx.x * D);
         }
     }
 }

@@ -29,6 +29,8 @@ SHAPES = {
     "longest feed-forward": dict(vocab=600, dim=992, heads=31, layers=2, ff=8192),
     "more heads than tiles": dict(vocab=260, dim=1024, heads=32, layers=1, ff=64),
     "wide heads of 128": dict(vocab=1000, dim=1024, heads=8, layers=2, ff=8160),       # one workgroup a head would take longer: the chain
+    "a block a workgroup": dict(vocab=512, dim=256, heads=8, layers=2, ff=2016),        # one workgroup less than there may be
+    "workgroups without blocks": dict(vocab=8000, dim=128, heads=4, layers=2, ff=96),
     "large vocabulary": dict(vocab=32000, dim=1024, heads=16, layers=1, ff=64),        # a quarter of the CUs would take longer
 }
 CHAIN = {"wide heads of 128", "large vocabulary"}
