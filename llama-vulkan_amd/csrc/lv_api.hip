@@ -2454,9 +2454,14 @@ static void launch_short_rows(hipStream_t st, const ShortArgs &a, uint32_t rt, u
 // and with three parts (T 0 and 1) above the choice, 16 and 19 us gate and up, 11 and 13 q, k and v (768 tiles):
 //   gate and up, RT 2/3/4/6: T 0 3.8/2.4/4.0/0, T 1 7.8/4.6/6.5/0; q, k and v: T 0 3.3/0/0.7/2.9, T 1 5.1/0/0.9/3.4
 //   down, RT 4 slices 1/2/3/4: T 0 9.3/1.2/0/0, T 1 13.5/2.3/0.2/0, RT 2: T 0 4.0/-0.8/1.4/0.5, T 1 8.4/-0.4/3.3/1.3
+// Up to 16 tokens the slice that arrives last also adds the others up, one after the other, and nobody else runs by then.  Whole prompts in us
+// with a slice more at 0.25, 1.5, 3 and 5 (7B: Wo and down as RT 4 with 4 slices, RT 2 with 2 for Wo, RT 2 with 2 for both, and the same):
+//   T 0: 7B q4_0 3 tokens 1846/-/1793/1790, 8 1875/-/1825/1826, 8 layers of q8_0 6 tokens 624/-/606/606, 13B q4_0 8 628/-/625/644, q8_0 5 832/-/824/841
+//   T 1: 7B q4_0 10 tokens 2250/2233/2265/-, 14 2290/2269/2294/-, 8 layers of q8_0 9 678/670/672/-, 13B q4_0 12 774/774/778/816, q8_0 13 969/967/968/996
 static void short_plan(uint32_t tiles, uint32_t nb, uint32_t T, int qt, bool sliced, uint32_t *best_rt, uint32_t *best_chunks)
 {
     const uint32_t chunks = nb / 4;
+    const double more = T == 0 ? 3 : T == 1 ? 1.5 : 0.25 * T;
     double best = 1e30;
     for (uint32_t rt : {2u, 3u, 4u, 6u}) {
         if (!short_fits(qt, T, rt)) continue;
@@ -2464,7 +2469,7 @@ static void short_plan(uint32_t tiles, uint32_t nb, uint32_t T, int qt, bool sli
             const uint32_t per = (chunks + s - 1) / s;
             if ((chunks + per - 1) / per != s) continue;
             const uint32_t steps = (per + kShortWaves - 1) / kShortWaves, held = ((tiles + rt - 1) / rt * s + 255) / 256;
-            const double cost = held * steps * (rt + 1.5) + 0.25 * (T ? T : 1) * (s - 1);
+            const double cost = held * steps * (rt + 1.5) + more * (s - 1);
             if (cost < best) { best = cost; *best_rt = rt; *best_chunks = per; }
         }
     }
