@@ -2768,7 +2768,8 @@ static int launch_short_attention(hipStream_t st, const lv_session *s, const Sho
     ShortAttnArgs a{};
     a.kcache = kv_ptr(s, layer, 0); a.vcache = kv_ptr(s, layer, 1); a.q = b.q; a.trig_abs = s->trig_abs;
     a.pos0 = pos; a.n = n; a.heads = hp.heads; a.backlog = s->backlog; a.tiles_per_split = per; a.num = b.num; a.den = b.den;
-    if (splits == 1) { a.act = b.act; a.tiles = short_tiles(n); a.q8 = ftype == LV_Q8_0; }
+    a.tiles = short_tiles(n); a.q8 = ftype == LV_Q8_0; a.counters = b.counters;
+    if (splits == 1 || n < kPrefillMin) a.act = b.act;
     const size_t lds = (size_t)512 * hp.rot;
     switch (hp.rot) {
 #define LV_SHORT_ATTN(R)                                                                                                              \
@@ -2787,7 +2788,7 @@ static int launch_short_attention(hipStream_t st, const lv_session *s, const Sho
     default: return fail(LV_ERR_ARG, "attention: head size %u (32, 64 and 128 are built)", hp.rot);
     }
     HIP_TRY(hipGetLastError());
-    if (splits == 1) return LV_OK;
+    if (a.act) return LV_OK;
     ShortCombineArgs c{};
     c.num = b.num; c.den = b.den; c.splits = splits; c.n = n; c.heads = hp.heads; c.rot = hp.rot; c.tiles = short_tiles(n); c.act = b.act;
     const dim3 grid((hp.dim / 8 + 255) / 256, n);

@@ -640,7 +640,8 @@ struct ShortAttnArgs {
     uint32_t pos0, n, heads, backlog;  // row z sits at pos0 + z
     uint32_t tiles_per_split;          // tiles of 64 positions
     float *num, *den;
-    uint8_t *act;                      // with one split: the output projection's activations, `tiles` token tiles, in place of num and den
+    uint8_t *act;                      // the output projection's activations, `tiles` token tiles; short_attn_kernel: with one split, in place of num and den
+    uint32_t *counters;                // short_attn_exact_kernel: one a head, zero before and after
     uint32_t tiles, q8;
 };
 // grid (heads, splits)
@@ -876,6 +877,48 @@ __global__ __launch_bounds__(256, 2) void short_attn_kernel(ShortAttnArgs a)
         }
 }
 
+__device__ __forceinline__ void short_act_row(const ShortAttnArgs &a, uint32_t k, uint32_t z, float4 va, float4 vb, float den)
+{
+    va.x /= den; va.y /= den; va.z /= den; va.w /= den;
+    vb.x /= den; vb.y /= den; vb.z /= den; vb.w /= den;
+    float f[8];
+    if (a.q8) short_order<8>(f, va, vb, short_exact(a.tiles));
+    else short_order<4>(f, va, vb, short_exact(a.tiles));
+    short_put(a.act, k / 32, z, k % 32 / 8, a.tiles, f);
+}
+// The end of a workgroup that has written its split of head h through to memory: the last of a head's splits to arrive adds them up, in their
+// order, and makes the output projection's operands of them.  short_attn_combine_kernel in its place: us of 8 layers of 7B q8_0, 4 tokens behind 1000
+// rows 668 and 651 so, 8 behind 300 645 and 635, 15 behind 1900 787 and 779; 13B q4_0, 8 behind 1500 731 and 721.  With more tokens a head
+// is too much for one workgroup (17 behind 150 844 and 850, 45 behind 619 1042 and 1077, 64 behind 1900 1249 and 1306).
+template <int R> __device__ __forceinline__ void short_attn_last(const ShortAttnArgs &a, uint32_t h)
+{
+    __shared__ uint32_t arrived;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(&a.counters[h], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (arrived != gridDim.y - 1) return;
+    if (threadIdx.x == 0) a.counters[h] = 0u;
+    const uint32_t D = a.heads * R;
+    for (uint32_t i = threadIdx.x; i < a.n * (R / 8); i += 256) {
+        const uint32_t z = i / (R / 8), k = h * R + i % (R / 8) * 8;
+        float4 va = make_float4(0.f, 0.f, 0.f, 0.f), vb = va;
+        float den = 0.f;
+#pragma unroll 4
+        for (uint32_t s = 0; s < gridDim.y; s++) {
+            const size_t part = (size_t)s * a.n + z;
+            const uint64_t *p = reinterpret_cast<const uint64_t *>(a.num + part * D + k);
+            float2 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = __builtin_bit_cast(float2, __hip_atomic_load(p + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            den += __uint_as_float(ld_dev(reinterpret_cast<const uint32_t *>(a.den + part * a.heads + h)));
+            va.x += v[0].x; va.y += v[0].y; va.z += v[1].x; va.w += v[1].y;
+            vb.x += v[2].x; vb.y += v[2].y; vb.z += v[3].x; vb.w += v[3].y;
+        }
+        short_act_row(a, k, z, va, vb, den);
+    }
+}
+
 // Attention of 2 to 15 tokens: fp32 throughout, on the fp32 matrix instruction, whose 16 columns are the step's queries.  attention_kernel
 // reads a head's cache rows and rotations again for every query (15 queries behind 1900 positions: 0.9 GB through the L2s); here they are read
 // once, rotated in registers and multiplied with all queries, 64 instructions per 16 positions whatever n is.  A layer of 7B, us with what makes
@@ -1014,26 +1057,23 @@ __global__ __launch_bounds__(256, 2) void short_attn_exact_kernel(ShortAttnArgs 
         return s;
     };
     auto weight = [&](uint32_t z) { return (den_s[0][z] + den_s[1][z]) + (den_s[2][z] + den_s[3][z]); };
-    if (a.act) {
+    if (gridDim.y == 1) {
         for (uint32_t i = t; i < a.n * C8; i += 256) {
-            const uint32_t z = i / C8, c = i % C8, d = (c >> 2) * 32, og = c & 3;
-            const float w = weight(z);
-            float4 va = total(z, d + 8 * og), vb = total(z, d + 8 * og + 4);
-            va.x /= w; va.y /= w; va.z /= w; va.w /= w;
-            vb.x /= w; vb.y /= w; vb.z /= w; vb.w /= w;
-            float f[8];
-            if (a.q8) short_order<8>(f, va, vb, true);
-            else short_order<4>(f, va, vb, true);
-            short_put(a.act, (h * R + d) / 32, z, og, a.tiles, f);
+            const uint32_t z = i / C8, d = i % C8 * 8;
+            short_act_row(a, h * R + d, z, total(z, d), total(z, d + 4), weight(z));
         }
         return;
     }
     const size_t part = (size_t)blockIdx.y * a.n;
     for (uint32_t i = t; i < a.n * (R / 4); i += 256) {
         const uint32_t z = i / (R / 4), d = i % (R / 4) * 4;
-        *reinterpret_cast<float4 *>(a.num + (part + z) * D + (size_t)h * R + d) = total(z, d);
+        const float4 s = total(z, d);
+        uint64_t *p = reinterpret_cast<uint64_t *>(a.num + (part + z) * D + (size_t)h * R + d);
+        __hip_atomic_store(p, __builtin_bit_cast(uint64_t, make_float2(s.x, s.y)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p + 1, __builtin_bit_cast(uint64_t, make_float2(s.z, s.w)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if ((uint32_t)t < a.n) a.den[(part + t) * H + h] = weight(t);
+    if ((uint32_t)t < a.n) st_dev(a.den + (part + t) * H + h, weight(t));
+    short_attn_last<R>(a, h);
 }
 
 // numerators and denominators of all splits, in order -> the output projection's activations.  grid (D / 8 / 256 rounded up, n)

@@ -104,6 +104,33 @@ def test_attention_of_short_steps_behind_long_contexts(lva, ctx, tmp_path, befor
     a.close(); b.close(); model.close()
 
 
+@pytest.mark.parametrize("rot,heads", [(32, 4), (64, 8), (128, 3)])
+@pytest.mark.parametrize("before,n", [(63, 2), (64, 15), (1500, 2), (1500, 15)])
+def test_parts_of_short_attention_put_together_by_the_last(lva, ctx, tmp_path, rot, heads, before, n):
+    """two parts and the most there are, fewest and most tokens; two layers and two steps, so that a count left over would show"""
+    path = str(tmp_path / "heads.ggml")
+    lva.write_model(path, wtype=lva.LV_Q4_0, seed=12, vocab=512, dim=rot * heads, heads=heads, layers=2, ff=512)
+    model = lva.Model(ctx, path)
+    total = before + 2 * n
+    toks = lva.synth_tokens(total, 3, 512, seed=n)
+    a, b = lva.Session(model, total), lva.Session(model, total)
+    b.set_path(lva.PATH_KERNELS)
+    a.begin(toks[:before], 0)
+    a.wait()
+    for layer in (0, 1):
+        for which in (0, 1):
+            b.kv_write(layer, which, a.kv(layer, which, before))
+    for s in (a, b):
+        s.keep_all_logits()
+    for at in (before, before + n):
+        a.begin(toks[at:at + n], at)
+        got = a.logits_rows(0, n)
+        for i in range(n):
+            b.begin(toks[at + i:at + i + 1], at + i)
+            close(got[i], b.logits())
+    a.close(); b.close(); model.close()
+
+
 # steps of 65 to 256 tokens (csrc/lv_mid.h), and what is left of a longer one: every edge of the token tiles and of the two groups of them
 MIDDLE = [(name, 0, n) for name in ("q4_64", "q8_128") for n in (65, 80, 81, 96, 97, 128, 129, 160, 161, 192, 193, 256)]
 MIDDLE += [(name, 37, n) for name in [*SHAPES, "q4_64_v1", "q8_64_v1"] for n in (70, 120, 170)]
