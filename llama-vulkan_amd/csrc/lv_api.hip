@@ -1370,29 +1370,12 @@ static int build_mega(lv_model *m)
     return LV_OK;
 }
 
-// Which models take lv_small.h's launch for a token: those whose operator chain has ten launches a layer (below the streaming kernels' 2048
-// rows) and whose work a few workgroups do in less time than those launches take to follow one another.  A head's three projections are one
-// workgroup's work, at most kSmallHeadTiles tiles a wave were looked at; then both times are estimated, in us behind 100 rows of context:
-//   launch  17 + layers (9.6 + 1.1 tiles a wave of a head's projections + 0.95 tiles a wave of the other products) + 1.26 of the output's
-//   chain   25 + layers (42 + 0.125 MB) + 0.06 MB of the output
-// a fit of 110 shapes of width 64 to 1024, 300 to 128256 rows of output, 7 % off the launch's and 14 % off the chain's measured times at most.
-// Measured, launch and chain: width 256, 2 layers 53 and 117; 512, 8 layers 198 and 361; 768, 12 layers 464 and 568.  A large vocabulary is
-// what a quarter of the chip is too little for: 640 wide, 4 layers, 128256 rows 260 and 240, 1024, 1 layer, 203 and 116.
-constexpr uint32_t kSmallHeadTiles = 12;
-// One workgroup also walks a head's cache rows, where the chain splits them over several: 80 ns more of a layer for every 1000 elements of
-// them, so what the launch gains bounds the context, and so do the rows that were looked at.  Width 512, 4 heads of 128, 4 layers 148 and
-// 191 us behind 100 rows, 199 and 205 behind 1000, 257 and 221 behind 2000; width 256, 4 heads of 64, 76 and 118 behind 2000.
-constexpr uint32_t kSmallRowElements = 131072;
-// Partial sums (lv_small.h) save two hand-overs a layer, 4 to 5 us, and every workgroup reads this many floats a layer instead of 3 D + F.
-// us a token, 4 layers unless said, without and with them (floats): width 256, ff 704, 2 layers 57 and 47 (6656), 8 layers 169 and 132; 256 and
-// 4096 90 and 78 (17408, two blocks a workgroup); 448 and 1216 107 and 98 (20160), q8_0 108 and 104; 384 and 2048 94 and 88 (29184), q8_0 96
-// and 93; 576 and 1536 140 and 142 (32832); 512 and 2048 101 and 102 (36864); 768 and 2048 143 and 155 (58368).
-constexpr uint32_t kSmallPartFloats = 30000;
+// a small model's token as one launch, where that is the faster way (lv_small_plan.h)
 static int build_small(lv_model *m)
 {
     const lv_hparams &hp = m->hp;
-    const uint32_t D = hp.dim, F = hp.ff, ft = m->output.ftype;
-    if (m->mega_kind || D > kSmallMaxDim || F > kSmallMaxFf || hp.heads > kSmallMaxWGs || m->ctx->props.multiProcessorCount < (int)kSmallMaxWGs) return LV_OK;
+    const uint32_t ft = m->output.ftype;
+    if (m->mega_kind || m->ctx->props.multiProcessorCount < (int)kSmallMaxWGs) return LV_OK;
     if (m->tok_ftype != LV_F32 && m->tok_ftype != LV_Q4_0 && m->tok_ftype != LV_Q8_0) return LV_OK;
     std::vector<SmallLayer> table;
     for (const LayerWeights &lw : m->layers) {
@@ -1400,27 +1383,11 @@ static int build_small(lv_model *m)
             if (x->ftype != ft || (x->view.scales_f32 != nullptr) != (m->output.view.scales_f32 != nullptr)) return LV_OK;
         table.push_back({lw.wq.view, lw.wk.view, lw.wv.view, lw.wo.view, lw.w1.view, lw.w2.view, lw.w3.view, lw.attn_norm, lw.ffn_norm});
     }
-    // tiles of `waves` waves of a matrix, the longest wave's
-    const auto tiles = [](uint32_t rows, uint32_t cols, uint32_t waves) -> uint32_t {
-        const uint32_t nb = cols / 32, lanes = 1u << small_lanes_log2(nb);
-        return ((rows * lanes + 63) / 64 + waves - 1) / waves * ((nb + lanes - 1) / lanes);
-    };
-    const uint32_t head = tiles(3 * hp.rot, D, kSmallWaves);
-    if (head > kSmallHeadTiles) return LV_OK;
-    // a pair of tiles a wave in the feed-forward, or four tiles of a large vocabulary
-    const uint32_t most = std::max(tiles(F, D, 1), tiles(hp.vocab, D, 1) / 4);
-    const uint32_t wgs = std::min(kSmallMaxWGs, std::max(hp.heads, (most + kSmallWaves - 1) / kSmallWaves)), waves = wgs * kSmallWaves;
-    const double mb = (ft == LV_Q4_0 ? 18 : 34) / 32e6, layer_mb = (4.0 * D * D + 3.0 * D * F) * mb, output_mb = (double)hp.vocab * D * mb;
-    const double launch = 17 + hp.layers * (9.6 + 1.1 * head + 0.95 * (tiles(D, D, waves) + 2 * tiles(F, D, waves) + tiles(D, F, waves))) + 1.26 * tiles(hp.vocab, D, waves);
-    const double chain = 25 + hp.layers * (42 + 0.125 * layer_mb) + 0.06 * output_mb;
-    if (launch >= chain) return LV_OK;
-    m->small_wgs = wgs;
-    const uint32_t own = small_parts(F, 1) <= kSmallMaxWGs ? 1 : 2, parts = small_parts(F, own);
-    if (parts <= kSmallMaxWGs && D * std::max(own, hp.rot / 32) <= kSmallPartBlocks * kSmallThreads && (hp.heads + parts) * D <= kSmallPartFloats) {
-        m->small_own = own;
-        m->small_wgs = std::max(wgs, parts);
-    }
-    m->small_elements = (uint32_t)std::min<double>(kSmallRowElements, (chain - launch) / hp.layers / 0.08 * 1000);
+    const SmallPlan plan = small_plan({hp.dim, hp.ff, hp.heads, hp.rot, hp.layers, hp.vocab, ft == LV_Q4_0 ? 18u : 34u});
+    if (!plan.wgs) return LV_OK;
+    m->small_wgs = plan.wgs;
+    m->small_own = plan.own;
+    m->small_elements = plan.elements;
     HIP_TRY(hipMalloc(reinterpret_cast<void **>(&m->small_layers), table.size() * sizeof(SmallLayer)));
     HIP_TRY(hipMemcpyAsync(m->small_layers, table.data(), table.size() * sizeof(SmallLayer), hipMemcpyHostToDevice, m->ctx->stream));
     HIP_TRY(hipStreamSynchronize(m->ctx->stream));
@@ -1963,12 +1930,18 @@ static int launch_mega(lv_session *s, uint32_t pos, uint32_t token, bool *refuse
     return mega_turn_end(s);
 }
 
+template <int QT, bool SF32, bool PARTS>
+static void launch_small_heads(const SmallArgs &a, uint32_t wgs, uint32_t rot, hipStream_t st)
+{
+    if (rot == 32) small_decode_kernel<QT, SF32, 32, PARTS><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
+    else if (rot == 64) small_decode_kernel<QT, SF32, 64, PARTS><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
+    else small_decode_kernel<QT, SF32, 128, PARTS><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
+}
 template <int QT, bool SF32>
 static void launch_small_kernel(const SmallArgs &a, uint32_t wgs, uint32_t rot, hipStream_t st)
 {
-    if (rot == 32) small_decode_kernel<QT, SF32, 32><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
-    else if (rot == 64) small_decode_kernel<QT, SF32, 64><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
-    else small_decode_kernel<QT, SF32, 128><<<dim3(wgs), dim3(kSmallThreads), 0, st>>>(a);
+    if (a.own) launch_small_heads<QT, SF32, true>(a, wgs, rot, st);
+    else launch_small_heads<QT, SF32, false>(a, wgs, rot, st);
 }
 
 // One token of a small model.  Its few workgroups wait for each other as the persistent kernel's do (turns: small_turn_begin).

@@ -10,7 +10,7 @@
 //
 // With partial sums, two hand-overs a layer instead of four: a head's workgroup multiplies its own o by its columns of Wo, a workgroup its
 // own blocks of ff by their columns of W2, and every reader adds the parts up.  More values are handed over, (heads + workgroups) D a
-// layer: for narrow models only (build_small).
+// layer: for narrow models only (lv_small_plan.h).
 //
 // Width 256, 2 layers: 53.6 us a token with four hand-overs a layer, 18.7 of them a layer; 47.9 with two, 14.2.
 // A wave takes tiles of 64 blocks: L lanes a row (a power of two, 8 to 64), 64 / L rows; the first kSmallDepth tiles of a phase are
@@ -19,14 +19,11 @@
 
 #include "lv_kernels.h"
 #include "lv_mega.h"
+#include "lv_small_plan.h"
 
 namespace lv {
 
-constexpr int kSmallThreads = 512, kSmallWaves = kSmallThreads / 64;
 constexpr int kSmallDepth = 4;             // tiles in flight a wave
-constexpr uint32_t kSmallMaxDim = 1024;    // two values of a normalised vector a thread
-constexpr uint32_t kSmallMaxFf = 8192;     // floats of LDS
-constexpr uint32_t kSmallMaxWGs = 64;      // each waits for the others: all of them, of four launches at once, find room beside one another
 
 struct SmallLayer {
     MatView wq, wk, wv, wo, w1, w2, w3;
@@ -48,13 +45,6 @@ struct SmallArgs {
     uint32_t layers, vocab, backlog, pos, token, D, F, heads, spin_limit;
     uint32_t own;              // 0, or with partial sums: feed-forward blocks of a workgroup, a power of two
 };
-
-// o, x1, ff, x2; with partial sums: one vector of every head and of every workgroup that has feed-forward blocks
-__host__ __device__ __forceinline__ uint32_t small_parts(uint32_t F, uint32_t own) { return (F / 32 + own - 1) / own; }
-__host__ __device__ __forceinline__ uint32_t small_layer_floats(uint32_t D, uint32_t F, uint32_t heads, uint32_t own) { return own ? (heads + small_parts(F, own)) * D : 3 * D + F; }
-constexpr uint32_t kSmallPartBlocks = 4;   // blocks a thread multiplies of a workgroup's own columns of Wo or W2, at most
-// lanes a row of nb blocks, as a power of two
-__host__ __device__ __forceinline__ int small_lanes_log2(uint32_t nb) { return nb <= 8 ? 3 : nb <= 16 ? 4 : nb <= 32 ? 5 : 6; }
 
 // Pointers to weights are kept as addresses of global memory: loads through a pointer that itself came from memory would otherwise be
 // ones that might go to LDS, which are waited for together with those.
@@ -337,7 +327,9 @@ struct SmallColumns {
     }
 };
 
-template <int QT, bool SF32, int R>
+// PARTS: with partial sums (args.own).  Instances of their own: the code of both ways in one made either 2 to 4 % slower (a line of code is
+// fetched from memory; 768 wide, 12 layers with four hand-overs 378 -> 392 us).
+template <int QT, bool SF32, int R, bool PARTS>
 __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a)
 {
     constexpr int LPR = R / 8, RPB = kSmallThreads / LPR, BATCH = 2;     // lanes a cache row, rows of the workgroup at once, times BATCH
@@ -350,9 +342,9 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
     const uint32_t D = a.D, F = a.F, nbD = D / 32, nbF = F / 32, G = gridDim.x, cur = a.pos;
     const uint32_t gw = blockIdx.x + wave * G, waves = G * kSmallWaves;   // consecutive tiles on different CUs
     const bool attends = blockIdx.x < a.heads;
-    const uint32_t per = small_layer_floats(D, F, a.heads, a.own);
+    const uint32_t own = PARTS ? a.own : 0, per = small_layer_floats(D, F, a.heads, own);
     // with partial sums: this workgroup's feed-forward blocks
-    const uint32_t parts = a.own ? small_parts(F, a.own) : 0, c0 = blockIdx.x * a.own, nown = blockIdx.x < parts ? min(a.own, nbF - c0) : 0;
+    const uint32_t parts = PARTS ? small_parts(F, own) : 0, c0 = blockIdx.x * own, nown = blockIdx.x < parts ? min(own, nbF - c0) : 0;
     float *const sums = xs;          // of parts, before xs is the norm
 
     for (uint32_t i = blockIdx.x * kSmallThreads + tid; i < a.layers * per; i += G * kSmallThreads) st_dev(a.xchg_rearm + i, __uint_as_float(kNotReady));
@@ -378,7 +370,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
         const SmallLayer &l = a.layer[ph == 4 ? 0 : li];
         float *const o = a.xchg + (size_t)li * per, *const x1 = o + D, *const ff = x1 + D, *const x2 = ff + F;   // o - D: the layer before's x2
         if (ph == 0 && !attends) continue;
-        if (a.own && (ph == 1 || ph == 3)) continue;
+        if (PARTS && (ph == 1 || ph == 3)) continue;
         float *const part1 = o, *const part2 = o + a.heads * D;      // with partial sums; part1 - parts D: the layer before's part2
 
         SmallGemv<QT, SF32> g;
@@ -394,12 +386,14 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
             g.part = R;
         }
         if (ph == 2) g.m1 = small_view<SF32>(&l.w1);
-        const bool mine = ph == 0 || (ph == 2 && a.own);             // a product of this workgroup alone
-        if (ph == 2 && a.own) g.row0 = 32 * c0;
-        g.start(mine ? wave : gw, mine ? kSmallWaves : waves, ph == 3 ? nbF : nbD, ph == 0 ? 3 * R : ph == 2 ? (a.own ? 32 * nown : F) : ph == 4 ? a.vocab : D);
+        const bool mine = ph == 0 || (ph == 2 && PARTS);             // a product of this workgroup alone
+        if (ph == 2 && PARTS) g.row0 = 32 * c0;
+        g.start(mine ? wave : gw, mine ? kSmallWaves : waves, ph == 3 ? nbF : nbD, ph == 0 ? 3 * R : ph == 2 ? (PARTS ? 32 * nown : F) : ph == 4 ? a.vocab : D);
         SmallColumns<QT, SF32> cols;
-        if (a.own && ph == 0) cols.fetch(small_view<SF32>(&l.wo), nbD, blockIdx.x * (R / 32), R / 32, R / 32, D);
-        if (a.own && ph == 2) cols.fetch(small_view<SF32>(&l.w2), nbF, c0, nown, a.own, D);
+        if constexpr (PARTS) {
+            if (ph == 0) cols.fetch(small_view<SF32>(&l.wo), nbD, blockIdx.x * (R / 32), R / 32, R / 32, D);
+            if (ph == 2) cols.fetch(small_view<SF32>(&l.w2), nbF, c0, nown, own, D);
+        }
 
         // the first cache rows come on their way before anything is waited for; the new row is in LDS only
         uint16_t *const kc = a.kv + (size_t)(2 * li) * a.backlog * D + blockIdx.x * R, *const vc = kc + (size_t)a.backlog * D;
@@ -424,7 +418,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
         const bool x_phase = ph != 1 && ph != 3;
         if (x_phase || (ph == 1 && !attends)) {
             const float *src = ph == 2 ? x1 : o - D;
-            if (a.own) {
+            if constexpr (PARTS) {
                 if (li && !(ph == 2 && attends)) small_add_parts(v, o - parts * D, parts, D, sums, a);
                 if (ph == 2) small_add_parts(v, part1, a.heads, D, sums, a);
             } else if (ph == 2 || li) small_poll_x(v, src, D, a);
@@ -444,14 +438,14 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
                 a.logits_host[r] = s;
             } else if (ph == 2) {
                 const float f = up * s / (__expf(-s) + 1.f);
-                if (a.own) xraw[r] = f;          // the residual is in registers
+                if constexpr (PARTS) xraw[r] = f;          // the residual is in registers
                 else small_publish(ff + r, f);
             }
             else small_publish((ph == 1 ? x1 : x2) + r, xraw[r] + s);
         });
-        if (a.own && ph == 2) {
+        if (PARTS && ph == 2) {
             lds_barrier();
-            if (nown) cols.publish(xraw, nown, a.own, D, part2 + blockIdx.x * D);
+            if (nown) cols.publish(xraw, nown, own, D, part2 + blockIdx.x * D);
         }
         if (ph != 0) continue;
 
@@ -514,10 +508,10 @@ __global__ __launch_bounds__(kSmallThreads) void small_decode_kernel(SmallArgs a
                 num += part[w][tid];
                 all += part[w][R];
             }
-            if (a.own) xraw[tid] = num / all;
+            if constexpr (PARTS) xraw[tid] = num / all;
             else small_publish(o + blockIdx.x * R + tid, num / all);
         }
-        if (a.own) {
+        if constexpr (PARTS) {
             lds_barrier();
             cols.publish(xraw, R / 32, R / 32, D, part1 + blockIdx.x * D);
         }

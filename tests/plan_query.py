@@ -1,0 +1,38 @@
+"""Asks the rules that choose kernels by sizes (csrc/lv_*_plan.h), compiled for the host."""
+import os
+import subprocess
+import tempfile
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llama-vulkan_amd", "csrc")
+SOURCE = r"""
+#include "lv_small_plan.h"
+#include <cstdio>
+#include <iostream>
+#include <string>
+int main()
+{
+    for (std::string what; std::cin >> what;) {
+        if (what == "small") {
+            lv::SmallShape m;
+            std::cin >> m.D >> m.F >> m.heads >> m.rot >> m.layers >> m.vocab >> m.block_bytes;
+            const lv::SmallPlan p = lv::small_plan(m);
+            printf("%u %u %u\n", p.wgs, p.own, p.elements);
+        }
+    }
+}
+"""
+_exe = []
+
+
+def ask(lines):
+    """a list of answers, tuples of numbers, to questions: ("small", dim, ff, heads, head size, layers, vocab, bytes of a block)"""
+    if not _exe:
+        d = tempfile.TemporaryDirectory()
+        src, exe = os.path.join(d.name, "main.cpp"), os.path.join(d.name, "main")
+        with open(src, "w") as f:
+            f.write(SOURCE)
+        subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, src, "-o", exe], check=True)
+        _exe.extend((exe, d))
+    text = "\n".join(" ".join(map(str, q)) for q in lines)
+    out = subprocess.run([_exe[0]], input=text, capture_output=True, text=True, check=True).stdout
+    return [tuple(map(int, line.split())) for line in out.splitlines()]

@@ -31,6 +31,9 @@ SHAPES = {
     "wide heads of 128": dict(vocab=1000, dim=1024, heads=8, layers=2, ff=8160),       # one workgroup a head would take longer: the chain
     "a block a workgroup": dict(vocab=512, dim=256, heads=8, layers=2, ff=2016),        # one workgroup less than there may be
     "workgroups without blocks": dict(vocab=8000, dim=128, heads=4, layers=2, ff=96),
+    "widest with partial sums": dict(vocab=700, dim=288, heads=9, layers=2, ff=1792),
+    "two blocks a workgroup": dict(vocab=512, dim=256, heads=4, layers=2, ff=4064),     # the last one has one
+    "narrowest without": dict(vocab=700, dim=320, heads=5, layers=2, ff=864),
     "large vocabulary": dict(vocab=32000, dim=1024, heads=16, layers=1, ff=64),        # a quarter of the CUs would take longer
 }
 CHAIN = {"wide heads of 128", "large vocabulary"}
