@@ -22,10 +22,13 @@ constexpr uint32_t small_layer_floats(uint32_t D, uint32_t F, uint32_t heads, ui
 // rows) and whose work a few workgroups do in less time than those launches take to follow one another.  A head's three projections are one
 // workgroup's work, at most kSmallHeadTiles tiles a wave were looked at; then both times are estimated, in us behind 100 rows of context:
 //   launch  17 + layers (9.6 + 1.1 tiles a wave of a head's projections + 0.95 tiles a wave of the other products) + 1.26 of the output's
-//   chain   25 + layers (42 + 0.125 MB) + 0.06 MB of the output
-// a fit of 110 shapes of width 64 to 1024, 300 to 128256 rows of output, 7 % off the launch's and 14 % off the chain's measured times at most.
+//           + 0.1 for 1000 logits; partial sums (below) 1.5 less a layer
+//   chain   25 + layers (42 + 0.125 MB) + 0.06 MB of the output + 0.27 for 1000 logits, which it copies
+// a fit of shapes of width 64 to 1024, 300 to 128256 rows of output, steps whose logits are read; over 140 of them 13 % off either way's
+// measured times at most (partial sums 16 %).
 // Measured, launch and chain: width 256, 2 layers 47 and 117; 512, 8 layers 198 and 361; 768, 12 layers 464 and 568.  A large vocabulary is
-// what a quarter of the chip is too little for: 640 wide, 4 layers, 128256 rows 260 and 240, 1024, 1 layer, 203 and 116.
+// what a quarter of the chip is too little for: 640 wide, 4 layers, 128256 rows 260 and 240, 1024, 1 layer, 203 and 116; of a narrow
+// model it is not: 256, 1 layer, 128256 rows 87 and 106, 128 wide 91 and 107.
 constexpr uint32_t kSmallHeadTiles = 12;
 // One workgroup also walks a head's cache rows, where the chain splits them over several: 80 ns more of a layer for every 1000 elements of
 // them, so what the launch gains bounds the context, and so do the rows that were looked at.  Width 512, 4 heads of 128, 4 layers 148 and
@@ -71,8 +74,8 @@ inline SmallPlan small_plan(const SmallShape &m)
     const uint32_t waves = p.wgs * kSmallWaves;
     const double mb = m.block_bytes / 32e6, layer_mb = (4.0 * m.D * m.D + 3.0 * m.D * m.F) * mb, output_mb = (double)m.vocab * m.D * mb;
     const double products = 0.95 * (tiles(m.D, m.D, waves) + 2 * tiles(m.F, m.D, waves) + tiles(m.D, m.F, waves));
-    const double launch = 17 + m.layers * (9.6 + 1.1 * head + products) + 1.26 * tiles(m.vocab, m.D, waves);
-    const double chain = 25 + m.layers * (42 + 0.125 * layer_mb) + 0.06 * output_mb;
+    const double launch = 17 + m.layers * (9.6 + 1.1 * head + products - (p.own ? 1.5 : 0.0)) + 1.26 * tiles(m.vocab, m.D, waves) + 0.1e-3 * m.vocab;
+    const double chain = 25 + m.layers * (42 + 0.125 * layer_mb) + 0.06 * output_mb + 0.27e-3 * m.vocab;
     if (launch >= chain) return {};
     p.elements = (uint32_t)std::min<double>(kSmallRowElements, (chain - launch) / m.layers / 0.08 * 1000);
     return p;
