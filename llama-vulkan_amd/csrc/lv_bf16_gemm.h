@@ -28,6 +28,7 @@
 #pragma once
 
 #include "../../include/llava_hip.h"
+#include "lv_bf_plan.h"
 #include "lv_device.h"
 
 namespace lv {
@@ -247,8 +248,6 @@ __device__ __forceinline__ bool bf_tile(const BfGemmArgs &a, uint32_t tile_token
 }
 inline uint32_t bf_grid(const BfGemmArgs &a) { return (a.row_tiles * a.token_tiles + 7) / 8 * 8; }
 
-constexpr int kBfTile = 128;       // tokens per workgroup, bf16
-constexpr int kBfStep = 64;
 constexpr int kBfRows = 128;       // rows of gemm_bf16_kernel's tile
 constexpr int kBfLdsBytes = 2 * (kBfRows + kBfTile) * kBfStep * 2;
 

@@ -814,81 +814,6 @@ template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs 
     }
 }
 
-// Which tiles a bf16 product takes, and into how many slices of K it is cut (`slices` at most; the reader of the result adds them up).
-// Time = rounds of workgroups over 256 CUs x K steps x a step's time, plus prologue and epilogue, plus writing and reading a slice more.
-// Fitted to launches whose weights come from HBM, as a model's do; wide tiles have the longer ends (products in a prompt, us, 128 x 128 and
-// 256 x 128: 100 x 2048 x 2048 31 35, x 3072 x 768 15 21, x 4096 x 512 12 16, 301 x 3072 x 768 16 21, x 8512 x 2048 33 35).  us, 128 x 128 tiles and 256 rows x 128, 160, 192 and 256 tokens:
-// 16 x 8848 x 2048 29 25 26 26 46; 100 x 8848 x 2048 32 35 35 35 52; 300 x 22016 x 4096 109 89 78 69 95; 500 x 18560 x 4096 135 124 135 80 108;
-// 777 x 22016 x 4096 193 159 148 145 191; 777 x 18560 x 4096 144 126 157 155 209; 777 x 2112 x 4096 57 53 76 72 101; 777 x 4096 x 11008 in two
-// slices 93 82 109 96 137, in three 124 106 82 79 101; 1000 x 8848 x 2048 63 66 45 46 62; 1100 x 18560 x 4096 204 187 168 174 210;
-// 1900 x 22016 x 4096 346 328 335 324 294; 2048 x 13600 x 4096 279 250 234 244 217; 2048 x 4096 x 8192 144 123 133 130 187.
-enum class BfTiles { k128, kWide, kWide160, kWide192, kWidest };
-struct BfPlan {
-    BfTiles tiles;
-    uint32_t slices;
-};
-static BfPlan bf_plan(uint32_t rows, uint32_t n, uint32_t kp, uint32_t slices)
-{
-    constexpr double kCus = 256, kWideEnds = 5;     // us more before the first step and behind the last one
-    struct Offer {
-        BfTiles tiles;
-        uint32_t tokens;
-        double busy, idle;      // us of a step, every CU at work and few of them
-    };
-    constexpr Offer offers[] = {{BfTiles::kWide, 128, 0.87, 0.67}, {BfTiles::kWide160, 160, 1.12, 0.92}, {BfTiles::kWide192, 192, 1.25, 0.90}, {BfTiles::kWidest, 256, 1.52, 1.34}};
-    BfPlan best{BfTiles::k128, 1};
-    double best_us = 1e30;
-    for (uint32_t s = 1; s <= slices; s++) {
-        const uint32_t steps = (kp / kBfStep + s - 1) / s;
-        if (s > 1 && steps < 8) break;
-        // a slice more is written and read again, from the L2s while all of them fit there
-        const double more = 8.0 + (s - 1) * (1.0 + ((uint64_t)s * n * rows * 4 < 32u << 20 ? 1e-6 : 2e-6) * n * rows);
-        auto take = [&](BfTiles t, double step_us, double ends) {
-            const double us = step_us * steps + ends + more;
-            if (us < best_us) {
-                best_us = us;
-                best = {t, s};
-            }
-        };
-        // two share a CU
-        const double small = (double)((rows + 127) / 128) * ((n + 127) / 128) * s, left = std::fmod(small, 2 * kCus);
-        take(BfTiles::k128, std::floor(small / (2 * kCus)) * 1.05 + (left > kCus ? 0.95 + 0.1 * left / kCus : left ? 0.78 : 0.0), 0);
-        for (const Offer &o : offers) {
-            const uint32_t whole = n / o.tokens, rest = n % o.tokens;
-            // the batch's rest: what its loads take whatever its tokens, and its products
-            const double part = !rest ? 0.0 : o.tiles == BfTiles::kWidest ? 1.0 : 0.6 + 0.4 * ((rest + 31) / 32 * 32) / o.tokens;
-            const uint32_t token_tiles = whole + (rest != 0);
-            const double tiles = (double)((rows + 255) / 256) * token_tiles * s, last = std::fmod(tiles, kCus);
-            take(o.tiles, (std::floor(tiles / kCus) * o.busy + (last ? o.idle + (o.busy - o.idle) * last / kCus : 0.0)) * (whole + part) / token_tiles, kWideEnds);
-        }
-    }
-    return best;
-}
-
-// Tokens of an expert's tiles, 128 or 160, and their order.  us of gate and up, and of down (64 experts, 8 a token, 2048 x 4096 and
-// 4096 x 1024): tiles of 128, a row tile after the other, then an expert after the other; tiles of 160 likewise.
-//    300 tokens            239 180 241 179   127 121 127 121
-//    900                   273 240 265 199   168 170 166 161
-//   1400                   280 250 327 310   227 198 228 221
-//   2048                   372 356 329 309   259 281 270 242
-//    600, unevenly chosen  226 214 226 219   136 142 133 148
-//   2048, unevenly chosen  356 364 344 372   272 282 257 279
-// Few tokens an expert: the weights' way from HBM counts, an expert after the other; 160 where an expert of the mean number of choices
-// and two standard deviations more then has fewer tiles, and where every round of workgroups is not one of few (32 experts, 4 a token, 2048
-// x 2048 and 2048 x 1024, 900 tokens: 128 85 and 52, 160 92 and 62).  Down of 48 tokens an expert and more in tiles of 128: its weights are half
-// as many and uneven experts decide (512 tokens of a prompt, unevenly chosen: 135 and 146).  Many: runs of one length whoever is chosen.
-struct ExpertPlan {
-    uint32_t tile;
-    bool by_expert, down_by_expert;
-};
-static ExpertPlan expert_plan(uint32_t n, uint32_t top, uint32_t experts, uint32_t rows)
-{
-    const double mean = (double)n * top / experts, many = mean + 2 * std::sqrt(mean);
-    if (mean >= 192) return {160, false, false};
-    const bool longer = experts * ((rows + 255) / 256) >= 512 && std::ceil(many / 160) < std::ceil(many / 128);
-    return {longer ? 160u : 128u, true, longer || mean < 48};
-}
-
 template <class K> static int launch_bf(hipStream_t st, K *k, const BfGemmArgs &a, int lds)
 {
     LV_TRY(allow_lds(k, lds));

@@ -5,6 +5,7 @@ import tempfile
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llama-vulkan_amd", "csrc")
 SOURCE = r"""
+#include "lv_bf_plan.h"
 #include "lv_small_plan.h"
 #include <cstdio>
 #include <iostream>
@@ -17,15 +18,23 @@ int main()
             std::cin >> m.D >> m.F >> m.heads >> m.rot >> m.layers >> m.vocab >> m.block_bytes;
             const lv::SmallPlan p = lv::small_plan(m);
             printf("%u %u %u\n", p.wgs, p.own, p.elements);
+        } else if (what == "product") {
+            uint32_t rows, n, kp, slices;
+            std::cin >> rows >> n >> kp >> slices;
+            const lv::BfPlan p = lv::bf_plan(rows, n, kp, slices);
+            printf("%d %u\n", (int)p.tiles, p.slices);
         }
     }
 }
 """
 _exe = []
+TILES = ("128x128", "256x128", "256x160", "256x192", "256x256")
 
 
 def ask(lines):
-    """a list of answers, tuples of numbers, to questions: ("small", dim, ff, heads, head size, layers, vocab, bytes of a block)"""
+    """a list of answers, tuples of numbers, to questions:
+    ("small", dim, ff, heads, head size, layers, vocab, bytes of a block) -> workgroups, blocks of a workgroup, cache elements
+    ("product", rows, tokens, columns, slices at most) -> TILES, slices"""
     if not _exe:
         d = tempfile.TemporaryDirectory()
         src, exe = os.path.join(d.name, "main.cpp"), os.path.join(d.name, "main")

@@ -40,12 +40,21 @@ def check_last(d, toks, want, tol):
 # tokens one beside a tile's edge; feed-forwards whose way down is cut into 2 and 4 slices, the last one shorter
 DENSE = [(40, 4100, 1100), (130, 2060, 1030), (700, 2060, 1025), (700, 4100, 1281), (300, 1100, 129), (300, 2113, 127), (257, 4160, 257),
          (1030, 3000, 255), (128, 2048, 513), (129, 1025, 65)]
-# 128 x 128 tiles in 3 slices; 256 x 128 in 1, 2, 3 and 4; 256 x 256 in 3; the last slice shorter
-DENSE += [(1536, 2500, 700), (4100, 1100, 900), (3000, 2060, 900), (2500, 2500, 777), (1536, 3000, 900), (4100, 3000, 900)]
-# 256 rows x 160 and x 192 tokens, every number of units of 32 tokens that a rest may have, one token beside a unit's end; 160 in two slices
+# products down in 1 to 4 slices (what the plan takes of each: test_host_plans.py)
+DENSE += [(1536, 2500, 700), (4100, 1100, 900), (3000, 2060, 900), (2500, 2500, 777), (1536, 3000, 900), (4100, 3000, 900), (4102, 2500, 897)]
+# few columns and many rows: 128 x 128, a rest of every number of units of 32 tokens
 DENSE += [(70, 5500, 641), (70, 7000, 513), (70, 8200, 385), (70, 11008, 257), (70, 8200, 449), (70, 4100, 960)]
 DENSE += [(70, 10240, 961), (70, 5500, 801), (70, 7000, 641), (70, 11008, 289), (70, 11008, 321), (70, 11008, 353)]
-DENSE += [(4102, 2500, 897)]
+# gate and up in 256 rows x 128, 160, 192 and 256 tokens: no rest, and rests of every number of units of 32, one token beside a unit's end
+WIDE_DENSE = [(2875, 286, 129), (4418, 306, 161), (929, 8448, 193), (1143, 8440, 225), (1103, 4325, 512)]
+WIDE_DENSE += [(327, 8923, 480), (323, 5868, 641), (327, 6574, 513), (325, 8533, 385), (321, 8272, 417), (367, 8343, 449)]
+WIDE_DENSE += [(257, 6324, 960), (260, 4994, 961), (393, 5410, 801), (261, 6857, 641), (385, 8237, 481), (129, 8953, 1281), (277, 6360, 929)]
+WIDE_DENSE += [(322, 7533, 1024), (326, 5958, 1025), (329, 8097, 801), (325, 6622, 897), (327, 6373, 1009)]
+# ... of 2 and 3 K steps, as many as the stages
+WIDE_DENSE += [(100, 15500, 1793), (100, 15000, 1921), (150, 16500, 1793), (150, 12500, 1921), (150, 12500, 897), (150, 10500, 1921)]
+# down in one slice of 160, 192 and 256 tokens, and in slices of 128, 160 and 192 of which the last one is shorter
+WIDE_DENSE += [(5995, 505, 1291), (8329, 505, 1122), (7681, 405, 1559), (7188, 1447, 257), (8815, 1760, 129), (5660, 2742, 129), (8281, 1540, 385), (7180, 4288, 257), (6414, 1974, 641)]
+DENSE += WIDE_DENSE
 # streams so wide that the sum of slices and the norm's input would not fit LDS side by side
 DENSE += [(20544, 1152, 33)]
 

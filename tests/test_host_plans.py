@@ -1,8 +1,9 @@
 """Rules that choose between kernels by sizes, on both sides of their borders, and the sizes that other tests rely on."""
 import pytest
 
+import test_gpu_block_tiles
 import test_gpu_small
-from plan_query import ask
+from plan_query import TILES, ask
 
 Q4, Q8 = 18, 34
 
@@ -57,3 +58,45 @@ def test_small_shapes_of_the_gpu_tests_take_the_ways_they_are_there_for():
             if wgs:
                 assert own == {"three blocks a row": 1, "one head, one block": 1, "head of 128": 1, "a block a workgroup": 1, "workgroups without blocks": 1,
                                "widest with partial sums": 1, "two columns a lane": 2, "two blocks a workgroup": 2}.get(name, 0), name
+
+
+def up(v, a):
+    return (v + a - 1) // a * a
+
+
+def dense_plans(shapes):
+    """of gate and up, and of down, in a feed-forward of (width, ff) and n tokens: tile, slices, K steps of a slice, units of 32 tokens in the rest"""
+    asked = []
+    for width, ff, n in shapes:
+        rows = up(2 * up(ff, 16), 128)
+        asked += [("product", rows, n, up(width, 64), 1), ("product", width, n, rows // 2, 4 if n <= 1024 else 1)]
+    for (_, rows, n, columns, _), (tile, slices) in zip(asked, ask(asked)):
+        yield TILES[tile], slices, columns // 64, -(-(n % int(TILES[tile][4:])) // 32)
+
+
+def test_dense_shapes_of_the_gpu_tests_reach_every_tile():
+    """with every rest of whole units: each is a loop of its own.  A plan that moves has to move the shapes too"""
+    plans = list(dense_plans(test_gpu_block_tiles.DENSE))
+    dense, store = plans[::2], plans[1::2]
+    for tile, units in ("256x128", 4), ("256x160", 5), ("256x192", 6):
+        assert {p[3] for p in dense if p[0] == tile} >= set(range(units)), tile
+    assert {p[3] for p in dense if p[0] == "256x256"} >= {0, 1, 2, 5, 8}      # its rests share one loop; a whole 128 tokens missing, and less
+    for tile, steps in ("128x128", 1), ("256x128", 3), ("256x160", 3), ("256x192", 2), ("256x256", 2):
+        assert min(p[2] for p in dense if p[0] == tile) <= steps, tile
+    for tile, slices in ("128x128", {1, 2, 3, 4}), ("256x128", {1, 2, 3, 4}), ("256x160", {1, 2, 4}), ("256x192", {1, 2}), ("256x256", {1}):
+        assert {p[1] for p in store if p[0] == tile} >= slices, tile
+    for tile in "128x128", "256x128", "256x160", "256x192":
+        assert any(p[0] == tile and p[1] > 1 and p[2] % p[1] for p in store), tile      # a last slice that is shorter
+
+
+@pytest.mark.parametrize("rows,n,columns,slices,want", [
+    # few workgroups take as long a step as they load: 128 x 128 (256 x 128 1.2 times as long)
+    (5248, 100, 5120, 1, ("128x128", 1)), (5248, 256, 5120, 1, ("128x128", 1)), (3200, 128, 3072, 1, ("128x128", 1)), (7296, 512, 7168, 1, ("128x128", 1)),
+    # slices of long rows in tiles of 160 tokens took 1.6 times what they were thought to
+    (7168, 460, 19392, 4, ("256x128", 2)), (7168, 512, 18432, 4, ("256x128", 2)),
+    # large products
+    (18560, 500, 4096, 1, ("256x192", 1)), (13600, 2048, 4096, 1, ("256x256", 1)), (8848, 1000, 2048, 1, ("256x160", 1)),
+])
+def test_tiles_of_products(rows, n, columns, slices, want):
+    tile, got = ask([("product", rows, n, columns, slices)])[0]
+    assert (TILES[tile], got) == want
