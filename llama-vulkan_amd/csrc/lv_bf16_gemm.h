@@ -285,14 +285,14 @@ __device__ __forceinline__ void bf_store_wave(const BfGemmArgs &a, const lv_f4 (
     }
 }
 
-template <int EP>
+template <int EP, bool GROUPED>
 __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(BfGemmArgs a)
 {
     constexpr int RM = kBfRows, STAGE = (RM + kBfTile) * kBfStep * 2;
     constexpr int LW = RM / 32, LX = kBfTile / 32;          // direct loads per wave and stage, 8 rows (1 KB) each
     extern __shared__ __attribute__((aligned(128))) uint8_t bf_lds[];
     uint32_t rt, expert, first, count;
-    if (!bf_tile<false>(a, kBfTile, rt, expert, first, count)) return;
+    if (!bf_tile<GROUPED>(a, kBfTile, rt, expert, first, count)) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, g4 = lane >> 4;
     const uint32_t kp = a.kp;
@@ -300,11 +300,16 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_kernel(BfGemmArgs a)
     const uint16_t *gw, *gx[LX];
     {
         const int r8 = lane >> 3, c = (lane & 7) ^ r8;
-        gw = a.w + ((size_t)rt * RM + wave * (RM / 4) + r8) * kp + c * 8;
+        gw = a.w + ((size_t)expert * a.expert_rows + (size_t)rt * RM + wave * (RM / 4) + r8) * kp + c * 8;
 #pragma unroll
         for (int i = 0; i < LX; i++) {
             const int row = wave * (kBfTile / 4) + i * 8 + r8;
-            gx[i] = static_cast<const uint16_t *>(a.x) + ((size_t)first + row) * a.ldx + c * 8;
+            size_t xr = (size_t)first + row;
+            if constexpr (GROUPED) {
+                const uint32_t p = first + min((uint32_t)row, count - 1);
+                xr = a.gather ? a.slots[p] / a.top : p;
+            }
+            gx[i] = static_cast<const uint16_t *>(a.x) + xr * a.ldx + c * 8;
         }
     }
     const uint32_t k_lo = EP == kEpStore && a.k_slice ? blockIdx.z * a.k_slice : 0;

@@ -77,28 +77,49 @@ inline BfPlan bf_plan(uint32_t rows, uint32_t n, uint32_t kp, uint32_t slices)
     return best;
 }
 
-// Tokens of an expert's tiles, 128 or 160, and their order.  us of gate and up, and of down (64 experts, 8 a token, 2048 x 4096 and
-// 4096 x 1024): tiles of 128, a row tile after the other, then an expert after the other; tiles of 160 likewise.
-//    300 tokens            239 180 241 179   127 121 127 121
-//    900                   273 240 265 199   168 170 166 161
-//   1400                   280 250 327 310   227 198 228 221
-//   2048                   372 356 329 309   259 281 270 242
-//    600, unevenly chosen  226 214 226 219   136 142 133 148
-//   2048, unevenly chosen  356 364 344 372   272 282 257 279
-// Few tokens an expert: the weights' way from HBM counts, an expert after the other; 160 where an expert of the mean number of choices
-// and two standard deviations more then has fewer tiles, and where every round of workgroups is not one of few (32 experts, 4 a token, 2048
-// x 2048 and 2048 x 1024, 900 tokens: 128 85 and 52, 160 92 and 62).  Down of 48 tokens an expert and more in tiles of 128: its weights are half
-// as many and uneven experts decide (512 tokens of a prompt, unevenly chosen: 135 and 146).  Many: runs of one length whoever is chosen.
+// A layer's two products of chosen experts, over tiles of at most kBfTile tokens, an expert's each: 128 x 128 or 256 rows x 128
 struct ExpertPlan {
-    uint32_t tile;
-    bool by_expert, down_by_expert;
+    BfTiles gate_up, down;
+    bool gate_up_by_expert;      // an expert after the other, not a row tile after the other
 };
-inline ExpertPlan expert_plan(uint32_t n, uint32_t top, uint32_t experts, uint32_t rows)
+struct ExpertShape {
+    uint32_t experts, top, rows, kp, down_rows, down_kp;      // rows: of an expert's gate and up
+};
+// How many tiles an expert has: choices spread about their mean as a normal variable, a little wider than even chances make them
+inline double expert_tiles(double mean, uint32_t tile)
 {
-    const double mean = (double)n * top / experts, many = mean + 2 * std::sqrt(mean);
-    if (mean >= 192) return {160, false, false};
-    const bool longer = experts * ((rows + 255) / 256) >= 512 && std::ceil(many / 160) < std::ceil(many / 128);
-    return {longer ? 160u : 128u, true, longer || mean < 48};
+    const double spread = std::sqrt(2 * (mean + 0.03 * mean * mean));
+    double tiles = 1 - std::exp(-mean);
+    for (uint32_t k = 1; k < 4096; k++) {
+        const double p = 0.5 * std::erfc((k * (double)tile + 0.5 - mean) / spread);
+        if (p < 1e-3) break;
+        tiles += p;
+    }
+    return tiles;
+}
+// By the estimate of bf_plan, the ends of wide tiles longer still: an expert's rows are gathered, and its tiles end at other times than others'.
+// Us a layer in prompts of models of several layers (experts, a token's, feed-forward x width, tokens), 256 rows x 128, a row tile after the other,
+// and what is more or less with: gate and up an expert after the other; 128 x 128 tiles of gate and up, of down; 256 rows x 160 tokens
+//   8, 2, 512 x 1024       100  155    -0   -2  -5    +1      512  197   -0   -2   -5   +11     1600  339    0   -2   -5   +11
+//   16, 4, 512 x 512       100  139    -1   -4  -5     0      512  174    0   -3   -5    +9     1600  292    0   -2   -4    +9
+//   64, 8, 512 x 2048      100  254     0   -1  -1    +1      512  358   -1   +6   -5    +4     1600  631   +2   +9   +1    -7
+//   32, 4, 1024 x 2048     128  255    -2   -3  -4    +1      512  345   +3   +7   -1    -2     1600  604   +5   +9   +4   -14
+//   64, 8, 1024 x 4096     100  522   -26  -10 -10    -2      512  692  +12  +32   +8    +1     1600 1304  +13  +48  +10   -14
+//   128, 8, 768 x 4096     100  550    -3   +1  -1     0      512  778   -8  +11   +1   +29     1600 1383   +2  +42   +3    +8
+//   8, 2, 7168 x 4096      100  530    +7   +2  -2    -2      512  685  +70  +33  +11    +8     1600 1403 +178  +61  +18   +28
+//   16, 2, 2048 x 8192     100  676    +4   +6  +3    -1      512 1021  +16  +37   +7    +6     1600 2271  +41  +43  +27   -63
+// An expert after the other reads weights as one run, which counts while there is little else to do; experts that are chosen unevenly then make
+// unequal runs for the XCDs.  Tiles of 160 tokens gain where more than 128 choose most experts and fewer than 160, which the mean does
+// not tell: 1.2 % slower in the mean of these and 280 more.
+inline ExpertPlan expert_plan(uint32_t n, const ExpertShape &e)
+{
+    constexpr double kEnds = 10;
+    const double mean = (double)n * e.top / e.experts, tiles = e.experts * expert_tiles(mean, kBfTile), share = std::fmin(1.0, (double)n * e.top / (tiles * kBfTile) + 0.125);
+    auto kind = [&](uint32_t rows, uint32_t kp) {
+        const double steps = kp / kBfStep, wide = bf_wide_step(kBfOffers[0], (rows + 255) / 256 * tiles) * bf_part(share) * steps + kEnds;
+        return bf_small_step((rows + 127) / 128 * tiles) * steps < wide ? BfTiles::k128 : BfTiles::kWide;
+    };
+    return {kind(e.rows, e.kp), kind(e.down_rows, e.down_kp), e.experts >= 128 || (e.experts >= 64 && mean < 32)};
 }
 
 }  // namespace lv

@@ -830,11 +830,10 @@ template <int EP, bool GROUPED, int WN> static int launch_wide(hipStream_t st, B
     return launch_bf(st, &gemm_wide_kernel<EP, GROUPED, WN>, a, wide_lds_bytes(WN));
 }
 
-// a product of n tokens.  `plan`: its tiles where they are settled already.  Grouped: `tile` tokens at most a tile of the list
-template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t experts = 1, uint32_t tile = kBfTile, const BfTiles *plan = nullptr)
+// a product of n tokens.  `plan`: its tiles where they are settled already, as an expert's are
+template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w, uint32_t n, uint32_t experts = 1, const BfTiles *plan = nullptr)
 {
-    if (f32) tile = kF32Tile;
-    const uint32_t token_tiles = (n + tile - 1) / tile;
+    const uint32_t tile = f32 ? kF32Tile : kBfTile, token_tiles = (n + tile - 1) / tile;
     a.w = w.w;
     a.kp = w.kp;
     a.rows = w.rows;
@@ -847,7 +846,9 @@ template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemm
         return LV_OK;
     }
     if constexpr (GROUPED) {
-        return tile == kBfTile ? launch_wide<EP, true, 64>(st, a) : launch_wide<EP, true, 80>(st, a);
+        if (*plan == BfTiles::kWide) return launch_wide<EP, true, 64>(st, a);
+        a.row_tiles = (w.rows + kBfRows - 1) / kBfRows;
+        return launch_bf(st, &gemm_bf16_kernel<EP, true>, a, kBfLdsBytes);
     } else {
         if constexpr (EP != kEpDecay && EP != kEpSigmoid) {      // those two have a few K steps only
             switch (plan ? *plan : a.k_slice ? BfTiles::k128 : bf_plan(w.rows, n, w.kp, 1).tiles) {
@@ -859,7 +860,7 @@ template <int EP, bool GROUPED> static int gemm(hipStream_t st, bool f32, BfGemm
             }
         }
         a.row_tiles = (w.rows + kBfRows - 1) / kBfRows;
-        return launch_bf(st, &gemm_bf16_kernel<EP>, a, kBfLdsBytes);
+        return launch_bf(st, &gemm_bf16_kernel<EP, false>, a, kBfLdsBytes);
     }
 }
 
@@ -880,7 +881,7 @@ static int gemm_output(hipStream_t st, bool f32, BfGemmArgs a, const BfMatrix &w
     }
     a.ldo = dp * p.slices;
     *slices = p.slices;
-    return gemm<kEpStore, false>(st, f32, a, w, n, 1, kBfTile, &p.tiles);
+    return gemm<kEpStore, false>(st, f32, a, w, n, 1, &p.tiles);
 }
 
 // calls fn(element, integral constant DP, integral constant R) for a layer's attention
@@ -1646,17 +1647,17 @@ static int step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx
         LV_TRY((gemm<kEpStore, false>(st, f32, rt, l.router, n)));
         route_rows_kernel<<<dim3(n), dim3(64), e.experts * 4ull, st>>>(w.z, ldz, z_parts, rt.slice_floats, e.experts, e.top, w.ids, w.scores);
         HIP_TRY(hipGetLastError());
-        const ExpertPlan plan = f32 ? ExpertPlan{kF32Tile, false, false} : expert_plan(n, e.top, e.experts, l.gu_rows);
-        sort_experts_kernel<<<dim3(1), dim3(1024), e.experts * 8ull, st>>>(w.ids, total, e.experts, plan.tile, w.slots, w.tiles);
+        const ExpertPlan plan = expert_plan(n, {e.experts, e.top, l.gu_rows, Dp, l.down_rows, l.down.kp});
+        sort_experts_kernel<<<dim3(1), dim3(1024), e.experts * 8ull, st>>>(w.ids, total, e.experts, f32 ? kF32Tile : kBfTile, w.slots, w.tiles);
         HIP_TRY(hipGetLastError());
         BfGemmArgs gu{};
-        gu.x = w.act; gu.ldx = Dp; gu.tiles = w.tiles; gu.slots = w.slots; gu.weights = w.scores; gu.top = e.top; gu.expert_rows = l.gu_rows; gu.gather = true; gu.by_expert = plan.by_expert;
+        gu.x = w.act; gu.ldx = Dp; gu.tiles = w.tiles; gu.slots = w.slots; gu.weights = w.scores; gu.top = e.top; gu.expert_rows = l.gu_rows; gu.gather = true;
+        gu.by_expert = !f32 && plan.gate_up_by_expert;
         gu.act = w.ff; gu.lda = l.down.kp;
-        LV_TRY((gemm<kEpGlu, true>(st, f32, gu, l.gate_up, total, e.experts, plan.tile)));
+        LV_TRY((gemm<kEpGlu, true>(st, f32, gu, l.gate_up, total, e.experts, &plan.gate_up)));
         BfGemmArgs dn{};
         dn.x = w.ff; dn.ldx = l.down.kp; dn.tiles = w.tiles; dn.slots = w.slots; dn.top = e.top; dn.expert_rows = l.down_rows; dn.out = w.y; dn.ldo = Dp;
-        dn.by_expert = plan.down_by_expert;
-        LV_TRY((gemm<kEpScatter, true>(st, f32, dn, l.down, total, e.experts, plan.tile)));
+        LV_TRY((gemm<kEpScatter, true>(st, f32, dn, l.down, total, e.experts, &plan.down)));
         parts = e.top;
     }
     if (trace || logits_all) {

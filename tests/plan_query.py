@@ -23,6 +23,12 @@ int main()
             std::cin >> rows >> n >> kp >> slices;
             const lv::BfPlan p = lv::bf_plan(rows, n, kp, slices);
             printf("%d %u\n", (int)p.tiles, p.slices);
+        } else if (what == "experts") {
+            uint32_t n;
+            lv::ExpertShape e;
+            std::cin >> n >> e.experts >> e.top >> e.rows >> e.kp >> e.down_rows >> e.down_kp;
+            const lv::ExpertPlan p = lv::expert_plan(n, e);
+            printf("%d %d %d\n", (int)p.gate_up, (int)p.down, (int)p.gate_up_by_expert);
         }
     }
 }
@@ -34,7 +40,8 @@ TILES = ("128x128", "256x128", "256x160", "256x192", "256x256")
 def ask(lines):
     """a list of answers, tuples of numbers, to questions:
     ("small", dim, ff, heads, head size, layers, vocab, bytes of a block) -> workgroups, blocks of a workgroup, cache elements
-    ("product", rows, tokens, columns, slices at most) -> TILES, slices"""
+    ("product", rows, tokens, columns, slices at most) -> TILES, slices
+    ("experts", tokens, experts, of a token, rows, columns, rows, columns) -> TILES of gate and up, of down, gate and up an expert after the other"""
     if not _exe:
         d = tempfile.TemporaryDirectory()
         src, exe = os.path.join(d.name, "main.cpp"), os.path.join(d.name, "main")

@@ -85,8 +85,14 @@ def test_slices_do_not_hang_on_what_came_before(lva, ctx):
             assert np.array_equal(d.run(toks, (n,)), first), n
 
 
-@pytest.mark.parametrize("width,ff,n,experts,top", [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4), (64, 24, 17, 3, 2),
-                                                      (130, 520, 230, 4, 2), (70, 300, 375, 3, 2)])      # tiles of 160 tokens
+# what the plan takes of each: test_host_plans.py
+EXPERTS = [(130, 1100, 900, 4, 2), (40, 2050, 513, 9, 3), (700, 700, 1281, 5, 2), (257, 130, 1030, 12, 4), (64, 24, 17, 3, 2), (130, 520, 230, 4, 2), (70, 300, 375, 3, 2)]
+# gate and up, down in tiles of 256 rows, one or several an expert; an expert after the other, with either tile, one or several
+EXPERTS += [(2886, 126, 52, 5, 2), (2080, 847, 539, 12, 3), (167, 2357, 43, 32, 2), (677, 2191, 1210, 24, 3), (138, 1381, 212, 130, 4), (1030, 200, 2000, 128, 9),
+            (40, 24, 1900, 128, 9), (103, 94, 116, 130, 4)]
+
+
+@pytest.mark.parametrize("width,ff,n,experts,top", EXPERTS)
 def test_expert_tiles(lva, ctx, width, ff, n, experts, top):
     cfg = bb.config(width=width, layers=[bb.layer(experts=experts, top=top, ff=ff)])
     W = bb.weights(cfg, seed=n)

@@ -89,6 +89,36 @@ def test_dense_shapes_of_the_gpu_tests_reach_every_tile():
         assert any(p[0] == tile and p[1] > 1 and p[2] % p[1] for p in store), tile      # a last slice that is shorter
 
 
+def experts(width, ff, n, count, top):
+    rows = up(2 * up(ff, 16), 128)
+    gate_up, down, by_expert = ask([("experts", n, count, top, rows, up(width, 64), up(width, 128), rows // 2)])[0]
+    return TILES[gate_up], TILES[down], bool(by_expert)
+
+
+def test_expert_shapes_of_the_gpu_tests_reach_every_tile_and_order():
+    seen = set()
+    for width, ff, n, count, top in test_gpu_block_tiles.EXPERTS:
+        gate_up, down, by_expert = experts(width, ff, n, count, top)
+        several = n * top > 128 * count
+        seen |= {("gate_up", gate_up, by_expert, several), ("down", down, several)}
+    assert seen == {("gate_up", t, o, s) for t in ("128x128", "256x128") for o in (False, True) for s in (False, True)} | {
+        ("down", t, s) for t in ("128x128", "256x128") for s in (False, True)}
+
+
+@pytest.mark.parametrize("width,ff,count,top,n,want", [
+    # small experts: 128 x 128 (256 rows x 128 or 160 tokens were 3 to 8 % of a prompt slower)
+    (1024, 512, 8, 2, 100, ("128x128", "128x128", False)), (1024, 512, 8, 2, 777, ("128x128", "128x128", False)), (512, 512, 16, 4, 512, ("128x128", "128x128", False)),
+    (1024, 512, 32, 4, 512, ("128x128", "128x128", False)),
+    # large ones: 256 x 128, a row tile after the other (an expert after the other up to 10 % slower)
+    (4096, 7168, 8, 2, 512, ("256x128", "256x128", False)), (4096, 7168, 8, 2, 1300, ("256x128", "256x128", False)), (8192, 2048, 16, 2, 640, ("256x128", "256x128", False)),
+    (2048, 1024, 32, 4, 900, ("256x128", "128x128", False)), (4096, 1024, 64, 8, 512, ("256x128", "256x128", False)), (4096, 1024, 64, 8, 2048, ("256x128", "256x128", False)),
+    # few tokens of many experts: an expert after the other
+    (4096, 1024, 64, 8, 100, ("256x128", "256x128", True)), (4096, 768, 128, 8, 640, ("256x128", "256x128", True)),
+])
+def test_tiles_of_chosen_experts(width, ff, count, top, n, want):
+    assert experts(width, ff, n, count, top) == want
+
+
 @pytest.mark.parametrize("rows,n,columns,slices,want", [
     # few workgroups take as long a step as they load: 128 x 128 (256 x 128 1.2 times as long)
     (5248, 100, 5120, 1, ("128x128", 1)), (5248, 256, 5120, 1, ("128x128", 1)), (3200, 128, 3072, 1, ("128x128", 1)), (7296, 512, 7168, 1, ("128x128", 1)),

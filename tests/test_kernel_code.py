@@ -90,4 +90,4 @@ def test_nothing_moves_between_matrix_products_of_tiles_with_units(code_objects)
                     if x == "s_nop 15":
                         inside, halves = False, halves + 1
             assert not inside and halves == 2 * (5 if "ELi80E" in name else 6), (name, halves)
-    assert seen == 8      # three epilogues of each, and of 160 tokens the experts' two
+    assert seen == 6      # three epilogues of each
