@@ -2721,6 +2721,10 @@ static int launch_short_norm(hipStream_t st, const ShortBuffers &b, const float 
     return LV_OK;
 }
 
+// Floats of a head's parts up to which the workgroup that arrives last adds them up instead of a launch of its own.  us a layer with it against
+// the launch, means of 14 models, 2 to 15 tokens behind 70 to 3900 rows: heads of 64 and 32 -1.3, and -1.0 at their most (15360); heads of 128 up
+// to 10000 -0.9, 13000 to 15000 -0.5, 15000 to 18000 -0.3, 18000 to 20000 0, 23000 and more +0.5 (+1.6 at most, 12 heads, 15 tokens behind 1900).
+constexpr uint32_t kShortLastFloats = 18000;
 static int launch_short_attention(hipStream_t st, const lv_session *s, const ShortBuffers &b, uint32_t layer, uint32_t pos, uint32_t n, uint32_t ftype)
 {
     const lv_hparams &hp = s->model->hp;
@@ -2742,7 +2746,7 @@ static int launch_short_attention(hipStream_t st, const lv_session *s, const Sho
     a.kcache = kv_ptr(s, layer, 0); a.vcache = kv_ptr(s, layer, 1); a.q = b.q; a.trig_abs = s->trig_abs;
     a.pos0 = pos; a.n = n; a.heads = hp.heads; a.backlog = s->backlog; a.tiles_per_split = per; a.num = b.num; a.den = b.den;
     a.tiles = short_tiles(n); a.q8 = ftype == LV_Q8_0; a.counters = b.counters;
-    if (splits == 1 || n < kPrefillMin) a.act = b.act;
+    if (splits == 1 || (n < kPrefillMin && n * splits * hp.rot <= kShortLastFloats)) a.act = b.act;
     const size_t lds = (size_t)512 * hp.rot;
     switch (hp.rot) {
 #define LV_SHORT_ATTN(R)                                                                                                              \

@@ -640,7 +640,7 @@ struct ShortAttnArgs {
     uint32_t pos0, n, heads, backlog;  // row z sits at pos0 + z
     uint32_t tiles_per_split;          // tiles of 64 positions
     float *num, *den;
-    uint8_t *act;                      // the output projection's activations, `tiles` token tiles; short_attn_kernel: with one split, in place of num and den
+    uint8_t *act;                      // the output projection's activations, `tiles` token tiles, or null: num and den are for short_attn_combine_kernel
     uint32_t *counters;                // short_attn_exact_kernel: one a head, zero before and after
     uint32_t tiles, q8;
 };
@@ -1073,7 +1073,7 @@ __global__ __launch_bounds__(256, 2) void short_attn_exact_kernel(ShortAttnArgs 
         __hip_atomic_store(p + 1, __builtin_bit_cast(uint64_t, make_float2(s.z, s.w)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if ((uint32_t)t < a.n) st_dev(a.den + (part + t) * H + h, weight(t));
-    short_attn_last<R>(a, h);
+    if (a.act) short_attn_last<R>(a, h);
 }
 
 // numerators and denominators of all splits, in order -> the output projection's activations.  grid (D / 8 / 256 rounded up, n)

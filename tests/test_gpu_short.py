@@ -105,9 +105,10 @@ def test_attention_of_short_steps_behind_long_contexts(lva, ctx, tmp_path, befor
 
 
 @pytest.mark.parametrize("rot,heads", [(32, 4), (64, 8), (128, 3)])
-@pytest.mark.parametrize("before,n", [(63, 2), (64, 15), (1500, 2), (1500, 15)])
+@pytest.mark.parametrize("before,n", [(63, 2), (64, 15), (800, 10), (800, 11), (1500, 2), (1500, 15)])
 def test_parts_of_short_attention_put_together_by_the_last(lva, ctx, tmp_path, rot, heads, before, n):
-    """two parts and the most there are, fewest and most tokens; two layers and two steps, so that a count left over would show"""
+    """two parts and the most there are, fewest and most tokens; two layers and two steps, so that a count left over would show.  Of heads of 128
+    the last part to arrive adds up 10 tokens behind 800 rows, a launch of its own 11"""
     path = str(tmp_path / "heads.ggml")
     lva.write_model(path, wtype=lva.LV_Q4_0, seed=12, vocab=512, dim=rot * heads, heads=heads, layers=2, ff=512)
     model = lva.Model(ctx, path)
