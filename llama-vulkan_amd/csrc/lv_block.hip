@@ -787,15 +787,16 @@ template <int MODE, int INPUT, int R, int DEPTH> static int launch_gemv(hipStrea
     return LV_OK;
 }
 
+// rows of the busiest wave, which walks r of them together
+static uint32_t gemv_rows_in_turn(uint32_t units, uint32_t r)
+{
+    constexpr uint32_t kWaves = 16 * 256;
+    return ((units + r - 1) / r + kWaves - 1) / kWaves * r;
+}
 // Rows a wave walks together: two where there are enough of them, one where the last round of waves would then be far from full
 // (us for two and one: 32000 x 4096 40.9 and 42.5, 16384 x 4096 22.5 and 23.5, 32000 x 2048 22.0 and 23.1, 9000 x 4096 16.3 and 15.4,
 // 8848 x 2048 9.4 and 8.3).
-static uint32_t gemv_rows_together(uint32_t units)
-{
-    constexpr uint32_t kWaves = 16 * 256;
-    auto rows_in_turn = [&](uint32_t r) { return ((units + r - 1) / r + kWaves - 1) / kWaves * r; };      // of the busiest wave
-    return units < 8192 || rows_in_turn(1) * 4 <= rows_in_turn(2) * 3 ? 1 : 2;
-}
+static uint32_t gemv_rows_together(uint32_t units) { return units < 8192 || gemv_rows_in_turn(units, 1) * 4 <= gemv_rows_in_turn(units, 2) * 3 ? 1 : 2; }
 
 template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs &a)
 {
@@ -803,11 +804,16 @@ template <int MODE, int INPUT> static int gemv(hipStream_t st, const BfGemvArgs 
                        (INPUT == kInGroups ? group_sums(a.group.groups, gemv_waves(INPUT)) * 4ull : 0);
     // Three or four loads of a wave ahead: enough while every one of them is waited for by itself, and what is asked for first keeps the
     // input waiting.  us, one row, 2, 3, 4, 5 and 8 ahead: 8848 x 2048 9.0 8.3 8.5 8.9 10.3; 18560 x 4096 behind four streams 27.9 27.8 27.5 28.4
-    // 29.0; 6144 x 1536 5.7 5.7 5.9 7.0 7.1; two rows, 1, 2, 3 and 4 ahead: 32000 x 2048 22.0 22.0 22.1 22.5.  Pairs of gate and up one at a
-    // time (two, one: 8 experts of 2048 x 4096 25.6 and 23.2, 22016 x 4096 32.7 and 30.8), and so a workgroup of 16 waves.
+    // 29.0; 6144 x 1536 5.7 5.7 5.9 7.0 7.1; two rows, 1, 2, 3 and 4 ahead: 32000 x 2048 22.0 22.0 22.1 22.5.  Experts' pairs of gate and up one
+    // at a time (two, one: 8 experts of 2048 x 4096 25.6 and 23.2), and so the rows of a workgroup of 16 waves.  Pairs of a dense feed-forward two
+    // at a time where no wave then has more of them, in a token's layer: us more or less than one at a time with three loads ahead, one with two
+    // ahead, two: 27648 x 5120 -1.2 -3.4, 28672 x 4096 -0.7 -2.0, 44032 x 8192 -0.5 -7.8, 11008 x 2048 -0.5 -0.7; otherwise 22016 x 4096 -0.2 +3.0,
+    // 36864 x 7168 -2.0 +4.7, 5632 x 1024 -0.4 +0.9.
     if constexpr (MODE == kGemvExperts) return launch_gemv<MODE, INPUT, 1, 3>(st, a, a.top * (a.expert_rows / 2), lds);
-    else if constexpr (MODE == kGemvGlu) return launch_gemv<MODE, INPUT, 1, 3>(st, a, a.rows / 2, lds);
-    else {
+    else if constexpr (MODE == kGemvGlu) {
+        const uint32_t units = a.rows / 2;
+        return gemv_rows_in_turn(units, 2) <= gemv_rows_in_turn(units, 1) ? launch_gemv<MODE, INPUT, 2, 2>(st, a, units, lds) : launch_gemv<MODE, INPUT, 1, 2>(st, a, units, lds);
+    } else {
         if constexpr (gemv_threads(INPUT) == 512)
             if (gemv_rows_together(a.rows) == 2) return launch_gemv<MODE, INPUT, 2, 2>(st, a, a.rows, lds);
         return launch_gemv<MODE, INPUT, 1, 3>(st, a, a.rows, lds);
