@@ -30,6 +30,10 @@ struct BfOffer {
 };
 constexpr BfOffer kBfOffers[] = {{BfTiles::kWide, 128, 0.87, 0.76}, {BfTiles::kWide160, 160, 1.12, 0.87}, {BfTiles::kWide192, 192, 1.24, 0.88}, {BfTiles::kWidest, 256, 1.54, 1.27}};
 
+// 128 tokens, one round, half of them or fewer in the rest: its tile is done with a step sooner, runs ahead and brings the weights of its rows to
+// the L2 for the other tiles (5248 rows x 5120: 512 and 640 tokens 84 us, 900, seven tiles and four tokens, 72; measured from 512 rows on)
+constexpr double kBfAhead = 0.67;
+
 // us of a K step of all rounds
 inline double bf_small_step(double tiles)      // two share a CU
 {
@@ -68,7 +72,10 @@ inline BfPlan bf_plan(uint32_t rows, uint32_t n, uint32_t kp, uint32_t slices)
         for (const BfOffer &o : kBfOffers) {
             const uint32_t whole = n / o.tokens, rest = n % o.tokens, token_tiles = whole + (rest != 0);
             const double part = !rest ? 0.0 : o.tiles == BfTiles::kWidest ? 1.0 : bf_part((rest + 31) / 32 * 32.0 / o.tokens);
-            const double us = bf_wide_step(o, (double)((rows + 255) / 256) * token_tiles * s) * (whole + part) / token_tiles * steps + kBfWideEnds + more;
+            const double tiles = (double)((rows + 255) / 256) * token_tiles * s;
+            double step_us = bf_wide_step(o, tiles) * (whole + part) / token_tiles;
+            if (o.tiles == BfTiles::kWide && tiles <= kBfCus && whole && rest && rest <= 64 && rows >= 512) step_us = std::fmin(step_us, kBfAhead + 0.5 * (o.busy - kBfAhead) * tiles / kBfCus);
+            const double us = step_us * steps + kBfWideEnds + more;
             // 160 and 192 tokens, slices of long rows: up to 1.6 times the estimate (460 x 7168 x 19392, 160 in three 240, 128 in two 149), so only
             // where they gain more than a little
             take(o.tiles, s > 1 && (o.tokens == 160 || o.tokens == 192) ? 1.04 * us : us);

@@ -53,7 +53,7 @@ WIDE_DENSE += [(322, 7533, 1024), (326, 5958, 1025), (329, 8097, 801), (325, 662
 # ... of 2 and 3 K steps, as many as the stages
 WIDE_DENSE += [(100, 15500, 1793), (100, 15000, 1921), (150, 16500, 1793), (150, 12500, 1921), (150, 12500, 897), (150, 10500, 1921)]
 # down in one slice of 160, 192 and 256 tokens, and in slices of 128, 160 and 192 of which the last one is shorter
-WIDE_DENSE += [(5995, 505, 1291), (8329, 505, 1122), (7681, 405, 1559), (7188, 1447, 257), (8815, 1760, 129), (5660, 2742, 129), (8281, 1540, 385), (7180, 4288, 257), (6414, 1974, 641)]
+WIDE_DENSE += [(5995, 505, 1291), (8329, 505, 1122), (7681, 405, 1559), (7188, 1447, 257), (8815, 1760, 129), (5660, 2742, 129), (8251, 1675, 385), (7180, 4288, 257), (6524, 2700, 641)]
 DENSE += WIDE_DENSE
 # streams so wide that the sum of slices and the norm's input would not fit LDS side by side
 DENSE += [(20544, 1152, 33)]

@@ -122,6 +122,8 @@ def test_tiles_of_chosen_experts(width, ff, count, top, n, want):
 @pytest.mark.parametrize("rows,n,columns,slices,want", [
     # few workgroups take as long a step as they load: 128 x 128 (256 x 128 1.2 times as long)
     (5248, 100, 5120, 1, ("128x128", 1)), (5248, 256, 5120, 1, ("128x128", 1)), (3200, 128, 3072, 1, ("128x128", 1)), (7296, 512, 7168, 1, ("128x128", 1)),
+    # but with a rest that runs ahead of the other tiles of its rows
+    (2112, 777, 4096, 1, ("256x128", 1)), (5248, 900, 5120, 1, ("256x128", 1)),
     # slices of long rows in tiles of 160 tokens took 1.6 times what they were thought to
     (7168, 460, 19392, 4, ("256x128", 2)), (7168, 512, 18432, 4, ("256x128", 2)),
     # large products
