@@ -11,8 +11,8 @@
 // holds token l % 16 and four consecutive weight rows 4 * (l / 16) .. + 3, i.e. one 16-byte store into the token's row.
 //
 // Tiles, K step 64, both operands in LDS by direct loads, four waves:
-//   gemm_bf16_kernel        128 rows x 128 tokens, waves of 64 x 64, two stages, two workgroups a CU: few tiles, and short K
-//   gemm_wide_kernel<64>    256 rows x 128 tokens, waves of 128 x 64, three stages, one workgroup a CU
+//   gemm_bf16_kernel        128 rows x 128 tokens, waves of 64 x 64, two stages, two workgroups a CU: few tiles, and short K; small experts
+//   gemm_wide_kernel<64>    256 rows x 128 tokens, waves of 128 x 64, three stages, one workgroup a CU; large experts
 //   gemm_wide_kernel<80>    256 rows x 160 tokens, waves of 128 x 80, three stages
 //   gemm_wide_kernel<96>    256 rows x 192 tokens, waves of 128 x 96, two stages
 //   gemm_wide_kernel<128>   256 rows x 256 tokens, waves of 128 x 128 (all 256 accumulation registers), two stages
@@ -21,8 +21,9 @@
 // A 64 x 64 wave reads 8 KB of LDS per 16 matrix instructions, as long as those take, and the direct loads write LDS as well: LDS
 // bounds it at three quarters of the matrix rate.  Larger waves read 6 or 4 KB.  One wave per SIMD hides nothing by itself: the
 // wide kernels spell the order out, the next half step's operand reads and the direct loads one by one between the products.
-// Measured, us (TFLOP/s): 2048 tokens x 13600 x 4096 240 (952), 239 (957), 196 (1165); x 4096 x 8192
-// 130, 116, 154 (128 x 128, 256 x 128 and 256 x 256; all five: bf_plan).
+// Measured on one matrix again and again, which the infinity cache then holds, us (TFLOP/s): 2048 tokens x 13600 x 4096 240 (952), 239 (957),
+// 196 (1165); x 4096 x 8192 130, 116, 154 (128 x 128, 256 x 128 and 256 x 256).  On weights from HBM, as in a model: 279 (818), 250 (913), 217
+// (1052); 144, 123, 187 (all five tiles: lv_bf_plan.h).
 // A row of a tile is 128 bytes; its eight 16-byte chunks are stored in the order chunk ^ (row % 8), so that the 16 rows an MFMA
 // operand reads at one k spread over all banks.
 #pragma once
@@ -225,7 +226,7 @@ __device__ __forceinline__ void bf_store_glu(const BfGemmArgs &a, uint32_t posit
 // instead of two).  A run goes through the token tiles of one row tile after the other, so that an XCD reads a weight tile into its L2
 // once (the batch's rest behind all whole tiles instead, to fill gaps: 777 x 18560 x 4096 122 -> 129 us).
 // by_expert: through the row tiles of one token tile after the other.  An expert's token tiles read its weights at one time, gathered
-// activations come from L2 as well; but experts that are chosen unevenly then make unequal runs.
+// activations come from L2 as well; but experts that are chosen unevenly then make unequal runs (both measured: lv_bf_plan.h).
 template <bool GROUPED>
 __device__ __forceinline__ bool bf_tile(const BfGemmArgs &a, uint32_t tile_tokens, uint32_t &rt, uint32_t &expert, uint32_t &first, uint32_t &count)
 {

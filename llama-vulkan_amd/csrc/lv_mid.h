@@ -11,7 +11,8 @@
 //
 // Measured, us, 7B q8_0, gate and up: 48 tokens 47 -> 32 (three row tiles a workgroup, activations through registers, before), 128 tokens
 // 92 -> 54 (tiles of 256 rows x 128 tokens on the prompt copy, 88 workgroups); q, k and v 26 -> 22, 89 -> 39.  At 48 tokens the loads alone
-// take 28 (the weights alone 22, the activations alone 15), the arithmetic alone 20, launch and sum 7 of each.  The barrier in the
+// take 28 (the weights alone 22, the activations alone 15), the arithmetic alone 20, launch and sum 7 of each: loads bound it, the activations'
+// beside the weights' (vector units at work 42 % of the time, matrix cores 27).  The barrier in the
 // middle of a stage and everything read a token tile ahead instead of at its start: 128 tokens 60 -> 54.
 #pragma once
 
