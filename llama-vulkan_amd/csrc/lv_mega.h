@@ -408,6 +408,7 @@ __device__ __forceinline__ void gemv_phase(MegaTile (&q)[S::DEPTH], const MegaWa
     for (int i = 0; i < NT4; i++) {
         if (i < NT) {
             const int slot = (SEQ0 + i) % S::DEPTH;
+            behind_first(i, NT);
             const MegaTile t = q[slot];
             p[i & 3] = tile_dot<S>(t, xr, xsum);
             mw.fetch(q[slot], SEQ0 + i + S::DEPTH, layer);
@@ -435,6 +436,7 @@ __device__ __forceinline__ void gemv_phase_d(MegaTile (&q)[S::DEPTH], const Mega
     for (int i = 0; i < NT4; i++) {
         if (i < NT) {
             const int slot = (SEQ0 + i) % S::DEPTH;
+            behind_first(i, NT);
             const MegaTile t = q[slot];
             p[i & 3] = tile_dot<S>(t, xr, xsum);
             mw.fetch(q[slot], SEQ0 + i + S::DEPTH, layer);
@@ -891,6 +893,7 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
                 mega_e_tile<S>(w, i, row, slab);
                 if (i > 0 && i % S::E_SPARE_ROWS == 0 && w >= S::NSF) load_slab(xr, xsum, xs, slab * 64 + lane, slab * 64 + lane < S::NBF);
                 const int slot = (S::SEQ_E + i) % S::DEPTH;
+                behind_first(i, S::TE);
                 const MegaTile t = q[slot];
                 p[i & 3] = tile_dot<S>(t, xr, xsum);
                 mw.fetch(q[slot], S::SEQ_E + i + S::DEPTH, layer);
@@ -926,6 +929,7 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
 #pragma unroll
         for (int i = 0; i < S::HEAD; i++) {
             const int slot = i % S::DEPTH;
+            behind_first(i, S::HEAD);
             const MegaTile t = q[slot];
             p[i & 3] = tile_dot<S>(t, xr, xsum);
             mw.fetch_head(q[slot], i + S::DEPTH);
