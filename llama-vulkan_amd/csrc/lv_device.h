@@ -249,18 +249,23 @@ __device__ __forceinline__ float q8_block_dot(const uint4 &qa, const uint4 &qb, 
     return acc;
 }
 
-// A wave's place in the queue of its SIMD, by how far it is: step i of n.  Between two waves that could issue the older one goes first, so one
-// of a SIMD's two runs through its steps, then waits at the barrier with all it has asked for in registers, while the other walks the rest with
-// nobody to fill its gaps.  With a priority that falls by a level every eighth of the steps (four levels, twice over) the one that is behind goes
-// first, and both end together.  us a token of the persistent kernel without it and with, 7B q4_0 at position 511, 13B q4_0, 8 layers, at 287:
-// 970 945, 368 351; falling once over all steps 953 351, with every step 948 353, every other step 947 351, one level in the middle 954 355.
-__device__ __forceinline__ void behind_first(uint32_t i, uint32_t n)
+// step(0) .. step(N - 1), unrolled, with the wave's place in the queue of its SIMD by how far it is.  Between two waves that could issue the
+// older one goes first, so one of a SIMD's two runs through its steps, then waits at the barrier with all it has asked for in registers, while the
+// other walks the rest with nobody to fill its gaps.  With a priority that falls by a level every eighth of the steps (four levels, twice over) the
+// one that is behind goes first, and both end together.  us a token of the persistent kernel without it and with: 7B q4_0 at position 511 969 949,
+// q8_0, 8 layers, at 2039 429 426; 13B, 8 layers, q4_0 at 287 371 351, q8_0 at 511 560 550.  q4_0 of 7B and 13B in other steps: falling once over
+// all 953 351, with every step 948 353, every other one 947 351, one level in the middle 954 355.
+template <int N, int EIGHTH = 0, class Step>
+__device__ __forceinline__ void behind_first(Step &&step)
 {
-    switch (i * 8 / n & 3) {
-    case 0: __builtin_amdgcn_s_setprio(3); break;
-    case 1: __builtin_amdgcn_s_setprio(2); break;
-    case 2: __builtin_amdgcn_s_setprio(1); break;
-    default: __builtin_amdgcn_s_setprio(0); break;
+    if constexpr (EIGHTH < 8) {
+        constexpr int from = (EIGHTH * N + 7) / 8, to = (EIGHTH * N + N + 7) / 8;
+        if constexpr (from < to) {
+            __builtin_amdgcn_s_setprio(3 - EIGHTH % 4);
+#pragma unroll
+            for (int i = from; i < to; i++) step(i);
+        }
+        behind_first<N, EIGHTH + 1>(step);
     }
 }
 

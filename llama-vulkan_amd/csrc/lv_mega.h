@@ -404,11 +404,9 @@ __device__ __forceinline__ void gemv_phase(MegaTile (&q)[S::DEPTH], const MegaWa
 {
     constexpr int NT4 = round_up(NT, 4);
     float p[4];
-#pragma unroll
-    for (int i = 0; i < NT4; i++) {
+    auto step = [&](int i) {
         if (i < NT) {
             const int slot = (SEQ0 + i) % S::DEPTH;
-            behind_first(i, NT);
             const MegaTile t = q[slot];
             p[i & 3] = tile_dot<S>(t, xr, xsum);
             mw.fetch(q[slot], SEQ0 + i + S::DEPTH, layer);
@@ -421,7 +419,10 @@ __device__ __forceinline__ void gemv_phase(MegaTile (&q)[S::DEPTH], const MegaWa
             const int row = rset * NT + ii;
             if (active && (mw.lane & 15) == 0 && row < rows && ii < NT) red[row * NS + slab] = s;
         }
-    }
+    };
+    behind_first<NT>(step);
+#pragma unroll
+    for (int i = NT; i < NT4; i++) step(i);
 }
 
 // A D-wide GEMV phase (input vector of D floats, ROWS rows per workgroup): waves on a full slab take one row per tile, waves
@@ -432,11 +433,9 @@ __device__ __forceinline__ void gemv_phase_d(MegaTile (&q)[S::DEPTH], const Mega
 {
     constexpr int NT = S::tiles_d(ROWS), TH = S::tiles_half(ROWS), NT4 = round_up(NT, 4), NS = S::NSD;
     float p[4];
-#pragma unroll
-    for (int i = 0; i < NT4; i++) {
+    auto step = [&](int i) {
         if (i < NT) {
             const int slot = (SEQ0 + i) % S::DEPTH;
-            behind_first(i, NT);
             const MegaTile t = q[slot];
             p[i & 3] = tile_dot<S>(t, xr, xsum);
             mw.fetch(q[slot], SEQ0 + i + S::DEPTH, layer);
@@ -463,7 +462,10 @@ __device__ __forceinline__ void gemv_phase_d(MegaTile (&q)[S::DEPTH], const Mega
                 if (mw.actD && (ln & 15) == 0 && row < ROWS && ii < NT) red[row * NS + mw.sD] = s;
             }
         }
-    }
+    };
+    behind_first<NT>(step);
+#pragma unroll
+    for (int i = NT; i < NT4; i++) step(i);
 }
 
 template <int NS>
@@ -887,13 +889,11 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
         if constexpr (S::E_REDEAL) {
             // every wave TE tiles; the spare waves change their column slab every E_SPARE_ROWS tiles and fetch its activations anew
             float p[4];
-#pragma unroll
-            for (int i = 0; i < S::TE; i++) {
+            behind_first<S::TE>([&](int i) {
                 int row, slab;
                 mega_e_tile<S>(w, i, row, slab);
                 if (i > 0 && i % S::E_SPARE_ROWS == 0 && w >= S::NSF) load_slab(xr, xsum, xs, slab * 64 + lane, slab * 64 + lane < S::NBF);
                 const int slot = (S::SEQ_E + i) % S::DEPTH;
-                behind_first(i, S::TE);
                 const MegaTile t = q[slot];
                 p[i & 3] = tile_dot<S>(t, xr, xsum);
                 mw.fetch(q[slot], S::SEQ_E + i + S::DEPTH, layer);
@@ -903,7 +903,7 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
                     mega_e_tile<S>(w, i - 3, r0, sl);       // the four tiles are four consecutive rows of one slab
                     if ((lane & 15) == 0) red[(r0 + quad_partial_of_lane(lane)) * S::NSF + sl] = sum4;
                 }
-            }
+            });
         } else {
             gemv_phase<S, S::SEQ_E, S::TE, S::NSF>(q, mw, layer, xr, xsum, mw.sF, mw.rF, mw.actF, S::ROWS_E, red);
         }
@@ -926,10 +926,8 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
         const int rows = (int)mw.vocab_rows, per_set = cdiv(rows, S::WPF), per_half = S::HALFD ? cdiv(cdiv(rows, 2), S::WPH) : 0;
         // the head's slots are numbered from 0; tiles beyond per_set read the dummy tile
         float p[4];
-#pragma unroll
-        for (int i = 0; i < S::HEAD; i++) {
+        behind_first<S::HEAD>([&](int i) {
             const int slot = i % S::DEPTH;
-            behind_first(i, S::HEAD);
             const MegaTile t = q[slot];
             p[i & 3] = tile_dot<S>(t, xr, xsum);
             mw.fetch_head(q[slot], i + S::DEPTH);
@@ -950,7 +948,7 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
                     if (mw.actD && (lane & 15) == 0 && ii < per_set && row < rows) red[row * S::NSD + mw.sD] = s;
                 }
             }
-        }
+        });
         lds_barrier();
         // logits out; on the way the greedy pick (llava_session.cpp:144-152: index of the first strict maximum):
         // every workgroup hands its best (value, index) to workgroup 0 like any other hand-over
