@@ -198,12 +198,13 @@ struct lv_model {
 };
 
 // Shape classes the persistent kernel is compiled for: LLaMA-7B and LLaMA-13B layer shapes, q4_0 and q8_0.
-// Eight wavefronts per workgroup (two per SIMD leave each wave 256 registers, which buys a queue 8 q4_0 tiles or 4 q8_0 tiles
-// deep; twelve waves with the shallow queue the register file then allows lost 6-13 %).  The 13B classes ran on seven waves
+// Eight wavefronts per workgroup (two per SIMD leave each wave 256 registers, which buys a queue 8 to 10 q4_0 tiles or 4 q8_0 tiles
+// deep; twelve waves with the shallow queue the register file then allows lost 6-13 %).  Ten of 7B q4_0: its layer has 50 tiles a wave, so no slot
+// of the sequence is empty (us a token at position 511, 8, 9 and 10: 949 940 923; 13B q4_0, 83 tiles, 8 layers, at 287: 7 359, 8 351, 10 354).  The 13B classes ran on seven waves
 // while a wave was tied to one of three column slabs, the third half empty; with the half slab's tiles carrying two rows
 // and the waves dealt 3 + 3 + 2 (MegaShapeBase) all eight work in the D-wide phases: 13B q4_0 544 -> 592-607 tok/s, 13B q8_0
 // 357-370 -> 379-392.
-using Mega7Bq4 = MegaShape<4096, 11008, 32, 8, 4, 8>;
+using Mega7Bq4 = MegaShape<4096, 11008, 32, 8, 4, 10>;
 using Mega7Bq8 = MegaShape<4096, 11008, 32, 8, 8, 4>;
 using Mega13Bq4 = MegaShape<5120, 13824, 40, 8, 4, 8>;
 using Mega13Bq8 = MegaShape<5120, 13824, 40, 8, 8, 4>;
