@@ -49,6 +49,11 @@ constexpr int kStatusXcd = 3;           // word that tells whether workgroup 0 h
 // (1-2 us), and the second try pays that again.  Sleeping this many 64-clock units first makes the first try
 // succeed; measured optimum, flat between 16 and 32.
 constexpr int kPollDelay = 24;
+// Rows of context up to which a head's attention is one workgroup's work: it sends the head's output itself, and the hand-over of partial sums (1.2 us
+// a layer) falls away; the head's other workgroups go on to wait for the outputs.  us a token without and with, behind 20, 63, 94 and 127 rows: 7B
+// q4_0 891 848, 890 856, 891 874, 892 885; q8_0, 8 layers, 378 366, 378 367, 377 372, 377 375; 13B, 8 layers, q4_0 349 338, 350 341, 347 346,
+// 347 349; q8_0 543 531, 543 533, 544 536, 543 538.
+constexpr uint32_t kMegaAlone = 96;
 
 __device__ __forceinline__ uint32_t ld_dev(const uint32_t *p)
 {
@@ -652,6 +657,7 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
     float xr[32];
     float xsum;
 
+    const bool alone = pos < kMegaAlone;
     for (uint32_t layer = 0; layer < a.layers; layer++) {
         float *xc = a.xchg + (size_t)layer * S::XCHG_LAYER, *xlc = a.xl + (size_t)layer * S::LOCAL_LAYER;
         const float *norm_w = a.norms + (size_t)layer * 2 * D;
@@ -693,10 +699,10 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
         // ================= B: attention chunk (head h, chunk c) ================================================
         {
             const int h = place.h, c = place.c;
-            if (place.attends) {
+            if (place.attends && (c == 0 || !alone)) {
                 const uint32_t n_valid = pos + 1;
                 uint32_t chunk = (n_valid + S::CPH - 1) / S::CPH;
-                chunk = (chunk + 3) & ~3u;
+                chunk = alone ? n_valid : (chunk + 3) & ~3u;
                 const uint32_t p_begin = min((uint32_t)c * chunk, n_valid), p_end = min(p_begin + chunk, n_valid);
                 const int sub = lane & 15, rsel = w * 4 + (lane >> 4);
                 constexpr int RPR = NW * 4;   // cache rows per round of the workgroup
@@ -819,15 +825,21 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
                     float t = 0.f;
 #pragma unroll
                     for (int i = 0; i < NW; i++) t += l.attn_red[i * (R + 1) + st];
+                    if (alone) {
+                        float d = 0.f;
+#pragma unroll
+                        for (int i = 0; i < NW; i++) d += l.attn_red[i * (R + 1) + R];
+                        if (st < R) st_dev(xc + S::OFF_O + h * R + st, t / d);      // every workgroup of the device reads this one
+                    }
                     // read by chunk 0 of this head, on this XCD
-                    if (xcd_local) xlc[S::OFF_PART + (h * S::CPH + c) * S::PART + st] = t;
+                    else if (xcd_local) xlc[S::OFF_PART + (h * S::CPH + c) * S::PART + st] = t;
                     else st_dev(xlc + S::OFF_PART + (h * S::CPH + c) * S::PART + st, t);
                 }
             }
         }
 
         // ================= B': combine the chunks of head b (one wait for numerators and denominators) ==========
-        if (place.attends && place.c == 0 && st < R) {
+        if (place.attends && place.c == 0 && !alone && st < R) {
             float nd[2 * S::CPH];
             const uint32_t *hp = reinterpret_cast<const uint32_t *>(xlc + S::OFF_PART + (size_t)place.h * S::CPH * S::PART);
             uint32_t spins = 0;

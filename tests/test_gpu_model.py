@@ -277,6 +277,29 @@ def test_persistent_kernel_hands_over_alike_inside_an_xcd_and_at_device_scope(lv
     a.close(); b.close(); model.close()
 
 
+def test_attention_by_one_workgroup_a_head_and_by_several(lva, ctx, wide_model):
+    """up to 96 rows of context one workgroup does a head's attention, behind them several hand partial sums over: both sides of the line, and
+    the last row before it again, against the operator chain and between the two transports of the hand-overs"""
+    model = lva.Model(ctx, wide_model)
+    a, b, ops = (lva.Session(model, 128) for _ in range(3))
+    b.set_xcd_handover(False)
+    ops.set_path(lva.PATH_KERNELS)
+    toks = lva.synth_tokens(101, 3, 2048, seed=6)
+    for s in (a, b, ops):
+        s.begin(toks[:93], 0)
+        s.wait()
+    for i in (93, 94, 95, 96, 97, 98, 95, 96, 99):
+        got = []
+        for s in (a, b, ops):
+            s.begin([toks[i]], i)
+            got.append(s.logits())
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)), i
+        assert np.max(np.abs(got[0] - got[2])) <= 3e-4 * np.max(np.abs(got[2])), i   # two fp32 summation orders
+    for s in (a, b, ops):
+        s.close()
+    model.close()
+
+
 def test_persistent_kernel_refused_for_other_shapes(lva, ctx, tiny_models):
     model = lva.Model(ctx, tiny_models["tiny_q4"])
     s = lva.Session(model, 128)

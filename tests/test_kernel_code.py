@@ -45,6 +45,15 @@ def test_short_products_fit_their_registers(spills):
     assert {n: v for n, v in short.items() if v > 32} == {}
 
 
+def test_persistent_kernels_keep_their_queue_in_registers(code_objects):
+    """a loop over tiles that is too long to be unrolled indexes the queue at run time, in scratch memory: three times as long a token"""
+    scratch = {}
+    for f in code_objects:
+        notes = subprocess.run([tool("llvm-readelf"), "--notes", f], check=True, capture_output=True, text=True).stdout
+        scratch.update((n, int(v)) for n, v in re.findall(r"\.name:\s+(_Z\S+mega_decode_kernel\S+)\n(?:(?!\.name:\s+_Z).*\n)*?\s+\.private_segment_fixed_size:\s+(\d+)", notes))
+    assert len(scratch) == 6 and set(scratch.values()) == {0}, scratch
+
+
 def test_nothing_moves_between_matrix_products_in_inline_assembly(code_objects):
     """gemm_wide_kernel with 256-token tiles names its matrix instructions in inline assembly, where the compiler knows nothing of the
     states that have to lie between one of them and a move of its registers: it must have no move, no spill and no other matrix
