@@ -246,8 +246,8 @@ struct lv_session {
     uint32_t *cfg_host = nullptr;  // pinned staging of the same
     float *logits_host = nullptr;     // pinned, written by logits_out_kernel
     uint32_t *argmax_host = nullptr;  // behind them in the same allocation, written by argmax_kernel
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
+    hipGraph_t graph[2] = {};         // of a token; [1]: its logits go to logits_host as well (block models)
+    hipGraphExec_t graph_exec[2] = {};
     bool use_graph = true;
     int path = LV_PATH_AUTO;
     // workspace of the batched prompt path, allocated at first use: activations for pf_cap tokens
@@ -1577,10 +1577,12 @@ extern "C" int lv_model_arena_bytes(const lv_model *m, uint64_t *bytes)
 // -----------------------------------------------------------------------------------------------------------
 static void drop_graph(lv_session *s)
 {
-    if (s->graph_exec) (void)hipGraphExecDestroy(s->graph_exec);
-    if (s->graph) (void)hipGraphDestroy(s->graph);
-    s->graph_exec = nullptr;
-    s->graph = nullptr;
+    for (int i = 0; i < 2; i++) {
+        if (s->graph_exec[i]) (void)hipGraphExecDestroy(s->graph_exec[i]);
+        if (s->graph[i]) (void)hipGraphDestroy(s->graph[i]);
+        s->graph_exec[i] = nullptr;
+        s->graph[i] = nullptr;
+    }
 }
 
 extern "C" int lv_session_destroy(lv_session *s)
@@ -2042,11 +2044,12 @@ static int embed_token(lv_session *s, uint32_t pos, uint32_t idx, uint32_t token
 
 // The embedded token through every layer (llava_layer.cpp:53-73 + llava_command_buffer.cpp:38-39).  Its cache row is
 // cfg[0] + idx.  With_head = also compute the logits.
-static int record_token(lv_session *s, uint32_t idx, bool with_head)
+// send: a block model's logits go to logits_host as well
+static int record_token(lv_session *s, uint32_t idx, bool with_head, bool send = false)
 {
     if (s->block) {
         const BlockTrace t = block_trace(s);
-        return block_step_token(s->block, s->cfg, idx, with_head ? s->logits : nullptr, s->trace ? &t : nullptr);
+        return block_step_token(s->block, s->cfg, idx, with_head ? s->logits : nullptr, send ? s->logits_host : nullptr, s->trace ? &t : nullptr);
     }
     const lv_model *m = s->model;
     const lv_hparams &hp = m->hp;
@@ -2240,12 +2243,12 @@ static int launch_prefill_norm(hipStream_t st, lv_session *s, const float *w, ui
 // Rows idx0 .. idx0+n-1 of the step at once (llava_layer.cpp:39-75 with batch > 1).  Row z sees cache rows
 // 0..pos+z: all K/V rows of the chunk are appended before any row attends, rows above its own are masked.
 static int record_mid_layers(lv_session *s, uint32_t idx0, uint32_t n, float *const parts[kGemmMaxMats], uint32_t *pending_out);
-// mid: the products of lv_mid.h, n at most kMidTokens
-static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_head, uint32_t row_base, bool mid)
+// mid: the products of lv_mid.h, n at most kMidTokens; send: as in record_token
+static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_head, uint32_t row_base, bool mid, bool send)
 {
     if (s->block) {
         const BlockTrace t = block_trace(s);
-        return block_step_batch(s->block, s->cfg, s->cfg_host[0] + idx0, idx0, n, with_head ? s->logits : nullptr,
+        return block_step_batch(s->block, s->cfg, s->cfg_host[0] + idx0, idx0, n, with_head ? s->logits : nullptr, send ? s->logits_host : nullptr,
                                 s->all_logits ? s->logits_all + (size_t)(row_base + idx0) * s->model->hp.vocab : nullptr, s->trace ? &t : nullptr);
     }
     const lv_model *m = s->model;
@@ -2959,7 +2962,8 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
     s->have_logits = false;
     s->pick_in_status = false;
     s->logits_on_host = false;
-    // Whoever has read the last step's logits reads this one's: the persistent kernel then sends them to the host itself
+    // Whoever has read the last step's logits reads this one's: the persistent kernel and a block model's output product then send them to the
+    // host themselves
     const bool send_logits = s->logits_were_read && !s->all_logits;
     s->logits_were_read = false;
     s->logits_rows = 0;
@@ -2978,6 +2982,7 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
             s->logits_cap = n;
         }
     }
+    const bool block_sends = send_logits && s->block;      // the output product of a block model sends them
     const uint32_t n_rows = n, V = s->model->hp.vocab;
     uint32_t row_base = 0;          // rows of this step already launched on the persistent kernel when the rest takes another path
     if (s->trace) {
@@ -3060,9 +3065,9 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
         }
         s->logits_on_host = true;
     } else if (n == 1 && (path == LV_PATH_GRAPH || (path == LV_PATH_PERSISTENT && s->use_graph)) && !s->trace) {
-        if (!s->graph_exec) {
+        if (!s->graph_exec[block_sends]) {
             HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-            int rc = record_token(s, 0, true);
+            int rc = record_token(s, 0, true, block_sends);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(s->stream, &g);
             if (rc != LV_OK) {
@@ -3070,26 +3075,29 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
                 return rc;
             }
             HIP_TRY(e);
-            s->graph = g;
-            HIP_TRY(hipGraphInstantiate(&s->graph_exec, s->graph, nullptr, nullptr, 0));
+            s->graph[block_sends] = g;
+            HIP_TRY(hipGraphInstantiate(&s->graph_exec[block_sends], g, nullptr, nullptr, 0));
         }
         LV_TRY(embed_token(s, pos, 0, tokens[0]));
-        HIP_TRY(hipGraphLaunch(s->graph_exec, s->stream));
+        HIP_TRY(hipGraphLaunch(s->graph_exec[block_sends], s->stream));
+        s->logits_on_host = block_sends;
         if (s->all_logits) HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)row_base * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
     } else if (batch) {
         for (uint32_t i = 0; i < n; i += batch_max) {
             const uint32_t m = n - i < batch_max ? n - i : batch_max;
-            LV_TRY(record_prefill(s, i, m, i + m == n, row_base, mid && m == rest));
+            LV_TRY(record_prefill(s, i, m, i + m == n, row_base, mid && m == rest, block_sends && i + m == n));
         }
+        s->logits_on_host = block_sends;
     } else {
         // rows are evaluated one after the other: row z sees cache rows 0..pos+z, which is what the batched
         // shaders compute (every row's K/V is appended before any row attends, and rows above are masked)
         for (uint32_t i = 0; i < n; i++) {
             LV_TRY(embed_token(s, pos, i, tokens[i]));
-            LV_TRY(record_token(s, i, s->all_logits || i + 1 == n));
+            LV_TRY(record_token(s, i, s->all_logits || i + 1 == n, block_sends && i + 1 == n));
             if (s->all_logits)
                 HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)(row_base + i) * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
         }
+        s->logits_on_host = block_sends;
     }
     if (s->block) block_session_advance(s->block, pos + n);
     s->in_flight = true;

@@ -71,7 +71,7 @@ struct GroupInput {
 struct BfGemvArgs {
     const uint16_t *w;
     uint32_t rows, kp;
-    float *out;
+    float *out, *host;           // host: null or pinned memory that gets a kGemvRows product as well, as its rows are done
     NormInput norm;
     const float *x;              // kInPlain
     BranchInput branch;
@@ -580,6 +580,7 @@ __global__ __launch_bounds__(gemv_threads(INPUT)) void bf16_gemv_kernel(BfGemvAr
                         a.out[u] = glu_f(a.act, v0) * v1;
                     } else {
                         a.out[u] = v0;
+                        if (MODE == kGemvRows && a.host) a.host[u] = v0;
                     }
                 }
             }

@@ -35,11 +35,11 @@ struct BlockTrace {
 // A token into the residual, at pos + idx; leaves pos in cfg[0].
 int block_embed_token(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx, uint32_t token);
 // The embedded token at position cfg[0] + idx through the layers, as launches on the session's stream (capturable).  logits: null or
-// vocab floats.
-int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *logits, const BlockTrace *trace);
+// vocab floats; logits_host: null or pinned memory that gets them too.
+int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *logits, float *logits_host, const BlockTrace *trace);
 // Tokens cfg[1 + idx0] .. of the step at position pos on, n of them together.  logits_all: null or [n][vocab]; logits_last: null or
-// vocab floats.
-int block_step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_all,
+// vocab floats, without logits_all in logits_host (null or pinned memory) too.
+int block_step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_host, float *logits_all,
                      const BlockTrace *trace);
 // to be called when a step's launches are on the stream: the state stands at pos from now on
 void block_session_advance(BlockSession *s, uint32_t pos);

@@ -1183,7 +1183,7 @@ static int token_ssm(BlockSession *s, size_t i, const uint32_t *cfg, uint32_t id
     return gemv<kGemvRows, kInGroups>(s->st, o);
 }
 
-int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *logits, const BlockTrace *trace)
+int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *logits, float *logits_host, const BlockTrace *trace)
 {
     const BlockModel *m = s->m;
     hipStream_t st = s->st;
@@ -1251,7 +1251,7 @@ int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *
     }
     if (logits) {
         BfGemvArgs h{};
-        h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits; h.same_order = 1;
+        h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits; h.host = logits_host; h.same_order = 1;
         res.feed(h, m->final, nullptr, false);
         LV_TRY(gemv_residual<kGemvRows>(m, st, h));
     }
@@ -1568,7 +1568,7 @@ template <class T> static int batch_ssm(BlockSession *s, size_t i, uint32_t pos,
 }
 
 template <class T>
-static int step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_all, const BlockTrace *trace)
+static int step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_host, float *logits_all, const BlockTrace *trace)
 {
     constexpr bool f32 = sizeof(T) == 4;
     const BlockModel *m = s->m;
@@ -1678,7 +1678,7 @@ static int step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx
     } else if (logits_last) {
         BfGemvArgs h{};
         h.same_order = 1;
-        h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits_last;
+        h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits_last; h.host = logits_host;
         const float *x = w.x + (size_t)(n - 1) * m->copies * Dp;
         if (m->hp.streams) {
             if (parts > 1) {       // the launch's head takes one vector: the last token's streams take it in beforehand
@@ -1709,10 +1709,10 @@ static int step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx
     return LV_OK;
 }
 
-int block_step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_all, const BlockTrace *trace)
+int block_step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_host, float *logits_all, const BlockTrace *trace)
 {
-    return s->m->f32 ? step_batch<float>(s, cfg, pos, idx0, n, logits_last, logits_all, trace)
-                     : step_batch<uint16_t>(s, cfg, pos, idx0, n, logits_last, logits_all, trace);
+    return s->m->f32 ? step_batch<float>(s, cfg, pos, idx0, n, logits_last, logits_host, logits_all, trace)
+                     : step_batch<uint16_t>(s, cfg, pos, idx0, n, logits_last, logits_host, logits_all, trace);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------

@@ -71,3 +71,26 @@ def test_grouped_input(lva, ctx, heads, vdim, groups):
     want = zo.forward(toks, bb.as_float(W), cfg)[0]
     with block_device.Device(lva, zb.upload(ctx, cfg, W, lva.LV_F32), 512) as d:
         assert rel(d.run(toks, (1,)), want) < 2e-4
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_logits_of_steps_read_or_not(lva, ctx, f32):
+    """a step behind one whose logits were read sends its own to the host from the output product: the same bits whatever was read before,
+    for one token, several one by one and a batch, and as the greedy pick; 1003 rows of output"""
+    cfg = bb.config(width=320, vocab=1003, layers=[bb.layer(experts=5, top=2, ff=72)])
+    model = bb.upload(ctx, cfg, bb.weights(cfg, seed=5), lva.LV_F32 if f32 else lva.LV_BF16)
+    a, b = lva.Session(model, 128), lva.Session(model, 128)
+    toks = tokens_for(cfg, 80, 2)
+    pos = 0
+    for i, n in enumerate((1, 1, 1, 3, 1, 20, 1, 17, 2, 1, 18, 1, 1)):
+        a.begin(toks[pos:pos + n], pos)
+        want = a.logits()                                # every step
+        b.begin(toks[pos:pos + n], pos)
+        if i % 3 == 0:
+            b.wait()
+        else:
+            assert np.array_equal(b.logits().view(np.uint32), want.view(np.uint32)), i
+            assert np.array_equal(b.logits().view(np.uint32), want.view(np.uint32)), i
+        assert b.argmax() == int(want.argmax()) == a.argmax(), i
+        pos += n
+    a.close(); b.close(); model.close()
