@@ -246,8 +246,8 @@ struct lv_session {
     uint32_t *cfg_host = nullptr;  // pinned staging of the same
     float *logits_host = nullptr;     // pinned, written by logits_out_kernel
     uint32_t *argmax_host = nullptr;  // behind them in the same allocation, written by argmax_kernel
-    hipGraph_t graph[2] = {};         // of a token; [1]: its logits go to logits_host as well (block models)
-    hipGraphExec_t graph_exec[2] = {};
+    hipGraph_t graph = nullptr;       // of a token; a block model's without its output product, whose destinations change from step to step
+    hipGraphExec_t graph_exec = nullptr;
     bool use_graph = true;
     int path = LV_PATH_AUTO;
     // workspace of the batched prompt path, allocated at first use: activations for pf_cap tokens
@@ -1577,12 +1577,10 @@ extern "C" int lv_model_arena_bytes(const lv_model *m, uint64_t *bytes)
 // -----------------------------------------------------------------------------------------------------------
 static void drop_graph(lv_session *s)
 {
-    for (int i = 0; i < 2; i++) {
-        if (s->graph_exec[i]) (void)hipGraphExecDestroy(s->graph_exec[i]);
-        if (s->graph[i]) (void)hipGraphDestroy(s->graph[i]);
-        s->graph_exec[i] = nullptr;
-        s->graph[i] = nullptr;
-    }
+    if (s->graph_exec) (void)hipGraphExecDestroy(s->graph_exec);
+    if (s->graph) (void)hipGraphDestroy(s->graph);
+    s->graph_exec = nullptr;
+    s->graph = nullptr;
 }
 
 extern "C" int lv_session_destroy(lv_session *s)
@@ -2043,13 +2041,12 @@ static int embed_token(lv_session *s, uint32_t pos, uint32_t idx, uint32_t token
 }
 
 // The embedded token through every layer (llava_layer.cpp:53-73 + llava_command_buffer.cpp:38-39).  Its cache row is
-// cfg[0] + idx.  With_head = also compute the logits.
-// send: a block model's logits go to logits_host as well
-static int record_token(lv_session *s, uint32_t idx, bool with_head, bool send = false)
+// cfg[0] + idx.  With_head = also compute the logits (a block model's: block_head_token).
+static int record_token(lv_session *s, uint32_t idx, bool with_head)
 {
     if (s->block) {
         const BlockTrace t = block_trace(s);
-        return block_step_token(s->block, s->cfg, idx, with_head ? s->logits : nullptr, send ? s->logits_host : nullptr, s->trace ? &t : nullptr);
+        return block_step_token(s->block, s->cfg, idx, s->trace ? &t : nullptr);
     }
     const lv_model *m = s->model;
     const lv_hparams &hp = m->hp;
@@ -2243,7 +2240,7 @@ static int launch_prefill_norm(hipStream_t st, lv_session *s, const float *w, ui
 // Rows idx0 .. idx0+n-1 of the step at once (llava_layer.cpp:39-75 with batch > 1).  Row z sees cache rows
 // 0..pos+z: all K/V rows of the chunk are appended before any row attends, rows above its own are masked.
 static int record_mid_layers(lv_session *s, uint32_t idx0, uint32_t n, float *const parts[kGemmMaxMats], uint32_t *pending_out);
-// mid: the products of lv_mid.h, n at most kMidTokens; send: as in record_token
+// mid: the products of lv_mid.h, n at most kMidTokens; send: a block model's logits go to logits_host as well
 static int record_prefill(lv_session *s, uint32_t idx0, uint32_t n, bool with_head, uint32_t row_base, bool mid, bool send)
 {
     if (s->block) {
@@ -3065,9 +3062,9 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
         }
         s->logits_on_host = true;
     } else if (n == 1 && (path == LV_PATH_GRAPH || (path == LV_PATH_PERSISTENT && s->use_graph)) && !s->trace) {
-        if (!s->graph_exec[block_sends]) {
+        if (!s->graph_exec) {
             HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-            int rc = record_token(s, 0, true, block_sends);
+            int rc = record_token(s, 0, true);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(s->stream, &g);
             if (rc != LV_OK) {
@@ -3075,11 +3072,12 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
                 return rc;
             }
             HIP_TRY(e);
-            s->graph[block_sends] = g;
-            HIP_TRY(hipGraphInstantiate(&s->graph_exec[block_sends], g, nullptr, nullptr, 0));
+            s->graph = g;
+            HIP_TRY(hipGraphInstantiate(&s->graph_exec, s->graph, nullptr, nullptr, 0));
         }
         LV_TRY(embed_token(s, pos, 0, tokens[0]));
-        HIP_TRY(hipGraphLaunch(s->graph_exec[block_sends], s->stream));
+        HIP_TRY(hipGraphLaunch(s->graph_exec, s->stream));
+        if (s->block) LV_TRY(block_head_token(s->block, s->logits, block_sends ? s->logits_host : nullptr));
         s->logits_on_host = block_sends;
         if (s->all_logits) HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)row_base * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
     } else if (batch) {
@@ -3093,7 +3091,8 @@ extern "C" int lv_step_begin(lv_session *s, const uint32_t *tokens, uint32_t n, 
         // shaders compute (every row's K/V is appended before any row attends, and rows above are masked)
         for (uint32_t i = 0; i < n; i++) {
             LV_TRY(embed_token(s, pos, i, tokens[i]));
-            LV_TRY(record_token(s, i, s->all_logits || i + 1 == n, block_sends && i + 1 == n));
+            LV_TRY(record_token(s, i, s->all_logits || i + 1 == n));
+            if (s->block && (s->all_logits || i + 1 == n)) LV_TRY(block_head_token(s->block, s->logits, block_sends ? s->logits_host : nullptr));
             if (s->all_logits)
                 HIP_TRY(hipMemcpyAsync(s->logits_all + (size_t)(row_base + i) * V, s->logits, (size_t)V * 4, hipMemcpyDeviceToDevice, s->stream));
         }

@@ -34,9 +34,13 @@ struct BlockTrace {
 
 // A token into the residual, at pos + idx; leaves pos in cfg[0].
 int block_embed_token(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx, uint32_t token);
-// The embedded token at position cfg[0] + idx through the layers, as launches on the session's stream (capturable).  logits: null or
-// vocab floats; logits_host: null or pinned memory that gets them too.
-int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *logits, float *logits_host, const BlockTrace *trace);
+// The embedded token at position cfg[0] + idx through the layers, as launches on the session's stream (capturable).
+int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, const BlockTrace *trace);
+// The logits of the token that these launches have carried, as one launch behind them: vocab floats; logits_host: null or pinned memory that
+// gets them too.  It is no part of a captured graph, since that memory changes from step to step: a graph for each of its two cost a session that
+// reads some steps' logits and not others' 105 us at the second one and 5 us at every change.  Launched behind the graph it ends sooner too: us of
+// a step of one layer whose logits are read, inside and behind, 32000 x 2048 89 86, x 4096 134 130, 128256 x 2048 160 153, x 256 89 86.
+int block_head_token(BlockSession *s, float *logits, float *logits_host);
 // Tokens cfg[1 + idx0] .. of the step at position pos on, n of them together.  logits_all: null or [n][vocab]; logits_last: null or
 // vocab floats, without logits_all in logits_host (null or pinned memory) too.
 int block_step_batch(BlockSession *s, uint32_t *cfg, uint32_t pos, uint32_t idx0, uint32_t n, float *logits_last, float *logits_host, float *logits_all,

@@ -117,6 +117,7 @@ struct BlockSession {
     void *ql = nullptr;                // latent attention: queries (latent_put)
     float2 *turn = nullptr;            // the model's frequencies as (cos, sin) at the token's position
     uint32_t *ids = nullptr, *counters = nullptr, *last = nullptr;      // last: the sequence's last token, at [position % 2]
+    BfGemvArgs head{};                 // the output product behind block_step_token's launches, but for where its logits go
     Workspace ws;
 };
 
@@ -1183,7 +1184,7 @@ static int token_ssm(BlockSession *s, size_t i, const uint32_t *cfg, uint32_t id
     return gemv<kGemvRows, kInGroups>(s->st, o);
 }
 
-int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *logits, float *logits_host, const BlockTrace *trace)
+int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, const BlockTrace *trace)
 {
     const BlockModel *m = s->m;
     hipStream_t st = s->st;
@@ -1249,13 +1250,18 @@ int block_step_token(BlockSession *s, const uint32_t *cfg, uint32_t idx, float *
         }
         LV_TRY(keep_end((uint32_t)m->order.size() - 1));
     }
-    if (logits) {
-        BfGemvArgs h{};
-        h.w = m->head.w; h.rows = m->hp.vocab; h.kp = Dp; h.out = logits; h.host = logits_host; h.same_order = 1;
-        res.feed(h, m->final, nullptr, false);
-        LV_TRY(gemv_residual<kGemvRows>(m, st, h));
-    }
+    s->head = BfGemvArgs{};
+    s->head.w = m->head.w; s->head.rows = m->hp.vocab; s->head.kp = Dp; s->head.same_order = 1;
+    res.feed(s->head, m->final, nullptr, false);
     return LV_OK;
+}
+
+int block_head_token(BlockSession *s, float *logits, float *logits_host)
+{
+    BfGemvArgs h = s->head;
+    h.out = logits;
+    h.host = logits_host;
+    return gemv_residual<kGemvRows>(s->m, s->st, h);
 }
 
 // router logits of a batch: K in at most so many slices, each a multiple of so many columns

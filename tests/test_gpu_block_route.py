@@ -5,6 +5,8 @@ Small integers as embeddings, norm weights of one and router rows that come in e
 pair.  The plain evaluation chooses by the same rule (choose_experts); a wrong pick is an error of order one.
 
 And the inputs of one-token products, on both sides of the sizes up to which they are held in registers."""
+import time
+
 import numpy as np
 import pytest
 
@@ -94,3 +96,32 @@ def test_logits_of_steps_read_or_not(lva, ctx, f32):
         assert b.argmax() == int(want.argmax()) == a.argmax(), i
         pos += n
     a.close(); b.close(); model.close()
+
+
+def test_reading_some_steps_makes_no_second_graph(lva, ctx):
+    """us of the steps at which a session starts and stops to read logits, beside those of a session that always reads: the fastest of nine
+    sessions.  A token's graph is made at the first of them; a second one took as long as two of these steps"""
+    cfg = bb.config(width=320, vocab=1003, layers=[bb.layer(experts=5, top=2, ff=72) for _ in range(3)])
+    model = bb.upload(ctx, cfg, bb.weights(cfg, seed=6), lva.LV_BF16)
+    toks = tokens_for(cfg, 24, 1)
+
+    def steps(read):
+        s = lva.Session(model, 128)
+        s.begin(toks[:4], 0)
+        s.logits()
+        out = []
+        for i in range(4, len(toks)):
+            t = time.perf_counter()
+            s.begin(toks[i:i + 1], i)
+            s.logits() if read(i) else s.argmax()
+            out.append(time.perf_counter() - t)
+        s.close()
+        return out[1:]                                   # behind the one that makes the graph
+
+    def fastest(read):
+        return np.min([steps(read) for _ in range(9)], axis=0)
+
+    always = np.median(fastest(lambda i: True))
+    for read in (lambda i: i % 2 == 0, lambda i: i >= 12, lambda i: i < 12, lambda i: False):
+        assert fastest(read).max() < 1.5 * always, (fastest(read) * 1e6, always * 1e6)
+    model.close()
