@@ -75,19 +75,30 @@ def test_grouped_input(lva, ctx, heads, vdim, groups):
         assert rel(d.run(toks, (1,)), want) < 2e-4
 
 
-@pytest.mark.parametrize("f32", [False, True])
-def test_logits_of_steps_read_or_not(lva, ctx, f32):
+# an output row a wave, two together (from 8192 rows on; an odd number leaves half a task), and residuals of up to 2, 4 and 8 streams
+@pytest.mark.parametrize("streams,width,vocab,f32", [(0, 320, 1003, False), (0, 320, 1003, True), (0, 96, 32001, False), (2, 72, 1003, False),
+                                                     (3, 44, 32001, False), (5, 44, 1003, False), (5, 44, 32001, False)])
+def test_logits_of_steps_read_or_not(lva, ctx, streams, width, vocab, f32):
     """a step behind one whose logits were read sends its own to the host from the output product: the same bits whatever was read before,
-    for one token, several one by one and a batch, and as the greedy pick; 1003 rows of output"""
-    cfg = bb.config(width=320, vocab=1003, layers=[bb.layer(experts=5, top=2, ff=72)])
-    model = bb.upload(ctx, cfg, bb.weights(cfg, seed=5), lva.LV_F32 if f32 else lva.LV_BF16)
+    for one token, several one by one and a batch, with and without all rows' logits kept, and as the greedy pick"""
+    compute = lva.LV_F32 if f32 else lva.LV_BF16
+    if streams:
+        cfg = zb.config(width=width, vocab=vocab, streams=streams)
+        model = zb.upload(ctx, cfg, zb.weights(cfg, seed=5), compute)
+    else:
+        cfg = bb.config(width=width, vocab=vocab, layers=[bb.layer(experts=5, top=2, ff=72)])
+        model = bb.upload(ctx, cfg, bb.weights(cfg, seed=5), compute)
     a, b = lva.Session(model, 128), lva.Session(model, 128)
     toks = tokens_for(cfg, 80, 2)
     pos = 0
     for i, n in enumerate((1, 1, 1, 3, 1, 20, 1, 17, 2, 1, 18, 1, 1)):
         a.begin(toks[pos:pos + n], pos)
         want = a.logits()                                # every step
+        kept = i in (4, 6, 11)                           # behind a step that was read and behind one that was not
+        b.keep_all_logits(kept)
         b.begin(toks[pos:pos + n], pos)
+        if kept:
+            assert n == 1 and np.array_equal(b.logits_rows(0, 1)[0].view(np.uint32), want.view(np.uint32)), i
         if i % 3 == 0:
             b.wait()
         else:
