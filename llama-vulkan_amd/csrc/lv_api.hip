@@ -208,7 +208,8 @@ using Mega7Bq4 = MegaShape<4096, 11008, 32, 8, 4, 10>;
 using Mega7Bq8 = MegaShape<4096, 11008, 32, 8, 8, 4>;
 using Mega13Bq4 = MegaShape<5120, 13824, 40, 8, 4, 8>;
 using Mega13Bq8 = MegaShape<5120, 13824, 40, 8, 8, 4>;
-// the same for version-1 files (fp32 block scales; the reference loads q4_0 of that version only, llava_buffer.cpp:66-71)
+// the same for version-1 files (fp32 block scales; the reference loads q4_0 of that version only, llava_buffer.cpp:66-71); no other depth than 8
+// was measured for them
 using Mega7Bq4v1 = MegaShapeV1<4096, 11008, 32, 8, 4, 8>;
 using Mega13Bq4v1 = MegaShapeV1<5120, 13824, 40, 8, 4, 8>;
 constexpr int kMegaKinds = 6;
@@ -244,7 +245,7 @@ struct lv_session {
     uint32_t *attn_counters = nullptr;
     uint32_t *cfg = nullptr;       // device: [0] = pos, [1..] = token ids of the step
     uint32_t *cfg_host = nullptr;  // pinned staging of the same
-    float *logits_host = nullptr;     // pinned, written by logits_out_kernel
+    float *logits_host = nullptr;     // pinned: the logits that lv_logits_read hands out, written by logits_out_kernel or by the step itself (logits_on_host)
     uint32_t *argmax_host = nullptr;  // behind them in the same allocation, written by argmax_kernel
     hipGraph_t graph = nullptr;       // of a token; a block model's without its output product, whose destinations change from step to step
     hipGraphExec_t graph_exec = nullptr;
@@ -269,7 +270,7 @@ struct lv_session {
     uint32_t wait_limit = 0;              // polls per hand-over of the persistent kernel; 0 = default
     bool xcd_handover = true;             // the persistent kernel may keep a head's hand-overs inside its XCD (lv_session_set_xcd_handover)
     bool logits_on_host = false;          // the last step left its logits in logits_host as well
-    bool logits_were_read = false;        // lv_logits_read has read the last step's logits: the persistent kernel sends the next step's along
+    bool logits_were_read = false;        // lv_logits_read has read the last step's logits: the persistent kernel and block models send the next step's along
     bool pick_in_status = false;          // the last step ran the persistent kernel, whose greedy pick is in status_host
     bool mega_step = false;               // the step in flight ran the persistent kernel, or that of a small model
     uint32_t small_n = 0;                 // tokens of the step in flight where it ran the latter; they are in cfg_host

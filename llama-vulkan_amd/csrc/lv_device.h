@@ -252,9 +252,10 @@ __device__ __forceinline__ float q8_block_dot(const uint4 &qa, const uint4 &qb, 
 // step(0) .. step(N - 1), unrolled, with the wave's place in the queue of its SIMD by how far it is.  Between two waves that could issue the
 // older one goes first, so one of a SIMD's two runs through its steps, then waits at the barrier with all it has asked for in registers, while the
 // other walks the rest with nobody to fill its gaps.  With a priority that falls by a level every eighth of the steps (four levels, twice over) the
-// one that is behind goes first, and both end together.  us a token of the persistent kernel without it and with: 7B q4_0 at position 511 969 949,
-// q8_0, 8 layers, at 2039 429 426; 13B, 8 layers, q4_0 at 287 371 351, q8_0 at 511 560 550.  q4_0 of 7B and 13B in other steps: falling once over
-// all 953 351, with every step 948 353, every other one 947 351, one level in the middle 954 355.
+// one that is behind goes first, and both end together.  Fewer than eight steps leave levels out (four: 3 1 3 1; seven: 3 2 1 0 3 2 1), and the two
+// waves stay at the last one until their next steps; eight and more end at 0.  us a token of the persistent kernel without it and with: 7B q4_0 at
+// position 511 969 949, q8_0, 8 layers, at 2039 429 426; 13B, 8 layers, q4_0 at 287 371 351, q8_0 at 511 560 550.  q4_0 of 7B and 13B in other
+// steps: falling once over all 953 351, with every step 948 353, every other one 947 351, one level in the middle 954 355.
 template <int N, int EIGHTH = 0, class Step>
 __device__ __forceinline__ void behind_first(Step &&step)
 {

@@ -613,8 +613,9 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
 // A step's logits into pinned memory.  The runtime's copy to ordinary memory goes through its own staging buffer, one piece of work
 // for its copy engine or blit kernel and a wait of its own: behind a kernel of 80 us 93.5 us until 128 KB are there, this kernel, the
 // stream's wait and a memcpy 85; behind one of 5 us 73 against 19.
-// The persistent kernel, small models' launches and a block model's output product write them there themselves (the last: turns of 32 tokens 7960 ->
-// 7880 us at width 2048, 7400 -> 7280 at 4096), so this is left to prompts of LLaMA files and to the first step whose logits are read.
+// Where the last step's logits were read, the persistent kernel and a block model's output product write them there themselves, and small models'
+// launches always do.  So this is left to LLaMA files' prompts, short steps and tokens of the operator chain, to steps behind one that was not read,
+// and to steps that keep all rows' logits.
 __global__ __launch_bounds__(256) void logits_out_kernel(float *__restrict__ host, const float *__restrict__ logits, uint32_t n)
 {
     const uint32_t i = (blockIdx.x * 256 + threadIdx.x) * 4;

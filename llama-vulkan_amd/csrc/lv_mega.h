@@ -3,13 +3,14 @@
 // Why: at batch 1 a layer is five tiny dependent GEMVs (1-6 us of HBM time each).  Launched one by one
 // they spend more time draining, launching and refilling the memory pipeline than streaming weights.
 // Here one workgroup per CU stays resident for the whole token; every wavefront walks its own contiguous
-// weight stream with a register queue (8 q4_0 tiles or 4 q8_0 tiles deep) of 128-bit loads that keeps running across the phase
+// weight stream with a register queue (8 or 10 q4_0 tiles or 4 q8_0 tiles deep) of 128-bit loads that keeps running across the phase
 // boundaries, so HBM stays busy while the workgroups exchange the small activation vectors.
 //
 // Phases of a layer (llava_layer.cpp:53-73), each separated by a data hand-over through HBM/L2:
 //   A  norm + [Wq;Wk;Wv] x        -> q, new K/V row (fp16 into the cache)
-//   B  single-query attention, 8 (or 6) position chunks per head -> partial numerators / denominators
-//   B' combine the chunks         -> o
+//   B  single-query attention: up to kMegaAlone rows of context one workgroup a head -> o;
+//      behind them 8 (or 6) position chunks per head -> partial numerators / denominators,
+//   B' and one workgroup a head combines them         -> o
 //   C  x += Wo o                  -> x1
 //   D  norm + (W3 x1)*silu(W1 x1) -> ff
 //   E  x1 += W2 ff                -> x2 (next layer's x)
@@ -50,9 +51,10 @@ constexpr int kStatusXcd = 3;           // word that tells whether workgroup 0 h
 // succeed; measured optimum, flat between 16 and 32.
 constexpr int kPollDelay = 24;
 // Rows of context up to which a head's attention is one workgroup's work: it sends the head's output itself, and the hand-over of partial sums (1.2 us
-// a layer) falls away; the head's other workgroups go on to wait for the outputs.  us a token without and with, behind 20, 63, 94 and 127 rows: 7B
-// q4_0 891 848, 890 856, 891 874, 892 885; q8_0, 8 layers, 378 366, 378 367, 377 372, 377 375; 13B, 8 layers, q4_0 349 338, 350 341, 347 346,
-// 347 349; q8_0 543 531, 543 533, 544 536, 543 538.
+// a layer) falls away; the head's other workgroups go on to wait for the outputs.  One line for all classes, up to which each of them gains: behind
+// 127 rows 13B q4_0 loses, the others still gain a little.  us a token without and with, behind 20, 63, 94 and 127 rows: 7B q4_0 891 848, 890 856,
+// 891 874, 892 885; q8_0, 8 layers, 378 366, 378 367, 377 372, 377 375; 13B, 8 layers, q4_0 349 338, 350 341, 347 346, 347 349; q8_0 543 531,
+// 543 533, 544 536, 543 538.
 constexpr uint32_t kMegaAlone = 96;
 
 __device__ __forceinline__ uint32_t ld_dev(const uint32_t *p)
@@ -696,7 +698,7 @@ __global__ __launch_bounds__(S::NW * 64, 1) void mega_decode_kernel(MegaArgs a)
             else st_dev(xlc + S::OFF_QKV + which * D + col, out);
         }
 
-        // ================= B: attention chunk (head h, chunk c) ================================================
+        // ================= B: attention (head h, chunk c; alone: all rows in chunk 0) ============================
         {
             const int h = place.h, c = place.c;
             if (place.attends && (c == 0 || !alone)) {
